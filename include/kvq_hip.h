@@ -296,6 +296,24 @@ int kvq_prefill_attn(const void* query, const void* key, const void* value, int 
                      int64_t batch, int64_t max_q_len, int num_heads, int num_kv_heads,
                      int head_size, float scale, int causal, void* out, void* stream);
 
+/* Host-side (no GPU call): the plan of kvq_prefill_attn_planned for a batch of
+ * q_lens / kv_lens (int64 [batch]), int32 [2 (batch + 1) + 2 units] in `plan`:
+ * cu_seqlens_q, cu_seqlens_k, then (request, tile) of every 128-row tile (a row
+ * is one query of one head of a GQA group) in the order they should start.
+ * Returns the number of tiles (units), KVQ_ERR_CAPACITY when they exceed
+ * cap_units, or KVQ_ERR_INVALID. */
+int64_t kvq_plan_prefill_attn(const int64_t* q_lens, const int64_t* kv_lens, int64_t batch,
+                              int num_heads, int num_kv_heads, int head_size, int causal,
+                              int32_t* plan, int64_t cap_units);
+
+/* kvq_prefill_attn over a plan of kvq_plan_prefill_attn copied to the device:
+ * only tiles with rows are launched, the longest first.  bf16 / fp16 and head
+ * sizes 64, 128 and 256; KVQ_ERR_GEOMETRY otherwise. */
+int kvq_prefill_attn_planned(const void* query, const void* key, const void* value, int dtype,
+                             const int32_t* plan, int64_t batch, int64_t num_units,
+                             int num_heads, int num_kv_heads, int head_size, float scale,
+                             int causal, void* out, void* stream);
+
 /* ---- INT8 dynamic per-channel ------------------------------------------- */
 
 /* First-K/V scales in the activation dtype: amax over tokens per (head, dim),

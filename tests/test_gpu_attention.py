@@ -88,3 +88,39 @@ def test_prefill_attention_growing_and_shrinking_row_maxima(gpu_device, d, dtype
         q.to(gpu_device), k.to(gpu_device), v.to(gpu_device), q_lens, kv_lens, scale, True
     )
     torch.testing.assert_close(got.float().cpu(), want, atol=1e-2, rtol=1e-2)
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("hq,kvh", [(10, 2), (7, 1), (3, 3)])
+def test_prefill_attention_head_rows_across_tiles(gpu_device, d, hq, kvh):
+    """Rows of a GQA group's heads share a tile: groups that do not divide the
+    128-row tile, requests that end inside a wave, next to an empty one, one
+    without keys and one with fewer keys than queries (rows before the first
+    key are zero), through the plan and through the grid without one."""
+    from vllm_ascend_quantized_kv_cache.ops import _native
+    from vllm_ascend_quantized_kv_cache.ops.attention import prefill_attention
+
+    g = torch.Generator().manual_seed(d + hq)
+    q_lens = [129, 0, 33, 4, 9]
+    kv_lens = [193, 7, 33, 0, 5]
+    dtype = torch.bfloat16
+    q = torch.randn(sum(q_lens), hq, d, generator=g).to(dtype)
+    k = torch.randn(sum(kv_lens), kvh, d, generator=g).to(dtype)
+    v = torch.randn(sum(kv_lens), kvh, d, generator=g).to(dtype)
+    live = sum(q_lens[:3])
+    want = torch.zeros(q.shape)
+    want[:live] = ref.attention(q[:live], k[: sum(kv_lens[:3])], v[: sum(kv_lens[:3])],
+                                q_lens[:3], kv_lens[:3], d ** -0.5, True)
+    want[-5:] = ref.attention(q[-5:], k[-5:], v[-5:], [5], [5], d ** -0.5, True)
+    qg, kg, vg = (x.to(gpu_device) for x in (q, k, v))
+    got = prefill_attention(qg, kg, vg, q_lens, kv_lens, d ** -0.5, True)
+    torch.testing.assert_close(got.float().cpu(), want, atol=1e-2, rtol=1e-2)
+    cu = torch.tensor([[0, 129, 129, 162, 166, 175], [0, 193, 200, 233, 233, 238]],
+                      dtype=torch.int32, device=gpu_device)
+    out = torch.full_like(qg, 7.0)
+    rc = _native.lib().kvq_prefill_attn(
+        qg.data_ptr(), kg.data_ptr(), vg.data_ptr(), _native.dtype_code(dtype),
+        cu[0].data_ptr(), cu[1].data_ptr(), 5, 129, hq, kvh, d, d ** -0.5, 1, out.data_ptr(),
+        _native.stream_of(qg))
+    assert rc == 0
+    torch.testing.assert_close(out, got, atol=0, rtol=0)

@@ -10,9 +10,9 @@
 // position lk - lq + i; with `causal`, key positions past it are masked
 // (pkg/methods/kivi_int4/semantics.py:285-299).
 //
-// bf16/fp16 inputs with head_size 64 or 128 run prefill_attn_fa_kernel
+// bf16/fp16 inputs with head_size 64, 128 or 256 run prefill_attn_fa_kernel
 // (64-key blocks, DMA-staged K, transposed V, described at the kernel).  The
-// kernel below covers the rest (fp32 inputs, head_size 32 and 256):
+// kernel below covers the rest (fp32 inputs, head_size 32):
 // one workgroup = 4 waves = 64 query rows of one query head; each wave owns
 // 16 rows.  Keys/values stream through LDS in 32-token blocks.
 //   S^T = K * Q^T   (v_mfma_f32_16x16x32_{bf16,f16}): A = K rows from LDS
@@ -22,6 +22,9 @@
 //                   A = V^T read from the LDS block.
 // Online softmax in the log2 domain, fp32 accumulation, output in the input
 // dtype (fp32 inputs run through bf16 operands).
+#include <algorithm>
+#include <vector>
+
 #include "kvq_common.h"
 
 namespace {
@@ -241,16 +244,20 @@ prefill_attn_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* _
     for (int r = 0; r < 4; ++r) orow[16 * j + 4 * kg + r] = from_f32<T>(o[j][r] * inv);
 }
 
-// ---- 64-key-block kernel for 16-bit inputs, D in {64, 128} ------------------
-// One workgroup = 4 waves x 32 query rows (two 16-row MFMA column groups) of one
-// query head; key/value blocks of 64 tokens, double-buffered in LDS with one
-// barrier per block:
+// ---- 64-key-block kernel for 16-bit inputs, D in {64, 128, 256} -------------
+// One workgroup = 4 waves x 32 rows (two 16-row MFMA column groups) of one
+// request and kv head; key/value blocks of 64 tokens, double-buffered in LDS
+// with one barrier per block.  Row R of a (request, kv head) is query R / rep
+// of query head kvhead * rep + R % rep: the GQA group's heads share a tile, so
+// the tile's queries sit rep times closer together (fewer keys masked along
+// the diagonal), a short prompt fills its tile, and each key block is staged
+// once for the group instead of once per head.
 //   K  [64][D]    written by global_load_lds (16-byte lanes); the 16-byte
 //                 column of each row is XOR-swizzled by the row so that the
 //                 16 rows one score MFMA reads sit in different banks;
 //   V  [64][D]    written by global_load_lds too, row-major; 16-byte column
 //                 c of row r stored at c ^ (2*(r % 4) + 8*((r / 4) % 2)) (the
-//                 second term at D = 128), so that the rows the transposing
+//                 second term at D >= 128), so that the rows the transposing
 //                 reads of one LDS cycle cover sit in different banks.
 // Keys run one block ahead of values: the step of block i computes block i's
 // softmax and PV and block i+1's scores, whose MFMAs interleave with block
@@ -271,8 +278,6 @@ prefill_attn_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* _
 // fma and exp2 per score; the offset bookkeeping (new offset, rescale factor)
 // sits in the branch that the lazy offset rarely takes.
 
-constexpr int kFaGroupRows = 128;  // query rows per workgroup
-constexpr int kFaXcds = 8;         // XCDs workgroup ids are dealt over
 constexpr int kFaBlock = 64;  // keys per block
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) v4s* lds_v4s_ptr;
@@ -303,18 +308,28 @@ struct FaLds {
   static constexpr int BYTES = 2 * BUF;
 };
 
-// NG 16-row query column groups per wave; the workgroup's 8 / NG waves cover
-// 128 rows and share the LDS blocks.  The launcher uses NG = 2 (4 waves of 32
-// rows, 2 waves per SIMD): each LDS operand feeds two MFMAs.  NG = 1 (8 waves
-// of 16 rows, 4 per SIMD) measured 26% slower on config 4 (twice the LDS reads
-// per MFMA, and spills at the 128-VGPR limit of 4 waves per SIMD).
+// NG 16-row column groups per wave; the workgroup's 8 / NG waves cover 128 rows
+// and share the LDS blocks, at two waves per SIMD (fa_ng below):
+//   D <= 128: NG = 2 (4 waves of 32 rows, two workgroups a CU): each LDS operand
+//     feeds two MFMAs.  NG = 1 measured 26% slower on 8 x 2048 queries over
+//     10240 keys (twice the LDS reads per MFMA, and spills at the 128-VGPR limit
+//     of 4 waves per SIMD).
+//   D = 256: NG = 1 (8 waves of 16 rows; the blocks take 128 KB, one workgroup
+//     a CU): 242 VGPRs, 245 us on 6 ragged prompts of 200 - 2048 rows with 3000
+//     keys of history (8 heads on 1 kv head); the fallback kernel took 1612.
+//     NG = 2 needs about 400 registers, one wave per SIMD and accumulator moves:
+//     322 us, and 335 with its operand reads a step ahead.
+template <int D>
+constexpr int fa_ng() { return D == 256 ? 1 : 2; }
+
 template <typename T, int D, int NG>
 __global__ void __launch_bounds__(64 * (8 / NG))
-__attribute__((amdgpu_waves_per_eu(4 / NG, 4 / NG)))
+__attribute__((amdgpu_waves_per_eu(2, 2)))
 prefill_attn_fa_kernel(const T* __restrict__ q, const T* __restrict__ k,
                        const T* __restrict__ v, const int32_t* __restrict__ cu_q,
-                       const int32_t* __restrict__ cu_k, int hq, int kvh, float qscale,
-                       int causal, int qblocks, int batch, T* __restrict__ out) {
+                       const int32_t* __restrict__ cu_k, const int32_t* __restrict__ units,
+                       int tiles, int hq, int kvh, FastDiv rep_div, float qscale, int causal,
+                       T* __restrict__ out) {
   using O = typename Op<T>::type;
   using L = FaLds<D>;
   constexpr int kFaWaves = 8 / NG;
@@ -334,28 +349,25 @@ prefill_attn_fa_kernel(const T* __restrict__ q, const T* __restrict__ k,
   extern __shared__ __align__(16) char lds[];
   const uint32_t lds0 = lds_addr(lds);  // LDS byte address of the buffers (DMA M0)
 
-  // Workgroup ids go to the XCDs round-robin.  The rep * qblocks workgroups
-  // that stream one (request, kv head)'s K/V run on one XCD, one such pair
-  // after another, so that XCD's L2 keeps the pair's blocks between them;
-  // inside a pair the heavy query blocks (more keys under the causal mask)
-  // come first, the pair's query heads interleaved.
-  const int rep = hq / kvh;
-  const int per_pair = rep * qblocks;
-  const int xcd = static_cast<int>(blockIdx.x) % kFaXcds;
-  const int xj = static_cast<int>(blockIdx.x) / kFaXcds;
-  const int pair = xcd + kFaXcds * (xj / per_pair);
-  if (pair >= batch * kvh) return;  // padding of the last round
-  const int w = xj % per_pair;
-  const int b = pair / kvh;
-  const int kvhead = pair - b * kvh;
-  const int head = kvhead * rep + w % rep;
-  const int qb = qblocks - 1 - w / rep;
+  // Workgroup ids go to the XCDs round-robin: with 8 kv heads each XCD runs one
+  // kv head of every tile, in the order of the unit list (a request's tiles
+  // one after another where its keys outgrow an L2, so that the XCD's L2 keeps
+  // them between its tiles); with fewer kv heads a request's tiles spread over
+  // all XCDs.
+  const int rep = static_cast<int>(rep_div.d);
+  const int unit = static_cast<int>(blockIdx.x) / kvh;
+  const int kvhead = static_cast<int>(blockIdx.x) - unit * kvh;
+  // without a unit list: every request's `tiles` tiles, the last (most keys
+  // under the causal mask) first
+  const int b = units ? units[2 * unit] : unit / tiles;
+  const int tile = units ? units[2 * unit + 1] : tiles - 1 - unit % tiles;
   const int q_start = cu_q[b];
   const int lq = cu_q[b + 1] - q_start;
   const int k_start = cu_k[b];
   const int lk = cu_k[b + 1] - k_start;
-  const int row0 = qb * (kFaRows * kFaWaves);
-  if (row0 >= lq || lk <= 0) return;  // uniform over the workgroup
+  const int rows = lq * rep;  // rows of this (request, kv head)
+  const int row0 = tile * (kFaRows * kFaWaves);
+  if (row0 >= rows) return;  // uniform over the workgroup
   const int tid = threadIdx.x;
   // wave-uniform; saying so keeps the DMA destinations in scalar registers
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -363,64 +375,74 @@ prefill_attn_fa_kernel(const T* __restrict__ q, const T* __restrict__ k,
   const int n = lane & 15;
   const int kg = lane >> 4;
   const int wrow0 = row0 + wave * kFaRows;
-  const int last_row = min(row0 + kFaRows * kFaWaves, lq) - 1;
-  const int kv_end = causal ? min(lk, lk - lq + last_row + 1) : lk;
+  auto query_of = [&](int row) { return static_cast<int>(rep_div.div(static_cast<uint32_t>(row))); };
+  const int last_row = min(row0 + kFaRows * kFaWaves, rows) - 1;
+  const int kv_end = causal ? min(lk, lk - lq + query_of(last_row) + 1) : lk;
   const int nblk = (kv_end + kFaBlock - 1) / kFaBlock;
-  const int wave_last = min(wrow0 + kFaRows, lq) - 1;  // < wrow0 when the wave has no rows
-  const int wave_last_pos = lk - lq + wave_last;
+  const int wave_last = min(wrow0 + kFaRows, rows) - 1;  // < wrow0 when the wave has no rows
+  // kv positions of the wave's first and last query
+  const int wave_first_pos = lk - lq + query_of(wrow0);
+  const int wave_last_pos = lk - lq + query_of(wave_last);
 
-  // Q^T operands: group g2, k-step s: query row wrow0 + 16*g2 + n, dims 32s + 8kg + i
-  // (unscaled: exact in the operand type)
+  // element offset of row R in q and out
+  auto row_offset = [&](int row) -> int64_t {
+    const int i = query_of(row);
+    return (static_cast<int64_t>(q_start + i) * hq + kvhead * rep + (row - i * rep)) * D;
+  };
+  if (lk <= 0) {  // uniform: nothing to attend to
+    for (int r = tid >> 4; r < kFaRows * kFaWaves; r += 4 * kFaWaves)
+      if (row0 + r < rows)
+        for (int c = tid & 15; c < D; c += 16) out[row_offset(row0 + r) + c] = from_f32<T>(0.0f);
+    return;
+  }
+
+  // Q^T operands: group g2, k-step s: row wrow0 + 16*g2 + n, dims 32s + 8kg + i
+  // (unscaled: exact in the operand type; loaded with the first blocks below)
   u8v qop[NG][KS];
   int my_pos[NG];
   bool live[NG];
 #pragma unroll
   for (int g2 = 0; g2 < NG; ++g2) {
     const int row = wrow0 + 16 * g2 + n;
-    live[g2] = row < lq;
-    my_pos[g2] = lk - lq + row;
-    const T* qrow = q + (static_cast<int64_t>(q_start + (live[g2] ? row : 0)) * hq + head) * D;
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      u8v x = load_op8(qrow + 32 * s + 8 * kg);
-      if (!live[g2]) x = u8v{0, 0, 0, 0, 0, 0, 0, 0};
-      qop[g2][s] = x;
-    }
+    live[g2] = row < rows;
+    my_pos[g2] = lk - lq + query_of(row);
   }
 
   // ---- staging ----
   const T* kbase = k + (static_cast<int64_t>(k_start) * kvh + kvhead) * D;
   const T* vbase = v + (static_cast<int64_t>(k_start) * kvh + kvhead) * D;
   const int64_t row_stride = static_cast<int64_t>(kvh) * D;
-  // per-lane byte offsets of the K and V rows this lane moves (row r of the
-  // block, swizzled piece), relative to the block's first row: 32-bit, so
-  // that every DMA is a uniform base plus a lane offset
-  uint32_t koff[KINST], voff[KINST];
-  int krow[KINST];
-#pragma unroll
-  for (int i = 0; i < KINST; ++i) {
-    const int inst = wave * KINST + i;
-    const int r = inst * RPI + lane / PPR;  // block row of this lane
-    krow[i] = r;
-    koff[i] = static_cast<uint32_t>((r * row_stride + 8 * ((lane % PPR) ^ (r % PPR))) * 2);
-    voff[i] = static_cast<uint32_t>((r * row_stride + 8 * ((lane % PPR) ^ vswz(r))) * 2);
-  }
-  // DMA of block rows kb .. kb + 63 of `base` into `dst` with the lane
-  // offsets `off`; in the last block rows past the end read the last row
-  // (masked later)
-  auto issue_rows = [&](const T* base, const uint32_t (&off)[KINST], char* dst, int kb) {
+  // DMA instruction i of a wave moves block rows c .. c + RPI - 1, c = RPI *
+  // (wave * KINST + i): lane l the 16-byte column (l % PPR) ^ swz(row) of row
+  // c + l / PPR.  Both swizzles split over the bits of the row, swz(c + l / PPR)
+  // = swz(c) ^ swz(l / PPR), and a row's columns are the low bits of its
+  // offset, so one offset per lane and side serves every instruction: the
+  // instruction adds row c to the uniform base and xors 16 * swz(c).
+  auto kswz = [](int r) { return r % PPR; };
+  const uint32_t row_bytes = static_cast<uint32_t>(row_stride * 2);
+  const int lane_row = lane / PPR;
+  const uint32_t koff = lane_row * row_bytes + 16 * ((lane % PPR) ^ kswz(lane_row));
+  const uint32_t voff = lane_row * row_bytes + 16 * ((lane % PPR) ^ vswz(lane_row));
+  // DMA of block rows kb .. kb + 63 of `base` into `dst`; in the last block
+  // rows past the end read the last row (masked later)
+  auto issue_rows = [&](const T* base, uint32_t off, auto swz, char* dst, int kb) {
     const char* gb = reinterpret_cast<const char*>(base + static_cast<int64_t>(kb) * row_stride);
     if (kb + kFaBlock <= lk) {  // uniform: only the last block clamps
 #pragma unroll
-      for (int i = 0; i < KINST; ++i)
-        dma16_so(gb, off[i], lds0 + static_cast<uint32_t>(dst - lds) + 1024u * (wave * KINST + i));
+      for (int i = 0; i < KINST; ++i) {
+        const int c = RPI * (wave * KINST + i);
+        dma16_so(gb + static_cast<uint32_t>(c) * row_bytes, off ^ (16u * swz(c)),
+                 lds0 + static_cast<uint32_t>(dst - lds) + 1024u * (wave * KINST + i));
+      }
     } else {
 #pragma unroll
       for (int i = 0; i < KINST; ++i) {
         // rows past the end step back to row lk - 1 - kb of the block (>= 0),
         // so the offset from the block's first row stays non-negative
-        const int back = kb + krow[i] >= lk ? kb + krow[i] - (lk - 1) : 0;
-        dma16_so(gb, off[i] - static_cast<uint32_t>(back) * static_cast<uint32_t>(row_stride * 2),
+        const int c = RPI * (wave * KINST + i);
+        const int over = kb + c + lane_row - (lk - 1);
+        const int r = c - (over > 0 ? over : 0);
+        dma16_so(gb, (off ^ (16u * swz(c))) + static_cast<uint32_t>(r) * row_bytes,
                  lds0 + static_cast<uint32_t>(dst - lds) + 1024u * (wave * KINST + i));
       }
     }
@@ -480,6 +502,26 @@ prefill_attn_fa_kernel(const T* __restrict__ q, const T* __restrict__ k,
       a[s] = *reinterpret_cast<const u8v*>(sk + r * D + 8 * piece);
     }
   };
+  // the V^T operands of k-step ks, half jh of the dim blocks
+  auto v_reads = [&](const char* sv, int ks, int jh, u8v (&a)[DB / 2]) {
+#pragma unroll
+    for (int jj = 0; jj < DB / 2; ++jj) {
+      const int j = jh * (DB / 2) + jj;
+      v4s part[2];
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) {
+        // keys 32 ks + 16 hh + 4 kg + k, k = 0..3
+        const int r = 32 * ks + 16 * hh + 4 * kg + tr_row;
+        const int pos = (2 * j + tr_chunk) ^ vswz(r);
+        part[hh] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (lds_v4s_ptr)(sv + r * (2 * D) + 16 * pos + tr_half));
+      }
+      a[jj] = u8v{static_cast<uint16_t>(part[0][0]), static_cast<uint16_t>(part[0][1]),
+                  static_cast<uint16_t>(part[0][2]), static_cast<uint16_t>(part[0][3]),
+                  static_cast<uint16_t>(part[1][0]), static_cast<uint16_t>(part[1][1]),
+                  static_cast<uint16_t>(part[1][2]), static_cast<uint16_t>(part[1][3])};
+    }
+  };
   auto k_mfmas = [&](const u8v (&a)[KS], f4 (&acc)[NG]) {
 #pragma unroll
     for (int s = 0; s < KS; ++s)
@@ -488,9 +530,21 @@ prefill_attn_fa_kernel(const T* __restrict__ q, const T* __restrict__ k,
   };
 
   // prologue: keys of blocks 0 and 1, values of block 0; scores of block 0
-  issue_rows(kbase, koff, kbuf0, 0);
-  if (nblk > 1) issue_rows(kbase, koff, kbuf1, kFaBlock);
-  issue_rows(vbase, voff, vbuf0, 0);
+  issue_rows(kbase, koff, kswz, kbuf0, 0);
+  if (nblk > 1) issue_rows(kbase, koff, kswz, kbuf1, kFaBlock);
+  issue_rows(vbase, voff, vswz, vbuf0, 0);
+  // the query rows go out behind the DMAs, so that one wait covers both
+#pragma unroll
+  for (int g2 = 0; g2 < NG; ++g2) {
+    const T* qrow = q + row_offset(live[g2] ? wrow0 + 16 * g2 + n : 0);
+#pragma unroll
+    for (int s = 0; s < KS; ++s) qop[g2][s] = load_op8(qrow + 32 * s + 8 * kg);
+  }
+#pragma unroll
+  for (int g2 = 0; g2 < NG; ++g2)
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+      if (!live[g2]) qop[g2][s] = u8v{0, 0, 0, 0, 0, 0, 0, 0};
   wait_vmcnt<0>();  // landed in LDS
   __syncthreads();
   f4 sacc[4][NG];
@@ -515,13 +569,13 @@ prefill_attn_fa_kernel(const T* __restrict__ q, const T* __restrict__ k,
   auto step = [&](const char* __restrict__ kn, const char* __restrict__ vc,
                   char* __restrict__ kd, char* __restrict__ vd, int i) {
     const int kb = i * kFaBlock;
-    if (i + 2 < nblk) issue_rows(kbase, koff, kd, kb + 2 * kFaBlock);
-    if (i + 1 < nblk) issue_rows(vbase, voff, vd, kb + kFaBlock);
+    if (i + 2 < nblk) issue_rows(kbase, koff, kswz, kd, kb + 2 * kFaBlock);
+    if (i + 1 < nblk) issue_rows(vbase, voff, vswz, vd, kb + kFaBlock);
     if (active(i)) {
       // ---- online softmax of block i per query column ----
       // the max runs over raw scores (qscale > 0), the exponent is one fma:
       // p = 2^(qscale * s + m_off)
-      const bool full = kb + kFaBlock <= lk && (!causal || kb + kFaBlock - 1 <= lk - lq + wrow0);
+      const bool full = kb + kFaBlock <= lk && (!causal || kb + kFaBlock - 1 <= wave_first_pos);
       if (!full) {  // uniform: one branch, then a compare per score
 #pragma unroll
         for (int g2 = 0; g2 < NG; ++g2) {
@@ -621,40 +675,24 @@ prefill_attn_fa_kernel(const T* __restrict__ q, const T* __restrict__ k,
           pop[g2][ks] = __builtin_bit_cast(u8v, make_uint4(pw[g2][ks][0], pw[g2][ks][1],
                                                            pw[g2][ks][2], pw[g2][ks][3]));
       // ---- O^T += V^T * P^T ----
-      const char* sv_base = vc;
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-      for (int jh = 0; jh < 2; ++jh) {
-        u8v a[DB / 2];  // half the dim blocks' V^T operands of this k-step, then the MFMAs
+        for (int jh = 0; jh < 2; ++jh) {
+          u8v a[DB / 2];  // half the dim blocks' V^T operands of this k-step, then the MFMAs
+          v_reads(vc, ks, jh, a);
+          __builtin_amdgcn_sched_barrier(0);  // keep the reads ahead of the MFMAs
 #pragma unroll
-        for (int jj = 0; jj < DB / 2; ++jj) {
-          const int j = jh * (DB / 2) + jj;
-          v4s part[2];
+          for (int jj = 0; jj < DB / 2; ++jj)
 #pragma unroll
-          for (int hh = 0; hh < 2; ++hh) {
-            // keys 32 ks + 16 hh + 4 kg + k, k = 0..3
-            const int r = 32 * ks + 16 * hh + 4 * kg + tr_row;
-            const int pos = (2 * j + tr_chunk) ^ vswz(r);
-            part[hh] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (lds_v4s_ptr)(sv_base + r * (2 * D) + 16 * pos + tr_half));
+            for (int g2 = 0; g2 < NG; ++g2)
+              o[jh * (DB / 2) + jj][g2] =
+                  mfma16(a[jj], pop[g2][ks], o[jh * (DB / 2) + jj][g2], O{});
+          if (jh == 1) {
+#pragma unroll
+            for (int g2 = 0; g2 < NG; ++g2) l_acc[g2] = mfma16(ones, pop[g2][ks], l_acc[g2], O{});
           }
-          a[jj] = u8v{static_cast<uint16_t>(part[0][0]), static_cast<uint16_t>(part[0][1]),
-                      static_cast<uint16_t>(part[0][2]), static_cast<uint16_t>(part[0][3]),
-                      static_cast<uint16_t>(part[1][0]), static_cast<uint16_t>(part[1][1]),
-                      static_cast<uint16_t>(part[1][2]), static_cast<uint16_t>(part[1][3])};
         }
-        __builtin_amdgcn_sched_barrier(0);  // keep the reads ahead of the MFMAs
-#pragma unroll
-        for (int jj = 0; jj < DB / 2; ++jj)
-#pragma unroll
-          for (int g2 = 0; g2 < NG; ++g2)
-            o[jh * (DB / 2) + jj][g2] = mfma16(a[jj], pop[g2][ks], o[jh * (DB / 2) + jj][g2], O{});
-        if (jh == 1) {
-#pragma unroll
-          for (int g2 = 0; g2 < NG; ++g2) l_acc[g2] = mfma16(ones, pop[g2][ks], l_acc[g2], O{});
-        }
-      }
       __builtin_amdgcn_s_setprio(0);
 #pragma unroll
       for (int kb2 = 0; kb2 < 4; ++kb2)
@@ -683,12 +721,61 @@ prefill_attn_fa_kernel(const T* __restrict__ q, const T* __restrict__ k,
     if (!live[g2]) continue;
     const float l = l_acc[g2][0];
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-    T* orow = out + (static_cast<int64_t>(q_start + wrow0 + 16 * g2 + n) * hq + head) * D;
+    T* orow = out + row_offset(wrow0 + 16 * g2 + n);
 #pragma unroll
     for (int j = 0; j < DB; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) orow[16 * j + 4 * kg + r] = from_f32<T>(o[j][g2][r] * inv);
+      *reinterpret_cast<uint2*>(orow + 16 * j + 4 * kg) =
+          make_uint2(pack_op2(o[j][g2][0] * inv, o[j][g2][1] * inv, O{}),
+                     pack_op2(o[j][g2][2] * inv, o[j][g2][3] * inv, O{}));
   }
+}
+
+constexpr int kFaTileRows = 128;  // rows (queries x heads of a GQA group) per workgroup
+
+// The 64-key-block kernel: 16-bit inputs, head sizes 64, 128 and 256, on a
+// device with its LDS.  `units` int32 [num_units, 2] = (request, tile) in
+// dispatch order, or NULL: num_units = batch * tiles, every request's `tiles`
+// tiles.  *launched: false when another kernel has to run.
+int launch_fa(const void* query, const void* key, const void* value, int dtype,
+              const int32_t* cu_q, const int32_t* cu_k, const int32_t* units, int64_t num_units,
+              int64_t tiles, int num_heads, int num_kv_heads, int head_size, float qscale,
+              int causal, void* out, hipStream_t s, bool* launched) {
+  *launched = false;
+  if (dtype != KVQ_DTYPE_BF16 && dtype != KVQ_DTYPE_F16) return KVQ_OK;
+  if (head_size != 64 && head_size != 128 && head_size != 256) return KVQ_OK;
+  int64_t lds_max = 0;  // LDS one workgroup may use on this device
+  const int lrc = device_lds_max(&lds_max);
+  if (lrc != KVQ_OK) return lrc;
+  const int64_t fa_lds = head_size == 64    ? FaLds<64>::BYTES
+                         : head_size == 128 ? FaLds<128>::BYTES
+                                            : FaLds<256>::BYTES;
+  if (fa_lds > lds_max) return KVQ_OK;
+  if (num_units * num_kv_heads > 0x7fffffff || tiles > 0x7fffffff / kFaTileRows)
+    return KVQ_ERR_INVALID;
+  const dim3 grid(static_cast<unsigned>(num_units * num_kv_heads));
+  const FastDiv rep_div = FastDiv::make(static_cast<uint32_t>(num_heads / num_kv_heads));
+#define KVQ_PREFILL_FA(TT, DD)                                                              \
+  hipLaunchKernelGGL((prefill_attn_fa_kernel<TT, DD, fa_ng<DD>()>), grid, dim3(64 * (8 / fa_ng<DD>())), \
+                     FaLds<DD>::BYTES, s, static_cast<const TT*>(query),                   \
+                     static_cast<const TT*>(key), static_cast<const TT*>(value), cu_q, cu_k, \
+                     units, static_cast<int>(tiles), num_heads, num_kv_heads, rep_div, qscale, \
+                     causal, static_cast<TT*>(out))
+#define KVQ_PREFILL_FA_D(TT)                        \
+  switch (head_size) {                              \
+    case 64: KVQ_PREFILL_FA(TT, 64); break;         \
+    case 128: KVQ_PREFILL_FA(TT, 128); break;       \
+    default: KVQ_PREFILL_FA(TT, 256); break;        \
+  }
+  if (dtype == KVQ_DTYPE_BF16) {
+    KVQ_PREFILL_FA_D(kvq::bf16)
+  } else {
+    KVQ_PREFILL_FA_D(kvq::f16)
+  }
+#undef KVQ_PREFILL_FA_D
+#undef KVQ_PREFILL_FA
+  KVQ_LAUNCH_CHECK();
+  *launched = true;
+  return KVQ_OK;
 }
 
 }  // namespace
@@ -708,35 +795,13 @@ extern "C" int kvq_prefill_attn(const void* query, const void* key, const void* 
   if (!(scale > 0.0f)) return KVQ_ERR_INVALID;  // the softmax max runs over raw scores
   hipStream_t s = static_cast<hipStream_t>(stream);
   const float qscale = scale * 1.4426950408889634f;
-  int64_t lds_max = 0;  // LDS one workgroup may use on this device
-  const int lrc = device_lds_max(&lds_max);
-  if (lrc != KVQ_OK) return lrc;
-  const int64_t fa_lds = head_size == 64 ? FaLds<64>::BYTES : FaLds<128>::BYTES;
-  constexpr int kFaNG = 2;
-  if ((dtype == KVQ_DTYPE_BF16 || dtype == KVQ_DTYPE_F16) &&
-      (head_size == 64 || head_size == 128) && fa_lds <= lds_max) {
-    const int64_t fab = (max_q_len + kFaGroupRows - 1) / kFaGroupRows;
-    const int64_t pairs = batch * num_kv_heads;
-    const int64_t wgs = (pairs + kFaXcds - 1) / kFaXcds * kFaXcds * (num_heads / num_kv_heads) * fab;
-    if (wgs > 0x7fffffff) return KVQ_ERR_INVALID;
-    const dim3 fgrid(static_cast<unsigned>(wgs));
-#define KVQ_PREFILL_FA(TT, DD)                                                              \
-    hipLaunchKernelGGL((prefill_attn_fa_kernel<TT, DD, kFaNG>), fgrid, dim3(64 * (8 / kFaNG)), \
-                       FaLds<DD>::BYTES, s, static_cast<const TT*>(query),                 \
-                       static_cast<const TT*>(key), static_cast<const TT*>(value),         \
-                       cu_seqlens_q, cu_seqlens_k, num_heads, num_kv_heads, qscale, causal, \
-                       static_cast<int>(fab), static_cast<int>(batch), static_cast<TT*>(out))
-    if (dtype == KVQ_DTYPE_BF16) {
-      if (head_size == 64) KVQ_PREFILL_FA(kvq::bf16, 64);
-      else KVQ_PREFILL_FA(kvq::bf16, 128);
-    } else {
-      if (head_size == 64) KVQ_PREFILL_FA(kvq::f16, 64);
-      else KVQ_PREFILL_FA(kvq::f16, 128);
-    }
-#undef KVQ_PREFILL_FA
-    KVQ_LAUNCH_CHECK();
-    return KVQ_OK;
-  }
+  const int64_t rows = max_q_len * (num_heads / num_kv_heads);
+  const int64_t tiles = (rows + kFaTileRows - 1) / kFaTileRows;
+  bool launched = false;
+  const int frc = launch_fa(query, key, value, dtype, cu_seqlens_q, cu_seqlens_k, nullptr,
+                            batch * tiles, tiles, num_heads, num_kv_heads, head_size, qscale,
+                            causal, out, s, &launched);
+  if (frc != KVQ_OK || launched) return frc;
   const int64_t qblocks = (max_q_len + 63) / 64;
   if (qblocks > 0x7fffffff) return KVQ_ERR_INVALID;
   const dim3 grid(static_cast<unsigned>(qblocks), num_heads, static_cast<unsigned>(batch));
@@ -755,4 +820,79 @@ extern "C" int kvq_prefill_attn(const void* query, const void* key, const void* 
 #undef KVQ_PREFILL
   KVQ_LAUNCH_CHECK();
   return KVQ_OK;
+}
+
+// Host side of a planned call: the cumulative lengths and the tiles in the
+// order they should start.  A tile's cost is its key blocks; long ones start
+// first, so that the last to end are short.  Where the keys and values an XCD
+// streams outgrow its 4 MB L2 twice over, a request's tiles stay together (the
+// requests by falling cost), so that one request's keys are in use at a time.
+extern "C" int64_t kvq_plan_prefill_attn(const int64_t* q_lens, const int64_t* kv_lens,
+                                         int64_t batch, int num_heads, int num_kv_heads,
+                                         int head_size, int causal, int32_t* plan,
+                                         int64_t cap_units) {
+  if (batch < 0 || (batch > 0 && (!q_lens || !kv_lens)) || !plan || num_kv_heads <= 0 ||
+      num_heads <= 0 || num_heads % num_kv_heads || head_size <= 0)
+    return KVQ_ERR_INVALID;
+  const int64_t rep = num_heads / num_kv_heads;
+  int32_t* cu_q = plan;
+  int32_t* cu_k = plan + batch + 1;
+  int32_t* units = plan + 2 * (batch + 1);
+  int64_t nq = 0, nk = 0, n = 0;
+  struct Unit {
+    int64_t group, cost;  // descending sort keys
+    int32_t b, tile;
+  };
+  std::vector<Unit> all;
+  all.reserve(static_cast<size_t>(cap_units > 0 ? cap_units : 0));
+  cu_q[0] = cu_k[0] = 0;
+  for (int64_t b = 0; b < batch; ++b) {
+    const int64_t lq = q_lens[b], lk = kv_lens[b];
+    if (lq < 0 || lk < 0) return KVQ_ERR_INVALID;
+    nq += lq;
+    nk += lk;
+    if (nq * rep > 0x7fffffff || nk > 0x7fffffff) return KVQ_ERR_INVALID;
+    cu_q[b + 1] = static_cast<int32_t>(nq);
+    cu_k[b + 1] = static_cast<int32_t>(nk);
+    const int64_t rows = lq * rep;
+    for (int64_t r0 = 0; r0 < rows; r0 += kFaTileRows, ++n) {
+      if (n >= cap_units) return KVQ_ERR_CAPACITY;
+      const int64_t last = (std::min<int64_t>(r0 + kFaTileRows, rows) - 1) / rep;
+      const int64_t end = causal ? std::min(lk, lk - lq + last + 1) : lk;
+      const int64_t cost = end <= 0 ? 0 : (end + kFaBlock - 1) / kFaBlock;
+      all.push_back({0, cost, static_cast<int32_t>(b), static_cast<int32_t>(r0 / kFaTileRows)});
+    }
+  }
+  const int64_t xcd_bytes = nk * head_size * 4 * std::max<int64_t>(1, num_kv_heads / 8);
+  if (xcd_bytes > (int64_t{8} << 20))
+    for (auto& u : all) u.group = q_lens[u.b] * kv_lens[u.b];
+  std::stable_sort(all.begin(), all.end(), [](const Unit& x, const Unit& y) {
+    if (x.group != y.group) return x.group > y.group;
+    if (x.group != 0 && x.b != y.b) return x.b < y.b;
+    return x.cost > y.cost;
+  });
+  for (int64_t i = 0; i < n; ++i) {
+    units[2 * i] = all[static_cast<size_t>(i)].b;
+    units[2 * i + 1] = all[static_cast<size_t>(i)].tile;
+  }
+  return n;
+}
+
+extern "C" int kvq_prefill_attn_planned(const void* query, const void* key, const void* value,
+                                        int dtype, const int32_t* plan, int64_t batch,
+                                        int64_t num_units, int num_heads, int num_kv_heads,
+                                        int head_size, float scale, int causal, void* out,
+                                        void* stream) {
+  if (batch == 0 || num_units == 0) return KVQ_OK;
+  if (!query || !key || !value || !plan || !out || batch < 0 || num_units < 0)
+    return KVQ_ERR_INVALID;
+  if (num_kv_heads <= 0 || num_heads % num_kv_heads) return KVQ_ERR_GEOMETRY;
+  if (!(scale > 0.0f)) return KVQ_ERR_INVALID;
+  bool launched = false;
+  const int rc = launch_fa(query, key, value, dtype, plan, plan + batch + 1,
+                           plan + 2 * (batch + 1), num_units, 0, num_heads, num_kv_heads,
+                           head_size, scale * 1.4426950408889634f, causal, out,
+                           static_cast<hipStream_t>(stream), &launched);
+  if (rc != KVQ_OK) return rc;
+  return launched ? KVQ_OK : KVQ_ERR_GEOMETRY;
 }
