@@ -685,3 +685,106 @@ def test_decode_combine_of_many_items_per_request(gpu_device):
         ring_k.to(gpu_device), ring_v.to(gpu_device), scale, g, split_tokens=128,
     )
     torch.testing.assert_close(got.float().cpu(), want, atol=1e-2, rtol=1e-2)
+
+
+def _split_decode_case(dev, d, kvh, g, bs, rep, dtype, plan_of, *, lens=None, stale=True):
+    """A decode over stale pages against the oracle; ``plan_of(seqs) -> plan``."""
+    from vllm_ascend_quantized_kv_cache.ops.kivi_decode import DecodeSeq, kivi_decode_attention
+
+    r_len = 128
+    lens = lens or [r_len * 9 + 3, 1, 700, 0, r_len * 5 + 64, 77, 2 * bs + 1, 3 * bs]
+    cpu, table, ring_k, ring_v, seqs, wk, wv, _, _ = _ring_case(
+        dev, d, kvh, g, bs, r_len, lens, seed=43, ring_dtype=dtype, stale=stale)
+    q = torch.randn(len(lens), kvh * rep, d, generator=torch.Generator().manual_seed(8)).to(dtype)
+    dk, dv = ref.dequant_gather(*cpu, table, torch.tensor(lens), torch.float32, g)
+    dk = ref.overlay_residual(dk, lens, wk)
+    dv = ref.overlay_residual(dv, lens, wv)
+    want = ref.attention(q.float(), dk, dv, [1] * len(lens), lens, d ** -0.5, causal=True)
+    dseqs = [DecodeSeq(n, hk, hv, row, ks_, vs_) for (n, hk, hv, row, ks_, vs_) in seqs]
+    plan = tuple(torch.from_numpy(x).to(dev) for x in plan_of(dseqs) if x is not None)
+    print(f"split decode d={d} kvh={kvh} g={g} bs={bs} rep={rep} {dtype}: {plan[1].shape[0]} items",
+          flush=True)
+    got = kivi_decode_attention(q.to(dev), to_dev(cpu, dev), table.to(dev), dseqs,
+                                ring_k.to(dev), ring_v.to(dev), d ** -0.5, g, plan=plan)
+    got = got.float().cpu()
+    assert torch.isfinite(got).all()
+    torch.testing.assert_close(got, want, atol=1e-2, rtol=1e-2)
+
+
+@pytest.mark.parametrize("d,kvh,g,bs,rep,dtype", [
+    (128, 1, 128, 128, 8, torch.bfloat16),   # key scales and minima in one DMA
+    (128, 2, 64, 128, 5, torch.float16),     # two key groups a page, two value groups
+    (128, 4, 64, 64, 16, torch.bfloat16),    # 64-position pages, unfolded
+    (128, 8, 64, 64, 7, torch.float16),      # 8 heads, but not the page-streaming pages
+    (256, 1, 128, 128, 8, torch.bfloat16),
+    (256, 2, 64, 128, 4, torch.float16),     # four value groups
+    (256, 1, 64, 64, 12, torch.bfloat16),
+    (256, 3, 128, 256, 1, torch.bfloat16),   # key groups of half a page, odd head count
+])
+@pytest.mark.parametrize("cu_count", [1, 3, 256])
+def test_split_decode_matches_oracle(gpu_device, d, kvh, g, bs, rep, dtype, cu_count):
+    """The split decode: pieces of many requests on one wave (1 CU), pieces of
+    one tile (256 CUs), runs that continue over items, merged and unmerged
+    partials; every byte past the histories holds NaN scales."""
+    from vllm_ascend_quantized_kv_cache.ops.kivi_decode import plan_decode_pieces
+
+    _split_decode_case(gpu_device, d, kvh, g, bs, rep, dtype,
+                       lambda s: plan_decode_pieces(s, kvh, cu_count))
+
+
+@pytest.mark.parametrize("g,bs", [(128, 128), (64, 64)])
+@pytest.mark.parametrize("paired", [False, True])
+def test_split_decode_without_pieces_head_256(gpu_device, g, bs, paired):
+    """Head size 256 runs every plan: fixed splits (an item a wave) and pairs of
+    even / odd 64-position chunks."""
+    from vllm_ascend_quantized_kv_cache.ops.kivi_decode import plan_decode_work
+
+    _split_decode_case(gpu_device, 256, 2, g, bs, 4, torch.bfloat16,
+                       lambda s: plan_decode_work(s, 128, paired=paired))
+
+
+def test_split_decode_two_pieces_a_wave_and_long_combine(gpu_device):
+    """Head size 256 with more pieces than the chip holds waves (two pieces a
+    wave), and a request of some 150 items, most of them merged away."""
+    from vllm_ascend_quantized_kv_cache.ops.kivi_decode import plan_decode_pieces
+
+    lens = [9000, 5, 2000, 128, 129] + [300] * 40
+    _split_decode_case(gpu_device, 256, 16, 128, 128, 1, torch.bfloat16,
+                       lambda s: plan_decode_pieces(s, 1, 256), lens=lens, stale=False)
+
+
+@pytest.mark.parametrize("d,kvh,g,bs", [(128, 2, 128, 128), (256, 1, 64, 64), (256, 2, 128, 128)])
+def test_split_decode_with_row_maxima_growing_every_tile(gpu_device, d, kvh, g, bs):
+    """Keys along one direction with a magnitude that grows with the position:
+    the running maximum rises on every tile, and the merged partials of a
+    workgroup's waves differ by many powers of two."""
+    from vllm_ascend_quantized_kv_cache.ops.kivi_decode import (
+        DecodeSeq,
+        kivi_decode_attention,
+        plan_decode,
+    )
+
+    r_len, lens, dtype = 128, [1500, 700], torch.bfloat16
+    u = torch.nn.functional.normalize(
+        torch.randn(kvh, d, generator=torch.Generator().manual_seed(3)), dim=-1)
+
+    def make(n, h_, d_, seed):
+        gen = torch.Generator().manual_seed(seed)
+        grow = torch.arange(n).float()[:, None, None] * (20.0 / n)
+        key = (grow * u + 0.05 * torch.randn(n, h_, d_, generator=gen)).to(dtype)
+        return key, torch.randn(n, h_, d_, generator=gen).to(dtype)
+
+    cpu, table, ring_k, ring_v, seqs, wk, wv, _, _ = _ring_case(
+        gpu_device, d, kvh, g, bs, r_len, lens, seed=45, ring_dtype=dtype, make=make)
+    rep = 4
+    q = (u.repeat_interleave(rep, 0)[None] * 3.0 * d ** 0.5).repeat(len(lens), 1, 1).to(dtype)
+    dk, dv = ref.dequant_gather(*cpu, table, torch.tensor(lens), torch.float32, g)
+    dk = ref.overlay_residual(dk, lens, wk)
+    dv = ref.overlay_residual(dv, lens, wv)
+    want = ref.attention(q.float(), dk, dv, [1] * len(lens), lens, d ** -0.5, causal=True)
+    dseqs = [DecodeSeq(n, hk, hv, row, ks_, vs_) for (n, hk, hv, row, ks_, vs_) in seqs]
+    dev = gpu_device
+    plan = tuple(torch.from_numpy(x).to(dev) for x in plan_decode(dseqs, kvh, 256))
+    got = kivi_decode_attention(q.to(dev), to_dev(cpu, dev), table.to(dev), dseqs,
+                                ring_k.to(dev), ring_v.to(dev), d ** -0.5, g, plan=plan)
+    torch.testing.assert_close(got.float().cpu(), want, atol=1e-2, rtol=1e-2)

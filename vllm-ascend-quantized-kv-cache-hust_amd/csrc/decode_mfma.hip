@@ -774,7 +774,7 @@ __device__ __forceinline__ void tr_item(
     if ((p & 63) == 0) p += cs - 64;
     return p;
   };
-  tr::QGroup qg;
+  tr::QGroup<> qg;
   auto step = [&](const char* __restrict__ cur, char* __restrict__ nxt, int p0, bool new_group) {
     const int p1 = next_tile(p0);
     if (p1 < pe) {
@@ -793,9 +793,9 @@ __device__ __forceinline__ void tr_item(
     if (pieces) __builtin_amdgcn_s_setprio(1);
     const uint32_t off = tr::lds_off(cur);
     if (p0 + GT <= pe)
-      tr::compute_tile<NVG, KSV, FOLD, true>(W, off, p0, pe, n, kg, qg, qscale, acc);
+      tr::compute_tile<NVG, KSV, FOLD, true>(W, off, p0, p0, pe, n, kg, qg, qscale, acc);
     else
-      tr::compute_tile<NVG, KSV, FOLD, false>(W, off, p0, pe, n, kg, qg, qscale, acc);
+      tr::compute_tile<NVG, KSV, FOLD, false>(W, off, p0, p0, pe, n, kg, qg, qscale, acc);
     if (pieces) __builtin_amdgcn_s_setprio(0);
   };
   if (p_first < pe) issue(my_lds, p_first, true);  // prologue: tile 0 into buffer 0
@@ -1113,6 +1113,25 @@ int launch_kivi_decode_mfma(const void* query, int q_dtype, int hq, int kvh, int
                             bool* tail_done) {
   *launched = false;
   *tail_done = false;
+  {
+    // the split decode: pieces that the page-streaming kernel does not take, and
+    // head size 256 with or without them
+    const bool with_pieces = pieces && num_pieces > 0;
+    bool split = false;
+    if (d == 256 || (with_pieces && !(qscale > 0.0f && qscale != INFINITY &&
+                                      coop_decode_applies(q_dtype, hq, kvh, d, ring_dtype, bs, g)))) {
+      const int src = launch_kivi_decode_split(
+          query, q_dtype, hq, kvh, d, qscale, kq, ks, km, vq, vs, vm, bs, g, nb, block_table,
+          maxb, seq_meta, work, num_work, with_pieces ? pieces : nullptr, num_pieces, ring_k,
+          ring_v, ring_dtype, ring_len, ws_o, ws_ml, s, &split);
+      if (src != KVQ_OK) return src;
+    }
+    if (split) {
+      *launched = true;
+      *tail_done = true;
+      return KVQ_OK;
+    }
+  }
   if (d != 128 || hq / kvh > 16 || g % 8 || d % g || g < 32 || g > 128) return KVQ_OK;
   if (bs <= 0 || (bs & (bs - 1))) return KVQ_OK;  // power-of-two pages (shift arithmetic)
   // tiles of 64 tokens (32 for G = 32): inside one key group and one page

@@ -100,10 +100,12 @@ __device__ __forceinline__ int ring_lane(int x, int ring_len) {
 // lane layout of the path that produced it: o[q][r] belongs to query head
 // 4*kg + r of the GQA group and one head dim fixed by (q, lane); m and l are
 // the log2-domain running max and sum of head n = lane % 16.
-struct Partial {
-  f4 o[8];
+template <int NB>
+struct PartialT {
+  f4 o[NB];
   float m, l;
 };
+using Partial = PartialT<8>;  // head size 128
 
 // Two waves of a workgroup (half 0 and half 1) split an item's positions; the
 // half-1 wave hands its partial to its half-0 partner through `xfer` (LDS of
@@ -141,7 +143,7 @@ __device__ __forceinline__ void merge_halves(Partial& p, float* __restrict__ xfe
   __syncthreads();  // the partner's region is free again
 }
 
-constexpr int kD = 128;
+constexpr int kD = 128;           // dims staged at a time
 constexpr int kTT = 32;           // positions per sub-tile
 constexpr int kKP = kD + 8;       // K row pitch (elements): rows stay 16-byte aligned
 constexpr int kKW = kTT / 8 + 1;  // key words of one dim covering a sub-tile (8-aligned start)
@@ -183,8 +185,11 @@ struct Rows8 {
 // c ^ 2 (r % 4)) and reach the PV MFMAs through transposing reads.  Int4 values
 // inside a tail (a value side without a window) are loaded and dequantized
 // where they are staged.
-template <typename T>
-__device__ __forceinline__ Partial tail_item(char* __restrict__ lds_raw, const T* __restrict__ query,
+// NH: the head size in 128-dim halves.  The halves of a sub-tile are staged one
+// after the other over the same LDS (scores add up over them, then each half's
+// values meet the probabilities), "the next sub-tile" above being the next half.
+template <typename T, int NH = 1>
+__device__ __forceinline__ PartialT<8 * NH> tail_item(char* __restrict__ lds_raw, const T* __restrict__ query,
                                           int hq, int kvh, float qscale,
                                           const uint32_t* __restrict__ kq,
                                           const float* __restrict__ ks,
@@ -199,6 +204,7 @@ __device__ __forceinline__ Partial tail_item(char* __restrict__ lds_raw, const T
                                           const T* __restrict__ ring_v, int ring_len,
                                           int half, int nhalf) {
   constexpr int D = kD;
+  constexpr int DT = NH * kD;  // the head size
   uint16_t* sk = reinterpret_cast<uint16_t*>(lds_raw);  // [kTT][kKP] int4 key hi parts
   uint16_t* skl = sk + kTT * kKP;                        // [kTT][kKP] int4 key lo parts
   char* sv = lds_raw;                                    // [kTT][D] value rows, after the scores
@@ -227,16 +233,16 @@ __device__ __forceinline__ Partial tail_item(char* __restrict__ lds_raw, const T
   // lane 0 of the request's ring row for head h; lanes lie 32-bit byte offsets
   // past it (a ring row of all heads is under 4 GiB), a uniform base plus a
   // lane offset per load
-  const char* rk_base = reinterpret_cast<const char*>(ring_k + (ring_row0 * kvh + h) * D);
-  const char* rv_base = reinterpret_cast<const char*>(ring_v + (ring_row0 * kvh + h) * D);
+  const char* rk_base = reinterpret_cast<const char*>(ring_k + (ring_row0 * kvh + h) * DT);
+  const char* rv_base = reinterpret_cast<const char*>(ring_v + (ring_row0 * kvh + h) * DT);
 
   // B operand of QK: q[head n][32*s4 + 8*kg + i], raw (the scale is applied in fp32)
-  u8v qb[4];
+  u8v qb[4 * NH];
   {
     const bool live = n < rep;
-    const T* qrow = query + (static_cast<int64_t>(b) * hq + h * rep + (live ? n : 0)) * D;
+    const T* qrow = query + (static_cast<int64_t>(b) * hq + h * rep + (live ? n : 0)) * DT;
 #pragma unroll
-    for (int s4 = 0; s4 < 4; ++s4) {
+    for (int s4 = 0; s4 < 4 * NH; ++s4) {
       const uint4 v = *reinterpret_cast<const uint4*>(qrow + 32 * s4 + 8 * kg);
       qb[s4] = __builtin_bit_cast(u8v, live ? v : make_uint4(0, 0, 0, 0));
     }
@@ -268,7 +274,7 @@ __device__ __forceinline__ Partial tail_item(char* __restrict__ lds_raw, const T
   };
   // int4 key words, scales and minima of positions [p, p + mk): the kKW words
   // of each of the lane's two dims (clamped into the range: every load valid)
-  auto load_key_words = [&](int p, int32_t pg, KeyWords& kw) {
+  auto load_key_words = [&](int p, int32_t pg, int hf, KeyWords& kw) {
     const int mk = count(p, khist);
     if (mk == 0) return;  // uniform
     const int first = p & ~7;
@@ -280,7 +286,7 @@ __device__ __forceinline__ Partial tail_item(char* __restrict__ lds_raw, const T
     for (int k = 0; k < kKW; ++k) {
       const int q = first + 8 * k;
       const int qq = q < p ? p : (q < p + mk ? q : p + mk - 1);
-      const int64_t r = (page_uniform(pg, p, qq) * kvh + h) * D;
+      const int64_t r = (page_uniform(pg, p, qq) * kvh + h) * DT + hf * D;
       const char* wb = reinterpret_cast<const char*>(kq + r * wpd + ((qq & (bs - 1)) >> 3));
       kw.w[0][k] = *reinterpret_cast<const uint32_t*>(wb + wo);
       kw.w[1][k] = *reinterpret_cast<const uint32_t*>(wb + wo + 4 * wpd);
@@ -288,7 +294,8 @@ __device__ __forceinline__ Partial tail_item(char* __restrict__ lds_raw, const T
 #pragma unroll
     for (int s = 0; s < 2; ++s) {  // the groups of positions p and p + mk - 1
       const int qq = s ? p + mk - 1 : p;
-      const int64_t r = (page_uniform(pg, p, qq) * kvh + h) * D * gpb + ((qq & (bs - 1)) >> gsh);
+      const int64_t r = ((page_uniform(pg, p, qq) * kvh + h) * DT + hf * D) * gpb +
+                        ((qq & (bs - 1)) >> gsh);
       const char* sb = reinterpret_cast<const char*>(ks + r);
       const char* mb = reinterpret_cast<const char*>(km + r);
       kw.sc[0][s] = *reinterpret_cast<const float*>(sb + so);
@@ -300,7 +307,7 @@ __device__ __forceinline__ Partial tail_item(char* __restrict__ lds_raw, const T
   // ring key rows: slot 4*jm + s4 holds row 16*jm + n of the sub-tile, dims
   // 32*s4 + 8*kg .. + 7; rows outside [mk, nt) read a row in the ring and are
   // not staged
-  auto load_ring_keys = [&](int p) {
+  auto load_ring_keys = [&](int p, int hf) {
     const int nt = (pe - p) < kTT ? (pe - p) : kTT;
     const int mk = count(p, khist);
     Rows8 kr;
@@ -309,7 +316,7 @@ __device__ __forceinline__ Partial tail_item(char* __restrict__ lds_raw, const T
       const int pi = 16 * jm + n;
       const int pc = pi < mk ? mk : (pi < nt ? pi : nt - 1);
       const int rl = ring_lane(kfirst + (p + pc - khist), ring_len);
-      const uint32_t off = static_cast<uint32_t>((rl * kvh * D + 8 * kg) * 2);
+      const uint32_t off = static_cast<uint32_t>((rl * kvh * DT + hf * D + 8 * kg) * 2);
 #pragma unroll
       for (int s4 = 0; s4 < 4; ++s4)
         kr.r[4 * jm + s4] = *reinterpret_cast<const w4*>(rk_base + off + 64 * s4);
@@ -317,7 +324,7 @@ __device__ __forceinline__ Partial tail_item(char* __restrict__ lds_raw, const T
     return kr;
   };
   // ring value rows: slot k holds row (lane / 16) + 4k, chunk lane % 16
-  auto load_ring_values = [&](int p) {
+  auto load_ring_values = [&](int p, int hf) {
     const int nt = (pe - p) < kTT ? (pe - p) : kTT;
     const int mv = count(p, vhist);
     Rows8 vr;
@@ -326,16 +333,17 @@ __device__ __forceinline__ Partial tail_item(char* __restrict__ lds_raw, const T
       const int pi = kg + 4 * k;
       const int pc = pi < mv ? mv : (pi < nt ? pi : nt - 1);
       const int rl = ring_lane(vfirst + (p + pc - vhist), ring_len);
-      vr.r[k] = *reinterpret_cast<const w4*>(rv_base + static_cast<uint32_t>((rl * kvh * D + 8 * n) * 2));
+      vr.r[k] = *reinterpret_cast<const w4*>(
+          rv_base + static_cast<uint32_t>((rl * kvh * DT + hf * D + 8 * n) * 2));
     }
     return vr;
   };
 
   float m_run = -INFINITY;
   float l_run = 0.0f;
-  f4 o_acc[8];
+  f4 o_acc[8 * NH];
 #pragma unroll
-  for (int q = 0; q < 8; ++q) o_acc[q] = f4{0.f, 0.f, 0.f, 0.f};
+  for (int q = 0; q < 8 * NH; ++q) o_acc[q] = f4{0.f, 0.f, 0.f, 0.f};
 
   const int step = kTT * nhalf;
   const int p_first = pb + kTT * half;
@@ -343,8 +351,8 @@ __device__ __forceinline__ Partial tail_item(char* __restrict__ lds_raw, const T
   Rows8 vr;
   int32_t pg_cur = load_pages(p_first);
   if (p_first < pe) {  // uniform
-    load_key_words(p_first, pg_cur, kw);
-    vr = load_ring_values(p_first);
+    load_key_words(p_first, pg_cur, 0, kw);
+    vr = load_ring_values(p_first, 0);
   }
   int32_t pg_next = load_pages(p_first + step);
 
@@ -360,8 +368,11 @@ __device__ __forceinline__ Partial tail_item(char* __restrict__ lds_raw, const T
     const int mk = __builtin_amdgcn_readfirstlane(count(p0, khist));
     const int mv = __builtin_amdgcn_readfirstlane(count(p0, vhist));
     const int p1 = p0 + step;
+    f4 sacc[kTT / 16];
+#pragma unroll
+    for (int hf = 0; hf < NH; ++hf) {
     // the ring key rows, in flight while the int4 keys are staged
-    const Rows8 kr = load_ring_keys(p0);
+    const Rows8 kr = load_ring_keys(p0, hf);
     // one wave: its LDS accesses take effect in program order, so the previous
     // sub-tile's reads are done before these writes
     // ---- key rows: int4 rows [0, mk) as hi and lo parts, ring rows [mk, nt)
@@ -407,20 +418,19 @@ __device__ __forceinline__ Partial tail_item(char* __restrict__ lds_raw, const T
       }
     }
     // ---- scores: S^T[token][head] for kTT/16 x 16 tokens ------------------------
-    f4 sacc[kTT / 16];
     // the key lo parts exist only for int4 keys: one uniform branch for the block
     auto scores = [&](auto with_lo) {
 #pragma unroll
       for (int jm = 0; jm < kTT / 16; ++jm) {
-        sacc[jm] = f4{0.f, 0.f, 0.f, 0.f};
+        if (hf == 0) sacc[jm] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int s4 = 0; s4 < 4; ++s4) {
           const int o = (16 * jm + n) * kKP + 32 * s4 + 8 * kg;
           const u8v a = *reinterpret_cast<const u8v*>(sk + o);
-          sacc[jm] = mfma16(a, qb[s4], sacc[jm], T{});
+          sacc[jm] = mfma16(a, qb[4 * hf + s4], sacc[jm], T{});
           if constexpr (decltype(with_lo)::value) {
             const u8v al = *reinterpret_cast<const u8v*>(skl + o);
-            sacc[jm] = mfma16(al, qb[s4], sacc[jm], T{});
+            sacc[jm] = mfma16(al, qb[4 * hf + s4], sacc[jm], T{});
           }
         }
       }
@@ -429,7 +439,11 @@ __device__ __forceinline__ Partial tail_item(char* __restrict__ lds_raw, const T
       scores(std::true_type{});
     else
       scores(std::false_type{});
-    if (p1 < pe) load_key_words(p1, pg_next, kw);  // uniform: the next sub-tile's int4 keys
+    if (hf + 1 < NH)
+      load_key_words(p0, pg_cur, hf + 1, kw);  // this sub-tile's next half
+    else if (p1 < pe)
+      load_key_words(p1, pg_next, 0, kw);  // uniform: the next sub-tile's int4 keys
+    }  // key halves
     float tmax = -INFINITY;
 #pragma unroll
     for (int jm = 0; jm < kTT / 16; ++jm) {
@@ -460,9 +474,11 @@ __device__ __forceinline__ Partial tail_item(char* __restrict__ lds_raw, const T
     for (int r = 0; r < 4; ++r) {
       const float ar = __shfl(alpha, 4 * kg + r, 64);
 #pragma unroll
-      for (int q = 0; q < 8; ++q) o_acc[q][r] *= ar;
+      for (int q = 0; q < 8 * NH; ++q) o_acc[q][r] *= ar;
     }
 
+#pragma unroll
+    for (int hf = 0; hf < NH; ++hf) {
     // ---- value rows into LDS (over the consumed key rows) -----------------------
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
@@ -479,9 +495,10 @@ __device__ __forceinline__ Partial tail_item(char* __restrict__ lds_raw, const T
         if (pi < mv) {
           const int p = p0 + pi;
           const int64_t vrow = ((blk << bsh) + (p & (bs - 1))) * kvh + h;
-          const uint32_t w = vq[vrow * (D / 8) + n];
-          const float sc = vs[vrow * (D >> gsh) + ((8 * n) >> gsh)];
-          const float mn = vm[vrow * (D >> gsh) + ((8 * n) >> gsh)];
+          const int c = hf * D + 8 * n;  // first dim of the lane's word
+          const uint32_t w = vq[vrow * (DT / 8) + hf * (D / 8) + n];
+          const float sc = vs[vrow * (DT >> gsh) + (c >> gsh)];
+          const float mn = vm[vrow * (DT >> gsh) + (c >> gsh)];
           uint32_t q[4];
 #pragma unroll
           for (int i = 0; i < 4; ++i)
@@ -518,29 +535,35 @@ __device__ __forceinline__ Partial tail_item(char* __restrict__ lds_raw, const T
                         static_cast<uint16_t>(part[0][2]), static_cast<uint16_t>(part[0][3]),
                         static_cast<uint16_t>(part[1][0]), static_cast<uint16_t>(part[1][1]),
                         static_cast<uint16_t>(part[1][2]), static_cast<uint16_t>(part[1][3])};
-        o_acc[q] = mfma16(ahi, bv, o_acc[q], T{});
-        o_acc[q] = mfma16(alo, bv, o_acc[q], T{});
+        o_acc[8 * hf + q] = mfma16(ahi, bv, o_acc[8 * hf + q], T{});
+        o_acc[8 * hf + q] = mfma16(alo, bv, o_acc[8 * hf + q], T{});
       }
     }
-    // the next sub-tile's values, then the block-table rows of the one after
-    if (p1 < pe) vr = load_ring_values(p1);
+    // the next values (this sub-tile's next half, or the next sub-tile), then the
+    // block-table rows of the one after
+    if (hf + 1 < NH)
+      vr = load_ring_values(p0, hf + 1);
+    else if (p1 < pe)
+      vr = load_ring_values(p1, 0);
+    }  // value halves
     pg_cur = pg_next;
     pg_next = load_pages(p1 + step);
   }
 
-  Partial res;
+  PartialT<8 * NH> res;
 #pragma unroll
-  for (int q = 0; q < 8; ++q) res.o[q] = o_acc[q];
+  for (int q = 0; q < 8 * NH; ++q) res.o[q] = o_acc[q];
   res.m = m_run;
   res.l = l_run;
   return res;
 }
 
-// Writes a tail partial for heads 0..rep-1 of kv head h's group: o[q][r] is
+// Writes a partial for heads 0..rep-1 of kv head h's group: o[q][r] is
 // O[head 4*kg + r][dim 16*q + n].
-__device__ __forceinline__ void tail_store(const Partial& p, int wi, int hq, int h, int rep,
-                                           int lane, float* __restrict__ ws_o,
-                                           float* __restrict__ ws_ml) {
+template <int NB>
+__device__ __forceinline__ void store_o(const PartialT<NB>& p, int wi, int hq, int h, int rep,
+                                        int lane, float* __restrict__ ws_o,
+                                        float* __restrict__ ws_ml) {
   const int n = lane & 15;
   const int kg = lane >> 4;
   const int64_t head0 = static_cast<int64_t>(wi) * hq + h * rep;
@@ -549,13 +572,18 @@ __device__ __forceinline__ void tail_store(const Partial& p, int wi, int hq, int
     const int hh = 4 * kg + r;
     if (hh < rep) {
 #pragma unroll
-      for (int q = 0; q < 8; ++q) ws_o[(head0 + hh) * kD + 16 * q + n] = p.o[q][r];
+      for (int q = 0; q < NB; ++q) ws_o[(head0 + hh) * (16 * NB) + 16 * q + n] = p.o[q][r];
     }
   }
   if (kg == 0 && n < rep) {
     ws_ml[2 * (head0 + n)] = p.m;
     ws_ml[2 * (head0 + n) + 1] = p.l;
   }
+}
+__device__ __forceinline__ void tail_store(const Partial& p, int wi, int hq, int h, int rep,
+                                           int lane, float* __restrict__ ws_o,
+                                           float* __restrict__ ws_ml) {
+  store_o<8>(p, wi, hq, h, rep, lane, ws_o, ws_ml);
 }
 
 }  // namespace tail

@@ -96,36 +96,37 @@ __device__ __forceinline__ v2i read_tr4(uint32_t off) {
   return __builtin_amdgcn_ds_read_tr4_b64_v2i32((lds_v2i_ptr)(uintptr_t)(off));
 }
 
-// Tile layout in 32-bit words (a wave's buffer is 64-byte aligned).
+// Tile layout in 32-bit words for head size D (128 or 256; a wave's buffer is
+// D/2-byte aligned).
 //   KW  key words in 16-byte slots: dim d's 32-token half h (two 16-token
 //       runs) at slot 2d + (h ^ ((d >> 2) & 1)).  A score read names 16
 //       consecutive dims at one run offset; the xor puts them on 8 different
 //       16-byte bank offsets.
 //   KS, KM  the key group's scale and minimum per dim, dim order.
-//   VW  value words: token t's 16-byte chunk c at slot 4t + (c ^ pi(t)),
-//       pi(t) = ((t >> 4) & 3) ^ ((t >> 1) & 1); a PV read names the 16
-//       tokens of a lane group (t = 16 jm + 4 g + r), which pi spreads over 8
-//       bank offsets.
+//   VW  value words: token t's 16-byte chunk c at slot (D/32) t + (c ^ pi(t)),
+//       pi(t) = ((t >> 4) & 3) ^ ((t >> 1) & 1) at D = 128 and 2 ((t >> 4) & 3)
+//       + ((t >> 1) & 1) at D = 256; a PV read names the 16 tokens of a lane
+//       group (t = 16 jm + 4 g + r), which pi spreads over 8 (16) bank offsets.
 //   VS, VM  [vg][s][g][i]: scale / min of value group vg of token
 //       tau(g, 8 s + slot_nib(i)), the token of PV slot i in k-step s for
 //       lane group g (tau(g, j) = 16 (j >> 2) + 4 g + (j & 3)).
-template <int NVG, bool KSV>
+template <int NVG, bool KSV, int DD = 128>
 struct Tile {
-  static constexpr int D = 128;
+  static constexpr int D = DD;
   static constexpr int GT = 64;
   static constexpr int KW = 0;
-  static constexpr int KS = KW + 1024;
-  static constexpr int KM = KS + 128;
-  static constexpr int VW = KM + 128;
-  static constexpr int VS = VW + 1024;
+  static constexpr int KS = KW + 8 * D;
+  static constexpr int KM = KS + D;
+  static constexpr int VW = KM + D;
+  static constexpr int VS = VW + 8 * D;
   static constexpr int VM = VS + 64 * NVG;
   static constexpr int WORDS = VM + 64 * NVG;
   static constexpr int BYTES = 4 * WORDS;
-  static_assert(BYTES % 64 == 0 && (4 * VW) % 64 == 0, "swizzle alignment");
+  static_assert(BYTES % (D / 2) == 0 && (4 * VW) % (D / 2) == 0, "swizzle alignment");
   // DMA instructions per tile (the waits count them)
-  static constexpr int KW_INST = 4;                  // 16-byte lanes
-  static constexpr int VW_INST = 4;                  // 16-byte lanes
-  static constexpr int KS_DMA = KSV ? 1 : 4;         // scale + min
+  static constexpr int KW_INST = D / 32;             // 16-byte lanes
+  static constexpr int VW_INST = D / 32;             // 16-byte lanes
+  static constexpr int KS_DMA = KSV ? D / 128 : D / 32;  // scale + min
   static constexpr int VS_DMA = 2 * NVG;             // 4-byte lanes, scale + min
   static constexpr int NINST = KW_INST + VW_INST + KS_DMA + VS_DMA;
   static constexpr int NINST_CONT = NINST - KS_DMA;  // same key group as the previous tile
@@ -204,31 +205,29 @@ __device__ __forceinline__ void issue_tile(char* buf, const LaneDma& ld, const u
 // pairs (16 VGPRs instead of 32 across the item) and widen where a key group
 // is prepared; bf16 pairs are pre-scaled (a bf16 exponent change is exact),
 // fp16 pairs scale in the widening fma.  Lanes past the group hold 0.
-template <typename TQ>
-struct QLane {
-  uint32_t w[4][4];  // pair p of k-step s: slots 2p (low half) and 2p + 1
-  __device__ __forceinline__ f2 get(int s, int p) const;
-};
-template <>
-__device__ __forceinline__ f2 QLane<bf16>::get(int s, int p) const {
+__device__ __forceinline__ f2 widen_pair(uint32_t w, int, bf16) {
   float lo, hi;
-  asm volatile("v_lshlrev_b32 %0, 16, %1" : "=v"(lo) : "v"(w[s][p]));
-  asm volatile("v_and_b32 %0, 0xffff0000, %1" : "=v"(hi) : "v"(w[s][p]));
+  asm volatile("v_lshlrev_b32 %0, 16, %1" : "=v"(lo) : "v"(w));
+  asm volatile("v_and_b32 %0, 0xffff0000, %1" : "=v"(hi) : "v"(w));
   return f2{lo, hi};
 }
-template <>
-__device__ __forceinline__ f2 QLane<f16>::get(int s, int p) const {
+__device__ __forceinline__ f2 widen_pair(uint32_t w, int p, f16) {
   // fp16 -> fp32 times 1 or 1/16, exact: x * c + 0 in the mixed-precision fma
   const float c = (p & 1) ? 0.0625f : 1.0f;
   float lo, hi;
-  asm volatile("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,0,0]" : "=v"(lo) : "v"(w[s][p]), "v"(c));
+  asm volatile("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,0,0]" : "=v"(lo) : "v"(w), "v"(c));
   asm volatile("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
                : "=v"(hi)
-               : "v"(w[s][p]), "v"(c));
+               : "v"(w), "v"(c));
   return f2{lo, hi};
 }
+template <typename TQ, int D = 128>
+struct QLane {
+  uint32_t w[D / 32][4];  // pair p of k-step s: slots 2p (low half) and 2p + 1
+  __device__ __forceinline__ f2 get(int s, int p) const { return widen_pair(w[s][p], p, TQ{}); }
+};
 template <>
-struct QLane<float> {
+struct QLane<float, 128> {
   float q[4][8];
   __device__ __forceinline__ f2 get(int s, int p) const { return f2{q[s][2 * p], q[s][2 * p + 1]}; }
 };
@@ -238,15 +237,15 @@ __device__ __forceinline__ uint16_t bits16(TQ x) {
   return __builtin_bit_cast(uint16_t, x);
 }
 
-template <typename TQ>
-__device__ __forceinline__ QLane<TQ> load_q(const TQ* __restrict__ query, int b, int hq, int h,
+template <typename TQ, int D = 128>
+__device__ __forceinline__ QLane<TQ, D> load_q(const TQ* __restrict__ query, int b, int hq, int h,
                                             int rep, int n, int kg, bool fold) {
-  QLane<TQ> ql;
+  QLane<TQ, D> ql;
   const int hn = fold ? (n & 7) : n;
   const bool live = hn < rep;
-  const TQ* qrow = query + (static_cast<int64_t>(b) * hq + h * rep + (live ? hn : 0)) * 128;
+  const TQ* qrow = query + (static_cast<int64_t>(b) * hq + h * rep + (live ? hn : 0)) * D;
 #pragma unroll
-  for (int s = 0; s < 4; ++s) {
+  for (int s = 0; s < D / 32; ++s) {
     float x[8];
     load8(qrow + 64 * (s >> 1) + 16 * kg + 8 * (s & 1), x);
 #pragma unroll
@@ -278,8 +277,9 @@ __device__ __forceinline__ QLane<TQ> load_q(const TQ* __restrict__ query, int b,
 // Folded (GQA groups of at most 8 heads): column n < 8 carries head n's hi
 // part and column n + 8 its lo part, so one MFMA per k-step gives both, and
 // a rotate-by-8 add sums them.
+template <int D = 128>
 struct QGroup {
-  h8 bq[4], bl[4];
+  h8 bq[D / 32], bl[D / 32];
   float kb;
 };
 
@@ -309,39 +309,44 @@ __device__ __forceinline__ float add_ror8(float x) {
   return x + __int_as_float(y);
 }
 
-template <typename TQ, int NVG, bool KSV, bool FOLD>
+template <typename TQ, int NVG, bool KSV, bool FOLD, int D = 128>
 __device__ __forceinline__ void prepare_group(const uint32_t* W, int n, int kg,
-                                              const QLane<TQ>& ql, float qscale, QGroup& qg) {
+                                              const QLane<TQ, D>& ql, float qscale,
+                                              QGroup<D>& qg) {
 #pragma clang fp contract(fast)
-  using T = Tile<NVG, KSV>;
+  using T = Tile<NVG, KSV, D>;
+  constexpr int KS = D / 32;
   const float* ksf = reinterpret_cast<const float*>(W + T::KS);
   const float* kmf = reinterpret_cast<const float*>(W + T::KM);
-  // the lane's 32 scales and minima (dims 64 P + 16 kg + 8 e + 0..7), all
-  // read before any is used
-  f4 sc[4][2], mn[4][2];
-#pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    const int base = 64 * (s >> 1) + 16 * kg + 8 * (s & 1);
-    sc[s][0] = *reinterpret_cast<const f4*>(ksf + base);
-    sc[s][1] = *reinterpret_cast<const f4*>(ksf + base + 4);
-    mn[s][0] = *reinterpret_cast<const f4*>(kmf + base);
-    mn[s][1] = *reinterpret_cast<const f4*>(kmf + base + 4);
-  }
   // folded: lo lanes (n >= 8) take x - hi, hi lanes x - 0
   const float nsel = (FOLD && n >= 8) ? -1.0f : 0.0f;
   const h2 one2 = h2{1.0f16, 1.0f16};
   // one partial sum per k-step: four short chains instead of one long one
-  float kb_u[4], kb_p[4], off[4];
+  float kb_u[KS], kb_p[KS], off[KS];
+  // 128 dims at a time: the lane's 32 scales and minima (dims 64 P + 16 kg +
+  // 8 e + 0..7), all read before any is used
+  f4 sc[4][2], mn[4][2];
 #pragma unroll
-  for (int s = 0; s < 4; ++s) {
+  for (int s = 0; s < KS; ++s) {
+    if (s % 4 == 0) {
+      if (s > 0) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int base = 64 * ((s + i) >> 1) + 16 * kg + 8 * (i & 1);
+        sc[i][0] = *reinterpret_cast<const f4*>(ksf + base);
+        sc[i][1] = *reinterpret_cast<const f4*>(ksf + base + 4);
+        mn[i][0] = *reinterpret_cast<const f4*>(kmf + base);
+        mn[i][1] = *reinterpret_cast<const f4*>(kmf + base + 4);
+      }
+    }
     kb_u[s] = kb_p[s] = off[s] = 0.0f;
     uint32_t ph[4], pl[4];
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
       const int d0 = slot_nib(2 * p), d1 = slot_nib(2 * p + 1);
       const f2 q = ql.get(s, p);
-      const float s0 = sc[s][d0 >> 2][d0 & 3], s1 = sc[s][d1 >> 2][d1 & 3];
-      const float m0 = mn[s][d0 >> 2][d0 & 3], m1 = mn[s][d1 >> 2][d1 & 3];
+      const float s0 = sc[s % 4][d0 >> 2][d0 & 3], s1 = sc[s % 4][d1 >> 2][d1 & 3];
+      const float m0 = mn[s % 4][d0 >> 2][d0 & 3], m1 = mn[s % 4][d1 >> 2][d1 & 3];
       const float x0 = q[0] * s0;
       const float x1 = q[1] * s1;
       if (p & 1)
@@ -365,6 +370,12 @@ __device__ __forceinline__ void prepare_group(const uint32_t* W, int n, int kg,
     if (!FOLD) qg.bl[s] = as_h8(pl[0], pl[1], pl[2], pl[3]);
   }
   // primed q are q / 16: their minima term is 16 * kb_p
+#pragma unroll
+  for (int s = 4; s < KS; ++s) {
+    kb_u[s & 3] += kb_u[s];
+    kb_p[s & 3] += kb_p[s];
+    off[s & 3] += off[s];
+  }
   const float kb = sum_kg((kb_u[0] + kb_u[1]) + (kb_u[2] + kb_u[3]) +
                           16.0f * ((kb_p[0] + kb_p[1]) + (kb_p[2] + kb_p[3])));
   float offs = sum_kg((off[0] + off[1]) + (off[2] + off[3]));
@@ -375,17 +386,17 @@ __device__ __forceinline__ void prepare_group(const uint32_t* W, int n, int kg,
 // Running state of one wave: softmax max / sum (log2 domain), the PV
 // accumulators o_acc[v] (dims 16 v + column), the constant-B MFMA sums that
 // remove the 1024 offset (one per value group), and the value-minima term.
-template <int NVG>
+template <int NVG, int DB = 8>
 struct Acc {
   float m_run, l_run;
-  f4 o_acc[8];
+  f4 o_acc[DB];
   f4 c_acc[NVG];
   float bias_v[NVG];
   __device__ __forceinline__ void init() {
     m_run = -INFINITY;
     l_run = 0.0f;
 #pragma unroll
-    for (int q = 0; q < 8; ++q) o_acc[q] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int q = 0; q < DB; ++q) o_acc[q] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int v = 0; v < NVG; ++v) {
       c_acc[v] = f4{0.f, 0.f, 0.f, 0.f};
@@ -401,31 +412,35 @@ struct Acc {
 __device__ __forceinline__ uint32_t key_read_base(uint32_t buf_off, int n, int kg) {
   return buf_off + 4 * Tile<1, false>::KW + 32 * (16 * kg + n) + 16 * ((n >> 2) & 1);
 }
+template <int D = 128>
 __device__ __forceinline__ uint32_t val_read_base(uint32_t buf_off, int n, int kg) {
   const int t = tau(kg, n);
-  const int pi = ((t >> 4) & 3) ^ ((t >> 1) & 1);
-  return buf_off + 4 * Tile<1, false>::VW + 64 * t + 16 * pi;
+  const int hi = (t >> 4) & 3, lo = (t >> 1) & 1;
+  const int pi = D == 128 ? hi ^ lo : 2 * hi + lo;
+  return buf_off + 4 * Tile<1, false, D>::VW + (D / 2) * t + 16 * pi;
 }
 
-// One tile: scores, softmax update and PV.  FULL: every token < pe.
+// One tile: scores, softmax update and PV.  FULL: every token in [pb, pe); else
+// at least one is.
 // Order: all eight key reads, the score MFMAs (the second k-step pair's reads
 // land behind the first pair's MFMAs), then all eight value reads, which land
 // behind the softmax; the PV MFMAs run k-step outer, so consecutive MFMAs
 // write different accumulators.
-template <int NVG, bool KSV, bool FOLD, bool FULL>
-__device__ __forceinline__ void compute_tile(const uint32_t* W, uint32_t buf_off, int p0, int pe,
-                                             int n, int kg, const QGroup& qg, float qscale,
-                                             Acc<NVG>& acc) {
+template <int NVG, bool KSV, bool FOLD, bool FULL, int D = 128>
+__device__ __forceinline__ void compute_tile(const uint32_t* W, uint32_t buf_off, int p0, int pb,
+                                             int pe, int n, int kg, const QGroup<D>& qg, float qscale,
+                                             Acc<NVG, D / 16>& acc) {
 #pragma clang fp contract(fast)
-  using T = Tile<NVG, KSV>;
-  static_assert(Tile<NVG, KSV>::KW == Tile<1, false>::KW && Tile<NVG, KSV>::VW == Tile<1, false>::VW,
+  using T = Tile<NVG, KSV, D>;
+  constexpr int DB = D / 16;
+  static_assert(T::KW == Tile<1, false>::KW && T::VW == Tile<1, false, D>::VW,
                 "read bases assume the common word offsets");
   const Consts cst;
   // ---- scores: S^T[token 16 jm + row][head] over k-steps s = 2P + e ----------------
   const uint32_t kbase = key_read_base(buf_off, n, kg);
-  v2i rk[2][4];
+  v2i rk[D / 64][4];
 #pragma unroll
-  for (int P = 0; P < 2; ++P)
+  for (int P = 0; P < D / 64; ++P)
 #pragma unroll
     for (int jm = 0; jm < 4; ++jm)
       rk[P][jm] = read_tr4(((kbase + 2048u * P) ^ (16u * (jm >> 1))) + 8u * (jm & 1));
@@ -433,7 +448,7 @@ __device__ __forceinline__ void compute_tile(const uint32_t* W, uint32_t buf_off
 #pragma unroll
   for (int j = 0; j < 4; ++j) sacc[j] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int P = 0; P < 2; ++P)
+  for (int P = 0; P < D / 64; ++P)
 #pragma unroll
     for (int e = 0; e < 2; ++e)
 #pragma unroll
@@ -445,10 +460,10 @@ __device__ __forceinline__ void compute_tile(const uint32_t* W, uint32_t buf_off
               __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qg.bl[2 * P + e], sacc[jm], 0, 0, 0);
       }
   // the value reads go out now and land while the softmax runs
-  const uint32_t vbase = val_read_base(buf_off, n, kg);
-  v2i rv[8];
+  const uint32_t vbase = val_read_base<D>(buf_off, n, kg);
+  v2i rv[DB];
 #pragma unroll
-  for (int v = 0; v < 8; ++v) rv[v] = read_tr4((vbase ^ (16u * (v >> 1))) + 8u * (v & 1));
+  for (int v = 0; v < DB; ++v) rv[v] = read_tr4((vbase ^ (16u * (v >> 1))) + 8u * (v & 1));
   __builtin_amdgcn_sched_barrier(0);
   if (FOLD) {
 #pragma unroll
@@ -464,7 +479,10 @@ __device__ __forceinline__ void compute_tile(const uint32_t* W, uint32_t buf_off
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       float sv = sacc[jm][r] * qscale + kb;
-      if (!FULL) sv = p0 + 16 * jm + 4 * kg + r < pe ? sv : -INFINITY;
+      if (!FULL) {
+        const int pos = p0 + 16 * jm + 4 * kg + r;
+        sv = pos >= pb && pos < pe ? sv : -INFINITY;
+      }
       sacc[jm][r] = sv;
     }
     tm[jm] = fmaxf(fmaxf(sacc[jm][0], sacc[jm][1]), fmaxf(sacc[jm][2], sacc[jm][3]));
@@ -489,7 +507,7 @@ __device__ __forceinline__ void compute_tile(const uint32_t* W, uint32_t buf_off
     for (int r = 0; r < 4; ++r) {
       const float ar = __shfl(alpha, 4 * kg + r, 64);
 #pragma unroll
-      for (int q = 0; q < 8; ++q) acc.o_acc[q][r] *= ar;
+      for (int q = 0; q < DB; ++q) acc.o_acc[q][r] *= ar;
 #pragma unroll
       for (int v = 0; v < NVG; ++v) acc.c_acc[v][r] *= ar;
     }
@@ -519,9 +537,10 @@ __device__ __forceinline__ void compute_tile(const uint32_t* W, uint32_t buf_off
         float sv = i < 4 ? s0[i] : s1[i - 4];
         float mv = i < 4 ? m0[i] : m1[i - 4];
         if (!FULL) {
-          // past the range p = 0, but the scale/min bytes are unwritten:
+          // outside the range p = 0, but the scale/min bytes may be unwritten:
           // select zeros so a stale NaN cannot reach the sums
-          const bool live = p0 + tau(kg, 8 * s + slot_nib(i)) < pe;
+          const int pos = p0 + tau(kg, 8 * s + slot_nib(i));
+          const bool live = pos >= pb && pos < pe;
           sv = live ? sv : 0.0f;
           mv = live ? mv : 0.0f;
         }
@@ -537,8 +556,8 @@ __device__ __forceinline__ void compute_tile(const uint32_t* W, uint32_t buf_off
       pa[vg] = as_h8(pack_h2(pp[0], pp[1]), a1, pack_h2(pp[4], pp[5]), a3);
     }
 #pragma unroll
-    for (int v = 0; v < 8; ++v) {
-      const int vg = NVG == 1 ? 0 : v / 4;
+    for (int v = 0; v < DB; ++v) {
+      const int vg = v / (DB / NVG);
       acc.o_acc[v] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
           pa[vg], codes(static_cast<uint32_t>(rv[v][s]), cst), acc.o_acc[v], 0, 0, 0);
     }
@@ -550,16 +569,16 @@ __device__ __forceinline__ void compute_tile(const uint32_t* W, uint32_t buf_off
 
 // Partial of the item for heads 4 kg + r (rows 8..15 repeat heads 0..7 when
 // folded and are not stored): o - offset + minima term.
-template <int NVG>
-__device__ __forceinline__ void finish(Acc<NVG>& acc, int kg, f4 (&o)[8]) {
+template <int NVG, int DB = 8>
+__device__ __forceinline__ void finish(Acc<NVG, DB>& acc, int kg, f4 (&o)[DB]) {
 #pragma unroll
   for (int v = 0; v < NVG; ++v) acc.bias_v[v] = sum_kg(acc.bias_v[v]);
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int hh = 4 * kg + r;
 #pragma unroll
-    for (int v = 0; v < 8; ++v) {
-      const int vg = NVG == 1 ? 0 : v / 4;
+    for (int v = 0; v < DB; ++v) {
+      const int vg = v / (DB / NVG);
       const float bv = __shfl(acc.bias_v[vg], hh, 64);
       o[v][r] = acc.o_acc[v][r] - acc.c_acc[vg][r] + bv;
     }

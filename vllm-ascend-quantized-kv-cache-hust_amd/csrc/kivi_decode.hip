@@ -298,8 +298,10 @@ namespace kvq {
 // readlane, and each lane accumulates columns lane + 64*k of sum_s w_s * o_s.
 // The o rows of the first kPre items are loaded before the (m, l) pass, so a
 // request with up to kPre items costs one round trip to memory instead of one
-// per few items.  Items with m = -inf (no position) carry weight 0 and their o
-// never reaches the sum (selected out, so stale bytes cannot turn it NaN).
+// per few items; of the others only those with weight are read, four at a time
+// (the split decode leaves most items of a long request to another's partial).
+// Items with m = -inf (no position) carry weight 0 and their o never reaches
+// the sum (selected out, so stale bytes cannot turn it NaN).
 template <typename TO, int KD>
 __global__ void __launch_bounds__(256)
 decode_combine_kernel(int hq, int d, const int32_t* __restrict__ seq_meta, int meta_stride,
@@ -369,8 +371,7 @@ decode_combine_kernel(int hq, int d, const int32_t* __restrict__ seq_meta, int m
         wsum += wgt * ls;
       }
     }
-    const int cnt = nw - s0 < 64 ? nw - s0 : 64;
-    int j0 = 0;
+    uint64_t live = __builtin_amdgcn_ballot_w64(wgt != 0.0f);
     if (s0 == 0) {
 #pragma unroll
       for (int j = 0; j < kPre; ++j) {
@@ -378,19 +379,27 @@ decode_combine_kernel(int hq, int d, const int32_t* __restrict__ seq_meta, int m
 #pragma unroll
         for (int k = 0; k < KD; ++k) acc[k] += wj != 0.0f ? wj * pre[j][k] : 0.0f;
       }
-      j0 = kPre;
+      live &= ~uint64_t{0} << kPre;
     }
     const float* row0 = rows + s0 * stride;
-#pragma unroll 4
-    for (int j = j0; j < cnt; ++j) {
-      const float wj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), j));
-      const float* row = row0 + j * stride;
+    while (live) {  // uniform; the rows with weight, in item order
+      float wj[4], x[4][KD];
 #pragma unroll
-      for (int k = 0; k < KD; ++k) {
-        const int c = lane + 64 * k;
-        const float x = row[c < d ? c : 0];  // columns past d are read in bounds, unused
-        acc[k] += wj != 0.0f ? wj * x : 0.0f;
+      for (int i = 0; i < 4; ++i) {
+        const int j = live ? __builtin_ctzll(live) : 0;
+        wj[i] = live ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), j)) : 0.0f;
+        live &= live - 1;  // 0 stays 0
+        const float* row = row0 + j * stride;
+#pragma unroll
+        for (int k = 0; k < KD; ++k) {
+          const int c = lane + 64 * k;
+          x[i][k] = row[c < d ? c : 0];  // columns past d are read in bounds, unused
+        }
       }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int k = 0; k < KD; ++k) acc[k] += wj[i] != 0.0f ? wj[i] * x[i][k] : 0.0f;
     }
   }
   wsum = sum_wave64(wsum);

@@ -439,6 +439,26 @@ inline int device_lds_max(int64_t* out) {
   return KVQ_OK;
 }
 
+// Compute units of the current device, cached per device likewise.
+inline int device_cu_count(int* out) {
+  static std::atomic<int> cache[64];
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return static_cast<int>(e);
+  if (dev < 0 || dev >= 64) {
+    *out = 0;
+    return KVQ_OK;
+  }
+  int v = cache[dev].load(std::memory_order_relaxed);
+  if (v == 0) {
+    e = hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e != hipSuccess) return static_cast<int>(e);
+    cache[dev].store(v, std::memory_order_relaxed);
+  }
+  *out = v;
+  return KVQ_OK;
+}
+
 }  // namespace kvq
 
 // Dispatch helpers for the C-ABI layer.

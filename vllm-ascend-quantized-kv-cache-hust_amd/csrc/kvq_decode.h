@@ -77,6 +77,22 @@ int launch_kivi_decode_coop(const void* query, int q_dtype, int hq, int kvh, int
                             const void* ring_v, int ring_dtype, int ring_len, float* ws_o,
                             float* ws_ml, hipStream_t s, bool* launched);
 
+// The split decode (decode_split.hip): head sizes 128 and 256, group 64 or 128,
+// pages of at least 64 positions (a power of two), GQA groups of at most 16
+// heads, 16-bit query and ring.  One wave per (pieces, kv head), four waves a
+// workgroup, merging their partials; items merged into another's partial get
+// m = -inf.  *launched tells the caller whether it ran (every kind then done).
+// Without pieces every item is one (kinds 0 and 1 only: the caller checks).
+bool split_decode_applies(int q_dtype, int hq, int kvh, int d, int ring_dtype, int bs, int g);
+int launch_kivi_decode_split(const void* query, int q_dtype, int hq, int kvh, int d, float qscale,
+                             const int32_t* kq, const float* ks, const float* km,
+                             const int32_t* vq, const float* vs, const float* vm, int bs, int g,
+                             int64_t nb, const int32_t* block_table, int64_t maxb,
+                             const int32_t* seq_meta, const int32_t* work, int64_t num_work,
+                             const int32_t* pieces, int64_t num_pieces, const void* ring_k,
+                             const void* ring_v, int ring_dtype, int ring_len, float* ws_o,
+                             float* ws_ml, hipStream_t s, bool* launched);
+
 // Standalone MFMA tail kernel for the kind-1 items, for geometries the int4
 // kernel does not cover.  *launched tells the caller whether kind-1 items still
 // need the generic kernel.
