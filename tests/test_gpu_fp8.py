@@ -229,3 +229,87 @@ def test_full_size_round_trip_of_grid_values(gpu_device):
     torch.cuda.synchronize()
     assert torch.equal(dk, x) and torch.equal(dv, x)
     assert torch.equal(views[1].view(-1, kvh)[slots], torch.exp2(k).view(t, kvh))
+
+
+def _decode_case(dev, lens, *, d, kvh, rep, bs, dtype, index, seed=5):
+    """A decode over pages whose unwritten bytes are NaN codes and scales."""
+    gen = torch.Generator().manual_seed(seed)
+    need = [-(-n // bs) for n in lens]
+    nb = sum(need) + 2
+    perm = torch.randperm(nb, generator=gen)
+    table = torch.full((len(lens), max(max(need), 1)), -1, dtype=index)
+    used = 0
+    for b, k in enumerate(need):
+        table[b, :k] = perm[used:used + k].to(index)
+        used += k
+    slots = [table[b, torch.arange(n) // bs].long() * bs + torch.arange(n) % bs
+             for b, n in enumerate(lens)]
+    _, _, views = _views(dev, nb, bs, kvh, d)
+    for i, v in enumerate(views):
+        v.fill_(0xFF if i % 2 == 0 else float("nan"))
+    x = [(torch.randn((sum(lens), kvh, d), generator=gen) * 10 ** float(e)).to(dtype)
+         for e in (0, -3)]  # small values: their scales leave the fp16 range
+    fp8_ops.fp8_per_token_head_store(x[0].to(dev), x[1].to(dev), torch.cat(slots).to(dev), *views)
+    q = torch.randn((len(lens), kvh * rep, d), generator=gen).to(dtype)
+    got = fp8_ops.fp8_per_token_head_attention(
+        q.to(dev), *views, table.to(dev), lens, [1] * len(lens), d ** -0.5,
+        block_table_host=table.numpy())
+    torch.cuda.synchronize()
+    dk, dv = ref.fp8_pth_gather(*[v.cpu() for v in views], table, lens, torch.float32)
+    live = [b for b, n in enumerate(lens) if n]
+    want = torch.zeros(q.shape)
+    want[live] = ref.attention(q[live].float(), dk, dv, [1] * len(live),
+                               [lens[b] for b in live], d ** -0.5, True)
+    # the output's rounding, on values of 1e-3
+    rel = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    torch.testing.assert_close(got.float().cpu(), want, atol=1e-3 * 2 * rel, rtol=2 * rel)
+
+
+@pytest.mark.parametrize("d,kvh,rep,bs,dtype,index", [
+    (128, 8, 4, 128, torch.bfloat16, torch.int32),   # the item's heads in one workgroup
+    (128, 1, 16, 16, torch.float16, torch.int64),
+    (128, 3, 7, 48, torch.bfloat16, torch.int64),
+    (128, 16, 1, 32, torch.float16, torch.int32),    # one wave per head
+    (256, 1, 8, 128, torch.bfloat16, torch.int32),
+    (256, 4, 5, 64, torch.float16, torch.int64),
+    (256, 8, 2, 16, torch.bfloat16, torch.int32),
+])
+def test_decode_over_paged_codes(gpu_device, d, kvh, rep, bs, dtype, index):
+    """One row per request, straight from the codes: lengths around the tile and
+    the 16-token group, an empty request, requests cut into several items."""
+    _decode_case(gpu_device, [150, 0, 1, 15, 16, 17, 31, 32, 33, 64, 700], d=d, kvh=kvh, rep=rep,
+                 bs=bs, dtype=dtype, index=index)
+
+
+def test_decode_over_paged_codes_long_request_and_large_batch(gpu_device):
+    """More requests than one launch carries, next to one of many items."""
+    lens = [9000] + [(37 * i) % 50 for i in range(800)]
+    _decode_case(gpu_device, lens, d=128, kvh=2, rep=2, bs=16, dtype=torch.bfloat16,
+                 index=torch.int32)
+
+
+def test_decode_row_forms_agree(gpu_device):
+    """Rows whose heads or tokens are strided, and an output of another dtype, give
+    the packed rows' result; a batch that is not one row per request and a
+    head size the decode does not take run the gathered path."""
+    bs, kvh, hq, nb = 16, 2, 4, 12
+    gen = torch.Generator().manual_seed(4)
+    for d in (128, 64):
+        _, _, views = _views(gpu_device, nb, bs, kvh, d)
+        x = torch.randn((nb * bs, kvh, d), generator=gen).to(torch.bfloat16).to(gpu_device)
+        fp8_ops.fp8_per_token_head_store(x, x, torch.arange(nb * bs, device=gpu_device), *views)
+        table = torch.arange(nb, device=gpu_device, dtype=torch.int32).view(3, 4)
+        lens = [50, 3, 64]
+        wide = torch.randn((3, hq, 2 * d), generator=gen).to(torch.bfloat16).to(gpu_device)
+        q = wide[:, :, ::2]
+        want = fp8_ops.fp8_per_token_head_attention(q.contiguous(), *views, table, lens, [1] * 3,
+                                                    d ** -0.5)
+        out = torch.empty((3, hq, d), dtype=torch.float32, device=gpu_device)
+        got = fp8_ops.fp8_per_token_head_attention(q, *views, table, lens, [1] * 3, d ** -0.5,
+                                                   out=out)
+        assert got is out and torch.equal(out.to(torch.bfloat16), want)
+        two = fp8_ops.fp8_per_token_head_attention(
+            torch.cat([q[:1], q]), *views, table, lens, [2, 1, 1], d ** -0.5)
+        torch.testing.assert_close(two[1:].float(), want.float(), **TOL)
+    with pytest.raises(RuntimeError, match="does not cover the longest sequence"):
+        fp8_ops.fp8_per_token_head_attention(q, *views, table, [65, 3, 64], [1] * 3, 0.1)

@@ -189,3 +189,11 @@ def test_int8_decode_with_row_maxima_growing_every_block(gpu_device, kvh, d, bs,
             v_aq.to(gpu_device), table.to(gpu_device), lens, scale, split_tokens=split,
         )
         torch.testing.assert_close(got.float().cpu(), want, atol=1e-2, rtol=1e-2)
+
+
+@pytest.mark.parametrize("rep", [1, 5, 16])
+@pytest.mark.parametrize("kvh,bs", [(1, 128), (2, 16), (8, 64)])
+def test_int8_decode_head_256_matches_oracle(gpu_device, rep, kvh, bs):
+    """Head size 256 on the MFMA kernel: heads of an item in one workgroup (1, 2)
+    and a wave per head (8), folded and unfolded GQA groups, split items."""
+    test_int8_decode_matches_oracle(gpu_device, rep, kvh, 256, bs)

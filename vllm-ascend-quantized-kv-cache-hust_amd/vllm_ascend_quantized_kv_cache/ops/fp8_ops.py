@@ -11,8 +11,10 @@ gfx950's round-to-nearest-even E4M3 conversion.
 
 The read path has no counterpart in the reference (its scheme stops at the
 store): ``fp8_per_token_head_dequant_gather`` turns paged codes into dense
-TND rows exactly as ``dequantize`` then ``.to(dtype)`` would, and
-``fp8_per_token_head_attention`` runs the MFMA attention kernel over them.
+TND rows exactly as ``dequantize`` then ``.to(dtype)`` would;
+``fp8_per_token_head_attention`` decodes (one row per request) straight from
+the paged codes (``kvq_fp8_pth_decode_attn``) and runs longer chunks on the
+MFMA attention kernel over the gathered rows.
 """
 
 from __future__ import annotations
@@ -186,25 +188,10 @@ def _check_live_blocks(rows, lens: list[int], *, max_blocks: int, num_blocks: in
             "fp8_per_token_head block_table references blocks outside the cache.")
 
 
-def fp8_per_token_head_dequant_gather(
-    k_data: torch.Tensor,
-    k_scale: torch.Tensor,
-    v_data: torch.Tensor,
-    v_scale: torch.Tensor,
-    block_table: torch.Tensor,
-    seq_lens: list[int],
-    target_dtype: torch.dtype,
-    *,
-    block_table_host=None,
-) -> tuple[torch.Tensor, torch.Tensor]:
-    """Paged E4M3 -> dense TND ``[sum seq_lens, KVH, D]`` in ``target_dtype``.
-
-    Element ``(p, h, i)`` of request ``b`` is ``float(code) * scale`` in fp32,
-    rounded to ``target_dtype``, read from slot ``block_table[b, p // Bs] * Bs
-    + p % Bs``.  Live block ids are checked on the host (``block_table_host``,
-    or the table read back once when only a device copy is given).
-    """
-    nb, bs, kvh, d = k_data.shape
+def _check_paged_read(k_data, k_scale, v_data, v_scale, block_table, seq_lens,
+                      block_table_host) -> tuple[list[int], torch.Tensor]:
+    """Checks of a read of the paged codes; ``(lengths, their table rows)``."""
+    nb, bs, kvh, _ = k_data.shape
     for name, t in (("key data", k_data), ("key scale", k_scale), ("value data", v_data),
                     ("value scale", v_scale)):
         _check_contiguous(name, t)
@@ -225,6 +212,30 @@ def fp8_per_token_head_dequant_gather(
     table = block_table[: len(lens)]
     rows = block_table_host if block_table_host is not None else table.cpu().numpy()
     _check_live_blocks(rows, lens, max_blocks=table.shape[1], num_blocks=nb, block_size=bs)
+    return lens, table
+
+
+def fp8_per_token_head_dequant_gather(
+    k_data: torch.Tensor,
+    k_scale: torch.Tensor,
+    v_data: torch.Tensor,
+    v_scale: torch.Tensor,
+    block_table: torch.Tensor,
+    seq_lens: list[int],
+    target_dtype: torch.dtype,
+    *,
+    block_table_host=None,
+) -> tuple[torch.Tensor, torch.Tensor]:
+    """Paged E4M3 -> dense TND ``[sum seq_lens, KVH, D]`` in ``target_dtype``.
+
+    Element ``(p, h, i)`` of request ``b`` is ``float(code) * scale`` in fp32,
+    rounded to ``target_dtype``, read from slot ``block_table[b, p // Bs] * Bs
+    + p % Bs``.  Live block ids are checked on the host (``block_table_host``,
+    or the table read back once when only a device copy is given).
+    """
+    nb, bs, kvh, d = k_data.shape
+    lens, table = _check_paged_read(k_data, k_scale, v_data, v_scale, block_table, seq_lens,
+                                    block_table_host)
     dev = k_data.device
     total = sum(lens)
     out_k = torch.empty((total, kvh, d), dtype=target_dtype, device=dev)
@@ -247,6 +258,55 @@ def fp8_per_token_head_dequant_gather(
     return out_k, out_v
 
 
+def _decode_applies(query, k_data, block_table, query_lens, scale) -> bool:
+    """The fused decode: one query row per request (every key then precedes it,
+    causal or not), 16-bit queries, head size 128 or 256, pages of whole
+    16-token groups, at most 16 query heads per kv head, everything on the GPU."""
+    if len(query_lens) != query.shape[0] or any(n != 1 for n in query_lens):
+        return False
+    bs, kvh, d = k_data.shape[1:]
+    hq = query.shape[1]
+    return (query.dim() == 3 and query.dtype in (torch.bfloat16, torch.float16)
+            and query.shape[2] == d and d in (128, 256) and bs % 16 == 0
+            and kvh > 0 and hq % kvh == 0 and hq // kvh <= 16 and scale > 0
+            and query.device.type == k_data.device.type == block_table.device.type == "cuda"
+            and block_table.dtype in (torch.int32, torch.int64))
+
+
+def _decode_attention(query, k_data, k_scale, v_data, v_scale, block_table, seq_lens, scale, out,
+                      block_table_host) -> torch.Tensor:
+    nb, bs, kvh, d = k_data.shape
+    batch, hq = query.shape[:2]
+    if out is None:
+        out = torch.empty_like(query)
+    if len(seq_lens) != batch:
+        raise ValueError(
+            f"fp8_per_token_head_attention: {batch} query rows, {len(seq_lens)} lengths")
+    if batch == 0:
+        return out
+    lens, table = _check_paged_read(k_data, k_scale, v_data, v_scale, block_table, seq_lens,
+                                    block_table_host)
+    _native.require_gpu_tensors("fp8_per_token_head_attention", k_scale, v_data, v_scale, out)
+    q = query.contiguous()
+    table = table.contiguous()
+    target = out if out.is_contiguous() and out.dtype == q.dtype else torch.empty_like(q)
+    lib = _native.lib()
+    lens_np = np.array(lens, dtype=np.int64)
+    nbytes = int(lib.kvq_fp8_pth_decode_workspace_bytes(lens_np.ctypes.data, batch, hq, kvh, d, bs))
+    _native.check(nbytes if nbytes < 0 else 0, "kvq_fp8_pth_decode_workspace_bytes")
+    ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=q.device)
+    rc = lib.kvq_fp8_pth_decode_attn(
+        _native.ptr(q), _native.dtype_code(q.dtype), batch, hq, kvh, d, float(scale),
+        _native.ptr(k_data), _native.ptr(k_scale), _native.ptr(v_data), _native.ptr(v_scale), nb,
+        bs, _native.ptr(table), _native.index_code(table.dtype), table.shape[1],
+        lens_np.ctypes.data, _native.ptr(ws), _native.ptr(target), _native.stream_of(q),
+    )
+    _native.check(rc, "kvq_fp8_pth_decode_attn")
+    if target is not out:
+        out.copy_(target)
+    return out
+
+
 def fp8_per_token_head_attention(
     query: torch.Tensor,
     k_data: torch.Tensor,
@@ -265,6 +325,9 @@ def fp8_per_token_head_attention(
     """Attention of TND ``query [sum query_lens, Hq, D]`` over the paged E4M3
     history: each request's rows are its last ``query_lens[b]`` positions of
     ``seq_lens[b]`` (decode: ``query_lens`` all 1)."""
+    if _decode_applies(query, k_data, block_table, query_lens, scale):
+        return _decode_attention(query, k_data, k_scale, v_data, v_scale, block_table, seq_lens,
+                                 scale, out, block_table_host)
     from .attention import prefill_attention
 
     key, value = fp8_per_token_head_dequant_gather(
