@@ -297,11 +297,11 @@ int kvq_prefill_attn(const void* query, const void* key, const void* value, int 
                      int head_size, float scale, int causal, void* out, void* stream);
 
 /* Host-side (no GPU call): the plan of kvq_prefill_attn_planned for a batch of
- * q_lens / kv_lens (int64 [batch]), int32 [2 (batch + 1) + 2 units] in `plan`:
- * cu_seqlens_q, cu_seqlens_k, then (request, tile) of every 128-row tile (a row
- * is one query of one head of a GQA group) in the order they should start.
+ * q_lens / kv_lens (int64 [batch]), int32 [2 (batch + 1) + units] in `plan`:
+ * cu_seqlens_q, cu_seqlens_k, then request | tile << 16 of every 128-row tile (a
+ * row is one query of one head of a GQA group) in the order they should start.
  * Returns the number of tiles (units), KVQ_ERR_CAPACITY when they exceed
- * cap_units, or KVQ_ERR_INVALID. */
+ * cap_units or a tile's 16 bits, or KVQ_ERR_INVALID. */
 int64_t kvq_plan_prefill_attn(const int64_t* q_lens, const int64_t* kv_lens, int64_t batch,
                               int num_heads, int num_kv_heads, int head_size, int causal,
                               int32_t* plan, int64_t cap_units);
@@ -313,6 +313,22 @@ int kvq_prefill_attn_planned(const void* query, const void* key, const void* val
                              const int32_t* plan, int64_t batch, int64_t num_units,
                              int num_heads, int num_kv_heads, int head_size, float scale,
                              int causal, void* out, void* stream);
+
+/* kvq_prefill_attn with the lengths on the host (int64 [batch], read during the
+ * call): the plan travels with the launch, nothing is copied to the device.
+ * Calls of few tiles over long keys cut each tile's keys into segments, whose
+ * partial results go to `workspace` (kvq_prefill_attn_lens_workspace_bytes for
+ * the same arguments: 0 when the keys stay whole, as they do with a smaller
+ * workspace), and merge them.  Geometry as kvq_prefill_attn_planned; batches
+ * whose plan does not fit a launch return KVQ_ERR_CAPACITY before anything is
+ * launched. */
+int64_t kvq_prefill_attn_lens_workspace_bytes(const int64_t* q_lens, const int64_t* kv_lens,
+                                              int64_t batch, int num_heads, int num_kv_heads,
+                                              int head_size, int causal);
+int kvq_prefill_attn_lens(const void* query, const void* key, const void* value, int dtype,
+                          const int64_t* q_lens, const int64_t* kv_lens, int64_t batch,
+                          int num_heads, int num_kv_heads, int head_size, float scale, int causal,
+                          void* workspace, int64_t workspace_bytes, void* out, void* stream);
 
 /* ---- INT8 dynamic per-channel ------------------------------------------- */
 

@@ -29,7 +29,7 @@ def test_plan_covers_every_tile_once(hq, kvh, d, q_lens, kv_lens, causal):
     b = len(q_lens)
     assert plan[: b + 1].tolist() == [0, *np.cumsum(q_lens)]
     assert plan[b + 1: 2 * (b + 1)].tolist() == [0, *np.cumsum(kv_lens)]
-    units = [tuple(u) for u in plan[2 * (b + 1):].reshape(-1, 2).tolist()]
+    units = [(u & 0xFFFF, u >> 16) for u in plan[2 * (b + 1):].tolist()]
     want = [(i, t) for i, m in enumerate(q_lens) for t in range(-(-m * rep // TILE_ROWS))]
     assert n == len(units) and sorted(units) == want
 
@@ -50,10 +50,38 @@ def test_plan_covers_every_tile_once(hq, kvh, d, q_lens, kv_lens, causal):
         assert cost == sorted(cost, reverse=True)
 
 
-def test_plan_refuses_unmatched_lengths():
+def test_plan_refuses_negative_lengths():
     from vllm_ascend_quantized_kv_cache.ops.attention import _plan
 
-    with pytest.raises(ValueError, match="query lengths"):
-        _plan([1, 2], [1], 8, 8, 128, True)
     with pytest.raises(RuntimeError, match="rejected"):
         _plan([1], [-1], 8, 8, 128, True)
+
+
+def test_plan_past_the_packed_range_keeps_the_lengths():
+    from vllm_ascend_quantized_kv_cache.ops.attention import _plan
+
+    many = [1] * 70000  # requests past 16 bits: the grid without a unit list
+    plan, n = _plan(many, many, 1, 1, 128, True)
+    assert n == -1
+    assert plan[:70001].tolist() == list(range(70001)) == plan[70001:].tolist()
+
+
+@pytest.mark.parametrize("q_lens,kv_lens,hq,kvh,d,cut", [
+    ([16], [8192], 8, 1, 128, True),       # one tile, long keys
+    ([16], [500], 8, 1, 128, False),       # too few blocks to cut
+    ([2048] * 8, [10240] * 8, 40, 8, 128, False),  # more tiles than slots
+    ([0, 0], [5, 5], 8, 1, 128, False),
+])
+def test_workspace_follows_the_cut(q_lens, kv_lens, hq, kvh, d, cut):
+    import ctypes
+
+    import torch
+
+    lib = _native.lib()
+    arr = ctypes.c_int64 * len(q_lens)
+    got = lib.kvq_prefill_attn_lens_workspace_bytes(arr(*q_lens), arr(*kv_lens), len(q_lens), hq,
+                                                    kvh, d, 1)
+    if torch.cuda.is_available() or not cut:
+        # partial rows of whole tiles, D + 2 floats each (without a GPU: no cut)
+        assert (got > 0) == cut if got != _native.KVQ_ERR_CAPACITY else not cut
+        assert got <= 0 or got % (128 * (d + 2) * 4) == 0

@@ -124,3 +124,44 @@ def test_prefill_attention_head_rows_across_tiles(gpu_device, d, hq, kvh):
         _native.stream_of(qg))
     assert rc == 0
     torch.testing.assert_close(out, got, atol=0, rtol=0)
+
+
+@pytest.mark.parametrize("d,hq,kvh,dtype", [(64, 4, 2, torch.float16), (128, 8, 1, torch.bfloat16),
+                                            (128, 5, 5, torch.float16), (256, 8, 1, torch.bfloat16)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_prefill_attention_keys_in_segments(gpu_device, d, hq, kvh, dtype, causal):
+    """Few tiles over long keys: every tile's keys in segments, merged.  Requests
+    much shorter than the longest one get segments without keys; scores grow
+    along the keys, so the segments' maxima differ by powers of two."""
+    from vllm_ascend_quantized_kv_cache.ops.attention import prefill_attention
+
+    g = torch.Generator().manual_seed(d + hq)
+    q_lens, kv_lens = [17, 1, 2, 3], [3000, 70, 2, 0]
+    u = torch.nn.functional.normalize(torch.randn(kvh, d, generator=g), dim=-1)
+    grow = torch.cat([torch.arange(n).float() * (20.0 / max(n, 1)) for n in kv_lens])
+    k = (grow[:, None, None] * u + 0.2 * torch.randn(sum(kv_lens), kvh, d, generator=g)).to(dtype)
+    v = torch.randn(sum(kv_lens), kvh, d, generator=g).to(dtype)
+    q = (u.repeat_interleave(hq // kvh, 0)[None] * d ** 0.5
+         + torch.randn(sum(q_lens), hq, d, generator=g)).to(dtype)
+    got = prefill_attention(q.to(gpu_device), k.to(gpu_device), v.to(gpu_device), q_lens, kv_lens,
+                            d ** -0.5, causal).float().cpu()
+    want = ref.attention(q[:20], k, v, q_lens[:3], kv_lens[:3], d ** -0.5, causal)
+    torch.testing.assert_close(got[:20], want, atol=1e-2, rtol=1e-2)
+    assert not got[20:].any()  # no keys
+
+
+def test_prefill_attention_batch_past_the_launch_argument(gpu_device):
+    """More requests, and more tiles, than the plan argument carries."""
+    from vllm_ascend_quantized_kv_cache.ops.attention import prefill_attention
+
+    g = torch.Generator().manual_seed(9)
+    for q_lens in ([3] * 200, [3, 70000, 4]):
+        kv_lens = [n + 2 if n < 100 else 200 for n in q_lens]
+        causal = max(q_lens) < 100
+        q = torch.randn(sum(q_lens), 1, 64, generator=g).to(torch.bfloat16)
+        k = torch.randn(sum(kv_lens), 1, 64, generator=g).to(torch.bfloat16)
+        v = torch.randn(sum(kv_lens), 1, 64, generator=g).to(torch.bfloat16)
+        want = ref.attention(q, k, v, q_lens, kv_lens, 0.125, causal)
+        got = prefill_attention(q.to(gpu_device), k.to(gpu_device), v.to(gpu_device), q_lens,
+                                kv_lens, 0.125, causal)
+        torch.testing.assert_close(got.float().cpu(), want, atol=1e-2, rtol=1e-2)

@@ -322,14 +322,36 @@ struct FaLds {
 template <int D>
 constexpr int fa_ng() { return D == 256 ? 1 : 2; }
 
+// A launch's tiles, as a kernel argument when they fit (small calls then copy
+// nothing to the device): int32 cu_q [batch + 1], cu_k [batch + 1], and the
+// units request | tile << 16 in dispatch order.
+constexpr int kPlanArgWords = 500;
+struct PlanArg {
+  int32_t w[kPlanArgWords];
+};
+// Read-only tables: uniform reads through the constant address space are
+// scalar loads.  The plan argument is the kernel's first and is read in place
+// (indexed by value, the compiler would copy it to scratch).
+typedef const __attribute__((address_space(4))) int32_t cint32;
+__device__ __forceinline__ cint32* as_const(const int32_t* p) { return (cint32*)(p); }
+
+// Where a call's keys are cut into `segs` segments per tile (few tiles, long
+// keys): the partial results, o [unit][kv head][seg][row of the tile][D] and
+// (m, l) per row, m in the log2 domain.
+struct SegWs {
+  float* o;
+  float* ml;
+  int segs;
+};
+
 template <typename T, int D, int NG>
 __global__ void __launch_bounds__(64 * (8 / NG))
 __attribute__((amdgpu_waves_per_eu(2, 2)))
-prefill_attn_fa_kernel(const T* __restrict__ q, const T* __restrict__ k,
+prefill_attn_fa_kernel(PlanArg plan_arg, const int32_t* __restrict__ plan, int batch,
+                       const T* __restrict__ q, const T* __restrict__ k,
                        const T* __restrict__ v, const int32_t* __restrict__ cu_q,
-                       const int32_t* __restrict__ cu_k, const int32_t* __restrict__ units,
-                       int tiles, int hq, int kvh, FastDiv rep_div, float qscale, int causal,
-                       T* __restrict__ out) {
+                       const int32_t* __restrict__ cu_k, int tiles, int hq, int kvh,
+                       FastDiv rep_div, float qscale, int causal, T* __restrict__ out, SegWs seg) {
   using O = typename Op<T>::type;
   using L = FaLds<D>;
   constexpr int kFaWaves = 8 / NG;
@@ -357,14 +379,26 @@ prefill_attn_fa_kernel(const T* __restrict__ q, const T* __restrict__ k,
   const int rep = static_cast<int>(rep_div.d);
   const int unit = static_cast<int>(blockIdx.x) / kvh;
   const int kvhead = static_cast<int>(blockIdx.x) - unit * kvh;
-  // without a unit list: every request's `tiles` tiles, the last (most keys
-  // under the causal mask) first
-  const int b = units ? units[2 * unit] : unit / tiles;
-  const int tile = units ? units[2 * unit + 1] : tiles - 1 - unit % tiles;
-  const int q_start = cu_q[b];
-  const int lq = cu_q[b + 1] - q_start;
-  const int k_start = cu_k[b];
-  const int lk = cu_k[b + 1] - k_start;
+  // without a unit list (cu_q): every request's `tiles` tiles, the last (most
+  // keys under the causal mask) first
+  int b, tile;
+  cint32 *cq, *ck;
+  if (cu_q) {
+    b = unit / tiles;
+    tile = tiles - 1 - unit % tiles;
+    cq = as_const(cu_q);
+    ck = as_const(cu_k);
+  } else {
+    cq = plan ? as_const(plan) : (cint32*)__builtin_amdgcn_kernarg_segment_ptr();
+    ck = cq + batch + 1;
+    const uint32_t u = static_cast<uint32_t>(ck[batch + 1 + unit]);
+    b = static_cast<int>(u & 0xffffu);
+    tile = static_cast<int>(u >> 16);
+  }
+  const int q_start = cq[b];
+  const int lq = cq[b + 1] - q_start;
+  const int k_start = ck[b];
+  const int lk = ck[b + 1] - k_start;
   const int rows = lq * rep;  // rows of this (request, kv head)
   const int row0 = tile * (kFaRows * kFaWaves);
   if (row0 >= rows) return;  // uniform over the workgroup
@@ -378,7 +412,12 @@ prefill_attn_fa_kernel(const T* __restrict__ q, const T* __restrict__ k,
   auto query_of = [&](int row) { return static_cast<int>(rep_div.div(static_cast<uint32_t>(row))); };
   const int last_row = min(row0 + kFaRows * kFaWaves, rows) - 1;
   const int kv_end = causal ? min(lk, lk - lq + query_of(last_row) + 1) : lk;
-  const int nblk = (kv_end + kFaBlock - 1) / kFaBlock;
+  int blk0 = 0, nblk = (kv_end + kFaBlock - 1) / kFaBlock;  // this workgroup's blocks [blk0, nblk)
+  if (seg.segs > 1) {
+    const int all = nblk > 0 ? nblk : 0, sg = static_cast<int>(blockIdx.y);
+    blk0 = static_cast<int>(static_cast<int64_t>(all) * sg / seg.segs);
+    nblk = static_cast<int>(static_cast<int64_t>(all) * (sg + 1) / seg.segs);
+  }
   const int wave_last = min(wrow0 + kFaRows, rows) - 1;  // < wrow0 when the wave has no rows
   // kv positions of the wave's first and last query
   const int wave_first_pos = lk - lq + query_of(wrow0);
@@ -389,6 +428,16 @@ prefill_attn_fa_kernel(const T* __restrict__ q, const T* __restrict__ k,
     const int i = query_of(row);
     return (static_cast<int64_t>(q_start + i) * hq + kvhead * rep + (row - i * rep)) * D;
   };
+  // row of this workgroup's first row in the segments' partial results
+  const int64_t seg_row0 =
+      (static_cast<int64_t>(blockIdx.x) * seg.segs + blockIdx.y) * (kFaRows * kFaWaves);
+  if (seg.segs > 1 && blk0 >= nblk) {  // uniform: a segment without keys
+    for (int r = tid; r < kFaRows * kFaWaves; r += 64 * kFaWaves) {
+      seg.ml[2 * (seg_row0 + r)] = -INFINITY;
+      seg.ml[2 * (seg_row0 + r) + 1] = 0.0f;
+    }
+    return;
+  }
   if (lk <= 0) {  // uniform: nothing to attend to
     for (int r = tid >> 4; r < kFaRows * kFaWaves; r += 4 * kFaWaves)
       if (row0 + r < rows)
@@ -529,10 +578,10 @@ prefill_attn_fa_kernel(const T* __restrict__ q, const T* __restrict__ k,
       for (int g2 = 0; g2 < NG; ++g2) acc[g2] = mfma16(a[s], qop[g2][s], acc[g2], O{});
   };
 
-  // prologue: keys of blocks 0 and 1, values of block 0; scores of block 0
-  issue_rows(kbase, koff, kswz, kbuf0, 0);
-  if (nblk > 1) issue_rows(kbase, koff, kswz, kbuf1, kFaBlock);
-  issue_rows(vbase, voff, vswz, vbuf0, 0);
+  // prologue: keys of the first two blocks, values and scores of the first
+  issue_rows(kbase, koff, kswz, kbuf0, blk0 * kFaBlock);
+  if (blk0 + 1 < nblk) issue_rows(kbase, koff, kswz, kbuf1, (blk0 + 1) * kFaBlock);
+  issue_rows(vbase, voff, vswz, vbuf0, blk0 * kFaBlock);
   // the query rows go out behind the DMAs, so that one wait covers both
 #pragma unroll
   for (int g2 = 0; g2 < NG; ++g2) {
@@ -552,7 +601,7 @@ prefill_attn_fa_kernel(const T* __restrict__ q, const T* __restrict__ k,
   for (int kb2 = 0; kb2 < 4; ++kb2)
 #pragma unroll
     for (int g2 = 0; g2 < NG; ++g2) sacc[kb2][g2] = f4{0.f, 0.f, 0.f, 0.f};
-  if (active(0)) {
+  if (active(blk0)) {
 #pragma unroll
     for (int kb2 = 0; kb2 < 4; ++kb2) {
       u8v a[KS];
@@ -646,7 +695,8 @@ prefill_attn_fa_kernel(const T* __restrict__ q, const T* __restrict__ k,
       // 16-key group c: its exponentials (pop[g2][c / 2], half c % 2) beside
       // the score MFMAs of the next block's group c
       // (the last step computes scores of stale keys it never uses: one
-      // branch-free block keeps the MFMAs and the exponentials interleavable)
+      // branch-free block keeps the MFMAs and the exponentials interleavable;
+      // the last step as code of its own spills 55 registers)
       f4 snext[4][NG];
 #pragma unroll
       for (int kb2 = 0; kb2 < 4; ++kb2)
@@ -703,7 +753,7 @@ prefill_attn_fa_kernel(const T* __restrict__ q, const T* __restrict__ k,
   };
   // two steps per iteration, so that each step's buffers are compile-time
   // LDS offsets (folded into the reads' immediates instead of per-read adds)
-  int i = 0;
+  int i = blk0;
   for (; i + 1 < nblk; i += 2) {
     step(kbuf1, vbuf0, kbuf0, vbuf1, i);
     __syncthreads();
@@ -715,6 +765,21 @@ prefill_attn_fa_kernel(const T* __restrict__ q, const T* __restrict__ k,
     __syncthreads();
   }
 
+  if (seg.segs > 1) {  // uniform: this segment's partial, merged by the kernel below
+#pragma unroll
+    for (int g2 = 0; g2 < NG; ++g2) {
+      if (!live[g2]) continue;
+      const int64_t r = seg_row0 + wave * kFaRows + 16 * g2 + n;
+#pragma unroll
+      for (int j = 0; j < DB; ++j)
+        *reinterpret_cast<f4*>(seg.o + r * D + 16 * j + 4 * kg) = o[j][g2];
+      if (kg == 0) {
+        seg.ml[2 * r] = m_run[g2] == -INFINITY ? -INFINITY : qscale * m_run[g2];
+        seg.ml[2 * r + 1] = l_acc[g2][0];
+      }
+    }
+    return;
+  }
   // o[j][g2][r] = O^T[dim 16j + 4kg + r][query 16*g2 + n]
 #pragma unroll
   for (int g2 = 0; g2 < NG; ++g2) {
@@ -732,39 +797,116 @@ prefill_attn_fa_kernel(const T* __restrict__ q, const T* __restrict__ k,
 
 constexpr int kFaTileRows = 128;  // rows (queries x heads of a GQA group) per workgroup
 
+// Merge of the segments of a tile's rows: one wave per row, 8 waves a workgroup,
+// blockIdx.y the tile's group of 8 rows.  A segment without keys for the row
+// (m = -inf) carries weight 0 and its o, possibly unwritten, is selected out.
+constexpr int kMergeRows = 8;
+template <typename T, int D>
+__global__ void __launch_bounds__(64 * kMergeRows)
+prefill_merge_kernel(PlanArg plan_arg, int batch, int hq, int kvh, FastDiv rep_div,
+                     T* __restrict__ out, SegWs seg) {
+  const int unit = static_cast<int>(blockIdx.x) / kvh;
+  const int kvhead = static_cast<int>(blockIdx.x) - unit * kvh;
+  cint32* cq = (cint32*)__builtin_amdgcn_kernarg_segment_ptr();
+  const uint32_t u = static_cast<uint32_t>(cq[2 * (batch + 1) + unit]);
+  const int b = static_cast<int>(u & 0xffffu), tile = static_cast<int>(u >> 16);
+  const int rep = static_cast<int>(rep_div.d);
+  const int q_start = cq[b];
+  const int rows = (cq[b + 1] - q_start) * rep;
+  const int lane = threadIdx.x & 63;
+  const int r = kMergeRows * blockIdx.y + (threadIdx.x >> 6);  // of the tile
+  const int row = tile * kFaTileRows + r;
+  if (row >= rows) return;  // whole wave: no barrier below
+  const int64_t first = static_cast<int64_t>(blockIdx.x) * seg.segs * kFaTileRows + r;
+  // lane s: segment s's (m, l); at most 32 segments
+  float m = -INFINITY, l = 0.0f;
+  if (lane < seg.segs) {
+    const float2 x = *reinterpret_cast<const float2*>(
+        seg.ml + 2 * (first + static_cast<int64_t>(lane) * kFaTileRows));
+    m = x.x;
+    l = x.y;
+  }
+  const float mx = max_wave64(m);
+  const float w = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mx);
+  const float lsum = sum_wave64(w * l);
+  constexpr int PL = D / 64;  // dims per lane
+  float acc[PL];
+#pragma unroll
+  for (int i = 0; i < PL; ++i) acc[i] = 0.0f;
+#pragma unroll 4
+  for (int s = 0; s < seg.segs; ++s) {
+    const float ws = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), s));
+    const float* o = seg.o + (first + static_cast<int64_t>(s) * kFaTileRows) * D + PL * lane;
+#pragma unroll
+    for (int i = 0; i < PL; ++i) acc[i] += ws != 0.0f ? ws * o[i] : 0.0f;
+  }
+  const float inv = lsum > 0.0f ? 1.0f / lsum : 0.0f;
+  const int i = static_cast<int>(rep_div.div(static_cast<uint32_t>(row)));
+  T* orow = out + (static_cast<int64_t>(q_start + i) * hq + kvhead * rep + (row - i * rep)) * D;
+#pragma unroll
+  for (int k = 0; k < PL; ++k) orow[PL * lane + k] = from_f32<T>(acc[k] * inv);
+}
+
 // The 64-key-block kernel: 16-bit inputs, head sizes 64, 128 and 256, on a
-// device with its LDS.  `units` int32 [num_units, 2] = (request, tile) in
-// dispatch order, or NULL: num_units = batch * tiles, every request's `tiles`
-// tiles.  *launched: false when another kernel has to run.
-int launch_fa(const void* query, const void* key, const void* value, int dtype,
-              const int32_t* cu_q, const int32_t* cu_k, const int32_t* units, int64_t num_units,
-              int64_t tiles, int num_heads, int num_kv_heads, int head_size, float qscale,
-              int causal, void* out, hipStream_t s, bool* launched) {
-  *launched = false;
+// device with its LDS.  The tiles come from `arg` (num_units units; the only
+// form that may be cut into segments), from a plan on the device, or from
+// cu_q / cu_k: num_units = batch * tiles, every request's `tiles` tiles.
+// *launched: false when another kernel has to run.
+struct FaTiles {
+  const PlanArg* arg;
+  const int32_t* plan;
+  const int32_t* cu_q;
+  const int32_t* cu_k;
+  int64_t batch, num_units, tiles;
+};
+
+int fa_applies(int dtype, int head_size, bool* applies) {
+  *applies = false;
   if (dtype != KVQ_DTYPE_BF16 && dtype != KVQ_DTYPE_F16) return KVQ_OK;
   if (head_size != 64 && head_size != 128 && head_size != 256) return KVQ_OK;
   int64_t lds_max = 0;  // LDS one workgroup may use on this device
   const int lrc = device_lds_max(&lds_max);
   if (lrc != KVQ_OK) return lrc;
-  const int64_t fa_lds = head_size == 64    ? FaLds<64>::BYTES
+  *applies = lds_max >= (head_size == 64    ? FaLds<64>::BYTES
                          : head_size == 128 ? FaLds<128>::BYTES
-                                            : FaLds<256>::BYTES;
-  if (fa_lds > lds_max) return KVQ_OK;
-  if (num_units * num_kv_heads > 0x7fffffff || tiles > 0x7fffffff / kFaTileRows)
+                                            : FaLds<256>::BYTES);
+  return KVQ_OK;
+}
+
+int launch_fa(const void* query, const void* key, const void* value, int dtype, const FaTiles& t,
+              int num_heads, int num_kv_heads, int head_size, float qscale, int causal, void* out,
+              SegWs seg, hipStream_t s, bool* launched) {
+  *launched = false;
+  bool applies = false;
+  const int arc = fa_applies(dtype, head_size, &applies);
+  if (arc != KVQ_OK || !applies) return arc;
+  if (t.num_units * num_kv_heads > 0x7fffffff || t.tiles > 0x7fffffff / kFaTileRows)
     return KVQ_ERR_INVALID;
-  const dim3 grid(static_cast<unsigned>(num_units * num_kv_heads));
+  const unsigned wgs = static_cast<unsigned>(t.num_units * num_kv_heads);
+  const dim3 grid(wgs, static_cast<unsigned>(seg.segs));
   const FastDiv rep_div = FastDiv::make(static_cast<uint32_t>(num_heads / num_kv_heads));
+  static const PlanArg none{};
+  const PlanArg& arg = t.arg ? *t.arg : none;
 #define KVQ_PREFILL_FA(TT, DD)                                                              \
-  hipLaunchKernelGGL((prefill_attn_fa_kernel<TT, DD, fa_ng<DD>()>), grid, dim3(64 * (8 / fa_ng<DD>())), \
-                     FaLds<DD>::BYTES, s, static_cast<const TT*>(query),                   \
-                     static_cast<const TT*>(key), static_cast<const TT*>(value), cu_q, cu_k, \
-                     units, static_cast<int>(tiles), num_heads, num_kv_heads, rep_div, qscale, \
-                     causal, static_cast<TT*>(out))
-#define KVQ_PREFILL_FA_D(TT)                        \
-  switch (head_size) {                              \
-    case 64: KVQ_PREFILL_FA(TT, 64); break;         \
-    case 128: KVQ_PREFILL_FA(TT, 128); break;       \
-    default: KVQ_PREFILL_FA(TT, 256); break;        \
+  {                                                                                          \
+    hipLaunchKernelGGL((prefill_attn_fa_kernel<TT, DD, fa_ng<DD>()>), grid,                  \
+                       dim3(64 * (8 / fa_ng<DD>())), FaLds<DD>::BYTES, s, arg, t.plan,       \
+                       static_cast<int>(t.batch), static_cast<const TT*>(query),             \
+                       static_cast<const TT*>(key), static_cast<const TT*>(value), t.cu_q,   \
+                       t.cu_k, static_cast<int>(t.tiles), num_heads, num_kv_heads, rep_div,  \
+                       qscale, causal, static_cast<TT*>(out), seg);                          \
+    if (seg.segs > 1)                                                                        \
+      hipLaunchKernelGGL((prefill_merge_kernel<TT, DD>),                                     \
+                         dim3(wgs, kFaTileRows / kMergeRows), dim3(64 * kMergeRows), 0, s,   \
+                         arg, static_cast<int>(t.batch), num_heads, num_kv_heads, rep_div,   \
+                         static_cast<TT*>(out), seg);                                        \
+    break;                                                                                   \
+  }
+#define KVQ_PREFILL_FA_D(TT)              \
+  switch (head_size) {                    \
+    case 64: KVQ_PREFILL_FA(TT, 64)       \
+    case 128: KVQ_PREFILL_FA(TT, 128)     \
+    default: KVQ_PREFILL_FA(TT, 256)      \
   }
   if (dtype == KVQ_DTYPE_BF16) {
     KVQ_PREFILL_FA_D(kvq::bf16)
@@ -798,9 +940,9 @@ extern "C" int kvq_prefill_attn(const void* query, const void* key, const void* 
   const int64_t rows = max_q_len * (num_heads / num_kv_heads);
   const int64_t tiles = (rows + kFaTileRows - 1) / kFaTileRows;
   bool launched = false;
-  const int frc = launch_fa(query, key, value, dtype, cu_seqlens_q, cu_seqlens_k, nullptr,
-                            batch * tiles, tiles, num_heads, num_kv_heads, head_size, qscale,
-                            causal, out, s, &launched);
+  const FaTiles t{nullptr, nullptr, cu_seqlens_q, cu_seqlens_k, batch, batch * tiles, tiles};
+  const int frc = launch_fa(query, key, value, dtype, t, num_heads, num_kv_heads, head_size,
+                            qscale, causal, out, SegWs{nullptr, nullptr, 1}, s, &launched);
   if (frc != KVQ_OK || launched) return frc;
   const int64_t qblocks = (max_q_len + 63) / 64;
   if (qblocks > 0x7fffffff) return KVQ_ERR_INVALID;
@@ -822,60 +964,108 @@ extern "C" int kvq_prefill_attn(const void* query, const void* key, const void* 
   return KVQ_OK;
 }
 
-// Host side of a planned call: the cumulative lengths and the tiles in the
-// order they should start.  A tile's cost is its key blocks; long ones start
-// first, so that the last to end are short.  Where the keys and values an XCD
-// streams outgrow its 4 MB L2 twice over, a request's tiles stay together (the
-// requests by falling cost), so that one request's keys are in use at a time.
-extern "C" int64_t kvq_plan_prefill_attn(const int64_t* q_lens, const int64_t* kv_lens,
-                                         int64_t batch, int num_heads, int num_kv_heads,
-                                         int head_size, int causal, int32_t* plan,
-                                         int64_t cap_units) {
-  if (batch < 0 || (batch > 0 && (!q_lens || !kv_lens)) || !plan || num_kv_heads <= 0 ||
-      num_heads <= 0 || num_heads % num_kv_heads || head_size <= 0)
-    return KVQ_ERR_INVALID;
-  const int64_t rep = num_heads / num_kv_heads;
-  int32_t* cu_q = plan;
-  int32_t* cu_k = plan + batch + 1;
-  int32_t* units = plan + 2 * (batch + 1);
+namespace {
+
+struct Unit {
+  int64_t group, cost;  // descending sort keys
+  uint32_t unit;        // request | tile << 16
+};
+
+// The tiles of a batch with their cost in key blocks; *most the largest cost.
+// KVQ_ERR_CAPACITY past `cap` tiles or outside the packed unit's range.
+int64_t plan_units(const int64_t* q_lens, const int64_t* kv_lens, int64_t batch, int64_t rep,
+                   int causal, int64_t cap, int64_t* most, std::vector<Unit>* all) {
   int64_t nq = 0, nk = 0, n = 0;
-  struct Unit {
-    int64_t group, cost;  // descending sort keys
-    int32_t b, tile;
-  };
-  std::vector<Unit> all;
-  all.reserve(static_cast<size_t>(cap_units > 0 ? cap_units : 0));
-  cu_q[0] = cu_k[0] = 0;
+  *most = 0;
   for (int64_t b = 0; b < batch; ++b) {
     const int64_t lq = q_lens[b], lk = kv_lens[b];
     if (lq < 0 || lk < 0) return KVQ_ERR_INVALID;
     nq += lq;
     nk += lk;
     if (nq * rep > 0x7fffffff || nk > 0x7fffffff) return KVQ_ERR_INVALID;
-    cu_q[b + 1] = static_cast<int32_t>(nq);
-    cu_k[b + 1] = static_cast<int32_t>(nk);
-    const int64_t rows = lq * rep;
-    for (int64_t r0 = 0; r0 < rows; r0 += kFaTileRows, ++n) {
-      if (n >= cap_units) return KVQ_ERR_CAPACITY;
-      const int64_t last = (std::min<int64_t>(r0 + kFaTileRows, rows) - 1) / rep;
+    const int64_t rows = lq * rep, tiles = (rows + kFaTileRows - 1) / kFaTileRows;
+    if (n + tiles > cap || tiles > 0x10000 || b > 0xffff) return KVQ_ERR_CAPACITY;
+    n += tiles;
+    for (int64_t t = 0; t < tiles; ++t) {
+      const int64_t last = (std::min<int64_t>((t + 1) * kFaTileRows, rows) - 1) / rep;
       const int64_t end = causal ? std::min(lk, lk - lq + last + 1) : lk;
       const int64_t cost = end <= 0 ? 0 : (end + kFaBlock - 1) / kFaBlock;
-      all.push_back({0, cost, static_cast<int32_t>(b), static_cast<int32_t>(r0 / kFaTileRows)});
+      *most = std::max(*most, cost);
+      if (all) all->push_back({0, cost, static_cast<uint32_t>(b | (t << 16))});
     }
   }
-  const int64_t xcd_bytes = nk * head_size * 4 * std::max<int64_t>(1, num_kv_heads / 8);
+  return n;
+}
+
+// Segments per tile.  A launch of fewer tiles than the chip holds workgroups
+// leaves the rest of it idle while each tile walks its keys alone (8 query
+// heads on 1 kv head, 16 rows over 8K keys: 128 blocks on 1 of 256 CUs), so its
+// keys are cut into as many segments as fill the chip, of at least 4 blocks
+// (a segment's start and end cost about 3), where that takes 8 blocks off the
+// longest tile, about what the merge costs.
+int64_t plan_segs(int64_t units, int64_t most, int kvh, int head_size) {
+  int cus = 0;
+  if (device_cu_count(&cus) != KVQ_OK || cus <= 0) return 1;
+  const int64_t slots = static_cast<int64_t>(cus) * (head_size == 256 ? 1 : 2);
+  const int64_t segs = std::min<int64_t>({slots / std::max<int64_t>(1, units * kvh), most / 4, 32});
+  return segs > 1 && most - most / segs >= 8 ? segs : 1;
+}
+
+int64_t seg_rows(int64_t units, int kvh, int64_t segs) { return units * kvh * segs * kFaTileRows; }
+
+bool plan_args_ok(const int64_t* q_lens, const int64_t* kv_lens, int64_t batch, int num_heads,
+                  int num_kv_heads, int head_size) {
+  return batch >= 0 && (batch == 0 || (q_lens && kv_lens)) && num_kv_heads > 0 && num_heads > 0 &&
+         num_heads % num_kv_heads == 0 && head_size > 0;
+}
+
+// Host side of a planned call: the cumulative lengths and the tiles in the
+// order they should start.  Long tiles start first, so that the last to end are
+// short.  Where the keys and values an XCD streams outgrow its 4 MB L2 twice
+// over, a request's tiles stay together (the requests by falling cost), so that
+// one request's keys are in use at a time.
+int64_t write_plan(const int64_t* q_lens, const int64_t* kv_lens, int64_t batch, int num_heads,
+                   int num_kv_heads, int head_size, int causal, int32_t* plan, int64_t cap_units,
+                   int64_t* most) {
+  std::vector<Unit> all;
+  const int64_t n = plan_units(q_lens, kv_lens, batch, num_heads / num_kv_heads, causal,
+                               cap_units, most, &all);
+  if (n < 0) return n;
+  int32_t* cu_q = plan;
+  int32_t* cu_k = plan + batch + 1;
+  cu_q[0] = cu_k[0] = 0;
+  for (int64_t b = 0; b < batch; ++b) {
+    cu_q[b + 1] = cu_q[b] + static_cast<int32_t>(q_lens[b]);
+    cu_k[b + 1] = cu_k[b] + static_cast<int32_t>(kv_lens[b]);
+  }
+  const int64_t xcd_bytes =
+      static_cast<int64_t>(cu_k[batch]) * head_size * 4 * std::max(1, num_kv_heads / 8);
   if (xcd_bytes > (int64_t{8} << 20))
-    for (auto& u : all) u.group = q_lens[u.b] * kv_lens[u.b];
+    for (auto& u : all) u.group = q_lens[u.unit & 0xffff] * kv_lens[u.unit & 0xffff];
   std::stable_sort(all.begin(), all.end(), [](const Unit& x, const Unit& y) {
     if (x.group != y.group) return x.group > y.group;
-    if (x.group != 0 && x.b != y.b) return x.b < y.b;
+    if (x.group != 0 && (x.unit & 0xffff) != (y.unit & 0xffff))
+      return (x.unit & 0xffff) < (y.unit & 0xffff);
     return x.cost > y.cost;
   });
-  for (int64_t i = 0; i < n; ++i) {
-    units[2 * i] = all[static_cast<size_t>(i)].b;
-    units[2 * i + 1] = all[static_cast<size_t>(i)].tile;
-  }
+  int32_t* units = plan + 2 * (batch + 1);
+  for (int64_t i = 0; i < n; ++i) units[i] = static_cast<int32_t>(all[static_cast<size_t>(i)].unit);
   return n;
+}
+
+int64_t plan_arg_cap(int64_t batch) { return kPlanArgWords - 2 * (batch + 1); }
+
+}  // namespace
+
+extern "C" int64_t kvq_plan_prefill_attn(const int64_t* q_lens, const int64_t* kv_lens,
+                                         int64_t batch, int num_heads, int num_kv_heads,
+                                         int head_size, int causal, int32_t* plan,
+                                         int64_t cap_units) {
+  if (!plan || !plan_args_ok(q_lens, kv_lens, batch, num_heads, num_kv_heads, head_size))
+    return KVQ_ERR_INVALID;
+  int64_t most = 0;
+  return write_plan(q_lens, kv_lens, batch, num_heads, num_kv_heads, head_size, causal, plan,
+                    cap_units, &most);
 }
 
 extern "C" int kvq_prefill_attn_planned(const void* query, const void* key, const void* value,
@@ -889,10 +1079,61 @@ extern "C" int kvq_prefill_attn_planned(const void* query, const void* key, cons
   if (num_kv_heads <= 0 || num_heads % num_kv_heads) return KVQ_ERR_GEOMETRY;
   if (!(scale > 0.0f)) return KVQ_ERR_INVALID;
   bool launched = false;
-  const int rc = launch_fa(query, key, value, dtype, plan, plan + batch + 1,
-                           plan + 2 * (batch + 1), num_units, 0, num_heads, num_kv_heads,
-                           head_size, scale * 1.4426950408889634f, causal, out,
+  const FaTiles t{nullptr, plan, nullptr, nullptr, batch, num_units, 0};
+  const int rc = launch_fa(query, key, value, dtype, t, num_heads, num_kv_heads, head_size,
+                           scale * 1.4426950408889634f, causal, out, SegWs{nullptr, nullptr, 1},
                            static_cast<hipStream_t>(stream), &launched);
   if (rc != KVQ_OK) return rc;
   return launched ? KVQ_OK : KVQ_ERR_GEOMETRY;
+}
+
+extern "C" int64_t kvq_prefill_attn_lens_workspace_bytes(const int64_t* q_lens,
+                                                         const int64_t* kv_lens, int64_t batch,
+                                                         int num_heads, int num_kv_heads,
+                                                         int head_size, int causal) {
+  if (!plan_args_ok(q_lens, kv_lens, batch, num_heads, num_kv_heads, head_size))
+    return KVQ_ERR_INVALID;
+  if (plan_arg_cap(batch) <= 0) return KVQ_ERR_CAPACITY;
+  int64_t most = 0;
+  const int64_t n = plan_units(q_lens, kv_lens, batch, num_heads / num_kv_heads, causal,
+                               plan_arg_cap(batch), &most, nullptr);
+  if (n <= 0) return n;
+  const int64_t segs = plan_segs(n, most, num_kv_heads, head_size);
+  return segs == 1 ? 0 : seg_rows(n, num_kv_heads, segs) * (head_size + 2) * 4;
+}
+
+extern "C" int kvq_prefill_attn_lens(const void* query, const void* key, const void* value,
+                                     int dtype, const int64_t* q_lens, const int64_t* kv_lens,
+                                     int64_t batch, int num_heads, int num_kv_heads,
+                                     int head_size, float scale, int causal, void* workspace,
+                                     int64_t workspace_bytes, void* out, void* stream) {
+  if (!plan_args_ok(q_lens, kv_lens, batch, num_heads, num_kv_heads, head_size))
+    return KVQ_ERR_INVALID;
+  if (batch == 0) return KVQ_OK;
+  if (!query || !key || !value || !out || !(scale > 0.0f)) return KVQ_ERR_INVALID;
+  bool applies = false;
+  const int arc = fa_applies(dtype, head_size, &applies);
+  if (arc != KVQ_OK) return arc;
+  if (!applies) return KVQ_ERR_GEOMETRY;
+  if (plan_arg_cap(batch) <= 0) return KVQ_ERR_CAPACITY;
+  PlanArg arg;
+  int64_t most = 0;
+  const int64_t n = write_plan(q_lens, kv_lens, batch, num_heads, num_kv_heads, head_size, causal,
+                               arg.w, plan_arg_cap(batch), &most);
+  if (n <= 0) return static_cast<int>(n);
+  // without the workspace (or on another device than it was sized on) the keys
+  // stay whole
+  SegWs seg{nullptr, nullptr, 1};
+  const int64_t segs = plan_segs(n, most, num_kv_heads, head_size);
+  const int64_t rows = seg_rows(n, num_kv_heads, segs);
+  if (segs > 1 && workspace && workspace_bytes >= rows * (head_size + 2) * 4) {
+    seg.o = static_cast<float*>(workspace);
+    seg.ml = seg.o + rows * head_size;
+    seg.segs = static_cast<int>(segs);
+  }
+  bool launched = false;
+  const FaTiles t{&arg, nullptr, nullptr, nullptr, batch, n, 0};
+  return launch_fa(query, key, value, dtype, t, num_heads, num_kv_heads, head_size,
+                   scale * 1.4426950408889634f, causal, out, seg,
+                   static_cast<hipStream_t>(stream), &launched);
 }
