@@ -783,15 +783,29 @@ prefill_attn_fa_kernel(PlanArg plan_arg, const int32_t* __restrict__ plan, int b
   // o[j][g2][r] = O^T[dim 16j + 4kg + r][query 16*g2 + n]
 #pragma unroll
   for (int g2 = 0; g2 < NG; ++g2) {
-    if (!live[g2]) continue;
     const float l = l_acc[g2][0];
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-    T* orow = out + row_offset(wrow0 + 16 * g2 + n);
+    T* orow = out + row_offset(live[g2] ? wrow0 + 16 * g2 + n : 0);
+    // two dim blocks' 8-byte pieces trade places between the lanes of a row's
+    // 16-lane groups, so that a lane stores 16 bytes: group kg the dims 16 (j +
+    // kg % 2) + 8 (kg / 2) .. + 7
+    // (8-byte stores: 106 against 103 us on 12 ragged prompts of 17 - 1500 rows,
+    // 32 heads on 8 kv heads; a tile's end took 2.7 us of its 29)
 #pragma unroll
-    for (int j = 0; j < DB; ++j)
-      *reinterpret_cast<uint2*>(orow + 16 * j + 4 * kg) =
-          make_uint2(pack_op2(o[j][g2][0] * inv, o[j][g2][1] * inv, O{}),
-                     pack_op2(o[j][g2][2] * inv, o[j][g2][3] * inv, O{}));
+    for (int j = 0; j < DB; j += 2) {
+      uint32_t w[2][2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const auto r = __builtin_amdgcn_permlane16_swap(
+            pack_op2(o[j][g2][2 * h] * inv, o[j][g2][2 * h + 1] * inv, O{}),
+            pack_op2(o[j + 1][g2][2 * h] * inv, o[j + 1][g2][2 * h + 1] * inv, O{}), false, false);
+        w[0][h] = r[0];
+        w[1][h] = r[1];
+      }
+      if (live[g2])
+        *reinterpret_cast<uint4*>(orow + 16 * (j + kg % 2) + 8 * (kg / 2)) =
+            make_uint4(w[0][0], w[0][1], w[1][0], w[1][1]);
+    }
   }
 }
 
