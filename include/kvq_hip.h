@@ -364,6 +364,15 @@ int kvq_int8_dequant_gather(const int8_t* key_cache, const int8_t* value_cache,
                             const int64_t* cu_seqlens, int64_t batch,
                             void* out_k, void* out_v, void* stream);
 
+/* The same with the lengths on the host (int64 [batch], read during the call):
+ * they travel with the launches, nothing is copied to the device. */
+int kvq_int8_dequant_gather_lens(const int8_t* key_cache, const int8_t* value_cache,
+                                 int64_t num_blocks, int block_size, int num_kv_heads,
+                                 int head_size, const void* k_aq, const void* v_aq, int dtype,
+                                 const int32_t* block_table, int64_t max_blocks,
+                                 const int64_t* seq_lens, int64_t batch, void* out_k, void* out_v,
+                                 void* stream);
+
 /* Fused INT8 decode attention with per-channel antiquant (offset 0):
  * K = int8 * k_aq[h, d], V = int8 * v_aq[h, d].
  *   query/out [batch, num_heads, D] of `dtype`; k_aq/v_aq [KVH*D] of `dtype`
@@ -413,6 +422,14 @@ int kvq_fp8_pth_gather(const uint8_t* k_data, const float* k_scale, const uint8_
                        int num_kv_heads, int head_size, const void* block_table,
                        int block_index_type, int64_t max_blocks, const int64_t* cu_seqlens,
                        int64_t batch, void* out_k, void* out_v, int out_dtype, void* stream);
+
+/* The same with the lengths on the host (int64 [batch], read during the call):
+ * they travel with the launches, nothing is copied to the device. */
+int kvq_fp8_pth_gather_lens(const uint8_t* k_data, const float* k_scale, const uint8_t* v_data,
+                            const float* v_scale, int64_t num_blocks, int block_size,
+                            int num_kv_heads, int head_size, const void* block_table,
+                            int block_index_type, int64_t max_blocks, const int64_t* seq_lens,
+                            int64_t batch, void* out_k, void* out_v, int out_dtype, void* stream);
 
 /* Fused decode attention over the paged E4M3 codes: one query row per request
  * over its seq_lens[b] positions (host int64 [batch]; 0 gives zeros),

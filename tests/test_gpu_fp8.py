@@ -158,6 +158,25 @@ def test_gather_matches_oracle_bit_exact(gpu_device, out_dtype, d, kvh):
         assert torch.equal(dk.cpu(), wk) and torch.equal(dv.cpu(), wv)
 
 
+@pytest.mark.parametrize("batch", [256, 257, 600])
+def test_gather_of_batches_past_one_launch(gpu_device, batch):
+    """A launch carries 256 requests' rows; short, empty and long ones on both
+    sides of the cuts."""
+    nb, bs, kvh, d = 40, 16, 2, 64
+    gen = torch.Generator().manual_seed(batch)
+    lens = torch.randint(0, 40, (batch,), generator=gen).tolist()
+    lens[0] = lens[-1] = 48
+    lens[255] = 0
+    table = torch.randint(0, nb, (batch, 3), generator=gen, dtype=torch.int32)
+    _, _, views = _views(gpu_device, nb, bs, kvh, d)
+    rows = [_inputs(nb * bs, kvh, d, torch.bfloat16, seed=s).to(gpu_device) for s in (1, 2)]
+    fp8_ops.fp8_per_token_head_store(*rows, torch.arange(nb * bs, device=gpu_device), *views)
+    dk, dv = fp8_ops.fp8_per_token_head_dequant_gather(*views, table.to(gpu_device), lens,
+                                                       torch.bfloat16)
+    wk, wv = ref.fp8_pth_gather(*[v.cpu() for v in views], table, lens, torch.bfloat16)
+    assert torch.equal(dk.cpu(), wk) and torch.equal(dv.cpu(), wv)
+
+
 def test_semantics_object_matches_oracle(gpu_device):
     sem = Fp8PerTokenHeadSemantics(type("Cfg", (), {"head_size": 128})())
     x = _inputs(33, 4, 128, torch.bfloat16, seed=9)

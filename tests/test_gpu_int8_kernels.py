@@ -92,6 +92,26 @@ def test_int8_dequant_gather_bit_exact(gpu_device, dtype):
     assert torch.equal(want_v, got_v.cpu())
 
 
+@pytest.mark.parametrize("batch", [256, 257, 600])
+def test_int8_dequant_gather_of_batches_past_one_launch(gpu_device, batch):
+    """A launch carries 256 requests' rows; short, empty and long ones on both
+    sides of the cuts."""
+    from vllm_ascend_quantized_kv_cache.ops.int8_ops import int8_dequant_gather
+
+    nb, bs, kvh, d, dtype = 40, 16, 2, 64, torch.bfloat16
+    gen = torch.Generator().manual_seed(batch)
+    lens = torch.randint(0, 40, (batch,), generator=gen).tolist()
+    lens[0] = lens[-1] = 48
+    lens[255] = 0
+    table = torch.randint(0, nb, (batch, 3), generator=gen, dtype=torch.int32)
+    kc, vc = torch.randint(-128, 128, (2, nb, bs, kvh, d), generator=gen, dtype=torch.int8)
+    _, _, _, k_inv, v_inv, k_aq, v_aq = _int8_state(gpu_device, 1, [8], kvh, d, bs, dtype, 3)
+    want = ref.int8_paged_dequant(kc, vc, table, lens, dtype, k_inv, v_inv)
+    got = int8_dequant_gather(kc.to(gpu_device), vc.to(gpu_device), table.to(gpu_device), lens,
+                              dtype, k_aq.to(gpu_device), v_aq.to(gpu_device))
+    assert torch.equal(got[0].cpu(), want[0]) and torch.equal(got[1].cpu(), want[1])
+
+
 @pytest.mark.parametrize("rep", [1, 4, 8])
 @pytest.mark.parametrize("kvh,d,bs", [(2, 64, 16), (8, 128, 128), (4, 128, 32), (16, 128, 64)])
 def test_int8_decode_matches_oracle(gpu_device, rep, kvh, d, bs):

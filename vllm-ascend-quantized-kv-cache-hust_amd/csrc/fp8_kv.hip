@@ -24,6 +24,8 @@
 // Gather: one thread per NCH chunks of W codes of one (position, head) row,
 // laid out as in the store, into dense TND rows of the activation dtype
 // (code * scale in fp32, then RNE).
+#include <algorithm>
+
 #include "kvq_common.h"
 
 namespace {
@@ -218,14 +220,14 @@ fp8_pth_store_kernel(const T* __restrict__ key, const T* __restrict__ value,
 
 template <typename TO, typename TB, int W, int NCH>
 __global__ void __launch_bounds__(256)
-fp8_pth_gather_kernel(const uint8_t* __restrict__ k_data, const float* __restrict__ k_scale,
-                      const uint8_t* __restrict__ v_data, const float* __restrict__ v_scale,
+fp8_pth_gather_kernel(CuArg cu_arg, const uint8_t* __restrict__ k_data,
+                      const float* __restrict__ k_scale, const uint8_t* __restrict__ v_data, const float* __restrict__ v_scale,
                       FastDiv bs, int kvh, int d, int64_t nb, const TB* __restrict__ block_table,
                       int64_t maxb, const int64_t* __restrict__ cu, FastDiv per_pos,
                       FastDiv per_head, TO* __restrict__ out_k, TO* __restrict__ out_v) {
   const int b = blockIdx.y;
-  const int64_t row0 = cu[b];
-  const int64_t len = cu[b + 1] - row0;
+  int64_t row0, len;
+  request_rows(cu, b, row0, len);
   const int half = d / NCH;
   // gid < 2^31 (the grid is checked on the host), so 32-bit division suffices
   const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
@@ -345,6 +347,44 @@ extern "C" int kvq_fp8_pth_store(const void* key, const void* value, int dtype,
   return KVQ_OK;
 }
 
+namespace {
+
+// A launch over `batch` requests of at most `rows` rows; the dense rows from
+// `cu` on the device, else from `arg`.
+int launch_fp8_gather(const kvq::CuArg& arg, const int64_t* cu, int64_t rows,
+                      const uint8_t* k_data, const float* k_scale, const uint8_t* v_data,
+                      const float* v_scale, int64_t num_blocks, int block_size, int num_kv_heads,
+                      int head_size, const void* block_table, int block_index_type,
+                      int64_t max_blocks, int64_t batch, void* out_k, void* out_v, int out_dtype,
+                      hipStream_t s) {
+  const int vec = head_size % 16 == 0 ? 16 : (head_size % 8 == 0 ? 8 : 4);
+  const int64_t per_pos = static_cast<int64_t>(num_kv_heads) * (head_size / vec);
+  const int64_t threads = rows * per_pos;
+  if (threads > 0x7fffffff - 255) return KVQ_ERR_INVALID;
+  const dim3 grid(static_cast<unsigned>((threads + 255) / 256), static_cast<unsigned>(batch));
+  const FastDiv bs_div = FastDiv::make(static_cast<uint32_t>(block_size));
+  const FastDiv pos_div = FastDiv::make(static_cast<uint32_t>(per_pos));
+  const FastDiv head_div = FastDiv::make(static_cast<uint32_t>(head_size / vec));
+#define KVQ_FP8_GATHER(W, NCH)                                                               \
+  hipLaunchKernelGGL((fp8_pth_gather_kernel<TO, TB, W, NCH>), grid, dim3(256), 0, s, arg,    \
+                     k_data, k_scale, v_data, v_scale, bs_div, num_kv_heads, head_size,      \
+                     num_blocks, static_cast<const TB*>(block_table), max_blocks, cu,        \
+                     pos_div, head_div, static_cast<TO*>(out_k), static_cast<TO*>(out_v))
+  KVQ_DISPATCH_FLOAT(out_dtype, TO,
+    KVQ_DISPATCH_INDEX(block_index_type, TB,
+      if (vec == 16)
+        KVQ_FP8_GATHER(8, 2);
+      else if (vec == 8)
+        KVQ_FP8_GATHER(8, 1);
+      else
+        KVQ_FP8_GATHER(4, 1)));
+#undef KVQ_FP8_GATHER
+  KVQ_LAUNCH_CHECK();
+  return KVQ_OK;
+}
+
+}  // namespace
+
 extern "C" int kvq_fp8_pth_gather(const uint8_t* k_data, const float* k_scale,
                                   const uint8_t* v_data, const float* v_scale,
                                   int64_t num_blocks, int block_size, int num_kv_heads,
@@ -357,30 +397,37 @@ extern "C" int kvq_fp8_pth_gather(const uint8_t* k_data, const float* k_scale,
       num_kv_heads <= 0 || batch > 65535)
     return KVQ_ERR_INVALID;
   if (head_size <= 0 || head_size % 4) return KVQ_ERR_GEOMETRY;
-  const int vec = head_size % 16 == 0 ? 16 : (head_size % 8 == 0 ? 8 : 4);
   // grid.x covers the longest request the table can describe
-  const int64_t per_pos = static_cast<int64_t>(num_kv_heads) * (head_size / vec);
-  const int64_t threads = max_blocks * block_size * per_pos;
-  if (threads > 0x7fffffff - 255) return KVQ_ERR_INVALID;
-  const dim3 grid(static_cast<unsigned>((threads + 255) / 256), static_cast<unsigned>(batch));
-  const FastDiv bs_div = FastDiv::make(static_cast<uint32_t>(block_size));
-  const FastDiv pos_div = FastDiv::make(static_cast<uint32_t>(per_pos));
-  const FastDiv head_div = FastDiv::make(static_cast<uint32_t>(head_size / vec));
-  hipStream_t s = static_cast<hipStream_t>(stream);
-#define KVQ_FP8_GATHER(W, NCH)                                                               \
-  hipLaunchKernelGGL((fp8_pth_gather_kernel<TO, TB, W, NCH>), grid, dim3(256), 0, s, k_data, \
-                     k_scale, v_data, v_scale, bs_div, num_kv_heads, head_size, num_blocks,  \
-                     static_cast<const TB*>(block_table), max_blocks, cu_seqlens, pos_div,   \
-                     head_div, static_cast<TO*>(out_k), static_cast<TO*>(out_v))
-  KVQ_DISPATCH_FLOAT(out_dtype, TO,
-    KVQ_DISPATCH_INDEX(block_index_type, TB,
-      if (vec == 16)
-        KVQ_FP8_GATHER(8, 2);
-      else if (vec == 8)
-        KVQ_FP8_GATHER(8, 1);
-      else
-        KVQ_FP8_GATHER(4, 1)));
-#undef KVQ_FP8_GATHER
-  KVQ_LAUNCH_CHECK();
-  return KVQ_OK;
+  return launch_fp8_gather(kvq::CuArg{}, cu_seqlens, max_blocks * block_size, k_data, k_scale,
+                           v_data, v_scale, num_blocks, block_size, num_kv_heads, head_size,
+                           block_table, block_index_type, max_blocks, batch, out_k, out_v,
+                           out_dtype, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int kvq_fp8_pth_gather_lens(const uint8_t* k_data, const float* k_scale,
+                                       const uint8_t* v_data, const float* v_scale,
+                                       int64_t num_blocks, int block_size, int num_kv_heads,
+                                       int head_size, const void* block_table,
+                                       int block_index_type, int64_t max_blocks,
+                                       const int64_t* seq_lens, int64_t batch, void* out_k,
+                                       void* out_v, int out_dtype, void* stream) {
+  if (batch == 0 || max_blocks == 0) return KVQ_OK;
+  if (!k_data || !k_scale || !v_data || !v_scale || !block_table || !seq_lens || !out_k ||
+      !out_v || batch < 0 || max_blocks < 0 || num_blocks <= 0 || block_size <= 0 ||
+      num_kv_heads <= 0 || batch > 65535)
+    return KVQ_ERR_INVALID;
+  if (head_size <= 0 || head_size % 4) return KVQ_ERR_GEOMETRY;
+  const int vec = head_size % 16 == 0 ? 16 : (head_size % 8 == 0 ? 8 : 4);
+  const int64_t table_rows = max_blocks * block_size;
+  if (table_rows * num_kv_heads * (head_size / vec) > 0x7fffffff - 255) return KVQ_ERR_INVALID;
+  const int64_t index_bytes = block_index_type == KVQ_INDEX_I64 ? 8 : 4;
+  return kvq::for_each_cu_arg(
+      seq_lens, batch,
+      [&](const kvq::CuArg& arg, int64_t first, int64_t n, int64_t longest) -> int {
+        const char* bt = static_cast<const char*>(block_table) + first * max_blocks * index_bytes;
+        return launch_fp8_gather(arg, nullptr, std::min(longest, table_rows), k_data, k_scale,
+                                 v_data, v_scale, num_blocks, block_size, num_kv_heads, head_size,
+                                 bt, block_index_type, max_blocks, n, out_k, out_v, out_dtype,
+                                 static_cast<hipStream_t>(stream));
+      });
 }

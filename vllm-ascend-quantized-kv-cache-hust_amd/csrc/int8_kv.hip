@@ -146,19 +146,20 @@ int8_quant_scatter_kernel(const T* __restrict__ key, const T* __restrict__ value
 
 template <typename T>
 __global__ void __launch_bounds__(256)
-int8_dequant_gather_kernel(const int8_t* __restrict__ kc, const int8_t* __restrict__ vc, int bs,
+int8_dequant_gather_kernel(CuArg cu_arg, const int8_t* __restrict__ kc, const int8_t* __restrict__ vc, int bs,
                            int64_t channels, const T* __restrict__ k_aq,
                            const T* __restrict__ v_aq, const int32_t* __restrict__ block_table,
                            int64_t maxb, const int64_t* __restrict__ cu, T* __restrict__ out_k,
                            T* __restrict__ out_v) {
   const int b = blockIdx.y;
-  const int64_t row0 = cu[b];
-  const int64_t len = cu[b + 1] - row0;
+  int64_t row0, len;
+  request_rows(cu, b, row0, len);
   const int64_t per_row = channels / 8;
   const int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (gid >= len * per_row) return;
   const int64_t p = gid / per_row;
   const int64_t c8 = (gid - p * per_row) * 8;
+  if (p / bs >= maxb) return;  // a length the table does not cover reads nothing past it
   const int64_t blk = block_table[static_cast<int64_t>(b) * maxb + p / bs];
   const int64_t src = (blk * bs + p % bs) * channels + c8;
   const uint2 kw = *reinterpret_cast<const uint2*>(kc + src);
@@ -356,6 +357,29 @@ extern "C" int kvq_int8_quant_scatter(const void* key, const void* value, int dt
   return KVQ_OK;
 }
 
+namespace {
+
+// A launch over `batch` requests of at most `rows` rows; the dense rows from
+// `cu` on the device, else from `arg`.
+int launch_dequant_gather(const kvq::CuArg& arg, const int64_t* cu, int64_t rows,
+                          const int8_t* key_cache, const int8_t* value_cache, int block_size,
+                          int64_t channels, const void* k_aq, const void* v_aq, int dtype,
+                          const int32_t* block_table, int64_t max_blocks, int64_t batch,
+                          void* out_k, void* out_v, hipStream_t s) {
+  const int64_t blocks = (rows * (channels / 8) + 255) / 256;
+  if (blocks > 0x7fffffff) return KVQ_ERR_INVALID;
+  const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(batch));
+  KVQ_DISPATCH_FLOAT(dtype, T,
+    hipLaunchKernelGGL((int8_dequant_gather_kernel<T>), grid, dim3(256), 0, s, arg, key_cache,
+                       value_cache, block_size, channels, static_cast<const T*>(k_aq),
+                       static_cast<const T*>(v_aq), block_table, max_blocks, cu,
+                       static_cast<T*>(out_k), static_cast<T*>(out_v)));
+  KVQ_LAUNCH_CHECK();
+  return KVQ_OK;
+}
+
+}  // namespace
+
 extern "C" int kvq_int8_dequant_gather(const int8_t* key_cache, const int8_t* value_cache,
                                        int64_t num_blocks, int block_size, int num_kv_heads,
                                        int head_size, const void* k_aq, const void* v_aq,
@@ -367,20 +391,38 @@ extern "C" int kvq_int8_dequant_gather(const int8_t* key_cache, const int8_t* va
       !out_v || batch < 0 || num_blocks <= 0 || block_size <= 0 || head_size % 8 ||
       num_kv_heads <= 0 || batch > 65535)
     return KVQ_ERR_INVALID;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const int64_t channels = static_cast<int64_t>(num_kv_heads) * head_size;
   // grid.x covers the longest request: max_blocks * block_size rows
-  const int64_t rows = max_blocks * block_size;
-  const int64_t blocks = (rows * (channels / 8) + 255) / 256;
-  if (blocks > 0x7fffffff) return KVQ_ERR_INVALID;
-  const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(batch));
-  KVQ_DISPATCH_FLOAT(dtype, T,
-    hipLaunchKernelGGL((int8_dequant_gather_kernel<T>), grid, dim3(256), 0, s, key_cache,
-                       value_cache, block_size, channels, static_cast<const T*>(k_aq),
-                       static_cast<const T*>(v_aq), block_table, max_blocks, cu_seqlens,
-                       static_cast<T*>(out_k), static_cast<T*>(out_v)));
-  KVQ_LAUNCH_CHECK();
-  return KVQ_OK;
+  return launch_dequant_gather(kvq::CuArg{}, cu_seqlens, max_blocks * block_size, key_cache,
+                               value_cache, block_size,
+                               static_cast<int64_t>(num_kv_heads) * head_size, k_aq, v_aq, dtype,
+                               block_table, max_blocks, batch, out_k, out_v,
+                               static_cast<hipStream_t>(stream));
+}
+
+extern "C" int kvq_int8_dequant_gather_lens(const int8_t* key_cache, const int8_t* value_cache,
+                                            int64_t num_blocks, int block_size, int num_kv_heads,
+                                            int head_size, const void* k_aq, const void* v_aq,
+                                            int dtype, const int32_t* block_table,
+                                            int64_t max_blocks, const int64_t* seq_lens,
+                                            int64_t batch, void* out_k, void* out_v,
+                                            void* stream) {
+  if (batch == 0) return KVQ_OK;
+  if (!key_cache || !value_cache || !k_aq || !v_aq || !block_table || !seq_lens || !out_k ||
+      !out_v || batch < 0 || num_blocks <= 0 || block_size <= 0 || head_size % 8 ||
+      num_kv_heads <= 0 || max_blocks <= 0 || batch > 65535)
+    return KVQ_ERR_INVALID;
+  const int64_t channels = static_cast<int64_t>(num_kv_heads) * head_size;
+  const int64_t table_rows = max_blocks * block_size;
+  if ((table_rows * (channels / 8) + 255) / 256 > 0x7fffffff) return KVQ_ERR_INVALID;
+  return kvq::for_each_cu_arg(
+      seq_lens, batch,
+      [&](const kvq::CuArg& arg, int64_t first, int64_t n, int64_t longest) -> int {
+        // past the table's pages a request's rows stay unwritten
+        return launch_dequant_gather(arg, nullptr, std::min(longest, table_rows), key_cache,
+                                     value_cache, block_size, channels, k_aq, v_aq, dtype,
+                                     block_table + first * max_blocks, max_blocks, n, out_k, out_v,
+                                     static_cast<hipStream_t>(stream));
+      });
 }
 
 extern "C" int64_t kvq_int8_decode_workspace_bytes(int64_t num_work, int num_heads,

@@ -90,6 +90,10 @@ SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
         _I,
         [_P, _P, _I64, _I, _I, _I, _P, _P, _I, _P, _I64, _P, _I64, _P, _P, _P],
     ),
+    "kvq_int8_dequant_gather_lens": (
+        _I,
+        [_P, _P, _I64, _I, _I, _I, _P, _P, _I, _P, _I64, _P, _I64, _P, _P, _P],
+    ),
     "kvq_selftest_mfma_f16": (_I, [_P, _P, _P, _P]),
     "kvq_selftest_lds_dma": (_I, [_P, _P, _P]),
     "kvq_selftest_lane_reductions": (_I, [_P, _P, _P]),
@@ -104,6 +108,10 @@ SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
         [_P, _P, _I, _P, _I, _I64, _I, _I, _P, _P, _P, _P, _I64, _I, _P],
     ),
     "kvq_fp8_pth_gather": (
+        _I,
+        [_P, _P, _P, _P, _I64, _I, _I, _I, _P, _I, _I64, _P, _I64, _P, _P, _I, _P],
+    ),
+    "kvq_fp8_pth_gather_lens": (
         _I,
         [_P, _P, _P, _P, _I64, _I, _I, _I, _P, _I, _I64, _P, _I64, _P, _P, _I, _P],
     ),

@@ -243,18 +243,15 @@ def fp8_per_token_head_dequant_gather(
     if total == 0:
         return out_k, out_v
     _native.require_gpu_tensors("fp8_per_token_head_dequant_gather", k_data, table)
-    cu = [0]
-    for n in lens:
-        cu.append(cu[-1] + n)
-    cu_t = torch.tensor(cu, dtype=torch.int64).to(dev, non_blocking=True)
+    lens_np = np.array(lens, dtype=np.int64)
     table = table.contiguous()
-    rc = _native.lib().kvq_fp8_pth_gather(
+    rc = _native.lib().kvq_fp8_pth_gather_lens(
         _native.ptr(k_data), _native.ptr(k_scale), _native.ptr(v_data), _native.ptr(v_scale),
         nb, bs, kvh, d, _native.ptr(table), _native.index_code(table.dtype), table.shape[1],
-        _native.ptr(cu_t), len(lens), _native.ptr(out_k), _native.ptr(out_v),
+        lens_np.ctypes.data, len(lens), _native.ptr(out_k), _native.ptr(out_v),
         _native.dtype_code(target_dtype), _native.stream_of(k_data),
     )
-    _native.check(rc, "kvq_fp8_pth_gather")
+    _native.check(rc, "kvq_fp8_pth_gather_lens")
     return out_k, out_v
 
 

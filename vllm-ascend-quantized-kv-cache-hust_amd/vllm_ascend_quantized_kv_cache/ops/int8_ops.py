@@ -119,16 +119,16 @@ def int8_dequant_gather(
     if total == 0:
         return out_k, out_v
     _native.require_gpu_tensors("int8_dequant_gather", key_cache, value_cache, block_table)
-    cu = torch.tensor(np.concatenate([[0], np.cumsum(seq_lens)]), dtype=torch.int64, device=dev)
+    lens = np.array(seq_lens, dtype=np.int64)
     bt = block_table.to(torch.int32).contiguous()
-    rc = _native.lib().kvq_int8_dequant_gather(
+    rc = _native.lib().kvq_int8_dequant_gather_lens(
         _native.ptr(key_cache), _native.ptr(value_cache), nb, bs, kvh, d,
         _native.ptr(k_aq.to(target_dtype).contiguous()),
         _native.ptr(v_aq.to(target_dtype).contiguous()), _native.dtype_code(target_dtype),
-        _native.ptr(bt), bt.shape[1], _native.ptr(cu), len(seq_lens), _native.ptr(out_k),
+        _native.ptr(bt), bt.shape[1], lens.ctypes.data, len(seq_lens), _native.ptr(out_k),
         _native.ptr(out_v), _native.stream_of(key_cache),
     )
-    _native.check(rc, "kvq_int8_dequant_gather")
+    _native.check(rc, "kvq_int8_dequant_gather_lens")
     return out_k, out_v
 
 
