@@ -687,7 +687,8 @@ def test_decode_combine_of_many_items_per_request(gpu_device):
     torch.testing.assert_close(got.float().cpu(), want, atol=1e-2, rtol=1e-2)
 
 
-def _split_decode_case(dev, d, kvh, g, bs, rep, dtype, plan_of, *, lens=None, stale=True):
+def _split_decode_case(dev, d, kvh, g, bs, rep, dtype, plan_of, *, lens=None, stale=True,
+                       q_offset=0):
     """A decode over stale pages against the oracle; ``plan_of(seqs) -> plan``."""
     from vllm_ascend_quantized_kv_cache.ops.kivi_decode import DecodeSeq, kivi_decode_attention
 
@@ -704,7 +705,9 @@ def _split_decode_case(dev, d, kvh, g, bs, rep, dtype, plan_of, *, lens=None, st
     plan = tuple(torch.from_numpy(x).to(dev) for x in plan_of(dseqs) if x is not None)
     print(f"split decode d={d} kvh={kvh} g={g} bs={bs} rep={rep} {dtype}: {plan[1].shape[0]} items",
           flush=True)
-    got = kivi_decode_attention(q.to(dev), to_dev(cpu, dev), table.to(dev), dseqs,
+    q_dev = torch.empty(q.numel() + q_offset, dtype=dtype, device=dev)[q_offset:].view(q.shape)
+    q_dev.copy_(q)
+    got = kivi_decode_attention(q_dev, to_dev(cpu, dev), table.to(dev), dseqs,
                                 ring_k.to(dev), ring_v.to(dev), d ** -0.5, g, plan=plan)
     got = got.float().cpu()
     assert torch.isfinite(got).all()
@@ -730,6 +733,15 @@ def test_split_decode_matches_oracle(gpu_device, d, kvh, g, bs, rep, dtype, cu_c
 
     _split_decode_case(gpu_device, d, kvh, g, bs, rep, dtype,
                        lambda s: plan_decode_pieces(s, kvh, cu_count))
+
+
+@pytest.mark.parametrize("d,kvh,rep", [(128, 2, 5), (256, 1, 8), (256, 1, 16)])
+def test_split_decode_query_off_its_alignment(gpu_device, d, kvh, rep):
+    """Queries 8 bytes off a 16-byte bound (the staging through LDS needs one)."""
+    from vllm_ascend_quantized_kv_cache.ops.kivi_decode import plan_decode_pieces
+
+    _split_decode_case(gpu_device, d, kvh, 128, 128, rep, torch.bfloat16,
+                       lambda s: plan_decode_pieces(s, kvh, 256), q_offset=4)
 
 
 @pytest.mark.parametrize("g,bs", [(128, 128), (64, 64)])

@@ -14,7 +14,7 @@
 //
 // Head size 256 had no MFMA path (the generic fp32 kernel: 4650 us for 64
 // requests of 1K-16K positions on 1 kv head, against 32 us for its 166 MB at
-// the copy rate).
+// the copy rate; 62 here).
 //
 // Tiles: 64 positions, decode_tr.h's layout and compute, double-buffered in the
 // wave's own LDS: the DMA of the next tile is in flight while one computes.  The
@@ -24,6 +24,14 @@
 //   D = 128: 2 workgroups a CU (8 x 19-20 KB of LDS), one piece a wave;
 //   D = 256: 1 workgroup a CU (4 x 38-40 KB), two pieces a wave where the plan
 //            has more of them than the chip holds waves.
+// What bounds it: at D = 256 the issue of one wave per SIMD (3.9 us a tile, of
+// them 0.95 waiting for its DMA, at 1500 vector and 300 scalar instructions), at
+// D = 128 the start: every wave's first tile, 20 MB over the chip, takes 5 - 6 of
+// 22 us on 40 requests of 1K-10K positions and 2 kv heads.  Hence the query rows
+// through LDS (the second tile leaves before the first is there), the key
+// group's operands kept over its two tiles, and MFMA results in ordinary
+// registers (a build flag): 69.1 -> 62.0 us on the 64 requests above, 58.4 ->
+// 52.6 on 20 of 0.5K-10K with 2 kv heads of 256, 40.5 -> 38.7 on the 40.
 #include <algorithm>
 
 #include "decode_tail.h"
@@ -132,16 +140,21 @@ kivi_decode_split_kernel(const TQ* __restrict__ query, int hq, int kvh, float qs
   const uint32_t ks_lane = static_cast<uint32_t>(KSV ? 16 * (lane % (D / 4)) : 4 * lane * gpb);
   const uint32_t vs_lane = static_cast<uint32_t>(
       4 * tr::tau((lane >> 3) & 3, 8 * (lane >> 5) + tr::slot_nib(lane & 7)) * kvh * NVG);
-  // DMA of the tile at position p of a request whose page there is blk
+  // DMA of the tile at position p of a request whose page there is blk.  At D =
+  // 128 the loops stay rolled: unrolled, their bases spill scalar registers
+  // (104 requests of 384 - 506 positions on 4 kv heads 37.7 us, rolled 37.0); at
+  // D = 256 rolled costs more than the spills (62.3 against 63.5).
+  constexpr int DMA_UNROLL = D == 256 ? 8 : 1;
   auto issue = [&](int64_t blk, int p, int buf) {
     const uint32_t m0 = my_off + static_cast<uint32_t>(buf * T::BYTES);
     const int off0 = p & (bs - 1);
     const int64_t krow = (blk * kvh + h) * D;
     const int64_t vtok = ((blk << bsh) + off0) * kvh + h;
     const char* kb = reinterpret_cast<const char*>(kq + krow * wpd + (off0 >> 3));
-#pragma unroll
-    for (int i = 0; i < T::KW_INST; ++i)
-      sdma16(kb + static_cast<int64_t>(128 * i) * wpd, k_lane, m0 + 4 * T::KW + 1024 * i);
+    const uint32_t kstep = 128u * static_cast<uint32_t>(wpd);
+#pragma unroll DMA_UNROLL
+    for (int i = 0; i < T::KW_INST; ++i, kb += kstep)
+      sdma16(kb, k_lane, m0 + 4 * T::KW + 1024 * i);
     const char* sb = reinterpret_cast<const char*>(ks + krow * gpb + (off0 >> gsh));
     const char* mb = reinterpret_cast<const char*>(km + krow * gpb + (off0 >> gsh));
     if constexpr (KSV && D == 256) {
@@ -159,11 +172,11 @@ kivi_decode_split_kernel(const TQ* __restrict__ query, int hq, int kvh, float qs
       }
     }
     const char* vb = reinterpret_cast<const char*>(vq + vtok * (D / 8));
-#pragma unroll
-    for (int i = 0; i < T::VW_INST; ++i) {
+    const uint32_t vstep = static_cast<uint32_t>(TPI * kvh * (D / 2));
+#pragma unroll DMA_UNROLL
+    for (int i = 0; i < T::VW_INST; ++i, vb += vstep) {
       const uint32_t pi = D == 128 ? i : 2 * (i >> 1);  // of token TPI * i
-      sdma16(vb + static_cast<int64_t>(TPI * i) * kvh * (D / 2), v_row + 16 * (v_chunk ^ pi),
-             m0 + 4 * T::VW + 1024 * i);
+      sdma16(vb, v_row + 16 * (v_chunk ^ pi), m0 + 4 * T::VW + 1024 * i);
     }
     const char* vsb = reinterpret_cast<const char*>(vs + vtok * NVG);
     const char* vmb = reinterpret_cast<const char*>(vm + vtok * NVG);
@@ -173,6 +186,21 @@ kivi_decode_split_kernel(const TQ* __restrict__ query, int hq, int kvh, float qs
       sdma4(vmb + 4 * vg, vs_lane, m0 + 4 * (T::VM + 64 * vg));
     }
   };
+  // The query rows of request b and this kv head into the second buffer: row r's
+  // 16-byte chunk c in its slot c ^ (r % 16), over the banks.
+  constexpr int QCH = D / 8;  // chunks per row
+  const bool q_aligned = (reinterpret_cast<uintptr_t>(query) & 15) == 0;
+  auto stage_q = [&](int b) {
+    const char* src = reinterpret_cast<const char*>(
+        query + (static_cast<int64_t>(b) * hq + h * rep) * D);
+#pragma unroll 1
+    for (int i = 0; i * 64 < rep * QCH; ++i) {
+      const int r = (64 * i + lane) / QCH, c = (lane % QCH) ^ (r & 15 & (QCH - 1));
+      sdma16(src, static_cast<uint32_t>(2 * D * min(r, rep - 1) + 16 * c),
+             my_off + static_cast<uint32_t>(T::BYTES) + 1024u * i);
+    }
+  };
+  static_assert(T::BYTES >= 16 * 2 * D, "16 query rows fit a tile buffer");
   auto page_of = [&](int b, int p) -> int64_t {
     const int64_t v = ctable[static_cast<int64_t>(b) * maxb + (p >> bsh)];
     return v < 0 ? 0 : (v >= nb ? nb - 1 : v);  // never leave the cache
@@ -213,13 +241,33 @@ kivi_decode_split_kernel(const TQ* __restrict__ query, int hq, int kvh, float qs
     int pb = cwork[4 * static_cast<int64_t>(it) + 1], pe = cwork[4 * static_cast<int64_t>(it) + 2];
     int p = kind >= 2 ? pb + 64 * (kind - 2) : pb & ~63;
     int64_t ahead = 0;  // page of the tile after the one issued last, in its item
+    // the query rows go ahead of the first tile, through the other buffer: a
+    // load to registers would be waited for with the tile behind it, and the
+    // second tile could not leave before the first is there
+    if (q_aligned) stage_q(run_b);
     if (p < pe) {
       issue(page_of(run_b, p), p, 0);
       ahead = page_of(run_b, p + st < pe ? p + st : pe - 1);
     }
-    const tr::QLane<TQ, D> ql = tr::load_q<TQ, D>(query, run_b, hq, h, rep, n, kg, FOLD);
+    tr::QLane<TQ, D> ql;
+    if (q_aligned) {
+      if (p < pe)
+        wait_vmcnt<T::NINST>();
+      else
+        wait_vmcnt<0>();
+      ql = tr::load_q_at<TQ, D>(
+          [&](int hn, int c) {
+            return reinterpret_cast<const TQ*>(my_lds + T::BYTES) + hn * D +
+                   8 * (c ^ (hn & 15 & (QCH - 1)));
+          },
+          rep, n, kg, FOLD);
+    } else {
+      ql = tr::load_q<TQ, D>(query, run_b, hq, h, rep, n, kg, FOLD);
+    }
     tr::Acc<NVG, DB> acc;
     acc.init();
+    tr::QGroup<D> qg;
+    int again = -1;  // the tile that shares the last prepared key group
     int cb = 0;
     while (p < pe) {
       // the tile after p: in this item, or the first of the item that continues it
@@ -247,8 +295,10 @@ kivi_decode_split_kernel(const TQ* __restrict__ query, int hq, int kvh, float qs
         wait_vmcnt<0>();
       }
       const uint32_t* W = reinterpret_cast<const uint32_t*>(my_lds + cb * T::BYTES);
-      tr::QGroup<D> qg;
-      tr::prepare_group<TQ, NVG, KSV, FOLD, D>(W, n, kg, ql, qscale, qg);
+      // the second tile of a 128-position key group runs on the first one's
+      // operands (unfolded, twice the operands, they spill if kept)
+      if (!FOLD || p != again) tr::prepare_group<TQ, NVG, KSV, FOLD, D>(W, n, kg, ql, qscale, qg);
+      again = ((p + 64) & (g - 1)) != 0 ? p + 64 : -1;
       const uint32_t off = my_off + static_cast<uint32_t>(cb * T::BYTES);
       if (p >= tb && p + 64 <= te)
         tr::compute_tile<NVG, KSV, FOLD, true, D>(W, off, p, tb, te, n, kg, qg, qscale, acc);

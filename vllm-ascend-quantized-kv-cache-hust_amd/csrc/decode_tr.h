@@ -237,17 +237,16 @@ __device__ __forceinline__ uint16_t bits16(TQ x) {
   return __builtin_bit_cast(uint16_t, x);
 }
 
-template <typename TQ, int D = 128>
-__device__ __forceinline__ QLane<TQ, D> load_q(const TQ* __restrict__ query, int b, int hq, int h,
-                                            int rep, int n, int kg, bool fold) {
+// at(hn, c): the 8 values of 16-byte chunk c of head hn's row.
+template <typename TQ, int D, typename F>
+__device__ __forceinline__ QLane<TQ, D> load_q_at(F&& at, int rep, int n, int kg, bool fold) {
   QLane<TQ, D> ql;
   const int hn = fold ? (n & 7) : n;
   const bool live = hn < rep;
-  const TQ* qrow = query + (static_cast<int64_t>(b) * hq + h * rep + (live ? hn : 0)) * D;
 #pragma unroll
   for (int s = 0; s < D / 32; ++s) {
     float x[8];
-    load8(qrow + 64 * (s >> 1) + 16 * kg + 8 * (s & 1), x);
+    load8(at(live ? hn : 0, 8 * (s >> 1) + 2 * kg + (s & 1)), x);
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
       float a = live ? x[slot_nib(2 * p)] : 0.0f;
@@ -268,6 +267,13 @@ __device__ __forceinline__ QLane<TQ, D> load_q(const TQ* __restrict__ query, int
     }
   }
   return ql;
+}
+
+template <typename TQ, int D = 128>
+__device__ __forceinline__ QLane<TQ, D> load_q(const TQ* __restrict__ query, int b, int hq, int h,
+                                               int rep, int n, int kg, bool fold) {
+  const TQ* rows = query + (static_cast<int64_t>(b) * hq + h * rep) * D;
+  return load_q_at<TQ, D>([&](int hn, int c) { return rows + hn * D + 8 * c; }, rep, n, kg, fold);
 }
 
 // B operands of one key group: Q' = q * key_scale as fp16 hi + lo parts (the
