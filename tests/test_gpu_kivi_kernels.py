@@ -765,6 +765,24 @@ def test_split_decode_two_pieces_a_wave_and_long_combine(gpu_device):
                        lambda s: plan_decode_pieces(s, 1, 256), lens=lens, stale=False)
 
 
+@pytest.mark.parametrize("d", [128, 256])
+def test_combine_of_item_counts_at_its_edges(gpu_device, d):
+    """15 to 18 items a request (rows ahead of the weights, or only the live ones
+    after them) and 63 to 67 (one chunk of weights, or two)."""
+    from vllm_ascend_quantized_kv_cache.ops.kivi_decode import plan_decode_work
+
+    lens = [128 * n + 1 for n in (14, 15, 16, 17, 62, 63, 64, 65)]
+    counts = []
+
+    def plan(seqs):
+        meta, work = plan_decode_work(seqs, 128)
+        counts.extend(meta[:, 7].tolist())
+        return meta, work
+
+    _split_decode_case(gpu_device, d, 1, 128, 128, 4, torch.bfloat16, plan, lens=lens, stale=False)
+    assert {16, 17} <= set(counts) and {64, 65} <= set(counts), counts
+
+
 @pytest.mark.parametrize("d,kvh,g,bs", [(128, 2, 128, 128), (256, 1, 64, 64), (256, 2, 128, 128)])
 def test_split_decode_with_row_maxima_growing_every_tile(gpu_device, d, kvh, g, bs):
     """Keys along one direction with a magnitude that grows with the position:

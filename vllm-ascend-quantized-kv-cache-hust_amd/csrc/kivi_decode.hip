@@ -296,10 +296,13 @@ namespace kvq {
 // head), four heads per workgroup.  Lane s holds item s's (m, l) of the current
 // chunk of 64 items; the weights 2^(m_s - max) go to every lane through
 // readlane, and each lane accumulates columns lane + 64*k of sum_s w_s * o_s.
-// The o rows of the first kPre items are loaded before the (m, l) pass, so a
-// request with up to kPre items costs one round trip to memory instead of one
-// per few items; of the others only those with weight are read, four at a time
-// (the split decode leaves most items of a long request to another's partial).
+// The o rows of a request with up to kPre items are loaded before the (m, l)
+// pass, one round trip to memory for the whole combine.  Of a longer request
+// only the rows with weight are read, kPre at a time, after the pass: the split
+// decode leaves most items of a long request to another's partial (2 requests of
+// 5K - 14K positions, some 100 items each: 21.5 us a decode with the first kPre
+// rows ahead and the others four at a time, 18.9 so; 64 requests of some 32
+// items at head size 256: 61.6 and 60.3).
 // Items with m = -inf (no position) carry weight 0 and their o never reaches
 // the sum (selected out, so stale bytes cannot turn it NaN).
 template <typename TO, int KD>
@@ -326,16 +329,19 @@ decode_combine_kernel(int hq, int d, const int32_t* __restrict__ seq_meta, int m
   }
   const int64_t stride = static_cast<int64_t>(hq) * d;
   const float* rows = ws_o + (static_cast<int64_t>(fw) * hq + hh) * d;
+  const bool few = nw <= kPre;  // uniform
   float pre[kPre][KD];
+  if (few) {
 #pragma unroll
-  for (int j = 0; j < kPre; ++j)
+    for (int j = 0; j < kPre; ++j)
 #pragma unroll
-    for (int k = 0; k < KD; ++k) {
-      const int c = lane + 64 * k;
-      // rows past the request or columns past d are read in bounds (item 0,
-      // column 0) and never used
-      pre[j][k] = rows[(j < nw ? j * stride : 0) + (c < d ? c : 0)];
-    }
+      for (int k = 0; k < KD; ++k) {
+        const int c = lane + 64 * k;
+        // rows past the request or columns past d are read in bounds (item 0,
+        // column 0) and never used
+        pre[j][k] = rows[(j < nw ? j * stride : 0) + (c < d ? c : 0)];
+      }
+  }
   // (m, l) of the first 64 items in one 8-byte load per lane, kept for the
   // weights below: one round trip to memory for the whole combine when the
   // request has at most 64 items
@@ -372,20 +378,20 @@ decode_combine_kernel(int hq, int d, const int32_t* __restrict__ seq_meta, int m
       }
     }
     uint64_t live = __builtin_amdgcn_ballot_w64(wgt != 0.0f);
-    if (s0 == 0) {
+    if (few) {
 #pragma unroll
       for (int j = 0; j < kPre; ++j) {
         const float wj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), j));
 #pragma unroll
         for (int k = 0; k < KD; ++k) acc[k] += wj != 0.0f ? wj * pre[j][k] : 0.0f;
       }
-      live &= ~uint64_t{0} << kPre;
+      break;
     }
     const float* row0 = rows + s0 * stride;
     while (live) {  // uniform; the rows with weight, in item order
-      float wj[4], x[4][KD];
+      float wj[kPre];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < kPre; ++i) {
         const int j = live ? __builtin_ctzll(live) : 0;
         wj[i] = live ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), j)) : 0.0f;
         live &= live - 1;  // 0 stays 0
@@ -393,13 +399,13 @@ decode_combine_kernel(int hq, int d, const int32_t* __restrict__ seq_meta, int m
 #pragma unroll
         for (int k = 0; k < KD; ++k) {
           const int c = lane + 64 * k;
-          x[i][k] = row[c < d ? c : 0];  // columns past d are read in bounds, unused
+          pre[i][k] = row[c < d ? c : 0];  // columns past d are read in bounds, unused
         }
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < kPre; ++i)
 #pragma unroll
-        for (int k = 0; k < KD; ++k) acc[k] += wj[i] != 0.0f ? wj[i] * x[i][k] : 0.0f;
+        for (int k = 0; k < KD; ++k) acc[k] += wj[i] != 0.0f ? wj[i] * pre[i][k] : 0.0f;
     }
   }
   wsum = sum_wave64(wsum);
