@@ -431,20 +431,22 @@ int kvq_fp8_pth_gather_lens(const uint8_t* k_data, const float* k_scale, const u
                             int block_index_type, int64_t max_blocks, const int64_t* seq_lens,
                             int64_t batch, void* out_k, void* out_v, int out_dtype, void* stream);
 
-/* Fused decode attention over the paged E4M3 codes: one query row per request
- * over its seq_lens[b] positions (host int64 [batch]; 0 gives zeros),
+/* Fused decode attention over the paged E4M3 codes: `rows` query rows per
+ * request, its last positions, over its seq_lens[b] positions (host int64
+ * [batch]; 0 gives zeros; causal: row j sees the first seq_lens[b] - rows + 1 + j),
  *   K = float(code) * k_scale[token, head], V likewise, softmax in fp32.
- * query/out [batch, num_heads, D] of `dtype` (bf16 / fp16), D 128 or 256,
+ * query/out [batch * rows, num_heads, D] of `dtype` (bf16 / fp16), D 128 or 256,
  * block_size % 16 == 0, at most 16 query heads per kv head; other geometries
  * return KVQ_ERR_GEOMETRY.  Block ids as for kvq_fp8_pth_gather.  The lengths
  * are read during the call and travel with the launches; `workspace` holds
  * kvq_fp8_pth_decode_workspace_bytes for the same lengths.
  * The read path the reference lacks for this scheme, as kvq_fp8_pth_gather
  * followed by kvq_prefill_attn would compute it, without the dense rows. */
-int64_t kvq_fp8_pth_decode_workspace_bytes(const int64_t* seq_lens, int64_t batch, int num_heads,
-                                           int num_kv_heads, int head_size, int block_size);
-int kvq_fp8_pth_decode_attn(const void* query, int dtype, int64_t batch, int num_heads,
-                            int num_kv_heads, int head_size, float scale, const uint8_t* k_data,
+int64_t kvq_fp8_pth_decode_workspace_bytes(const int64_t* seq_lens, int64_t batch, int64_t rows,
+                                           int num_heads, int num_kv_heads, int head_size,
+                                           int block_size);
+int kvq_fp8_pth_decode_attn(const void* query, int dtype, int64_t batch, int64_t rows, int causal,
+                            int num_heads, int num_kv_heads, int head_size, float scale, const uint8_t* k_data,
                             const float* k_scale, const uint8_t* v_data, const float* v_scale,
                             int64_t num_blocks, int block_size, const void* block_table,
                             int block_index_type, int64_t max_blocks, const int64_t* seq_lens,

@@ -250,7 +250,7 @@ def test_full_size_round_trip_of_grid_values(gpu_device):
     assert torch.equal(views[1].view(-1, kvh)[slots], torch.exp2(k).view(t, kvh))
 
 
-def _decode_case(dev, lens, *, d, kvh, rep, bs, dtype, index, seed=5):
+def _decode_case(dev, lens, *, d, kvh, rep, bs, dtype, index, seed=5, rows=1, causal=True):
     """A decode over pages whose unwritten bytes are NaN codes and scales."""
     gen = torch.Generator().manual_seed(seed)
     need = [-(-n // bs) for n in lens]
@@ -269,16 +269,18 @@ def _decode_case(dev, lens, *, d, kvh, rep, bs, dtype, index, seed=5):
     x = [(torch.randn((sum(lens), kvh, d), generator=gen) * 10 ** float(e)).to(dtype)
          for e in (0, -3)]  # small values: their scales leave the fp16 range
     fp8_ops.fp8_per_token_head_store(x[0].to(dev), x[1].to(dev), torch.cat(slots).to(dev), *views)
-    q = torch.randn((len(lens), kvh * rep, d), generator=gen).to(dtype)
+    q = torch.randn((rows * len(lens), kvh * rep, d), generator=gen).to(dtype)
     got = fp8_ops.fp8_per_token_head_attention(
-        q.to(dev), *views, table.to(dev), lens, [1] * len(lens), d ** -0.5,
+        q.to(dev), *views, table.to(dev), lens, [rows] * len(lens), d ** -0.5, causal=causal,
         block_table_host=table.numpy())
     torch.cuda.synchronize()
     dk, dv = ref.fp8_pth_gather(*[v.cpu() for v in views], table, lens, torch.float32)
-    live = [b for b, n in enumerate(lens) if n]
+    # only rows with a position to see reach the oracle; the others are zeros
+    live = [(b, min(rows, n) if causal else rows) for b, n in enumerate(lens) if n]
+    at = torch.cat([torch.arange(rows * b + rows - m, rows * (b + 1)) for b, m in live])
     want = torch.zeros(q.shape)
-    want[live] = ref.attention(q[live].float(), dk, dv, [1] * len(live),
-                               [lens[b] for b in live], d ** -0.5, True)
+    want[at] = ref.attention(q[at].float(), dk, dv, [m for _, m in live],
+                             [lens[b] for b, _ in live], d ** -0.5, causal)
     # the output's rounding, on values of 1e-3
     rel = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
     torch.testing.assert_close(got.float().cpu(), want, atol=1e-3 * 2 * rel, rtol=2 * rel)
@@ -298,6 +300,26 @@ def test_decode_over_paged_codes(gpu_device, d, kvh, rep, bs, dtype, index):
     the 16-token group, an empty request, requests cut into several items."""
     _decode_case(gpu_device, [150, 0, 1, 15, 16, 17, 31, 32, 33, 64, 700], d=d, kvh=kvh, rep=rep,
                  bs=bs, dtype=dtype, index=index)
+
+
+@pytest.mark.parametrize("d,kvh,rep,bs,dtype,rows", [
+    (128, 8, 4, 128, torch.bfloat16, 4),   # a full set of score columns
+    (128, 2, 7, 16, torch.float16, 2),     # 14 columns
+    (128, 1, 7, 64, torch.bfloat16, 5),    # three passes, the last of one row
+    (128, 16, 1, 32, torch.float16, 33),   # one wave per head; 16, 16 and 1 rows
+    (256, 1, 8, 128, torch.bfloat16, 3),
+    (256, 2, 16, 16, torch.float16, 2),    # a pass per row
+])
+@pytest.mark.parametrize("causal", [True, False])
+def test_decode_of_a_few_rows(gpu_device, d, kvh, rep, bs, dtype, rows, causal):
+    """Several rows per request in one pass over its codes, each with its own end:
+    ends on both sides of the tiles, requests shorter than their rows."""
+    assert fp8_ops._decode_applies(
+        torch.empty((rows, kvh * rep, d), dtype=dtype, device=gpu_device),
+        torch.empty((1, bs, kvh, d), dtype=torch.uint8, device=gpu_device),
+        torch.empty((1, 1), dtype=torch.int32, device=gpu_device), [rows], 0.1)
+    _decode_case(gpu_device, [150, 0, 1, 2, 16, 17, 31, 32, 33, 34, 64, 129, 700], d=d, kvh=kvh,
+                 rep=rep, bs=bs, dtype=dtype, index=torch.int32, rows=rows, causal=causal)
 
 
 def test_decode_over_paged_codes_long_request_and_large_batch(gpu_device):

@@ -239,13 +239,14 @@ __device__ __forceinline__ float add_ror8(float x) {
   return x + __int_as_float(y);
 }
 
+// pb, pe: the item's positions; pen: where those of the lane's column end.
 // FOLD (GQA groups of at most 8 heads): qh carries the hi part of head n in
 // columns n < 8 and the lo part of head n - 8 in columns n >= 8, so one MFMA
 // per k-step gives both partial scores and a rotate-by-8 add sums them (both
 // lanes then hold head n % 8's score; ql unused).
 template <typename TQ, int D, bool FOLD, bool FP8>
 __device__ __forceinline__ void compute_tile(const TileRegs<D, FP8>& t, int p, int pb, int pe,
-                                             const u4v (&qh)[D / 32], const u4v (&ql)[D / 32],
+                                             int pen, const u4v (&qh)[D / 32], const u4v (&ql)[D / 32],
                                              float sc, int g, SoftmaxState<D>& st) {
   // ---- S^T = K * Q'^T: 2 groups of 16 tokens ----
   f4 s[2];
@@ -285,7 +286,7 @@ __device__ __forceinline__ void compute_tile(const TileRegs<D, FP8>& t, int p, i
     for (int r = 0; r < 4; ++r) {
       const int tok = p + 16 * j + 4 * g + r;
       const float x = FP8 ? s[j][r] * (sc * t.ksc[j][r]) : s[j][r] * sc;
-      const float v = (tok >= pb && tok < pe) ? x : -INFINITY;
+      const float v = (tok >= pb && tok < pen) ? x : -INFINITY;
       s[j][r] = v;
       mx = fmaxf(mx, v);
     }
@@ -326,7 +327,7 @@ __device__ __forceinline__ void compute_tile(const TileRegs<D, FP8>& t, int p, i
       for (int k = 0; k < 2; ++k) {
         // past the item p = 0, but the scale may be unwritten: no 0 * NaN
         const int tok = p + 16 * j + 4 * g + r + k;
-        y[k] = tok >= pb && tok < pe ? s[j][r + k] * t.vsc[j][r + k] : 0.0f;
+        y[k] = tok >= pb && tok < pen ? s[j][r + k] * t.vsc[j][r + k] : 0.0f;
       }
       ph[u] = bf16x2_bits(y[0], y[1]);
       pl[u] = bf16x2_bits(y[0] - __uint_as_float(ph[u] << 16),
@@ -420,8 +421,9 @@ __device__ __forceinline__ int wave_prefix(int x, int lane) {
   return x;
 }
 
-// Request and positions of item wi; false past the last one (wave-uniform).
-__device__ __forceinline__ bool find_item(int wi, int lane, int& b, int& pb, int& pe) {
+// Request, its length and the positions of item wi; false past the last one
+// (wave-uniform).
+__device__ __forceinline__ bool find_item(int wi, int lane, int& b, int& l, int& pb, int& pe) {
   cint32* a = lens_arg();
   const int n = a[0], split = a[1];
   int base = 0;
@@ -432,7 +434,7 @@ __device__ __forceinline__ bool find_item(int wi, int lane, int& b, int& pb, int
     const uint64_t past = __builtin_amdgcn_ballot_w64(upto > wi);
     if (past) {
       const int at = __builtin_ctzll(past);
-      const int l = __builtin_amdgcn_readlane(len, at);
+      l = __builtin_amdgcn_readlane(len, at);
       const int first = __builtin_amdgcn_readlane(upto - items, at);
       b = c + at;
       pb = (wi - first) * split;
@@ -468,9 +470,22 @@ __device__ __forceinline__ void write_meta(int lane, int32_t* __restrict__ meta)
 // heads' K and V lines interleave in HBM, are requested together: the DRAM
 // pages open once for all heads instead of once per head (config-2 decode
 // 111.5 -> 101 us, one 8-wave workgroup per CU).
+//
+// E4M3 with several query rows per request (RowCols): the columns of the score
+// MFMA are the rows' heads, each with its own last position, so that 16 / rep
+// rows share one pass over the codes.  32 requests of 0.5K-8K positions, 32 heads
+// on 8 kv heads: 77 us for 4 rows, 138 for 8 (two passes), 246 for 16 (four);
+// gathered to dense rows first they take 294, 302 and 310.
+struct RowCols {
+  int rows;   // query rows of a request
+  int first;  // first of them in this pass
+  int take;   // rows of this pass, take * rep <= 16
+  int limit;  // positions the first row of the request sees; one more per row if step
+  int step;
+};
 template <typename TQ, int D, bool FOLD, bool FP8>
 __device__ __forceinline__ void decode_item(
-    const TQ* __restrict__ query, int hq, int kvh, int hpw, int h, float qscale,
+    const TQ* __restrict__ query, RowCols rc, int hq, int kvh, int hpw, int h, float qscale,
     const int8_t* __restrict__ kc, const int8_t* __restrict__ vc, const float* __restrict__ ks,
     const float* __restrict__ vs, int bs, int64_t nb, const TQ* __restrict__ k_aq,
     const TQ* __restrict__ v_aq, const void* __restrict__ table_row, int bt64, int wi, int b,
@@ -481,9 +496,18 @@ __device__ __forceinline__ void decode_item(
   const int g = lane >> 4;
   u4v qh[D / 32], ql[D / 32];
   float sc = qscale;
+  // column c's row among the request's rows * hq (E4M3), and the end of its positions
+  const int cols = FP8 ? rep * rc.take : rep;
+  auto col_head = [&](int c) {
+    const int j = FP8 ? c / rep : 0;
+    return (FP8 ? rc.first + j : 0) * hq + h * rep + (c - j * rep);
+  };
+  const int heads = FP8 ? rc.rows * hq : hq;
+  int pen = pe;
   if constexpr (FP8) {
-    const bool live = n < rep;
-    const TQ* qrow = query + (static_cast<int64_t>(b) * hq + h * rep + (live ? n : 0)) * D;
+    const bool live = n < cols;
+    pen = min(pe, rc.limit + rc.step * (rc.first + (live ? n / rep : 0)));
+    const TQ* qrow = query + (static_cast<int64_t>(b) * heads + col_head(live ? n : 0)) * D;
 #pragma unroll
     for (int s = 0; s < D / 32; ++s) {
       const u4v x = *reinterpret_cast<const u4v*>(qrow + (D / 4) * g + 8 * s);
@@ -573,7 +597,7 @@ __device__ __forceinline__ void decode_item(
     }
     TileRegs<D, FP8> t;
     read_tile_lds<D, FP8>(t, cur, g, n);
-    compute_tile<TQ, D, FOLD, FP8>(t, p, pb, pe, qh, ql, sc, g, st);
+    compute_tile<TQ, D, FOLD, FP8>(t, p, pb, pe, pen, qh, ql, sc, g, st);
   };
   if (p0 < pe) issue_tile_dma<D, FP8>(lds_i8, c, p0, lane);  // an empty range leaves m = -inf, l = 0
   int cur = 0;
@@ -593,12 +617,12 @@ __device__ __forceinline__ void decode_item(
 #pragma unroll
   for (int tt = 0; tt < DPL; ++tt)
     va[tt] = FP8 ? 1.0f : to_f32(v_aq[static_cast<int64_t>(h) * D + DPL * n + tt]);
-  const int64_t head0 = static_cast<int64_t>(wi) * hq + static_cast<int64_t>(h) * rep;
+  const int64_t head0 = static_cast<int64_t>(wi) * heads;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int hh = 4 * g + r;
-    if (hh < rep) {
-      float* dst = ws_o + (head0 + hh) * D + DPL * n;
+    if (hh < cols) {
+      float* dst = ws_o + (head0 + col_head(hh)) * D + DPL * n;
 #pragma unroll
       for (int w = 0; w < D / 64; ++w) {
         float4 x;
@@ -610,9 +634,10 @@ __device__ __forceinline__ void decode_item(
       }
     }
   }
-  if (g == 0 && n < rep) {
-    ws_ml[2 * (head0 + n)] = st.m;
-    ws_ml[2 * (head0 + n) + 1] = l;
+  if (g == 0 && n < cols) {
+    const int64_t hh = head0 + col_head(n);
+    ws_ml[2 * hh] = st.m;
+    ws_ml[2 * hh + 1] = l;
   }
 }
 
@@ -644,7 +669,7 @@ int8_decode_mfma_kernel(const TQ* __restrict__ query, int hq, int kvh, int hpw, 
     return;
   }
   const int b = wk[0];
-  decode_item<TQ, D, FOLD, false>(query, hq, kvh, hpw, h, qscale, kc, vc, nullptr, nullptr, bs, nb,
+  decode_item<TQ, D, FOLD, false>(query, RowCols{}, hq, kvh, hpw, h, qscale, kc, vc, nullptr, nullptr, bs, nb,
                                   k_aq, v_aq, block_table + static_cast<int64_t>(b) * maxb, 0, wi,
                                   b, wk[1], wk[2], lds_wg + wave * 2 * tile_bytes<D, false>(), lane,
                                   ws_o, ws_ml);
@@ -654,7 +679,8 @@ int8_decode_mfma_kernel(const TQ* __restrict__ query, int hq, int kvh, int hpw, 
 // leaves the combine's (first item, items) per request in meta.
 template <typename TQ, int D>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
-fp8_decode_mfma_kernel(SeqLens lens, const TQ* __restrict__ query, int hq, int kvh, int hpw,
+fp8_decode_mfma_kernel(SeqLens lens, const TQ* __restrict__ query, int rows, int take, int causal,
+                       int hq, int kvh, int hpw,
                        float qscale, const uint8_t* __restrict__ kc, const float* __restrict__ ks,
                        const uint8_t* __restrict__ vc, const float* __restrict__ vs, int bs,
                        int64_t nb, const void* __restrict__ block_table, int bt64, int64_t maxb,
@@ -666,11 +692,15 @@ fp8_decode_mfma_kernel(SeqLens lens, const TQ* __restrict__ query, int hq, int k
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int h = (blockIdx.x - wi * groups) * hpw + wave;
   const int lane = threadIdx.x & 63;
-  if (blockIdx.x == 0 && wave == 0) write_meta(lane, meta);
-  int b, pb, pe;
-  if (!find_item(wi, lane, b, pb, pe)) return;  // workgroup-uniform
+  if (blockIdx.x == 0 && blockIdx.y == 0 && wave == 0) write_meta(lane, meta);
+  int b, len, pb, pe;
+  if (!find_item(wi, lane, b, len, pb, pe)) return;  // workgroup-uniform
+  // blockIdx.y: the pass, `take` of the request's rows
+  const int first = static_cast<int>(blockIdx.y) * take;
+  const RowCols rc{rows, first, min(take, rows - first), causal ? len - rows + 1 : len,
+                   causal ? 1 : 0};
   const char* row = static_cast<const char*>(block_table) + b * maxb * (bt64 ? 8 : 4);
-  decode_item<TQ, D, false, true>(query, hq, kvh, hpw, h, qscale,
+  decode_item<TQ, D, false, true>(query, rc, hq, kvh, hpw, h, qscale,
                                   reinterpret_cast<const int8_t*>(kc),
                                   reinterpret_cast<const int8_t*>(vc), ks, vs, bs, nb, nullptr,
                                   nullptr, row, bt64, wi, b, pb, pe,
@@ -739,6 +769,8 @@ int64_t fp8_split(const int64_t* lens, int64_t n, int kvh, int d, int cus) {
   return split;
 }
 
+constexpr int64_t kMaxRowHeads = 65536;  // rows * query heads of a request (the combine's grid)
+
 struct Fp8Plan {
   int64_t first, n, split, items;  // requests [first, first + n) of one launch
 };
@@ -773,8 +805,10 @@ int64_t fp8_ws_bytes(int64_t items, int64_t n, int hq, int d) {
 }  // namespace
 
 extern "C" int64_t kvq_fp8_pth_decode_workspace_bytes(const int64_t* seq_lens, int64_t batch,
-                                                      int num_heads, int num_kv_heads,
-                                                      int head_size, int block_size) {
+                                                      int64_t rows, int num_heads,
+                                                      int num_kv_heads, int head_size,
+                                                      int block_size) {
+  if (rows <= 0 || rows * std::max(1, num_heads) > kMaxRowHeads) return KVQ_ERR_INVALID;
   if (batch < 0 || (batch > 0 && !seq_lens)) return KVQ_ERR_INVALID;
   if (!fp8_decode_geometry(num_heads, num_kv_heads, head_size, block_size))
     return KVQ_ERR_GEOMETRY;
@@ -782,14 +816,15 @@ extern "C" int64_t kvq_fp8_pth_decode_workspace_bytes(const int64_t* seq_lens, i
     if (seq_lens[b] < 0 || seq_lens[b] > 0x7fff0000) return KVQ_ERR_INVALID;
   int64_t most = 0;  // launches run one after another on one stream and share it
   const int rc = fp8_launches(seq_lens, batch, num_kv_heads, head_size, [&](const Fp8Plan& p) {
-    most = std::max(most, fp8_ws_bytes(p.items, p.n, num_heads, head_size));
+    most = std::max(most, fp8_ws_bytes(p.items, p.n, rows * num_heads, head_size));
     return KVQ_OK;
   });
   return rc != KVQ_OK ? KVQ_ERR_INVALID : most;
 }
 
-extern "C" int kvq_fp8_pth_decode_attn(const void* query, int dtype, int64_t batch, int num_heads,
-                                       int num_kv_heads, int head_size, float scale,
+extern "C" int kvq_fp8_pth_decode_attn(const void* query, int dtype, int64_t batch, int64_t rows,
+                                       int causal, int num_heads, int num_kv_heads,
+                                       int head_size, float scale,
                                        const uint8_t* k_data, const float* k_scale,
                                        const uint8_t* v_data, const float* v_scale,
                                        int64_t num_blocks, int block_size,
@@ -803,6 +838,7 @@ extern "C" int kvq_fp8_pth_decode_attn(const void* query, int dtype, int64_t bat
   if (block_index_type != KVQ_INDEX_I32 && block_index_type != KVQ_INDEX_I64)
     return KVQ_ERR_INVALID;
   if (!(scale > 0.0f)) return KVQ_ERR_INVALID;
+  if (rows <= 0 || rows * std::max(1, num_heads) > kMaxRowHeads) return KVQ_ERR_INVALID;
   if ((dtype != KVQ_DTYPE_BF16 && dtype != KVQ_DTYPE_F16) ||
       !fp8_decode_geometry(num_heads, num_kv_heads, head_size, block_size))
     return KVQ_ERR_GEOMETRY;
@@ -819,10 +855,13 @@ extern "C" int kvq_fp8_pth_decode_attn(const void* query, int dtype, int64_t bat
   const int bt64 = block_index_type == KVQ_INDEX_I64;
   hipStream_t s = static_cast<hipStream_t>(stream);
   float* ws_o = static_cast<float*>(workspace);
-  const int64_t row = static_cast<int64_t>(num_heads) * d * 2;  // bytes of a 16-bit query row
+  const int heads = static_cast<int>(rows) * num_heads;  // of a request
+  const int64_t row = static_cast<int64_t>(heads) * d * 2;  // bytes of its 16-bit query rows
+  const int take = std::min<int>(static_cast<int>(rows), 16 / (num_heads / kvh));
+  const unsigned passes = static_cast<unsigned>((rows + take - 1) / take);
   return fp8_launches(seq_lens, batch, kvh, d, [&](const Fp8Plan& p) -> int {
-    float* ws_ml = ws_o + p.items * num_heads * d;
-    int32_t* meta = reinterpret_cast<int32_t*>(ws_ml + 2 * p.items * num_heads);
+    float* ws_ml = ws_o + p.items * heads * d;
+    int32_t* meta = reinterpret_cast<int32_t*>(ws_ml + 2 * p.items * heads);
     // a launch with nothing to read still writes the table (and the zeros)
     const int64_t blocks = std::max<int64_t>(1, p.items) * (kvh / hpw);
     if (blocks > 0x7fffffff) return KVQ_ERR_INVALID;
@@ -833,9 +872,10 @@ extern "C" int kvq_fp8_pth_decode_attn(const void* query, int dtype, int64_t bat
     const char* q = static_cast<const char*>(query) + p.first * row;
     const char* bt = static_cast<const char*>(block_table) + p.first * max_blocks * (bt64 ? 8 : 4);
 #define KVQ_LAUNCH_FP8(TQ, D)                                                                  \
-  hipLaunchKernelGGL((fp8_decode_mfma_kernel<TQ, D>), dim3(static_cast<unsigned>(blocks)),     \
-                     dim3(64 * hpw), hpw * wave_lds, s, lens, reinterpret_cast<const TQ*>(q),  \
-                     num_heads, kvh, hpw, qscale, k_data, k_scale, v_data, v_scale, block_size, \
+  hipLaunchKernelGGL((fp8_decode_mfma_kernel<TQ, D>),                                          \
+                     dim3(static_cast<unsigned>(blocks), passes), dim3(64 * hpw),              \
+                     hpw * wave_lds, s, lens, reinterpret_cast<const TQ*>(q),                  \
+                     static_cast<int>(rows), take, causal, num_heads, kvh, hpw, qscale, k_data, k_scale, v_data, v_scale, block_size, \
                      num_blocks, bt, bt64, max_blocks, ws_o, ws_ml, meta)
     if (dtype == KVQ_DTYPE_BF16) {
       if (d == 128) KVQ_LAUNCH_FP8(kvq::bf16, 128); else KVQ_LAUNCH_FP8(kvq::bf16, 256);
@@ -844,7 +884,7 @@ extern "C" int kvq_fp8_pth_decode_attn(const void* query, int dtype, int64_t bat
     }
 #undef KVQ_LAUNCH_FP8
     KVQ_LAUNCH_CHECK();
-    return kvq::launch_decode_combine(dtype, p.n, num_heads, d, meta, 2, 0, ws_o, ws_ml,
+    return kvq::launch_decode_combine(dtype, p.n, heads, d, meta, 2, 0, ws_o, ws_ml,
                                       static_cast<char*>(out) + p.first * row, s);
   });
 }
