@@ -113,7 +113,7 @@ int kvq_kivi_ring_write(const void* src, int src_dtype, const int64_t* src_rows,
  * sources index [ring rows (ring_rows of them) ; input rows]; ring src are
  * input rows, ring dst ring rows.  Inputs and rings are [rows, KVH, D] of
  * `dtype`.  Precondition: no ring dst is a pack source of the same side (the
- * batch then has no order inside it).  Head size 128, group size 64 or 128,
+ * batch then has no order inside it).  Head size 128 or 256, group size 64 or 128,
  * bf16/fp16 only: other geometries return KVQ_ERR_GEOMETRY and the caller
  * uses the separate entry points.  n_key_pack % group_size == 0 with the
  * group rules of kvq_kivi_pack_key. */

@@ -159,3 +159,18 @@ def test_store_large_batch_matches_oracle(gpu_device, g):
         names = ("k_quant", "k_scale", "k_mn", "v_quant", "v_scale", "v_mn")
         for name, a, b in zip(names, want, got):
             assert torch.equal(a.view(torch.int32), b.cpu().view(torch.int32)), f"{name} differs"
+
+
+@pytest.mark.parametrize("g", [64, 128])
+@pytest.mark.parametrize("kvh", [1, 3])
+def test_store_heads_of_256(gpu_device, monkeypatch, g, kvh):
+    """Heads of 256 dims run as pairs of 128: the same batches as above, against
+    the oracle, and one launch against the separate ones."""
+    import sys
+
+    here = sys.modules[__name__]
+    monkeypatch.setattr(here, "D", 256)
+    monkeypatch.setattr(here, "KVH", kvh)
+    test_store_large_batch_matches_oracle(gpu_device, g)
+    for dtype in (torch.bfloat16, torch.float16):
+        test_store_one_launch_matches_separate_launches(gpu_device, "all", g, dtype)

@@ -340,13 +340,18 @@ extern "C" int kvq_kivi_gather_dequant(const int32_t* k_quant, const float* k_sc
     return KVQ_ERR_GEOMETRY;
   if (ring_meta && (!ring_k || !ring_v || ring_len <= 0)) return KVQ_ERR_INVALID;
   if (batch > 65535 || num_kv_heads > 65535 || max_blocks > 0x7fffffff) return KVQ_ERR_INVALID;
-  const size_t lds = sizeof(uint32_t) * (block_size / 8) * (head_size + 4) +
-                     2 * sizeof(float) * head_size * (block_size / group_size);
-  if (lds > 160 * 1024) return KVQ_ERR_GEOMETRY;
-  const dim3 grid(static_cast<unsigned>(max_blocks), static_cast<unsigned>(batch),
-                  num_kv_heads);
+  auto lds_bytes = [&]() {
+    return sizeof(uint32_t) * (block_size / 8) * (head_size + 4) +
+           2 * sizeof(float) * head_size * (block_size / group_size);
+  };
+  if (lds_bytes() > 160 * 1024) return KVQ_ERR_GEOMETRY;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int rdt = ring_meta ? ring_dtype : out_dtype;
+  if ((group_size == 64 || group_size == 128) && block_size % 32 == 0 && block_size <= 128)
+    halve_heads_of_256(num_kv_heads, head_size, group_size);
+  const size_t lds = lds_bytes();
+  const dim3 grid(static_cast<unsigned>(max_blocks), static_cast<unsigned>(batch),
+                  num_kv_heads);
   if (head_size == 128 && (group_size == 64 || group_size == 128) && block_size % 32 == 0 &&
       block_size <= 128) {
     const int64_t npages = batch * max_blocks;

@@ -181,8 +181,9 @@ def ring_write(
 
 
 def store_one_launch_supported(head_size: int, group_size: int, dtype: torch.dtype) -> bool:
-    """Geometries ``kvq_kivi_store`` runs (the others use the separate launches)."""
-    return head_size == 128 and group_size in (64, 128) and dtype in (torch.bfloat16, torch.float16)
+    """Geometries ``kvq_kivi_store`` runs (the others use the separate launches);
+    a head of 256 dims runs as two of 128."""
+    return head_size in (128, 256) and group_size in (64, 128) and dtype in (torch.bfloat16, torch.float16)
 
 
 def kivi_store(
