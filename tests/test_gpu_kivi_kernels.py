@@ -765,6 +765,49 @@ def test_split_decode_two_pieces_a_wave_and_long_combine(gpu_device):
                        lambda s: plan_decode_pieces(s, 1, 256), lens=lens, stale=False)
 
 
+@pytest.mark.parametrize("g,bs,rep", [(128, 128, 8), (64, 128, 12)])
+@pytest.mark.parametrize("size", [1.0, 1e-3, 3e4])
+def test_split_decode_head_256_keeps_its_precision(gpu_device, g, bs, rep, size):
+    """Head size 256 against 64 bits over the dequantized history: within the fp16
+    output's rounding, for small values, for values whose scales times a
+    probability of 1 come near the fp16 range, and for flat softmaxes (many
+    positions of small probability)."""
+    from vllm_ascend_quantized_kv_cache.ops.kivi_decode import (
+        DecodeSeq,
+        kivi_decode_attention,
+        plan_decode,
+    )
+
+    d, kvh, r_len, lens, dtype = 256, 1, 128, [6000, 700, 129, 40], torch.float16
+
+    def make(n, h_, d_, seed):
+        gen = torch.Generator().manual_seed(seed)
+        key = 0.05 * torch.randn(n, h_, d_, generator=gen)
+        value = size * (torch.rand(n, h_, d_, generator=gen) * 2 - 1)
+        return key.to(dtype), value.to(dtype)
+
+    cpu, table, ring_k, ring_v, seqs, wk, wv, _, _ = _ring_case(
+        gpu_device, d, kvh, g, bs, r_len, lens, seed=46, ring_dtype=dtype, make=make)
+    q = torch.randn(len(lens), rep, d, generator=torch.Generator().manual_seed(2)).to(dtype)
+    dk, dv = ref.dequant_gather(*cpu, table, torch.tensor(lens), torch.float32, g)
+    dk, dv = ref.overlay_residual(dk, lens, wk), ref.overlay_residual(dv, lens, wv)
+    at, want = 0, []
+    for b, n in enumerate(lens):
+        k, v = dk[at:at + n, 0].double(), dv[at:at + n, 0].double()
+        want.append(torch.softmax(q[b].double() @ k.T * d ** -0.5, -1) @ v)
+        at += n
+    want = torch.stack(want)
+    dseqs = [DecodeSeq(n, hk, hv, row, ks_, vs_) for (n, hk, hv, row, ks_, vs_) in seqs]
+    dev = gpu_device
+    plan = tuple(torch.from_numpy(x).to(dev) for x in plan_decode(dseqs, kvh, 256))
+    got = kivi_decode_attention(q.to(dev), to_dev(cpu, dev), table.to(dev), dseqs,
+                                ring_k.to(dev), ring_v.to(dev), d ** -0.5, g, plan=plan)
+    err = (got.double().cpu() - want).norm(dim=-1) / want.norm(dim=-1)
+    # a rounding to fp16 is 2^-11 / sqrt(3) of a value at most, in its binade 2^-12
+    # on average; the flat softmaxes leave values of 1e-2 * size, subnormal at 1e-3
+    assert err.max() < (3e-3 if size < 1 else 2.0 ** -11), err.tolist()
+
+
 @pytest.mark.parametrize("d", [128, 256])
 def test_combine_of_item_counts_at_its_edges(gpu_device, d):
     """15 to 18 items a request (rows ahead of the weights, or only the live ones

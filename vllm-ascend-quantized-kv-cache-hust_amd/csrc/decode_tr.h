@@ -88,6 +88,17 @@ __device__ __forceinline__ h8 key_codes(uint32_t w, const Consts& c) {
   return as_h8(p0, and_or(w, c.hi, c.magic), p2, and_or(w8, c.hi, c.magic));
 }
 
+// ... with the 1024 removed from all slots: c and, primed, 16c
+__device__ __forceinline__ h8 plain_codes(uint32_t w, const Consts& c) {
+  const uint32_t w8 = w >> 8;
+  const h2 off = h2{1024.0f16, 1024.0f16};
+  auto drop = [&](uint32_t x) {
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, x) - off);
+  };
+  return as_h8(drop(and_or(w, c.lo, c.magic)), drop(and_or(w, c.hi, c.magic)),
+               drop(and_or(w8, c.lo, c.magic)), drop(and_or(w8, c.hi, c.magic)));
+}
+
 __device__ __forceinline__ uint32_t lds_off(const void* p) {
   return static_cast<uint32_t>(
       reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) char*)(p)));
@@ -439,6 +450,12 @@ __device__ __forceinline__ void compute_tile(const uint32_t* W, uint32_t buf_off
 #pragma clang fp contract(fast)
   using T = Tile<NVG, KSV, D>;
   constexpr int DB = D / 16;
+  // P' (p times the value scale) as one fp16 against codes that keep their offset,
+  // or as fp16 hi + lo parts against plain codes.  Rounded once, P' disagrees
+  // with the fp32 p of the minima term, and the offset's sums cancel: 0.0005 of
+  // the output against 0.0002 at 64 bits' distance (fp16 queries, 256 dims,
+  // 1K-9K positions), for 60.1 against 64 us on 64 requests of 1K-16K.
+  constexpr bool kSplitP = D == 256;
   static_assert(T::KW == Tile<1, false>::KW && T::VW == Tile<1, false, D>::VW,
                 "read bases assume the common word offsets");
   const Consts cst;
@@ -495,6 +512,26 @@ __device__ __forceinline__ void compute_tile(const uint32_t* W, uint32_t buf_off
   }
   float tmax = fmaxf(fmaxf(tm[0], tm[1]), fmaxf(tm[2], tm[3]));
   tmax = max_rows4(tmax);
+  if constexpr (kSplitP) {
+    // p up to 2^4 instead of 1 (the partial's m is the exponent offset, so any
+    // will do): fp16 parts of small p, and of the 1/16 of the primed slots, then
+    // lose no bits to the subnormals.  Less where a value scale would overflow.
+    const int lane = 16 * kg + n;
+    const float* sv = reinterpret_cast<const float*>(W + T::VS) + lane;
+    float big = sv[0];
+#pragma unroll
+    for (int vg = 1; vg < NVG; ++vg) big = fmaxf(big, sv[64 * vg]);
+    if (!FULL) {
+      const int pos = p0 + tau((lane >> 3) & 3, 8 * (lane >> 5) + slot_nib(lane & 7));
+      big = pos >= pb && pos < pe ? big : 0.0f;
+    }
+    float shift = 4.0f;
+    if (__builtin_amdgcn_ballot_w64(big > 2048.0f) != 0) {  // uniform
+      big = max_wave64(big);
+      shift = 141.0f - static_cast<float>(__float_as_uint(big) >> 23);  // 2^shift * big < 2^15
+    }
+    tmax -= shift;
+  }
   const float m_new = fmaxf(acc.m_run, tmax);
   const float alpha = acc.m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(acc.m_run - m_new);
   float ps[4];
@@ -529,7 +566,7 @@ __device__ __forceinline__ void compute_tile(const uint32_t* W, uint32_t buf_off
   for (int s = 0; s < 2; ++s) {
     // P' of k-step s, value group vg: slot i holds token tau(kg, 8 s + slot_nib(i)),
     // whose p is sacc[2 s + (i & 1)][i >> 1]
-    h8 pa[NVG];
+    h8 pa[NVG], pl[NVG];
 #pragma unroll
     for (int vg = 0; vg < NVG; ++vg) {
       const f4 s0 = *reinterpret_cast<const f4*>(vsf + 64 * vg + 32 * s);
@@ -559,17 +596,33 @@ __device__ __forceinline__ void compute_tile(const uint32_t* W, uint32_t buf_off
           uint32_t, __builtin_bit_cast(h2, pack_h2(pp[2], pp[3])) * sixteenth);
       const uint32_t a3 = __builtin_bit_cast(
           uint32_t, __builtin_bit_cast(h2, pack_h2(pp[6], pp[7])) * sixteenth);
-      pa[vg] = as_h8(pack_h2(pp[0], pp[1]), a1, pack_h2(pp[4], pp[5]), a3);
+      const uint32_t a0 = pack_h2(pp[0], pp[1]), a2 = pack_h2(pp[4], pp[5]);
+      pa[vg] = as_h8(a0, a1, a2, a3);
+      if constexpr (kSplitP) {
+        const uint32_t h1 = pack_h2(pp[2], pp[3]), h3 = pack_h2(pp[6], pp[7]);
+        auto rest = [](float x0, float x1, uint32_t hi) {
+          return pack_h2(sub_half_sel<0>(x0, hi, -1.0f), sub_half_sel<1>(x1, hi, -1.0f));
+        };
+        const h2 l1 = __builtin_bit_cast(h2, rest(pp[2], pp[3], h1)) * sixteenth;
+        const h2 l3 = __builtin_bit_cast(h2, rest(pp[6], pp[7], h3)) * sixteenth;
+        pl[vg] = as_h8(rest(pp[0], pp[1], a0), __builtin_bit_cast(uint32_t, l1),
+                       rest(pp[4], pp[5], a2), __builtin_bit_cast(uint32_t, l3));
+      }
     }
 #pragma unroll
     for (int v = 0; v < DB; ++v) {
       const int vg = v / (DB / NVG);
-      acc.o_acc[v] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-          pa[vg], codes(static_cast<uint32_t>(rv[v][s]), cst), acc.o_acc[v], 0, 0, 0);
+      const uint32_t w = static_cast<uint32_t>(rv[v][s]);
+      const h8 bv = kSplitP ? plain_codes(w, cst) : codes(w, cst);
+      acc.o_acc[v] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[vg], bv, acc.o_acc[v], 0, 0, 0);
+      if constexpr (kSplitP)
+        acc.o_acc[v] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl[vg], bv, acc.o_acc[v], 0, 0, 0);
     }
 #pragma unroll
     for (int vg = 0; vg < NVG; ++vg)
-      acc.c_acc[vg] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[vg], ones_b, acc.c_acc[vg], 0, 0, 0);
+      if constexpr (!kSplitP)
+        acc.c_acc[vg] =
+            __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[vg], ones_b, acc.c_acc[vg], 0, 0, 0);
   }
 }
 
