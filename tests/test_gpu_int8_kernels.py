@@ -217,3 +217,27 @@ def test_int8_decode_head_256_matches_oracle(gpu_device, rep, kvh, bs):
     """Head size 256 on the MFMA kernel: heads of an item in one workgroup (1, 2)
     and a wave per head (8), folded and unfolded GQA groups, split items."""
     test_int8_decode_matches_oracle(gpu_device, rep, kvh, 256, bs)
+
+
+@pytest.mark.parametrize("rep", [4, 12])
+def test_int8_decode_head_256_keeps_its_precision(gpu_device, rep):
+    """Head size 256 with fp32 queries against 64 bits: the query and the
+    probabilities go through the MFMA as two fp16 parts, 22 bits each, so scores
+    of up to 16 (log2) move by 2^-18 and the result by about as much."""
+    from vllm_ascend_quantized_kv_cache.ops.int8_ops import int8_decode_attention
+
+    kvh, d, bs, lens, dtype = 1, 256, 64, [2000, 513, 33], torch.float32
+    table, kc, vc, k_inv, v_inv, k_aq, v_aq = _int8_state(gpu_device, 3, lens, kvh, d, bs, dtype, 8)
+    q = torch.randn(len(lens), rep, d, generator=torch.Generator().manual_seed(2)).to(dtype)
+    dk, dv = ref.int8_paged_dequant(kc, vc, table, lens, torch.float32, k_inv, v_inv)
+    want, at = [], 0
+    for b, n in enumerate(lens):
+        k, v = dk[at:at + n, 0].double(), dv[at:at + n, 0].double()
+        want.append(torch.softmax(q[b].double() @ k.T * d ** -0.5, -1) @ v)
+        at += n
+    want = torch.stack(want)
+    got = int8_decode_attention(q.to(gpu_device), kc.to(gpu_device), vc.to(gpu_device),
+                                k_aq.to(gpu_device), v_aq.to(gpu_device), table.to(gpu_device),
+                                lens, d ** -0.5)
+    err = (got.double().cpu() - want).norm(dim=-1) / want.norm(dim=-1)
+    assert err.max() < 2.0 ** -16, err.tolist()

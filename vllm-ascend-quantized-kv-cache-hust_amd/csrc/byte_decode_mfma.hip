@@ -369,10 +369,25 @@ __device__ __forceinline__ void compute_tile(const TileRegs<D, FP8>& t, int p, i
       }
     }
   } else {
-    const h8 a = as_h8(h2_bits(static_cast<_Float16>(s[0][0]), static_cast<_Float16>(s[0][1])),
-                       h2_bits(static_cast<_Float16>(s[0][2]), static_cast<_Float16>(s[0][3])),
-                       h2_bits(static_cast<_Float16>(s[1][0]), static_cast<_Float16>(s[1][1])),
-                       h2_bits(static_cast<_Float16>(s[1][2]), static_cast<_Float16>(s[1][3])));
+    // at 256 dims p goes as fp16 hi + lo parts, at 128 as one fp16
+    constexpr bool kSplitP = D == 256;
+    auto halves = [](const f4 (&x)[2]) {
+      return as_h8(h2_bits(static_cast<_Float16>(x[0][0]), static_cast<_Float16>(x[0][1])),
+                   h2_bits(static_cast<_Float16>(x[0][2]), static_cast<_Float16>(x[0][3])),
+                   h2_bits(static_cast<_Float16>(x[1][0]), static_cast<_Float16>(x[1][1])),
+                   h2_bits(static_cast<_Float16>(x[1][2]), static_cast<_Float16>(x[1][3])));
+    };
+    const h8 a = halves(s);
+    h8 al = a;
+    if constexpr (kSplitP) {
+      f4 rest[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          rest[j][r] = s[j][r] - static_cast<float>(static_cast<_Float16>(s[j][r]));
+      al = halves(rest);
+    }
     // the lane's 8 tokens (i = 4j + r), four dims per word
 #pragma unroll
     for (int w = 0; w < D / 64; ++w) {
@@ -384,6 +399,9 @@ __device__ __forceinline__ void compute_tile(const TileRegs<D, FP8>& t, int p, i
     const h8 b = as_h8(value_pair<K>(x[0], x[1]), value_pair<K>(x[2], x[3]),                 \
                        value_pair<K>(x[4], x[5]), value_pair<K>(x[6], x[7]));                \
     st.o[4 * w + K] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, st.o[4 * w + K], 0, 0, 0); \
+    if constexpr (kSplitP)                                                                   \
+      st.o[4 * w + K] =                                                                      \
+          __builtin_amdgcn_mfma_f32_16x16x32_f16(al, b, st.o[4 * w + K], 0, 0, 0);           \
   }
       KVQ_PV_TILE(0)
       KVQ_PV_TILE(1)
