@@ -507,7 +507,10 @@ prefill_attn_fa_kernel(PlanArg plan_arg, const int32_t* __restrict__ plan, int b
   // (-inf before the first finite score); m_off = -qscale * m_run (0 while
   // m_run is -inf), so p = 2^(qscale * s + m_off); m_thr = m_run + 8 / qscale,
   // the raw score past which the offset moves (lazy offset, below).
-  const float lazy_thr = 8.0f / qscale;  // qscale > 0
+  // At D = 256 the offset follows every new maximum: the largest p is then 1
+  // exactly, where the rounding of a p past 1 costs 3 - 8% more error in the
+  // output (254 against 244 us on the prompts of fa_ng above).
+  const float lazy_thr = D == 256 ? 0.0f : 8.0f / qscale;  // qscale > 0
   float m_run[NG], m_off[NG], m_thr[NG];
 #pragma unroll
   for (int g2 = 0; g2 < NG; ++g2) {
