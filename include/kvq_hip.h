@@ -174,10 +174,14 @@ int kvq_kivi_gather_dequant(const int32_t* k_quant, const float* k_scale, const 
  *               per piece (one per half of the kv heads) stream the piece's
  *               kind-0 items page by page, then run its tail items (plan with
  *               split_tokens 128 so that no two pieces share a page).
- *               Elsewhere, where the MFMA kernel runs both kinds, one wave
- *               per (piece, kv head) runs its piece's items in order in a
- *               single pass, so pieces of equal cost end together; else the
- *               pieces are ignored.
+ *               Elsewhere one wave per (piece, kv head) runs its piece's
+ *               items in order, int4 and tail alike, so pieces of equal cost
+ *               end together.  D 128 or 256 with group_size 64 or 128, blocks
+ *               of a power of two from 64 and 16-bit query and ring: four such
+ *               waves form a workgroup and leave one partial per request
+ *               between them (D 256 runs plans without pieces so too, an item
+ *               per wave); the items merged away carry m = -inf.  Where no
+ *               MFMA kernel runs both kinds the pieces are ignored.
  *   workspace   >= kvq_kivi_decode_workspace_bytes(num_work, num_heads, D)
  *   block_table int32 [batch, max_blocks]
  * Replaces the decode branch: _forward_kivi_paged_decode_attention

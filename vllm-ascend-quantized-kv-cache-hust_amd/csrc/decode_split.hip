@@ -14,7 +14,7 @@
 //
 // Head size 256 had no MFMA path (the generic fp32 kernel: 4650 us for 64
 // requests of 1K-16K positions on 1 kv head, against 32 us for its 166 MB at
-// the copy rate; 62 here).
+// the copy rate; 64 here, its combine included).
 //
 // Tiles: 64 positions, decode_tr.h's layout and compute, double-buffered in the
 // wave's own LDS: the DMA of the next tile is in flight while one computes.  The
@@ -24,14 +24,15 @@
 //   D = 128: 2 workgroups a CU (8 x 19-20 KB of LDS), one piece a wave;
 //   D = 256: 1 workgroup a CU (4 x 38-40 KB), two pieces a wave where the plan
 //            has more of them than the chip holds waves.
-// What bounds it: at D = 256 the issue of one wave per SIMD (3.9 us a tile, of
+// What bounds it: at D = 256 the issue of one wave per SIMD (some 5 us a tile, of
 // them 0.95 waiting for its DMA, at 1500 vector and 300 scalar instructions), at
 // D = 128 the start: every wave's first tile, 20 MB over the chip, takes 5 - 6 of
 // 22 us on 40 requests of 1K-10K positions and 2 kv heads.  Hence the query rows
 // through LDS (the second tile leaves before the first is there), the key
 // group's operands kept over its two tiles, and MFMA results in ordinary
 // registers (a build flag): 69.1 -> 62.0 us on the 64 requests above, 58.4 ->
-// 52.6 on 20 of 0.5K-10K with 2 kv heads of 256, 40.5 -> 38.7 on the 40.
+// 52.6 on 20 of 0.5K-10K with 2 kv heads of 256, 40.5 -> 38.7 on the 40.  (The
+// two parts of P that compute_tile takes at 256 dims then added 3 - 4 us.)
 #include <algorithm>
 
 #include "decode_tail.h"

@@ -10,7 +10,8 @@
 //
 // Work items (built by the host from the request lengths, no device sync):
 //   kind 0: a range where keys and values both come from int4 pages -- the
-//           MFMA kernel of decode_mfma.hip;
+//           MFMA kernels of decode_coop.hip, decode_split.hip and
+//           decode_mfma.hip;
 //   kind 1: tails where one side is already in the ring -- the tail path of
 //           decode_tail.h, run by the same launch in a second pass of its
 //           grid (after every kind-0 wave), or by the standalone tail kernel

@@ -315,7 +315,7 @@ struct FaLds {
 //     10240 keys (twice the LDS reads per MFMA, and spills at the 128-VGPR limit
 //     of 4 waves per SIMD).
 //   D = 256: NG = 1 (8 waves of 16 rows; the blocks take 128 KB, one workgroup
-//     a CU): 242 VGPRs, 245 us on 6 ragged prompts of 200 - 2048 rows with 3000
+//     a CU): 240 VGPRs, 254 us on 6 ragged prompts of 200 - 2048 rows with 3000
 //     keys of history (8 heads on 1 kv head); the fallback kernel took 1612.
 //     NG = 2 needs about 400 registers, one wave per SIMD and accumulator moves:
 //     322 us, and 335 with its operand reads a step ahead.
