@@ -744,6 +744,78 @@ def test_split_decode_query_off_its_alignment(gpu_device, d, kvh, rep):
                        lambda s: plan_decode_pieces(s, kvh, 256), q_offset=4)
 
 
+def _off_16(t, dev):
+    """A contiguous copy on ``dev`` that starts 8 bytes off a 16-byte bound."""
+    skip = 8 // t.element_size()
+    out = torch.empty(t.numel() + skip, dtype=t.dtype, device=dev)[skip:].view(t.shape)
+    assert out.data_ptr() % 16 == 8
+    return out.copy_(t)
+
+
+@pytest.mark.parametrize("side", range(6))
+def test_split_decode_head_256_cache_off_its_alignment(gpu_device, monkeypatch, side):
+    """Head size 256 over pages 8 bytes off a 16-byte bound, one array of the six."""
+    import sys
+
+    from vllm_ascend_quantized_kv_cache.ops.kivi_decode import plan_decode_pieces
+
+    monkeypatch.setattr(sys.modules[__name__], "to_dev", lambda arrays, dev: tuple(
+        _off_16(t, dev) if i == side else t.to(dev) for i, t in enumerate(arrays)))
+    _split_decode_case(gpu_device, 256, 1, 128, 128, 8, torch.bfloat16,
+                       lambda s: plan_decode_pieces(s, 1, 256), lens=[300, 129, 1, 700])
+
+
+def test_head_256_views_off_their_alignment(gpu_device):
+    """INT8 decode, dense attention, E4M3 decode and the int4 packs of contiguous
+    views that start 8 bytes off a 16-byte bound, against the same on one."""
+    from vllm_ascend_quantized_kv_cache.ops import fp8_ops, kivi_pack
+    from vllm_ascend_quantized_kv_cache.ops.attention import prefill_attention
+    from vllm_ascend_quantized_kv_cache.ops.int8_ops import int8_decode_attention
+
+    dev, d, kvh, bs, dtype = gpu_device, 256, 2, 64, torch.bfloat16
+    gen = torch.Generator().manual_seed(6)
+    lens = [130, 64, 17]
+    table = torch.randperm(8, generator=gen, dtype=torch.int32)[:6]
+    table = torch.tensor([[*table[:3]], [table[3], 0, 0], [table[4], 0, 0]], dtype=torch.int32)
+    rows = torch.randn((sum(lens), kvh, d), generator=gen).to(dtype)
+    q = torch.randn((len(lens), kvh * 4, d), generator=gen).to(dtype).to(dev)
+    # two results within a bf16 rounding or two of the sums each
+    tol = dict(atol=1e-2, rtol=1e-2)
+
+    both = [prefill_attention(q, put(rows, dev), put(rows.flip(0), dev), [1] * 3, lens, d ** -0.5,
+                              True) for put in (_off_16, torch.Tensor.to)]
+    torch.testing.assert_close(*both, **tol)
+
+    codes = torch.randint(-127, 128, (2, 8, bs, kvh, d), generator=gen, dtype=torch.int8)
+    aq = (torch.rand((kvh, d), generator=gen) / 100).to(dtype).to(dev)
+    both = [int8_decode_attention(q, put(codes[0], dev), put(codes[1], dev), aq, aq, table.to(dev),
+                                  lens, d ** -0.5) for put in (_off_16, torch.Tensor.to)]
+    torch.testing.assert_close(*both, **tol)
+
+    fp8 = torch.randint(0, 120, (2, 8, bs, kvh, d), generator=gen, dtype=torch.uint8)
+    fp8 |= torch.randint(0, 2, fp8.shape, generator=gen, dtype=torch.uint8) << 7
+    for dim in (128, 256):
+        scales = torch.rand((8, bs, kvh, 1), generator=gen).to(dev) / 100
+        both = [fp8_ops.fp8_per_token_head_attention(
+            q[..., :dim], put(fp8[0, ..., :dim], dev), scales, put(fp8[1, ..., :dim], dev), scales,
+            table.to(dev), lens, [1] * 3, dim ** -0.5, block_table_host=table.numpy())
+            for put in (_off_16, lambda t, to: t.to(to).contiguous())]
+        torch.testing.assert_close(*both, **tol)
+
+    slots = torch.arange(128, device=dev)
+    packed = []
+    for put in (_off_16, torch.Tensor.to):
+        x = put(rows[:128], dev)
+        pages = to_dev(empty_kivi_caches(2, bs, kvh, d, 64), dev)
+        kivi_pack.kivi_pack_key_cache(x, slots, *pages[:3], 64)
+        kivi_pack.kivi_pack_value_cache(x, slots, *pages[3:], 64)
+        packed.append(pages)
+        assert kivi_pack.kivi_store(x, x, x.view(1, 128, kvh, d), x.view(1, 128, kvh, d),
+                                    slots[:0], (0, 0, 0, 0), pages, 64) is (x.data_ptr() % 16 == 0)
+    for a, b in zip(*packed):
+        assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+
+
 @pytest.mark.parametrize("g,bs", [(128, 128), (64, 64)])
 @pytest.mark.parametrize("paired", [False, True])
 def test_split_decode_without_pieces_head_256(gpu_device, g, bs, paired):

@@ -736,6 +736,8 @@ int launch_int8_decode_mfma(const void* query, int dtype, int hq, int kvh, int d
                             float* ws_ml, hipStream_t s, bool* launched) {
   *launched = false;
   if ((d != 128 && d != 256) || hq / kvh > 16 || bs % 16) return KVQ_OK;
+  // rows of 256 bytes off the DMA's 16-byte lanes run the generic kernel
+  if (d == 256 && !aligned16(kc, vc)) return KVQ_OK;
   if (num_work * kvh > 0x7fffffff) return KVQ_ERR_INVALID;
   // all kv heads of an item in one workgroup when they fit (at most 8 waves
   // and their tile buffers in the workgroup's LDS), else one wave per head
@@ -858,7 +860,8 @@ extern "C" int kvq_fp8_pth_decode_attn(const void* query, int dtype, int64_t bat
   if (!(scale > 0.0f)) return KVQ_ERR_INVALID;
   if (rows <= 0 || rows * std::max(1, num_heads) > kMaxRowHeads) return KVQ_ERR_INVALID;
   if ((dtype != KVQ_DTYPE_BF16 && dtype != KVQ_DTYPE_F16) ||
-      !fp8_decode_geometry(num_heads, num_kv_heads, head_size, block_size))
+      !fp8_decode_geometry(num_heads, num_kv_heads, head_size, block_size) ||
+      !kvq::aligned16(k_data, v_data))  // 16-byte DMA lanes
     return KVQ_ERR_GEOMETRY;
   for (int64_t b = 0; b < batch; ++b)
     if (seq_lens[b] < 0 || seq_lens[b] > max_blocks * block_size) return KVQ_ERR_INVALID;

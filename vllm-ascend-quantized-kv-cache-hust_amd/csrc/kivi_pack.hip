@@ -1094,7 +1094,7 @@ extern "C" int kvq_kivi_pack_key(const void* src_a, int64_t n_a, const void* src
     return KVQ_ERR_GEOMETRY;
   if (num_tokens % group_size) return KVQ_ERR_INVALID;
   if (!src_index && n_a < num_tokens) return KVQ_ERR_INVALID;
-  if (src_dtype == KVQ_DTYPE_BF16 || src_dtype == KVQ_DTYPE_F16)
+  if ((src_dtype == KVQ_DTYPE_BF16 || src_dtype == KVQ_DTYPE_F16) && kvq::aligned16(src_a, src_b))
     halve_heads_of_256(num_kv_heads, head_size, group_size);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (pack_lds_applies(src_dtype, head_size, group_size, num_tokens, num_kv_heads) &&
@@ -1154,7 +1154,7 @@ extern "C" int kvq_kivi_pack_value(const void* src_a, int64_t n_a, const void* s
   if (!kivi_geometry_ok(num_kv_heads, head_size, group_size, block_size))
     return KVQ_ERR_GEOMETRY;
   if (!src_index && n_a < num_tokens) return KVQ_ERR_INVALID;
-  if (src_dtype == KVQ_DTYPE_BF16 || src_dtype == KVQ_DTYPE_F16)
+  if ((src_dtype == KVQ_DTYPE_BF16 || src_dtype == KVQ_DTYPE_F16) && kvq::aligned16(src_a, src_b))
     halve_heads_of_256(num_kv_heads, head_size, group_size);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (pack_lds_applies(src_dtype, head_size, group_size, num_tokens, num_kv_heads) &&
@@ -1248,7 +1248,8 @@ extern "C" int kvq_kivi_store(const void* key_input, const void* value_input, vo
   if (n_value_pack && (!v_quant || !v_scale || !v_mn)) return KVQ_ERR_INVALID;
   if (!kivi_geometry_ok(num_kv_heads, head_size, group_size, block_size))
     return KVQ_ERR_GEOMETRY;
-  halve_heads_of_256(num_kv_heads, head_size, group_size);
+  if (kvq::aligned16(key_input, value_input) && kvq::aligned16(ring_k, ring_v))
+    halve_heads_of_256(num_kv_heads, head_size, group_size);
   // the register key pack's geometry; callers fall back to the separate
   // pack and ring-write entry points elsewhere
   if (head_size != 128 || (group_size != 64 && group_size != 128) ||

@@ -23,6 +23,12 @@ struct bf16 {
 };
 using f16 = _Float16;
 
+// Both on 16-byte bounds (nullptr is): what 16-byte lanes of a global-to-LDS
+// DMA take.  A contiguous view into a larger buffer may start off them.
+inline bool aligned16(const void* a, const void* b) {
+  return ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) == 0;
+}
+
 __device__ __forceinline__ float to_f32(float v) { return v; }
 __device__ __forceinline__ float to_f32(f16 v) { return static_cast<float>(v); }
 __device__ __forceinline__ float to_f32(bf16 v) {

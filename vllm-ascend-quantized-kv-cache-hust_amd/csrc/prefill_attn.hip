@@ -877,10 +877,13 @@ struct FaTiles {
   int64_t batch, num_units, tiles;
 };
 
-int fa_applies(int dtype, int head_size, bool* applies) {
+// At head size 256 the keys and values are on 16-byte bounds, which their DMA
+// into LDS takes in 16-byte lanes; views off them run prefill_attn_kernel.
+int fa_applies(const void* key, const void* value, int dtype, int head_size, bool* applies) {
   *applies = false;
   if (dtype != KVQ_DTYPE_BF16 && dtype != KVQ_DTYPE_F16) return KVQ_OK;
   if (head_size != 64 && head_size != 128 && head_size != 256) return KVQ_OK;
+  if (head_size == 256 && !aligned16(key, value)) return KVQ_OK;
   int64_t lds_max = 0;  // LDS one workgroup may use on this device
   const int lrc = device_lds_max(&lds_max);
   if (lrc != KVQ_OK) return lrc;
@@ -895,7 +898,7 @@ int launch_fa(const void* query, const void* key, const void* value, int dtype, 
               SegWs seg, hipStream_t s, bool* launched) {
   *launched = false;
   bool applies = false;
-  const int arc = fa_applies(dtype, head_size, &applies);
+  const int arc = fa_applies(key, value, dtype, head_size, &applies);
   if (arc != KVQ_OK || !applies) return arc;
   if (t.num_units * num_kv_heads > 0x7fffffff || t.tiles > 0x7fffffff / kFaTileRows)
     return KVQ_ERR_INVALID;
@@ -1129,7 +1132,7 @@ extern "C" int kvq_prefill_attn_lens(const void* query, const void* key, const v
   if (batch == 0) return KVQ_OK;
   if (!query || !key || !value || !out || !(scale > 0.0f)) return KVQ_ERR_INVALID;
   bool applies = false;
-  const int arc = fa_applies(dtype, head_size, &applies);
+  const int arc = fa_applies(key, value, dtype, head_size, &applies);
   if (arc != KVQ_OK) return arc;
   if (!applies) return KVQ_ERR_GEOMETRY;
   if (plan_arg_cap(batch) <= 0) return KVQ_ERR_CAPACITY;

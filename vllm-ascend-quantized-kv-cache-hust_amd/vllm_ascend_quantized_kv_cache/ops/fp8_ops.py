@@ -337,7 +337,8 @@ def fp8_per_token_head_attention(
     ``seq_lens[b]`` (decode: ``query_lens`` all 1).  The same few rows for every
     request are scored straight from the codes; other batches gather them to
     dense rows first."""
-    if _decode_applies(query, k_data, block_table, query_lens, scale):
+    if (_decode_applies(query, k_data, block_table, query_lens, scale)
+            and (k_data.data_ptr() | v_data.data_ptr()) % 16 == 0):  # the kernel's DMA lanes
         rows = int(query_lens[0]) if len(query_lens) else 1
         return _decode_attention(query, k_data, k_scale, v_data, v_scale, block_table, seq_lens,
                                  rows, scale, causal, out, block_table_host)

@@ -207,6 +207,9 @@ def kivi_store(
     nb, kvh, d, pbs = kq.shape
     if not store_one_launch_supported(d, group_size, ring_k.dtype):
         return False
+    if d == 256 and any(t is not None and t.data_ptr() % 16
+                        for t in (key_input, value_input, ring_k, ring_v)):
+        return False  # off the 16-byte lanes of the kernel's DMA
     if sum(counts) == 0:
         return True
     _native.require_gpu_tensors("kivi store", ring_k, ring_v, jobs, kq, key_input, value_input)
