@@ -1110,23 +1110,23 @@ int launch_kivi_decode_mfma(const void* query, int q_dtype, int hq, int kvh, int
                             const int32_t* pieces, int64_t num_pieces,
                             const void* ring_k, const void* ring_v, int ring_dtype, int ring_len,
                             float* ws_o, float* ws_ml, hipStream_t s, bool* launched,
-                            bool* tail_done) {
+                            bool* tail_done, bool* split) {
   *launched = false;
   *tail_done = false;
+  *split = false;
   {
     // the split decode: pieces that the page-streaming kernel does not take, and
     // head size 256 with or without them
     const bool with_pieces = pieces && num_pieces > 0;
-    bool split = false;
     if (d == 256 || (with_pieces && !(qscale > 0.0f && qscale != INFINITY &&
                                       coop_decode_applies(q_dtype, hq, kvh, d, ring_dtype, bs, g)))) {
       const int src = launch_kivi_decode_split(
           query, q_dtype, hq, kvh, d, qscale, kq, ks, km, vq, vs, vm, bs, g, nb, block_table,
           maxb, seq_meta, work, num_work, with_pieces ? pieces : nullptr, num_pieces, ring_k,
-          ring_v, ring_dtype, ring_len, ws_o, ws_ml, s, &split);
+          ring_v, ring_dtype, ring_len, ws_o, ws_ml, s, split);
       if (src != KVQ_OK) return src;
     }
-    if (split) {
+    if (*split) {
       *launched = true;
       *tail_done = true;
       return KVQ_OK;

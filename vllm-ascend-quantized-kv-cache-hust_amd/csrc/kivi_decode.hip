@@ -297,16 +297,19 @@ namespace kvq {
 // head), four heads per workgroup.  Lane s holds item s's (m, l) of the current
 // chunk of 64 items; the weights 2^(m_s - max) go to every lane through
 // readlane, and each lane accumulates columns lane + 64*k of sum_s w_s * o_s.
-// The o rows of a request with up to kPre items are loaded before the (m, l)
-// pass, one round trip to memory for the whole combine.  Of a longer request
-// only the rows with weight are read, kPre at a time, after the pass: the split
-// decode leaves most items of a long request to another's partial (2 requests of
+// The o rows of the first kPre items are loaded before the (m, l) pass, so a
+// request with up to kPre items costs one round trip to memory instead of one
+// per few items.  SPARSE (after the split decode, which leaves most items of a
+// long request to another's partial): of a request of more than kPre items only
+// the rows with weight are read, kPre at a time, after the pass (2 requests of
 // 5K - 14K positions, some 100 items each: 21.5 us a decode with the first kPre
 // rows ahead and the others four at a time, 18.9 so; 64 requests of some 32
-// items at head size 256: 61.6 and 60.3).
+// items at head size 256: 61.6 and 60.3).  Behind the page-streaming decode,
+// whose items all have weight, it took 5.27 us against 4.88 (32 requests of 2K -
+// 16K positions, 40 heads on 8 kv heads).
 // Items with m = -inf (no position) carry weight 0 and their o never reaches
 // the sum (selected out, so stale bytes cannot turn it NaN).
-template <typename TO, int KD>
+template <typename TO, int KD, bool SPARSE>
 __global__ void __launch_bounds__(256)
 decode_combine_kernel(int hq, int d, const int32_t* __restrict__ seq_meta, int meta_stride,
                       int first_col, const float* __restrict__ ws_o,
@@ -330,7 +333,7 @@ decode_combine_kernel(int hq, int d, const int32_t* __restrict__ seq_meta, int m
   }
   const int64_t stride = static_cast<int64_t>(hq) * d;
   const float* rows = ws_o + (static_cast<int64_t>(fw) * hq + hh) * d;
-  const bool few = nw <= kPre;  // uniform
+  const bool few = !SPARSE || nw <= kPre;  // uniform
   float pre[kPre][KD];
   if (few) {
 #pragma unroll
@@ -378,17 +381,34 @@ decode_combine_kernel(int hq, int d, const int32_t* __restrict__ seq_meta, int m
         wsum += wgt * ls;
       }
     }
-    uint64_t live = __builtin_amdgcn_ballot_w64(wgt != 0.0f);
-    if (few) {
+    const int cnt = nw - s0 < 64 ? nw - s0 : 64;
+    int j0 = 0;
+    if (few && s0 == 0) {
 #pragma unroll
       for (int j = 0; j < kPre; ++j) {
         const float wj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), j));
 #pragma unroll
         for (int k = 0; k < KD; ++k) acc[k] += wj != 0.0f ? wj * pre[j][k] : 0.0f;
       }
-      break;
+      if (SPARSE) break;
+      j0 = kPre;
     }
     const float* row0 = rows + s0 * stride;
+    if constexpr (!SPARSE) {
+#pragma unroll 4
+      for (int j = j0; j < cnt; ++j) {
+        const float wj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), j));
+        const float* row = row0 + j * stride;
+#pragma unroll
+        for (int k = 0; k < KD; ++k) {
+          const int c = lane + 64 * k;
+          const float x = row[c < d ? c : 0];  // columns past d are read in bounds, unused
+          acc[k] += wj != 0.0f ? wj * x : 0.0f;
+        }
+      }
+      continue;
+    }
+    uint64_t live = __builtin_amdgcn_ballot_w64(wgt != 0.0f);
     while (live) {  // uniform; the rows with weight, in item order
       float wj[kPre];
 #pragma unroll
@@ -420,14 +440,16 @@ decode_combine_kernel(int hq, int d, const int32_t* __restrict__ seq_meta, int m
 
 int launch_decode_combine(int dtype, int64_t batch, int hq, int d, const int32_t* seq_meta,
                           int meta_stride, int first_col, const float* ws_o,
-                          const float* ws_ml, void* out, hipStream_t s) {
+                          const float* ws_ml, void* out, hipStream_t s, bool sparse) {
   if (d <= 0 || d > 256) return KVQ_ERR_GEOMETRY;
   const dim3 grid(static_cast<unsigned>(batch), (hq + 3) / 4);
   const int kd = (d + 63) / 64;
-#define KVQ_LAUNCH_COMBINE(KD)                                                              \
+#define KVQ_LAUNCH_COMBINE_S(KD, SP)                                                        \
   KVQ_DISPATCH_FLOAT(dtype, TO,                                                             \
-    hipLaunchKernelGGL((decode_combine_kernel<TO, KD>), grid, dim3(256), 0, s, hq, d,       \
+    hipLaunchKernelGGL((decode_combine_kernel<TO, KD, SP>), grid, dim3(256), 0, s, hq, d,   \
                        seq_meta, meta_stride, first_col, ws_o, ws_ml, static_cast<TO*>(out)))
+#define KVQ_LAUNCH_COMBINE(KD) \
+  if (sparse) { KVQ_LAUNCH_COMBINE_S(KD, true); } else { KVQ_LAUNCH_COMBINE_S(KD, false); }
   switch (kd) {
     case 1: KVQ_LAUNCH_COMBINE(1); break;
     case 2: KVQ_LAUNCH_COMBINE(2); break;
@@ -435,6 +457,7 @@ int launch_decode_combine(int dtype, int64_t batch, int hq, int d, const int32_t
     default: KVQ_LAUNCH_COMBINE(4); break;
   }
 #undef KVQ_LAUNCH_COMBINE
+#undef KVQ_LAUNCH_COMBINE_S
   KVQ_LAUNCH_CHECK();
   return KVQ_OK;
 }
@@ -475,13 +498,13 @@ extern "C" int kvq_kivi_decode_attn(const void* query, int q_dtype, int64_t batc
 
   // int4 items (kind 0), and the tail items (kind 1) in a second pass of the
   // same grid where the tail path applies
-  bool mfma = false, tail = false;
+  bool mfma = false, tail = false, split = false;
   int rc = kvq::launch_kivi_decode_mfma(query, q_dtype, num_heads, num_kv_heads, head_size,
                                        qscale, k_quant, k_scale, k_mn, v_quant, v_scale, v_mn,
                                        block_size, group_size, num_blocks, block_table,
                                        max_blocks, seq_meta, work, num_work, pieces,
                                        num_pieces, ring_k, ring_v, ring_dtype, ring_len, ws_o,
-                                       ws_ml, s, &mfma, &tail);
+                                       ws_ml, s, &mfma, &tail, &split);
   if (rc != KVQ_OK) return rc;
   if (!tail) {
     rc = kvq::launch_kivi_decode_tail_mfma(query, q_dtype, num_heads, num_kv_heads, head_size,
@@ -507,7 +530,7 @@ extern "C" int kvq_kivi_decode_attn(const void* query, int q_dtype, int64_t batc
     KVQ_LAUNCH_CHECK();
   }
   return kvq::launch_decode_combine(q_dtype, batch, num_heads, head_size, seq_meta, 8, 6, ws_o,
-                                    ws_ml, out, s);
+                                    ws_ml, out, s, split);
 }
 
 // ---- allocation-free decode --------------------------------------------------

@@ -51,7 +51,7 @@ inline bool tail_path_applies(int q_dtype, int hq, int kvh, int d, int ring_dtyp
 // covers, taking the kind-1 items too when the tail path applies: in a second
 // pass of the same grid, or, given pieces, in one pass of one wave per (piece,
 // kv head).  *launched / *tail_done tell the caller which kinds still need
-// another kernel.
+// another kernel, *split that the split decode ran (items merged).
 int launch_kivi_decode_mfma(const void* query, int q_dtype, int hq, int kvh, int d, float qscale,
                             const int32_t* kq, const float* ks, const float* km,
                             const int32_t* vq, const float* vs, const float* vm, int bs, int g,
@@ -59,7 +59,7 @@ int launch_kivi_decode_mfma(const void* query, int q_dtype, int hq, int kvh, int
                             const int32_t* seq_meta, const int32_t* work, int64_t num_work,
                             const int32_t* pieces, int64_t num_pieces, const void* ring_k, const void* ring_v, int ring_dtype, int ring_len,
                             float* ws_o, float* ws_ml, hipStream_t s, bool* launched,
-                            bool* tail_done);
+                            bool* tail_done, bool* split);
 
 // The page-streaming decode (decode_coop.hip): given pieces, one workgroup of
 // kvh waves per piece streams whole pages of the piece's int4 items for all kv
@@ -116,8 +116,9 @@ int launch_int8_decode_mfma(const void* query, int dtype, int hq, int kvh, int d
 
 // Merge each request's work items: out = sum_s 2^(m_s-M) o_s / sum_s 2^(m_s-M) l_s.
 // seq_meta row b holds (first_work, num_work) at columns first_col, first_col+1.
+// sparse: most items of a long request carry no weight (merged into another's).
 int launch_decode_combine(int dtype, int64_t batch, int hq, int d, const int32_t* seq_meta,
                           int meta_stride, int first_col, const float* ws_o, const float* ws_ml,
-                          void* out, hipStream_t s);
+                          void* out, hipStream_t s, bool sparse = false);
 
 }  // namespace kvq
