@@ -438,7 +438,8 @@ int kvq_fp8_pth_gather_lens(const uint8_t* k_data, const float* k_scale, const u
 /* Fused decode attention over the paged E4M3 codes: `rows` query rows per
  * request, its last positions, over its seq_lens[b] positions (host int64
  * [batch]; 0 gives zeros; causal: row j sees the first seq_lens[b] - rows + 1 + j),
- *   K = float(code) * k_scale[token, head], V likewise, softmax in fp32.
+ *   K = float(code) * k_scale[token, head] rounded to `dtype`, V likewise (the
+ *   gather's rows), softmax in fp32.
  * query/out [batch * rows, num_heads, D] of `dtype` (bf16 / fp16), D 128 or 256,
  * block_size % 16 == 0, at most 16 query heads per kv head; other geometries
  * return KVQ_ERR_GEOMETRY.  Block ids as for kvq_fp8_pth_gather.  The lengths

@@ -274,7 +274,8 @@ def _decode_case(dev, lens, *, d, kvh, rep, bs, dtype, index, seed=5, rows=1, ca
         q.to(dev), *views, table.to(dev), lens, [rows] * len(lens), d ** -0.5, causal=causal,
         block_table_host=table.numpy())
     torch.cuda.synchronize()
-    dk, dv = ref.fp8_pth_gather(*[v.cpu() for v in views], table, lens, torch.float32)
+    # the rows attended to are the gather's, in the query's dtype
+    dk, dv = (x.float() for x in ref.fp8_pth_gather(*[v.cpu() for v in views], table, lens, dtype))
     # only rows with a position to see reach the oracle; the others are zeros
     live = [(b, min(rows, n) if causal else rows) for b, n in enumerate(lens) if n]
     at = torch.cat([torch.arange(rows * b + rows - m, rows * (b + 1)) for b, m in live])
@@ -354,3 +355,45 @@ def test_decode_row_forms_agree(gpu_device):
         torch.testing.assert_close(two[1:].float(), want.float(), **TOL)
     with pytest.raises(RuntimeError, match="does not cover the longest sequence"):
         fp8_ops.fp8_per_token_head_attention(q, *views, table, [65, 3, 64], [1] * 3, 0.1)
+
+
+@pytest.mark.parametrize("d,rows,dtype", [(128, 1, torch.bfloat16), (256, 1, torch.bfloat16),
+                                          (128, 3, torch.bfloat16), (128, 1, torch.float16),
+                                          (256, 2, torch.float16)])
+def test_decode_attends_to_the_rows_the_gather_leaves(gpu_device, d, rows, dtype):
+    """The decode's keys and values are the gather's dense rows in the query's dtype:
+    with peaked scores (keys of outlier channels) their rounding shows in the
+    output, so a decode of unrounded rows answers otherwise than a gathered one."""
+    kvh, rep, bs, lens = 2, 4, 32, [2000, 65, 700, 31]
+    gen = torch.Generator().manual_seed(17)
+    need = [-(-n // bs) for n in lens]
+    table = torch.zeros((len(lens), max(need)), dtype=torch.int32)
+    perm = torch.randperm(sum(need), generator=gen).to(torch.int32)
+    for b, k in enumerate(need):
+        table[b, :k] = perm[sum(need[:b]):sum(need[:b + 1])]
+    slots = torch.cat([table[b, torch.arange(n) // bs].long() * bs + torch.arange(n) % bs
+                       for b, n in enumerate(lens)]).to(gpu_device)
+    _, _, views = _views(gpu_device, sum(need), bs, kvh, d)
+    channel = torch.exp(torch.randn((kvh, d), generator=gen))
+    key = (torch.randn((sum(lens), kvh, d), generator=gen) * channel).to(dtype)
+    value = torch.randn((sum(lens), kvh, d), generator=gen).to(dtype)
+    fp8_ops.fp8_per_token_head_store(key.to(gpu_device), value.to(gpu_device), slots, *views)
+    q = torch.randn((rows * len(lens), kvh * rep, d), generator=gen).to(dtype)
+    args = (*views, table.to(gpu_device), lens)
+    got = fp8_ops.fp8_per_token_head_attention(q.to(gpu_device), *args, [rows] * len(lens),
+                                               d ** -0.5, block_table_host=table.numpy())
+    dk, dv = (x.double().cpu() for x in fp8_ops.fp8_per_token_head_dequant_gather(*args, dtype))
+    at = 0
+    for b, n in enumerate(lens):
+        for j in range(rows):
+            k, v = dk[at:at + n - rows + 1 + j], dv[at:at + n - rows + 1 + j]
+            for h in range(kvh * rep):
+                s = k[:, h // rep] @ q[rows * b + j, h].double() * d ** -0.5
+                want = torch.softmax(s, 0) @ v[:, h // rep]
+                # the output's rounding (half a unit in the last place) and a part
+                # in 2^13 of the largest value for p's parts and the fp32 sums
+                ulp = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+                bound = ulp * want.abs() + v.abs().max() * 2.0 ** -13
+                off = (got[rows * b + j, h].double().cpu() - want).abs() - bound
+                assert off.max() <= 0, (b, j, h, off.max().item())
+        at += n

@@ -29,9 +29,8 @@
 //       (~22 bits): two MFMAs, or with GQA groups of at most 8 heads one MFMA
 //       whose columns n and n + 8 carry the two parts (FOLD).  The softmax
 //       scale * log2(e) and the inverse power of two multiply the fp32 scores.
-//   E4M3: codes convert in pairs (v_cvt_scalef32_pk_{bf16,f16}_fp8, exact), B is
-//       the query as it is, one MFMA of its dtype, and the token's key scale
-//       multiplies the fp32 score.
+//   E4M3: A is the dense row the gather would leave, code * scale rounded to the
+//       query's dtype (e4m3_rows); B is the query as it is, one MFMA.
 // PV (O = P * V), one 32-token k-step per tile:
 //   A = P (fp16), row = query head, k = token: lane (g, n) already holds p of
 //       tokens 16j + 4g + r (j = 0, 1; r = 0..3) for head n from the QK
@@ -40,9 +39,9 @@
 //       [(D/16) n, (D/16) (n + 1)) of its 8 token rows and builds code pairs from
 //       byte t of two rows (v_perm + or + packed subtract, exact).
 //   v_aq multiplies the output per dim at the end.
-//   E4M3: the rows' 4 x 4 byte blocks are transposed (v_perm) and converted in
-//       pairs to bf16; A is p times the token's value scale as two bf16 parts,
-//       hi + lo (about 16 bits), two MFMAs.
+//   E4M3: the rows' 4 x 4 byte blocks are transposed (v_perm) and become the
+//       gather's dense rows likewise; A is p as hi + lo parts of the query's
+//       dtype (16 bits of it at least), two MFMAs.
 // Online softmax in the log2 domain; each item leaves (m, l, o) per query head
 // for the log-sum-exp combine.
 //
@@ -66,7 +65,7 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u4v __attribute__((ext_vector_type(4)));
 
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
-typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+typedef float f2 __attribute__((ext_vector_type(2)));
 
 constexpr int kTile = 32;  // tokens per tile: two groups of 16
 constexpr uint32_t kExp64 = 0x64646464u;  // 0x64: high byte of fp16 1024 + u, u < 256
@@ -76,24 +75,34 @@ __device__ __forceinline__ h8 as_h8(uint32_t a, uint32_t b, uint32_t c, uint32_t
   u4v v = {a, b, c, d};
   return __builtin_bit_cast(h8, v);
 }
-__device__ __forceinline__ b8 as_b8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
-  u4v v = {a, b, c, d};
-  return __builtin_bit_cast(b8, v);
-}
-
 __device__ __forceinline__ uint32_t minus1152(uint32_t pair) {
   const h2 v = __builtin_bit_cast(h2, pair) - h2{1152.0f16, 1152.0f16};
   return __builtin_bit_cast(uint32_t, v);
 }
 
-// E4M3 codes (bytes 0, 1 or 2, 3 of x) as a bf16 / fp16 pair, exact.
-template <bool HI>
-__device__ __forceinline__ uint32_t fp8_pair(uint32_t x, bf16) {
-  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(x, 1.0f, HI));
+// Two fp32 values as a bf16 / fp16 pair (round to nearest even), and the pair back.
+__device__ __forceinline__ uint32_t pack2(float lo, float hi, bf16) { return bf16x2_bits(lo, hi); }
+__device__ __forceinline__ uint32_t pack2(float lo, float hi, f16) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{lo, hi}), h2));
 }
-template <bool HI>
-__device__ __forceinline__ uint32_t fp8_pair(uint32_t x, f16) {
-  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(x, 1.0f, HI));
+__device__ __forceinline__ f2 widen2(uint32_t w, bf16) {
+  return f2{__uint_as_float(w << 16), __uint_as_float(w & 0xffff0000u)};
+}
+__device__ __forceinline__ f2 widen2(uint32_t w, f16) {
+  const h2 v = __builtin_bit_cast(h2, w);
+  return f2{static_cast<float>(v[0]), static_cast<float>(v[1])};
+}
+
+// E4M3 codes (bytes 0, 1 or 2, 3 of x) times their scales, as a pair of dense
+// values in T: fp32 product, one rounding, to the bit what the gather leaves.
+// (Exact codes with the scales on the fp32 scores and probabilities take 66.5 us
+// a step of 32 requests of 0.5K-8K positions, 32 heads on 8 kv heads, and these
+// 74.5; but the decode would then answer otherwise than the same rows gathered:
+// 0.0047 apart, 0.06 at the worst element.)
+template <bool HI, typename T>
+__device__ __forceinline__ uint32_t e4m3_rows(uint32_t x, float s0, float s1, T) {
+  const auto v = __builtin_amdgcn_cvt_pk_f32_fp8(x, HI);
+  return pack2(v[0] * s0, v[1] * s1, T{});
 }
 __device__ __forceinline__ f4 mfma_q(u4v a, u4v b, f4 c, bf16) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, a),
@@ -127,12 +136,13 @@ __device__ __forceinline__ uint32_t h2_bits(_Float16 a, _Float16 b) {
 
 // One tile's codes in registers.  k[j][u]: the 16 bytes from D/4 g + 16 u on of
 // token 16j + n; v[j][r][w]: word w of bytes [D/16 n, D/16 (n + 1)) of token
-// 16j + 4g + r; ksc / vsc (E4M3): scales of tokens 16j + 4g + r.
+// 16j + 4g + r; ksc (E4M3): scale of token 16j + n, vsc: of tokens 16j + 4g + r.
 template <int D, bool FP8>
 struct TileRegs {
   uint4 k[2][D / 64];
   uint32_t v[2][4][D / 64];
-  f4 ksc[FP8 ? 2 : 1], vsc[FP8 ? 2 : 1];
+  float ksc[FP8 ? 2 : 1];
+  f4 vsc[FP8 ? 2 : 1];
 };
 
 struct WaveCtx {
@@ -218,9 +228,9 @@ __device__ __forceinline__ void read_tile_lds(TileRegs<D, FP8>& t, const char* b
       }
     }
     if constexpr (FP8) {
-      const float* sc = reinterpret_cast<const float*>(buf + 2 * kTile * D) + 16 * j + 4 * g;
-      t.ksc[j] = *reinterpret_cast<const f4*>(sc);
-      t.vsc[j] = *reinterpret_cast<const f4*>(sc + kTile);
+      const float* sc = reinterpret_cast<const float*>(buf + 2 * kTile * D) + 16 * j;
+      t.ksc[j] = sc[n];
+      t.vsc[j] = *reinterpret_cast<const f4*>(sc + kTile + 4 * g);
     }
   }
 }
@@ -258,8 +268,9 @@ __device__ __forceinline__ void compute_tile(const TileRegs<D, FP8>& t, int p, i
       const uint4& kw = t.k[j][ks / 2];
       const uint32_t w0 = ks % 2 ? kw.z : kw.x, w1 = ks % 2 ? kw.w : kw.y;
       if constexpr (FP8) {
-        const u4v a = {fp8_pair<false>(w0, TQ{}), fp8_pair<true>(w0, TQ{}),
-                       fp8_pair<false>(w1, TQ{}), fp8_pair<true>(w1, TQ{})};
+        const float k = t.ksc[j];
+        const u4v a = {e4m3_rows<false>(w0, k, k, TQ{}), e4m3_rows<true>(w0, k, k, TQ{}),
+                       e4m3_rows<false>(w1, k, k, TQ{}), e4m3_rows<true>(w1, k, k, TQ{})};
         s[j] = mfma_q(a, qh[ks], s[j], TQ{});
       } else {
         const uint32_t x0 = w0 ^ kFlip, x1 = w1 ^ kFlip;
@@ -285,7 +296,7 @@ __device__ __forceinline__ void compute_tile(const TileRegs<D, FP8>& t, int p, i
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int tok = p + 16 * j + 4 * g + r;
-      const float x = FP8 ? s[j][r] * (sc * t.ksc[j][r]) : s[j][r] * sc;
+      const float x = s[j][r] * sc;
       const float v = (tok >= pb && tok < pen) ? x : -INFINITY;
       s[j][r] = v;
       mx = fmaxf(mx, v);
@@ -318,23 +329,27 @@ __device__ __forceinline__ void compute_tile(const TileRegs<D, FP8>& t, int p, i
   }
   // ---- O += P * V: one k-step of 32 tokens ----
   if constexpr (FP8) {
-    uint32_t ph[4], pl[4];  // p * value scale of the lane's 8 tokens, hi and lo parts
+    uint32_t ph[4], pl[4];  // p of the lane's 8 tokens, hi and lo parts
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int j = u / 2, r = 2 * (u % 2);
-      float y[2];
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        // past the item p = 0, but the scale may be unwritten: no 0 * NaN
-        const int tok = p + 16 * j + 4 * g + r + k;
-        y[k] = tok >= pb && tok < pen ? s[j][r + k] * t.vsc[j][r + k] : 0.0f;
-      }
-      ph[u] = bf16x2_bits(y[0], y[1]);
-      pl[u] = bf16x2_bits(y[0] - __uint_as_float(ph[u] << 16),
-                          y[1] - __uint_as_float(ph[u] & 0xffff0000u));
+      ph[u] = pack2(s[j][r], s[j][r + 1], TQ{});
+      const f2 hi = widen2(ph[u], TQ{});
+      pl[u] = pack2(s[j][r] - hi[0], s[j][r + 1] - hi[1], TQ{});
     }
-    const b8 ah = as_b8(ph[0], ph[1], ph[2], ph[3]);
-    const b8 al = as_b8(pl[0], pl[1], pl[2], pl[3]);
+    const u4v ah = {ph[0], ph[1], ph[2], ph[3]}, al = {pl[0], pl[1], pl[2], pl[3]};
+    // rows past the item may hold NaN codes and scales (their p is 0)
+    const bool whole = p >= pb && p + kTile <= pe;  // uniform
+    f4 vsc[2] = {t.vsc[0], t.vsc[1]};
+    if (!whole) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int tok = p + 16 * j + 4 * g + r;
+          vsc[j][r] = tok >= pb && tok < pe ? vsc[j][r] : 0.0f;
+        }
+    }
 #pragma unroll
     for (int w = 0; w < D / 64; ++w) {
       uint32_t tr[4][2];  // byte b of the 8 tokens' words, tokens 4j .. 4j + 3 in [b][j]
@@ -343,7 +358,7 @@ __device__ __forceinline__ void compute_tile(const TileRegs<D, FP8>& t, int p, i
         uint32_t x[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) x[r] = t.v[j][r][w];
-        if (p < pb || p + kTile > pe) {  // uniform: rows past the item may hold NaN codes
+        if (!whole) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const int tok = p + 16 * j + 4 * g + r;
@@ -361,11 +376,13 @@ __device__ __forceinline__ void compute_tile(const TileRegs<D, FP8>& t, int p, i
       }
 #pragma unroll
       for (int b = 0; b < 4; ++b) {
-        const b8 v = as_b8(fp8_pair<false>(tr[b][0], bf16{}), fp8_pair<true>(tr[b][0], bf16{}),
-                           fp8_pair<false>(tr[b][1], bf16{}), fp8_pair<true>(tr[b][1], bf16{}));
+        const u4v v = {e4m3_rows<false>(tr[b][0], vsc[0][0], vsc[0][1], TQ{}),
+                       e4m3_rows<true>(tr[b][0], vsc[0][2], vsc[0][3], TQ{}),
+                       e4m3_rows<false>(tr[b][1], vsc[1][0], vsc[1][1], TQ{}),
+                       e4m3_rows<true>(tr[b][1], vsc[1][2], vsc[1][3], TQ{})};
         f4& o = st.o[4 * w + b];
-        o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, v, o, 0, 0, 0);
-        o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, v, o, 0, 0, 0);
+        o = mfma_q(ah, v, o, TQ{});
+        o = mfma_q(al, v, o, TQ{});
       }
     }
   } else {
@@ -492,8 +509,8 @@ __device__ __forceinline__ void write_meta(int lane, int32_t* __restrict__ meta)
 // E4M3 with several query rows per request (RowCols): the columns of the score
 // MFMA are the rows' heads, each with its own last position, so that 16 / rep
 // rows share one pass over the codes.  32 requests of 0.5K-8K positions, 32 heads
-// on 8 kv heads: 77 us for 4 rows, 138 for 8 (two passes), 246 for 16 (four);
-// gathered to dense rows first they take 294, 302 and 310.
+// on 8 kv heads: 75 us for 4 rows, 139 for 8 (two passes), 267 for 16 (four);
+// gathered to dense rows first they take 286, 294 and 302.
 struct RowCols {
   int rows;   // query rows of a request
   int first;  // first of them in this pass

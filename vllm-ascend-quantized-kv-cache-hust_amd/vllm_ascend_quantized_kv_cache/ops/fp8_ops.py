@@ -257,9 +257,11 @@ def fp8_per_token_head_dequant_gather(
 
 #: passes over a request's codes up to which its query rows take the fused
 #: decode instead of the dense gather (a pass scores 16 (row, head) columns).
-#: Three passes won on every shape measured (38 requests of 0.6K-7.9K positions,
-#: 14 heads on 2: 45 us for 2 rows, 54 for 4, against 100 and 103 gathered); four
-#: lose 8% on 16 short requests (82 us against 75), and eight lose up to 45%.
+#: Three passes win where the codes weigh (38 requests of 0.6K-7.9K positions, 14
+#: heads on 2: 34, 55 and 68 us for one to three passes against 86, 88 and 90
+#: gathered; 64 of 30-200, 56 heads on 8: 40 against 41) and are level where a few
+#: long requests leave the chip part empty (4 of 3K-16K, 8 heads on 2: 47 - 52
+#: against 44 - 49); four lose on 16 of 100-900 (40 against 37).
 DECODE_PASSES = 3
 
 
