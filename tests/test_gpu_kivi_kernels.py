@@ -880,6 +880,78 @@ def test_split_decode_head_256_keeps_its_precision(gpu_device, g, bs, rep, size)
     assert err.max() < (3e-3 if size < 1 else 2.0 ** -11), err.tolist()
 
 
+def _wide_error(dev, dtype, g, bs, rep, lens, make, q, scale):
+    """2-norm error per (request, head) of a decode at head size 256, one kv head,
+    relative to 64-bit attention over the dequantized history."""
+    from vllm_ascend_quantized_kv_cache.ops.kivi_decode import (
+        DecodeSeq,
+        kivi_decode_attention,
+        plan_decode,
+    )
+
+    d = 256
+    cpu, table, ring_k, ring_v, seqs, wk, wv, _, _ = _ring_case(
+        dev, d, 1, g, bs, 128, lens, seed=47, ring_dtype=dtype, make=make)
+    dk, dv = ref.dequant_gather(*cpu, table, torch.tensor(lens), torch.float32, g)
+    dk, dv = ref.overlay_residual(dk, lens, wk), ref.overlay_residual(dv, lens, wv)
+    want, at = [], 0
+    for b, n in enumerate(lens):
+        k, v = dk[at:at + n, 0].double(), dv[at:at + n, 0].double()
+        want.append(torch.softmax(q[b].double() @ k.T * scale, -1) @ v)
+        at += n
+    want = torch.stack(want)
+    dseqs = [DecodeSeq(n, hk, hv, row, ks_, vs_) for (n, hk, hv, row, ks_, vs_) in seqs]
+    plan = tuple(torch.from_numpy(x).to(dev) for x in plan_decode(dseqs, 1, 256))
+    got = kivi_decode_attention(q.to(dev), to_dev(cpu, dev), table.to(dev), dseqs,
+                                ring_k.to(dev), ring_v.to(dev), scale, g, plan=plan)
+    err = (got.double().cpu() - want).norm(dim=-1) / want.norm(dim=-1)
+    print(f"{dtype} g={g} rep={rep}: {err.max().item():.3g}", flush=True)
+    return err
+
+
+#: The output's rounding and nothing beside it: the rms error of a rounding to 8
+#: (11) bits, relative to a value at the bottom of its binade (0.0017 and 0.0002
+#: over a spread of values).
+WIDE_BOUND = {torch.bfloat16: 2.0 ** -7 / 12 ** 0.5, torch.float16: 2.0 ** -10 / 12 ** 0.5}
+
+
+@pytest.mark.parametrize("g,bs,rep", [(128, 128, 8), (64, 64, 12)])
+@pytest.mark.parametrize("size", [1e4, 1.0, 1e-2, 1e-3, 1e-4, 1e-5])
+def test_split_decode_head_256_values_of_any_size(gpu_device, g, bs, rep, size):
+    """Head size 256, bf16, down to values whose scales sit at their floor of 1e-6."""
+    def make(n, h_, d_, seed):
+        gen = torch.Generator().manual_seed(seed)
+        key = torch.randn(n, h_, d_, generator=gen).to(torch.bfloat16)
+        return key, (size * torch.randn(n, h_, d_, generator=gen)).to(torch.bfloat16)
+
+    lens = [9000, 1025, 300, 40]
+    q = torch.randn(len(lens), rep, 256, generator=torch.Generator().manual_seed(2))
+    err = _wide_error(gpu_device, torch.bfloat16, g, bs, rep, lens, make, q.to(torch.bfloat16),
+                      256 ** -0.5)
+    assert err.max() < WIDE_BOUND[torch.bfloat16], err.tolist()
+
+
+@pytest.mark.parametrize("g,bs,rep", [(128, 128, 8), (64, 128, 12)])
+def test_split_decode_head_256_values_shrinking_as_probabilities_grow(gpu_device, g, bs, rep):
+    """Values from 1e3 down to 1e-6 over a request whose probabilities grow by as
+    much: every position counts alike, and no tile's largest value scale tells
+    how small the products of another's probabilities are."""
+    u = torch.nn.functional.normalize(
+        torch.randn(256, generator=torch.Generator().manual_seed(3)), dim=0)
+
+    def make(n, h_, d_, seed):
+        gen = torch.Generator().manual_seed(seed)
+        at = torch.arange(n)[:, None, None] / n
+        key = 20.723 * at * u + 0.02 * torch.randn(n, h_, d_, generator=gen)  # 9 ln(10)
+        value = 10.0 ** (3 - 9 * at) * torch.randn(n, h_, d_, generator=gen)
+        return key.to(torch.bfloat16), value.to(torch.bfloat16)
+
+    lens = [6000, 700]
+    q = (16.0 * u).expand(len(lens), rep, 256).to(torch.bfloat16)
+    err = _wide_error(gpu_device, torch.bfloat16, g, bs, rep, lens, make, q, 1 / 16)
+    assert err.max() < WIDE_BOUND[torch.bfloat16], err.tolist()
+
+
 @pytest.mark.parametrize("d", [128, 256])
 def test_combine_of_item_counts_at_its_edges(gpu_device, d):
     """15 to 18 items a request (rows ahead of the weights, or only the live ones

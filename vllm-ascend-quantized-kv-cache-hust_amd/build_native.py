@@ -54,7 +54,7 @@ EXTRA_FLAGS = {
     "kivi_pack.hip": ["-fno-honor-nans"],
     "fp8_kv.hip": ["-fno-honor-nans"],
     # MFMA results in ordinary registers where a kernel may also use accumulation
-    # registers: the 256-dim decode otherwise copies its 72 running sums between
+    # registers: the 256-dim decode otherwise copies its 64 running sums between
     # the two files on every tile
     "decode_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }

@@ -32,7 +32,7 @@
 // group's operands kept over its two tiles, and MFMA results in ordinary
 // registers (a build flag): 69.1 -> 62.0 us on the 64 requests above, 58.4 ->
 // 52.6 on 20 of 0.5K-10K with 2 kv heads of 256, 40.5 -> 38.7 on the 40.  (The
-// two parts of P that compute_tile takes at 256 dims then added 3 - 4 us.)
+// parts of P' that compute_tile takes at 256 dims then added 4 us.)
 #include <algorithm>
 
 #include "decode_tail.h"

@@ -26,6 +26,20 @@
 //           accumulation);
 //   values  all slots keep it; a constant-B MFMA (1024 in every slot) over the
 //           same P' removes it (1024 * P' and 64 * P' at the primed slots).
+//
+// Head size 256, values: no offsets whose sums cancel, and parts of P' that neither
+// overflow nor lose bits to the subnormals (its calls had an fp32 kernel before).
+//   codes   a nibble in a byte is the E4M3 value c / 512 (0..7 its subnormals, 8..15
+//           the first normal binade), so one v_and_b32 per four codes and the
+//           paired E4M3 conversions give exact bf16 operands, 7 instructions for
+//           8 codes where the 1024 magic and its removal take 9.  The 512 goes to
+//           the fp32 results.
+//               slot i   0  1  2  3  4  5  6  7
+//               nibble   0  2  4  6  1  3  5  7
+//   P'      three bf16 parts, which hold an fp32 whole whatever its size.
+// 4 requests of 40 - 9K positions, 8 heads on 1 kv head, values of size 1e4 down to
+// 1e-5: 0.0018 - 0.0019 from 64 bits (the bf16 output's rounding) throughout, where
+// fp16 parts of P' were 0.09 off at 1e-5.
 #pragma once
 
 #include <type_traits>
@@ -38,6 +52,7 @@ namespace tr {
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 typedef float f2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u4v __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));
@@ -45,13 +60,23 @@ typedef __attribute__((address_space(3))) v2i* lds_v2i_ptr;
 
 constexpr uint32_t kMagic = 0x64006400u;  // fp16 1024.0 in both halves
 
-// nibble of slot i: 4*(i & 1) + (i >> 1)
+// nibble of slot i (at head size 128): 4*(i & 1) + (i >> 1)
 __host__ __device__ constexpr int slot_nib(int i) { return 4 * (i & 1) + (i >> 1); }
-__host__ __device__ constexpr bool slot_primed(int i) { return (i & 2) != 0; }
+// ... and at head size D
+template <int D>
+__host__ __device__ constexpr int slot_nib_of(int i) {
+  return D == 256 ? 2 * (i & 3) + (i >> 2) : slot_nib(i);
+}
+// slot_nib's inverse: where a tile's scale table holds the token of nibble j
+__host__ __device__ constexpr int nib_slot(int j) { return 2 * (j & 3) + (j >> 2); }
 
 __device__ __forceinline__ h8 as_h8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
   u4v v = {a, b, c, d};
   return __builtin_bit_cast(h8, v);
+}
+__device__ __forceinline__ b8 as_b8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+  u4v v = {a, b, c, d};
+  return __builtin_bit_cast(b8, v);
 }
 
 // The three constants of the conversion, held in VGPRs: v_and_or_b32 is a
@@ -88,16 +113,17 @@ __device__ __forceinline__ h8 key_codes(uint32_t w, const Consts& c) {
   return as_h8(p0, and_or(w, c.hi, c.magic), p2, and_or(w8, c.hi, c.magic));
 }
 
-// ... with the 1024 removed from all slots: c and, primed, 16c
-__device__ __forceinline__ h8 plain_codes(uint32_t w, const Consts& c) {
-  const uint32_t w8 = w >> 8;
-  const h2 off = h2{1024.0f16, 1024.0f16};
-  auto drop = [&](uint32_t x) {
-    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, x) - off);
+// The eight slots of the 8 codes in w at head size 256: c / 512, exact.
+__device__ __forceinline__ b8 codes_bf16(uint32_t w) {
+  const uint32_t e = w & 0x0f0f0f0fu, o = (w >> 4) & 0x0f0f0f0fu;
+  auto pair = [](uint32_t x, auto hi) {
+    return __builtin_bit_cast(
+        uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(x, 1.0f, decltype(hi)::value));
   };
-  return as_h8(drop(and_or(w, c.lo, c.magic)), drop(and_or(w, c.hi, c.magic)),
-               drop(and_or(w8, c.lo, c.magic)), drop(and_or(w8, c.hi, c.magic)));
+  return as_b8(pair(e, std::false_type{}), pair(e, std::true_type{}), pair(o, std::false_type{}),
+               pair(o, std::true_type{}));
 }
+constexpr float kCodeUnit = 512.0f;
 
 __device__ __forceinline__ uint32_t lds_off(const void* p) {
   return static_cast<uint32_t>(
@@ -402,12 +428,14 @@ __device__ __forceinline__ void prepare_group(const uint32_t* W, int n, int kg,
 
 // Running state of one wave: softmax max / sum (log2 domain), the PV
 // accumulators o_acc[v] (dims 16 v + column), the constant-B MFMA sums that
-// remove the 1024 offset (one per value group), and the value-minima term.
+// remove the 1024 offset (one per value group; no offset at head size 256, DB
+// 16), and the value-minima term.
 template <int NVG, int DB = 8>
 struct Acc {
+  static constexpr bool kOffset = DB == 8;
   float m_run, l_run;
   f4 o_acc[DB];
-  f4 c_acc[NVG];
+  f4 c_acc[kOffset ? NVG : 1];
   float bias_v[NVG];
   __device__ __forceinline__ void init() {
     m_run = -INFINITY;
@@ -416,7 +444,7 @@ struct Acc {
     for (int q = 0; q < DB; ++q) o_acc[q] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int v = 0; v < NVG; ++v) {
-      c_acc[v] = f4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (kOffset) c_acc[v] = f4{0.f, 0.f, 0.f, 0.f};
       bias_v[v] = 0.0f;
     }
   }
@@ -450,12 +478,7 @@ __device__ __forceinline__ void compute_tile(const uint32_t* W, uint32_t buf_off
 #pragma clang fp contract(fast)
   using T = Tile<NVG, KSV, D>;
   constexpr int DB = D / 16;
-  // P' (p times the value scale) as one fp16 against codes that keep their offset,
-  // or as fp16 hi + lo parts against plain codes.  Rounded once, P' disagrees
-  // with the fp32 p of the minima term, and the offset's sums cancel: 0.0005 of
-  // the output against 0.0002 at 64 bits' distance (fp16 queries, 256 dims,
-  // 1K-9K positions), for 60.1 against 64 us on 64 requests of 1K-16K.
-  constexpr bool kSplitP = D == 256;
+  constexpr bool kWide = D == 256;
   static_assert(T::KW == Tile<1, false>::KW && T::VW == Tile<1, false, D>::VW,
                 "read bases assume the common word offsets");
   const Consts cst;
@@ -512,26 +535,6 @@ __device__ __forceinline__ void compute_tile(const uint32_t* W, uint32_t buf_off
   }
   float tmax = fmaxf(fmaxf(tm[0], tm[1]), fmaxf(tm[2], tm[3]));
   tmax = max_rows4(tmax);
-  if constexpr (kSplitP) {
-    // p up to 2^4 instead of 1 (the partial's m is the exponent offset, so any
-    // will do): fp16 parts of small p, and of the 1/16 of the primed slots, then
-    // lose no bits to the subnormals.  Less where a value scale would overflow.
-    const int lane = 16 * kg + n;
-    const float* sv = reinterpret_cast<const float*>(W + T::VS) + lane;
-    float big = sv[0];
-#pragma unroll
-    for (int vg = 1; vg < NVG; ++vg) big = fmaxf(big, sv[64 * vg]);
-    if (!FULL) {
-      const int pos = p0 + tau((lane >> 3) & 3, 8 * (lane >> 5) + slot_nib(lane & 7));
-      big = pos >= pb && pos < pe ? big : 0.0f;
-    }
-    float shift = 4.0f;
-    if (__builtin_amdgcn_ballot_w64(big > 2048.0f) != 0) {  // uniform
-      big = max_wave64(big);
-      shift = 141.0f - static_cast<float>(__float_as_uint(big) >> 23);  // 2^shift * big < 2^15
-    }
-    tmax -= shift;
-  }
   const float m_new = fmaxf(acc.m_run, tmax);
   const float alpha = acc.m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(acc.m_run - m_new);
   float ps[4];
@@ -551,22 +554,21 @@ __device__ __forceinline__ void compute_tile(const uint32_t* W, uint32_t buf_off
       const float ar = __shfl(alpha, 4 * kg + r, 64);
 #pragma unroll
       for (int q = 0; q < DB; ++q) acc.o_acc[q][r] *= ar;
+      if constexpr (!kWide)
 #pragma unroll
-      for (int v = 0; v < NVG; ++v) acc.c_acc[v][r] *= ar;
+        for (int v = 0; v < NVG; ++v) acc.c_acc[v][r] *= ar;
     }
 #pragma unroll
     for (int v = 0; v < NVG; ++v) acc.bias_v[v] *= alpha;
   }
   // ---- PV: O[head][dim 16 v + col] += P'[head][token] * V[token][dim] -------------
-  const h8 ones_b = as_h8(kMagic, kMagic, kMagic, kMagic);
   const float* vsf = reinterpret_cast<const float*>(W + T::VS) + 8 * kg;
   const float* vmf = reinterpret_cast<const float*>(W + T::VM) + 8 * kg;
-  const h2 sixteenth = h2{0.0625f16, 0.0625f16};
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
-    // P' of k-step s, value group vg: slot i holds token tau(kg, 8 s + slot_nib(i)),
-    // whose p is sacc[2 s + (i & 1)][i >> 1]
-    h8 pa[NVG], pl[NVG];
+    // P' of k-step s, value group vg: slot i holds token tau(kg, 8 s + nibble of i),
+    // whose p is sacc[2 s + nibble / 4][nibble % 4]
+    u4v part[NVG][kWide ? 3 : 1];
 #pragma unroll
     for (int vg = 0; vg < NVG; ++vg) {
       const f4 s0 = *reinterpret_cast<const f4*>(vsf + 64 * vg + 32 * s);
@@ -576,13 +578,14 @@ __device__ __forceinline__ void compute_tile(const uint32_t* W, uint32_t buf_off
       float pp[8], bsum[2] = {0.0f, 0.0f};
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const float p = sacc[2 * s + (i & 1)][i >> 1];
-        float sv = i < 4 ? s0[i] : s1[i - 4];
-        float mv = i < 4 ? m0[i] : m1[i - 4];
+        const int j = slot_nib_of<D>(i), t = nib_slot(j);
+        const float p = sacc[2 * s + j / 4][j % 4];
+        float sv = t < 4 ? s0[t] : s1[t - 4];
+        float mv = t < 4 ? m0[t] : m1[t - 4];
         if (!FULL) {
           // outside the range p = 0, but the scale/min bytes may be unwritten:
           // select zeros so a stale NaN cannot reach the sums
-          const int pos = p0 + tau(kg, 8 * s + slot_nib(i));
+          const int pos = p0 + tau(kg, 8 * s + j);
           const bool live = pos >= pb && pos < pe;
           sv = live ? sv : 0.0f;
           mv = live ? mv : 0.0f;
@@ -591,38 +594,52 @@ __device__ __forceinline__ void compute_tile(const uint32_t* W, uint32_t buf_off
         bsum[i & 1] += p * mv;
       }
       acc.bias_v[vg] += bsum[0] + bsum[1];
-      // primed slots (pairs 1 and 3) carry 1/16: their codes read as 16c
-      const uint32_t a1 = __builtin_bit_cast(
-          uint32_t, __builtin_bit_cast(h2, pack_h2(pp[2], pp[3])) * sixteenth);
-      const uint32_t a3 = __builtin_bit_cast(
-          uint32_t, __builtin_bit_cast(h2, pack_h2(pp[6], pp[7])) * sixteenth);
-      const uint32_t a0 = pack_h2(pp[0], pp[1]), a2 = pack_h2(pp[4], pp[5]);
-      pa[vg] = as_h8(a0, a1, a2, a3);
-      if constexpr (kSplitP) {
-        const uint32_t h1 = pack_h2(pp[2], pp[3]), h3 = pack_h2(pp[6], pp[7]);
-        auto rest = [](float x0, float x1, uint32_t hi) {
-          return pack_h2(sub_half_sel<0>(x0, hi, -1.0f), sub_half_sel<1>(x1, hi, -1.0f));
-        };
-        const h2 l1 = __builtin_bit_cast(h2, rest(pp[2], pp[3], h1)) * sixteenth;
-        const h2 l3 = __builtin_bit_cast(h2, rest(pp[6], pp[7], h3)) * sixteenth;
-        pl[vg] = as_h8(rest(pp[0], pp[1], a0), __builtin_bit_cast(uint32_t, l1),
-                       rest(pp[4], pp[5], a2), __builtin_bit_cast(uint32_t, l3));
+      if constexpr (kWide) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          float a = pp[2 * u], b = pp[2 * u + 1];
+#pragma unroll
+          for (int k = 0; k < 3; ++k) {  // each difference is exact
+            const uint32_t w = bf16x2_bits(a, b);
+            part[vg][k][u] = w;
+            a -= __uint_as_float(w << 16);
+            b -= __uint_as_float(w & 0xffff0000u);
+          }
+        }
+      } else {
+        // primed slots (pairs 1 and 3) carry 1/16: their codes read as 16c
+        const h2 sixteenth = h2{0.0625f16, 0.0625f16};
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const uint32_t w = pack_h2(pp[2 * u], pp[2 * u + 1]);
+          part[vg][0][u] =
+              u & 1 ? __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, w) * sixteenth) : w;
+        }
       }
     }
 #pragma unroll
     for (int v = 0; v < DB; ++v) {
       const int vg = v / (DB / NVG);
       const uint32_t w = static_cast<uint32_t>(rv[v][s]);
-      const h8 bv = kSplitP ? plain_codes(w, cst) : codes(w, cst);
-      acc.o_acc[v] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[vg], bv, acc.o_acc[v], 0, 0, 0);
-      if constexpr (kSplitP)
-        acc.o_acc[v] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl[vg], bv, acc.o_acc[v], 0, 0, 0);
-    }
+      f4& o = acc.o_acc[v];
+      if constexpr (kWide) {
+        const b8 bv = codes_bf16(w);
 #pragma unroll
-    for (int vg = 0; vg < NVG; ++vg)
-      if constexpr (!kSplitP)
-        acc.c_acc[vg] =
-            __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[vg], ones_b, acc.c_acc[vg], 0, 0, 0);
+        for (int k = 0; k < 3; ++k)
+          o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, part[vg][k]), bv, o,
+                                                      0, 0, 0);
+      } else {
+        o = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, part[vg][0]),
+                                                   codes(w, cst), o, 0, 0, 0);
+      }
+    }
+    if constexpr (!kWide) {
+      const h8 ones_b = as_h8(kMagic, kMagic, kMagic, kMagic);
+#pragma unroll
+      for (int vg = 0; vg < NVG; ++vg)
+        acc.c_acc[vg] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+            __builtin_bit_cast(h8, part[vg][0]), ones_b, acc.c_acc[vg], 0, 0, 0);
+    }
   }
 }
 
@@ -639,7 +656,10 @@ __device__ __forceinline__ void finish(Acc<NVG, DB>& acc, int kg, f4 (&o)[DB]) {
     for (int v = 0; v < DB; ++v) {
       const int vg = v / (DB / NVG);
       const float bv = __shfl(acc.bias_v[vg], hh, 64);
-      o[v][r] = acc.o_acc[v][r] - acc.c_acc[vg][r] + bv;
+      if constexpr (Acc<NVG, DB>::kOffset)
+        o[v][r] = acc.o_acc[v][r] - acc.c_acc[vg][r] + bv;
+      else
+        o[v][r] = acc.o_acc[v][r] * kCodeUnit + bv;
     }
   }
 }
