@@ -952,6 +952,32 @@ def test_split_decode_head_256_values_shrinking_as_probabilities_grow(gpu_device
     assert err.max() < WIDE_BOUND[torch.bfloat16], err.tolist()
 
 
+@pytest.mark.parametrize("g,bs,rep", [(128, 128, 8), (64, 128, 12)])
+@pytest.mark.parametrize("dtype,q_size,k_size", [
+    (torch.bfloat16, 1e3, 1e3),    # a query times a key scale past 65504
+    (torch.bfloat16, 1e15, 1e15),
+    (torch.bfloat16, 1e-4, 1e-3),  # ... and below the fp16 subnormals
+    (torch.bfloat16, 1e-20, 1e-4),
+    (torch.float16, 400, 400),
+])
+def test_split_decode_head_256_keys_of_any_size(gpu_device, g, bs, rep, dtype, q_size, k_size):
+    """Queries and keys of any size, the score scale to match; the channels spread
+    over a factor of some hundred."""
+    channel = torch.exp(torch.randn(256, generator=torch.Generator().manual_seed(4)))
+
+    def make(n, h_, d_, seed):
+        gen = torch.Generator().manual_seed(seed)
+        key = k_size * channel * torch.randn(n, h_, d_, generator=gen)
+        return key.to(dtype), torch.randn(n, h_, d_, generator=gen).to(dtype)
+
+    lens = [3000, 129, 40]
+    q = q_size / channel * torch.randn(len(lens), rep, 256,
+                                       generator=torch.Generator().manual_seed(5))
+    err = _wide_error(gpu_device, dtype, g, bs, rep, lens, make, q.to(dtype),
+                      2 / 16 / q_size / k_size)
+    assert err.max() < WIDE_BOUND[dtype], err.tolist()
+
+
 @pytest.mark.parametrize("d", [128, 256])
 def test_combine_of_item_counts_at_its_edges(gpu_device, d):
     """15 to 18 items a request (rows ahead of the weights, or only the live ones

@@ -298,7 +298,7 @@ kivi_decode_split_kernel(const TQ* __restrict__ query, int hq, int kvh, float qs
       const uint32_t* W = reinterpret_cast<const uint32_t*>(my_lds + cb * T::BYTES);
       // the second tile of a 128-position key group runs on the first one's
       // operands (unfolded, twice the operands, they spill if kept)
-      if (!FOLD || p != again) tr::prepare_group<TQ, NVG, KSV, FOLD, D>(W, n, kg, ql, qscale, qg);
+      if (!FOLD || p != again) tr::prepare_group<TQ, NVG, KSV, FOLD>(W, n, kg, ql, qscale, qg);
       again = ((p + 64) & (g - 1)) != 0 ? p + 64 : -1;
       const uint32_t off = my_off + static_cast<uint32_t>(cb * T::BYTES);
       if (p >= tb && p + 64 <= te)

@@ -27,19 +27,24 @@
 //   values  all slots keep it; a constant-B MFMA (1024 in every slot) over the
 //           same P' removes it (1024 * P' and 64 * P' at the primed slots).
 //
-// Head size 256, values: no offsets whose sums cancel, and parts of P' that neither
-// overflow nor lose bits to the subnormals (its calls had an fp32 kernel before).
+// Head size 256 computes what fp32 arithmetic would for every finite input (its
+// calls had an fp32 kernel before this one): no offsets whose sums cancel, and
+// operand parts that neither overflow nor lose bits to the subnormals.
 //   codes   a nibble in a byte is the E4M3 value c / 512 (0..7 its subnormals, 8..15
 //           the first normal binade), so one v_and_b32 per four codes and the
-//           paired E4M3 conversions give exact bf16 operands, 7 instructions for
-//           8 codes where the 1024 magic and its removal take 9.  The 512 goes to
-//           the fp32 results.
+//           paired E4M3 conversions give exact fp16 (keys) and bf16 (values)
+//           operands, 7 instructions for 8 codes where the 1024 magic and its
+//           removal take 9.  The 512 goes to the fp32 results.
 //               slot i   0  1  2  3  4  5  6  7
 //               nibble   0  2  4  6  1  3  5  7
-//   P'      three bf16 parts, which hold an fp32 whole whatever its size.
+//   keys    Q' = q * key_scale, times the power of two per head and key group that
+//           puts the largest of them in [2^14, 2^15), as fp16 hi + lo parts: an
+//           error of 2^-40 of the largest or 2^-23 of its own value.
+//   values  P' as three bf16 parts, which hold an fp32 whole whatever its size.
 // 4 requests of 40 - 9K positions, 8 heads on 1 kv head, values of size 1e4 down to
 // 1e-5: 0.0018 - 0.0019 from 64 bits (the bf16 output's rounding) throughout, where
-// fp16 parts of P' were 0.09 off at 1e-5.
+// fp16 parts of P' were 0.09 off at 1e-5; queries times key scales of 1e30 or 1e-24
+// likewise, where fp16 parts without the power of two gave NaN and noise.
 #pragma once
 
 #include <type_traits>
@@ -114,6 +119,15 @@ __device__ __forceinline__ h8 key_codes(uint32_t w, const Consts& c) {
 }
 
 // The eight slots of the 8 codes in w at head size 256: c / 512, exact.
+__device__ __forceinline__ h8 codes_f16(uint32_t w) {
+  const uint32_t e = w & 0x0f0f0f0fu, o = (w >> 4) & 0x0f0f0f0fu;
+  auto pair = [](uint32_t x, auto hi) {
+    return __builtin_bit_cast(
+        uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(x, 1.0f, decltype(hi)::value));
+  };
+  return as_h8(pair(e, std::false_type{}), pair(e, std::true_type{}), pair(o, std::false_type{}),
+               pair(o, std::true_type{}));
+}
 __device__ __forceinline__ b8 codes_bf16(uint32_t w) {
   const uint32_t e = w & 0x0f0f0f0fu, o = (w >> 4) & 0x0f0f0f0fu;
   auto pair = [](uint32_t x, auto hi) {
@@ -238,7 +252,7 @@ __device__ __forceinline__ void issue_tile(char* buf, const LaneDma& ld, const u
 
 // The lane's query values: head n of the GQA group (n & 7 when folded),
 // dims 64 P + 16 kg + 8 e + slot_nib(i) in k-step s = 2 P + e, slot i, with
-// the primed slots scaled by 1/16 (exact).  16-bit inputs stay packed as slot
+// the primed slots scaled by 1/16 (exact; none are at head size 256).  16-bit inputs stay packed as slot
 // pairs (16 VGPRs instead of 32 across the item) and widen where a key group
 // is prepared; bf16 pairs are pre-scaled (a bf16 exponent change is exact),
 // fp16 pairs scale in the widening fma.  Lanes past the group hold 0.
@@ -261,7 +275,9 @@ __device__ __forceinline__ f2 widen_pair(uint32_t w, int p, f16) {
 template <typename TQ, int D = 128>
 struct QLane {
   uint32_t w[D / 32][4];  // pair p of k-step s: slots 2p (low half) and 2p + 1
-  __device__ __forceinline__ f2 get(int s, int p) const { return widen_pair(w[s][p], p, TQ{}); }
+  __device__ __forceinline__ f2 get(int s, int p) const {
+    return widen_pair(w[s][p], D == 256 ? 0 : p, TQ{});
+  }
 };
 template <>
 struct QLane<float, 128> {
@@ -286,13 +302,13 @@ __device__ __forceinline__ QLane<TQ, D> load_q_at(F&& at, int rep, int n, int kg
     load8(at(live ? hn : 0, 8 * (s >> 1) + 2 * kg + (s & 1)), x);
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
-      float a = live ? x[slot_nib(2 * p)] : 0.0f;
-      float c = live ? x[slot_nib(2 * p + 1)] : 0.0f;
+      float a = live ? x[slot_nib_of<D>(2 * p)] : 0.0f;
+      float c = live ? x[slot_nib_of<D>(2 * p + 1)] : 0.0f;
       if constexpr (std::is_same<TQ, float>::value) {
         ql.q[s][2 * p] = (p & 1) ? a * 0.0625f : a;
         ql.q[s][2 * p + 1] = (p & 1) ? c * 0.0625f : c;
       } else {
-        if constexpr (std::is_same<TQ, bf16>::value) {
+        if constexpr (std::is_same<TQ, bf16>::value && D == 128) {
           if (p & 1) {  // exact: the widened input times a power of two
             a *= 0.0625f;
             c *= 0.0625f;
@@ -320,10 +336,12 @@ __device__ __forceinline__ QLane<TQ, D> load_q(const TQ* __restrict__ query, int
 // Folded (GQA groups of at most 8 heads): column n < 8 carries head n's hi
 // part and column n + 8 its lo part, so one MFMA per k-step gives both, and
 // a rotate-by-8 add sums them.
+// Head size 256: Q' times a power of two, no offset, and qs the factor of the
+// scores the MFMAs leave (qscale, the power of two and the codes' unit).
 template <int D = 128>
 struct QGroup {
   h8 bq[D / 32], bl[D / 32];
-  float kb;
+  float kb, qs;
 };
 
 // x - sel * (fp16 half of `pair`), exact in fp32: sel is 1 or 0.
@@ -352,44 +370,39 @@ __device__ __forceinline__ float add_ror8(float x) {
   return x + __int_as_float(y);
 }
 
-template <typename TQ, int NVG, bool KSV, bool FOLD, int D = 128>
+template <typename TQ, int NVG, bool KSV, bool FOLD>
 __device__ __forceinline__ void prepare_group(const uint32_t* W, int n, int kg,
-                                              const QLane<TQ, D>& ql, float qscale,
-                                              QGroup<D>& qg) {
+                                              const QLane<TQ>& ql, float qscale, QGroup<>& qg) {
 #pragma clang fp contract(fast)
-  using T = Tile<NVG, KSV, D>;
-  constexpr int KS = D / 32;
+  using T = Tile<NVG, KSV>;
   const float* ksf = reinterpret_cast<const float*>(W + T::KS);
   const float* kmf = reinterpret_cast<const float*>(W + T::KM);
+  // the lane's 32 scales and minima (dims 64 P + 16 kg + 8 e + 0..7), all
+  // read before any is used
+  f4 sc[4][2], mn[4][2];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const int base = 64 * (s >> 1) + 16 * kg + 8 * (s & 1);
+    sc[s][0] = *reinterpret_cast<const f4*>(ksf + base);
+    sc[s][1] = *reinterpret_cast<const f4*>(ksf + base + 4);
+    mn[s][0] = *reinterpret_cast<const f4*>(kmf + base);
+    mn[s][1] = *reinterpret_cast<const f4*>(kmf + base + 4);
+  }
   // folded: lo lanes (n >= 8) take x - hi, hi lanes x - 0
   const float nsel = (FOLD && n >= 8) ? -1.0f : 0.0f;
   const h2 one2 = h2{1.0f16, 1.0f16};
   // one partial sum per k-step: four short chains instead of one long one
-  float kb_u[KS], kb_p[KS], off[KS];
-  // 128 dims at a time: the lane's 32 scales and minima (dims 64 P + 16 kg +
-  // 8 e + 0..7), all read before any is used
-  f4 sc[4][2], mn[4][2];
+  float kb_u[4], kb_p[4], off[4];
 #pragma unroll
-  for (int s = 0; s < KS; ++s) {
-    if (s % 4 == 0) {
-      if (s > 0) __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int base = 64 * ((s + i) >> 1) + 16 * kg + 8 * (i & 1);
-        sc[i][0] = *reinterpret_cast<const f4*>(ksf + base);
-        sc[i][1] = *reinterpret_cast<const f4*>(ksf + base + 4);
-        mn[i][0] = *reinterpret_cast<const f4*>(kmf + base);
-        mn[i][1] = *reinterpret_cast<const f4*>(kmf + base + 4);
-      }
-    }
+  for (int s = 0; s < 4; ++s) {
     kb_u[s] = kb_p[s] = off[s] = 0.0f;
     uint32_t ph[4], pl[4];
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
       const int d0 = slot_nib(2 * p), d1 = slot_nib(2 * p + 1);
       const f2 q = ql.get(s, p);
-      const float s0 = sc[s % 4][d0 >> 2][d0 & 3], s1 = sc[s % 4][d1 >> 2][d1 & 3];
-      const float m0 = mn[s % 4][d0 >> 2][d0 & 3], m1 = mn[s % 4][d1 >> 2][d1 & 3];
+      const float s0 = sc[s][d0 >> 2][d0 & 3], s1 = sc[s][d1 >> 2][d1 & 3];
+      const float m0 = mn[s][d0 >> 2][d0 & 3], m1 = mn[s][d1 >> 2][d1 & 3];
       const float x0 = q[0] * s0;
       const float x1 = q[1] * s1;
       if (p & 1)
@@ -413,17 +426,66 @@ __device__ __forceinline__ void prepare_group(const uint32_t* W, int n, int kg,
     if (!FOLD) qg.bl[s] = as_h8(pl[0], pl[1], pl[2], pl[3]);
   }
   // primed q are q / 16: their minima term is 16 * kb_p
-#pragma unroll
-  for (int s = 4; s < KS; ++s) {
-    kb_u[s & 3] += kb_u[s];
-    kb_p[s & 3] += kb_p[s];
-    off[s & 3] += off[s];
-  }
   const float kb = sum_kg((kb_u[0] + kb_u[1]) + (kb_u[2] + kb_u[3]) +
                           16.0f * ((kb_p[0] + kb_p[1]) + (kb_p[2] + kb_p[3])));
   float offs = sum_kg((off[0] + off[1]) + (off[2] + off[3]));
   if (FOLD) offs = add_ror8(offs);  // hi column + lo column of the head
   qg.kb = (kb - 1024.0f * offs) * qscale;
+}
+
+// The same at head size 256.
+template <typename TQ, int NVG, bool KSV, bool FOLD>
+__device__ __forceinline__ void prepare_group(const uint32_t* W, int n, int kg,
+                                              const QLane<TQ, 256>& ql, float qscale,
+                                              QGroup<256>& qg) {
+#pragma clang fp contract(fast)
+  using T = Tile<NVG, KSV, 256>;
+  const float* ksf = reinterpret_cast<const float*>(W + T::KS) + 16 * kg;
+  const float* kmf = reinterpret_cast<const float*>(W + T::KM) + 16 * kg;
+  float x[8][8];  // q * scale in slot order
+  float kbs[4] = {0.0f, 0.0f, 0.0f, 0.0f}, amax = 0.0f;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    const int base = 64 * (s >> 1) + 8 * (s & 1);
+    const f4 sc[2] = {*reinterpret_cast<const f4*>(ksf + base),
+                      *reinterpret_cast<const f4*>(ksf + base + 4)};
+    const f4 mn[2] = {*reinterpret_cast<const f4*>(kmf + base),
+                      *reinterpret_cast<const f4*>(kmf + base + 4)};
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int d0 = slot_nib_of<256>(2 * p), d1 = slot_nib_of<256>(2 * p + 1);
+      const f2 q = ql.get(s, p);
+      x[s][2 * p] = q[0] * sc[d0 >> 2][d0 & 3];
+      x[s][2 * p + 1] = q[1] * sc[d1 >> 2][d1 & 3];
+      kbs[s & 3] += q[0] * mn[d0 >> 2][d0 & 3] + q[1] * mn[d1 >> 2][d1 & 3];
+      amax = fmaxf(amax, fmaxf(fabsf(x[s][2 * p]), fabsf(x[s][2 * p + 1])));
+    }
+  }
+  amax = max_rows4(amax);  // over the head's lanes
+  // 2^e * amax in [2^14, 2^15); an amax under 2^-87 stays below
+  int e = 141 - static_cast<int>(__float_as_uint(amax) >> 23);
+  e = e < -113 ? -113 : (e > 100 ? 100 : e);
+  const float up = __uint_as_float(static_cast<uint32_t>(127 + e) << 23);
+  const float nsel = (FOLD && n >= 8) ? -1.0f : 0.0f;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    uint32_t ph[4], pl[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const float x0 = x[s][2 * p] * up, x1 = x[s][2 * p + 1] * up;
+      const uint32_t hi = pack_h2(x0, x1);
+      if (FOLD) {
+        ph[p] = pack_h2(sub_half_sel<0>(x0, hi, nsel), sub_half_sel<1>(x1, hi, nsel));
+      } else {
+        ph[p] = hi;
+        pl[p] = pack_h2(sub_half_sel<0>(x0, hi, -1.0f), sub_half_sel<1>(x1, hi, -1.0f));
+      }
+    }
+    qg.bq[s] = as_h8(ph[0], ph[1], ph[2], ph[3]);
+    if (!FOLD) qg.bl[s] = as_h8(pl[0], pl[1], pl[2], pl[3]);
+  }
+  qg.kb = sum_kg((kbs[0] + kbs[1]) + (kbs[2] + kbs[3])) * qscale;
+  qg.qs = qscale * (kCodeUnit * __uint_as_float(static_cast<uint32_t>(127 - e) << 23));
 }
 
 // Running state of one wave: softmax max / sum (log2 domain), the PV
@@ -499,7 +561,8 @@ __device__ __forceinline__ void compute_tile(const uint32_t* W, uint32_t buf_off
     for (int e = 0; e < 2; ++e)
 #pragma unroll
       for (int jm = 0; jm < 4; ++jm) {
-        const h8 a = key_codes(static_cast<uint32_t>(rk[P][jm][e]), cst);
+        const uint32_t w = static_cast<uint32_t>(rk[P][jm][e]);
+        const h8 a = kWide ? codes_f16(w) : key_codes(w, cst);
         sacc[jm] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qg.bq[2 * P + e], sacc[jm], 0, 0, 0);
         if (!FOLD)
           sacc[jm] =
@@ -518,13 +581,13 @@ __device__ __forceinline__ void compute_tile(const uint32_t* W, uint32_t buf_off
       for (int r = 0; r < 4; ++r) sacc[jm][r] = add_ror8(sacc[jm][r]);
   }
   // lane (kg, n) holds head n (n & 7 folded) at tokens 16 jm + 4 kg + r
-  const float kb = qg.kb;
+  const float kb = qg.kb, qs = kWide ? qg.qs : qscale;
   float tm[4];
 #pragma unroll
   for (int jm = 0; jm < 4; ++jm) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      float sv = sacc[jm][r] * qscale + kb;
+      float sv = sacc[jm][r] * qs + kb;
       if (!FULL) {
         const int pos = p0 + 16 * jm + 4 * kg + r;
         sv = pos >= pb && pos < pe ? sv : -INFINITY;
