@@ -880,7 +880,7 @@ def test_split_decode_head_256_keeps_its_precision(gpu_device, g, bs, rep, size)
     assert err.max() < (3e-3 if size < 1 else 2.0 ** -11), err.tolist()
 
 
-def _wide_error(dev, dtype, g, bs, rep, lens, make, q, scale):
+def _wide_error(dev, dtype, g, bs, rep, lens, make, q, scale, split=None):
     """2-norm error per (request, head) of a decode at head size 256, one kv head,
     relative to 64-bit attention over the dequantized history."""
     from vllm_ascend_quantized_kv_cache.ops.kivi_decode import (
@@ -891,7 +891,7 @@ def _wide_error(dev, dtype, g, bs, rep, lens, make, q, scale):
 
     d = 256
     cpu, table, ring_k, ring_v, seqs, wk, wv, _, _ = _ring_case(
-        dev, d, 1, g, bs, 128, lens, seed=47, ring_dtype=dtype, make=make)
+        dev, d, 1, g, bs, 128, lens, seed=47, ring_dtype=dtype, make=make, split=split)
     dk, dv = ref.dequant_gather(*cpu, table, torch.tensor(lens), torch.float32, g)
     dk, dv = ref.overlay_residual(dk, lens, wk), ref.overlay_residual(dv, lens, wv)
     want, at = [], 0
@@ -976,6 +976,72 @@ def test_split_decode_head_256_keys_of_any_size(gpu_device, g, bs, rep, dtype, q
     err = _wide_error(gpu_device, dtype, g, bs, rep, lens, make, q.to(dtype),
                       2 / 16 / q_size / k_size)
     assert err.max() < WIDE_BOUND[dtype], err.tolist()
+
+
+@pytest.mark.parametrize("rep", [8, 12])
+@pytest.mark.parametrize("dtype,size,offset", [
+    (torch.bfloat16, 1.0, 3008.0),  # channels far from zero: a key's detail is its last bits
+    (torch.bfloat16, 1e-4, 0.0),
+    (torch.float16, 1.0, 256.0),
+    (torch.float16, 1e-6, 0.0),     # int4 keys below the fp16 subnormals
+    (torch.float16, 1e6, 0.0),      # ... and past its range
+])
+def test_tail_head_256_int4_keys(gpu_device, rep, dtype, size, offset):
+    """Tails whose keys are int4 and whose values are still in the ring."""
+    lens = [129, 255, 256]
+
+    def make(n, h_, d_, seed):
+        gen = torch.Generator().manual_seed(seed)
+        key = size * torch.randn(n, h_, d_, generator=gen)
+        key[(n - 1) // 128 * 128:] = 0.0  # the ring's: nothing but the offset
+        return key + offset, torch.randn(n, h_, d_, generator=gen).to(dtype)
+
+    q = torch.randn(len(lens), rep, 256, generator=torch.Generator().manual_seed(6))
+    q = (q - q.mean(-1, keepdim=True)).to(dtype)
+    err = _wide_error(gpu_device, dtype, 128, 128, rep, lens, make, q, 1 / 16 / size)
+    assert err.max() < WIDE_BOUND[dtype], err.tolist()
+
+
+@pytest.mark.parametrize("rep", [8, 12])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_tail_head_256_probabilities(gpu_device, rep, dtype):
+    """Two ring positions whose probabilities differ in their last bits only and whose
+    values cancel but for that, beside one of the largest probability and no
+    value: a 16-bit probability would be some hundredth of the result off."""
+    step = 2.0 ** -6 if dtype == torch.bfloat16 else 2.0 ** -2
+
+    def make(n, h_, d_, seed):
+        gen = torch.Generator().manual_seed(seed)
+        key, value = torch.zeros(n, h_, d_), torch.randn(n, h_, d_, generator=gen).to(dtype)
+        key[1:, :, 0] = -1.0
+        key[2, :, 1] = step
+        value[0], value[2] = 0.0, -value[1]
+        return key.to(dtype), value
+
+    q = torch.zeros(3, rep, 256)
+    q[:, :, 0], q[:, :, 1] = 4.0 + torch.arange(rep) / 4, 0.25
+    err = _wide_error(gpu_device, dtype, 128, 128, rep, [3, 3, 3], make, q.to(dtype), 1 / 16)
+    assert err.max() < WIDE_BOUND[dtype], err.tolist()
+
+
+@pytest.mark.parametrize("rep", [8, 12])
+@pytest.mark.parametrize("dtype,size", [(torch.bfloat16, 1.0), (torch.float16, 1.0),
+                                        (torch.bfloat16, 1e-5), (torch.float16, 1e-3)])
+def test_tail_head_256_int4_values(gpu_device, rep, dtype, size):
+    """Tails whose values are int4 and whose keys are still in the ring, as a
+    caller's own window rule may leave them."""
+    def make(n, h_, d_, seed):
+        gen = torch.Generator().manual_seed(seed)
+        value = size * torch.randn(n, h_, d_, generator=gen)
+        value[n // 2:] = value[n // 2:].to(dtype)
+        return torch.randn(n, h_, d_, generator=gen).to(dtype), value
+
+    lens = [100, 61, 14]
+    q = torch.randn(len(lens), rep, 256, generator=torch.Generator().manual_seed(7)).to(dtype)
+    err = _wide_error(gpu_device, dtype, 64, 128, rep, lens, make, q, 1 / 16,
+                      split=lambda n: (0, n // 2))
+    # fp16 outputs of 1e-4 at the smallest size: 2^-25 / sqrt(3) of each is subnormal
+    assert err.max() < WIDE_BOUND[dtype] + (3e-4 if size == 1e-3 else 0), err.tolist()
 
 
 @pytest.mark.parametrize("d", [128, 256])

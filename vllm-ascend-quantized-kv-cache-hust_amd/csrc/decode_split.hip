@@ -31,8 +31,8 @@
 // through LDS (the second tile leaves before the first is there), the key
 // group's operands kept over its two tiles, and MFMA results in ordinary
 // registers (a build flag): 69.1 -> 62.0 us on the 64 requests above, 58.4 ->
-// 52.6 on 20 of 0.5K-10K with 2 kv heads of 256, 40.5 -> 38.7 on the 40.  (The
-// parts of P' that compute_tile takes at 256 dims then added 4 us.)
+// 52.6 on 20 of 0.5K-10K with 2 kv heads of 256, 40.5 -> 38.7 on the 40.  (What
+// keeps fp32's bits at 256 dims then added 6 us: P' 4, the tails 2.)
 #include <algorithm>
 
 #include "decode_tail.h"
@@ -80,7 +80,8 @@ constexpr int kSplitWaves = 4;
 template <int D, int NVG, bool KSV>
 constexpr int wave_bytes() {
   constexpr int two = 2 * tr::Tile<NVG, KSV, D>::BYTES;
-  return two > tail::kLdsBytes ? two : tail::kLdsBytes;
+  constexpr int tail = D == 256 ? tail::kLdsBytesWide : tail::kLdsBytes;
+  return two > tail ? two : tail;
 }
 
 template <typename TQ, int D, int NVG, bool KSV, bool FOLD>

@@ -148,6 +148,7 @@ constexpr int kTT = 32;           // positions per sub-tile
 constexpr int kKP = kD + 8;       // K row pitch (elements): rows stay 16-byte aligned
 constexpr int kKW = kTT / 8 + 1;  // key words of one dim covering a sub-tile (8-aligned start)
 constexpr int kLdsBytes = 2 * kTT * kKP * 2;
+constexpr int kLdsBytesWide = 3 * kTT * kKP * 2;  // head size 256
 static_assert(kTT * kD * 2 <= kLdsBytes, "the V rows fit the key region they reuse");
 
 typedef short v4s __attribute__((ext_vector_type(4)));
@@ -188,6 +189,13 @@ struct Rows8 {
 // NH: the head size in 128-dim halves.  The halves of a sub-tile are staged one
 // after the other over the same LDS (scores add up over them, then each half's
 // values meet the probabilities), "the next sub-tile" above being the next half.
+// A head of two halves keeps what the fp32 kernel its calls had before kept:
+//   bf16   int4 keys and p as three parts (24 bits) instead of two;
+//   fp16   int4 keys times the power of two that brings the sub-tile's to
+//          [2^14, 2^15), and p times 2^14, so that their two parts (22 bits)
+//          neither overflow nor meet the subnormals;
+//   int4 values inside a tail meet p in fp32, outside the MFMAs (rare: a plan of
+//          the caller's own).
 template <typename T, int NH = 1>
 __device__ __forceinline__ PartialT<8 * NH> tail_item(char* __restrict__ lds_raw, const T* __restrict__ query,
                                           int hq, int kvh, float qscale,
@@ -205,8 +213,12 @@ __device__ __forceinline__ PartialT<8 * NH> tail_item(char* __restrict__ lds_raw
                                           int half, int nhalf) {
   constexpr int D = kD;
   constexpr int DT = NH * kD;  // the head size
+  constexpr bool kWide = NH == 2, kScaled = kWide && std::is_same<T, f16>::value;
+  constexpr int kParts = kWide && !kScaled ? 3 : 2;  // of an int4 key, and of p
+  constexpr float kLift = kScaled ? 16384.0f : 1.0f;  // p's, and o's while it runs
   uint16_t* sk = reinterpret_cast<uint16_t*>(lds_raw);  // [kTT][kKP] int4 key hi parts
-  uint16_t* skl = sk + kTT * kKP;                        // [kTT][kKP] int4 key lo parts
+  constexpr int kPlane = kTT * kKP;                      // ... and their lower parts behind
+  float* sp = reinterpret_cast<float*>(lds_raw + kTT * D * 2);  // [kTT][16] p (int4 values)
   char* sv = lds_raw;                                    // [kTT][D] value rows, after the scores
   // opaque to the optimizer: the lane-dependent set-up below is recomputed per
   // item instead of being hoisted out of the caller's item loop, where it
@@ -377,7 +389,19 @@ __device__ __forceinline__ PartialT<8 * NH> tail_item(char* __restrict__ lds_raw
     // sub-tile's reads are done before these writes
     // ---- key rows: int4 rows [0, mk) as hi and lo parts, ring rows [mk, nt)
     // as they are (their lo parts zero, read only when the sub-tile has int4 rows)
+    float up = 1.0f, down = 1.0f;
     if (mk > 0) {
+      if constexpr (kScaled) {
+        float big = 0.0f;  // of the sub-tile's keys
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          big = fmaxf(big, fabsf(kw.mn[i / 2][i % 2]) + 15.0f * fabsf(kw.sc[i / 2][i % 2]));
+        big = max_wave64(big);
+        int e = 141 - static_cast<int>(__float_as_uint(big) >> 23);
+        e = e < -113 ? -113 : (e > 100 ? 100 : e);
+        up = __uint_as_float(static_cast<uint32_t>(127 + e) << 23);
+        down = __uint_as_float(static_cast<uint32_t>(127 - e) << 23);
+      }
       // words realigned to the sub-tile (word k: positions p0 + 8k .. + 7), so
       // that row t = 8k + j is nibble j of word k and no row needs a test:
       // rows past mk are overwritten by the ring rows below or masked
@@ -396,10 +420,14 @@ __device__ __forceinline__ PartialT<8 * NH> tail_item(char* __restrict__ lds_raw
                                         gb ? kw.mn[0][1] : kw.mn[0][0]);
           const float x1 = kivi_dequant((a1 >> (4 * j)) & 0xfu, gb ? kw.sc[1][1] : kw.sc[1][0],
                                         gb ? kw.mn[1][1] : kw.mn[1][0]);
-          const uint32_t hi = pack2<T>(x0, x1);
-          *reinterpret_cast<uint32_t*>(sk + t * kKP + c0) = hi;
-          *reinterpret_cast<uint32_t*>(skl + t * kKP + c0) =
-              pack2<T>(x0 - half_f32<T>(hi, 0), x1 - half_f32<T>(hi, 1));
+          float y0 = kScaled ? x0 * up : x0, y1 = kScaled ? x1 * up : x1;
+#pragma unroll
+          for (int k3 = 0; k3 < kParts; ++k3) {
+            const uint32_t part = pack2<T>(y0, y1);
+            *reinterpret_cast<uint32_t*>(sk + k3 * kPlane + t * kKP + c0) = part;
+            y0 -= half_f32<T>(part, 0);
+            y1 -= half_f32<T>(part, 1);
+          }
         }
       }
     }
@@ -414,25 +442,38 @@ __device__ __forceinline__ PartialT<8 * NH> tail_item(char* __restrict__ lds_raw
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const int o = (16 * (i >> 2) + n) * kKP + 32 * (i & 3) + 8 * kg;
-        if (i < 4 ? ring0 : ring1) *reinterpret_cast<w4*>(skl + o) = w4{0, 0, 0, 0};
+#pragma unroll
+        for (int k3 = 1; k3 < kParts; ++k3)
+          if (i < 4 ? ring0 : ring1) *reinterpret_cast<w4*>(sk + k3 * kPlane + o) = w4{0, 0, 0, 0};
       }
     }
     // ---- scores: S^T[token][head] for kTT/16 x 16 tokens ------------------------
-    // the key lo parts exist only for int4 keys: one uniform branch for the block
+    // the lower key parts exist only for int4 keys: one uniform branch for the block
     auto scores = [&](auto with_lo) {
 #pragma unroll
       for (int jm = 0; jm < kTT / 16; ++jm) {
-        if (hf == 0) sacc[jm] = f4{0.f, 0.f, 0.f, 0.f};
+        f4 acc = kScaled || hf == 0 ? f4{0.f, 0.f, 0.f, 0.f} : sacc[jm];
 #pragma unroll
         for (int s4 = 0; s4 < 4; ++s4) {
           const int o = (16 * jm + n) * kKP + 32 * s4 + 8 * kg;
           const u8v a = *reinterpret_cast<const u8v*>(sk + o);
-          sacc[jm] = mfma16(a, qb[4 * hf + s4], sacc[jm], T{});
+          acc = mfma16(a, qb[4 * hf + s4], acc, T{});
           if constexpr (decltype(with_lo)::value) {
-            const u8v al = *reinterpret_cast<const u8v*>(skl + o);
-            sacc[jm] = mfma16(al, qb[4 * hf + s4], sacc[jm], T{});
+#pragma unroll
+            for (int k3 = 1; k3 < kParts; ++k3) {
+              const u8v al = *reinterpret_cast<const u8v*>(sk + k3 * kPlane + o);
+              acc = mfma16(al, qb[4 * hf + s4], acc, T{});
+            }
           }
         }
+        if constexpr (kScaled) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {  // ring rows came unscaled
+            if (decltype(with_lo)::value && 16 * jm + 4 * kg + r < mk) acc[r] *= down;
+            acc[r] = hf == 0 ? acc[r] : sacc[jm][r] + acc[r];
+          }
+        }
+        sacc[jm] = acc;
       }
     };
     if (mk > 0)
@@ -484,10 +525,33 @@ __device__ __forceinline__ PartialT<8 * NH> tail_item(char* __restrict__ lds_raw
     for (int k = 0; k < 8; ++k) {
       const int pi = kg + 4 * k;
       // positions past the item: p = 0 there, and zero V keeps 0 * V exact
-      const w4 x = pi < nt ? vr.r[k] : w4{0, 0, 0, 0};
+      const w4 x = pi < nt && (!kWide || pi >= mv) ? vr.r[k] : w4{0, 0, 0, 0};
       *reinterpret_cast<w4*>(sv + pi * (2 * D) + 16 * (n ^ (2 * (pi & 3)))) = x;
     }
-    if (mv > 0) {  // uniform: int4 values (rare), loaded and dequantized over their rows
+    if (kWide && mv > 0) {  // uniform: int4 values (rare)
+      if (hf == 0) {
+#pragma unroll
+        for (int jm = 0; jm < kTT / 16; ++jm)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) sp[(16 * jm + 4 * kg + r) * 16 + n] = sacc[jm][r];
+      }
+#pragma unroll 1
+      for (int t = 0; t < mv; ++t) {
+        const int64_t vrow =
+            ((page_uniform(pg_cur, p0, p0 + t) << bsh) + ((p0 + t) & (bs - 1))) * kvh + h;
+        const f4 pr = *reinterpret_cast<const f4*>(sp + 16 * t + 4 * kg) * kLift;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          const int c = hf * D + 16 * q + n;
+          const float x = kivi_dequant((vq[vrow * (DT / 8) + (c >> 3)] >> (4 * (c & 7))) & 0xfu,
+                                       vs[vrow * (DT >> gsh) + (c >> gsh)],
+                                       vm[vrow * (DT >> gsh) + (c >> gsh)]);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o_acc[8 * hf + q][r] += pr[r] * x;
+        }
+      }
+    }
+    if (!kWide && mv > 0) {  // uniform: likewise, dequantized over their rows
 #pragma unroll 1
       for (int k = 0; k < 8; ++k) {
         const int pi = kg + 4 * k;
@@ -513,13 +577,15 @@ __device__ __forceinline__ PartialT<8 * NH> tail_item(char* __restrict__ lds_raw
     // ---- O += P V: slot i of lane group kg is token 32*st + 16*(i/4) + 4*kg + i%4
 #pragma unroll
     for (int st = 0; st < kTT / 32; ++st) {
-      u8v ahi, alo;
+      u8v pa[kParts];
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const float p = sacc[2 * st + i / 4][i % 4];
-        const float hi = to_f32(from_f32<T>(p));
-        ahi[i] = bits_of<T>(p);
-        alo[i] = bits_of<T>(p - hi);
+        float p = sacc[2 * st + i / 4][i % 4] * kLift;
+#pragma unroll
+        for (int k3 = 0; k3 < kParts; ++k3) {
+          pa[k3][i] = bits_of<T>(p);
+          p -= to_f32(from_f32<T>(p));
+        }
       }
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
@@ -535,8 +601,9 @@ __device__ __forceinline__ PartialT<8 * NH> tail_item(char* __restrict__ lds_raw
                         static_cast<uint16_t>(part[0][2]), static_cast<uint16_t>(part[0][3]),
                         static_cast<uint16_t>(part[1][0]), static_cast<uint16_t>(part[1][1]),
                         static_cast<uint16_t>(part[1][2]), static_cast<uint16_t>(part[1][3])};
-        o_acc[8 * hf + q] = mfma16(ahi, bv, o_acc[8 * hf + q], T{});
-        o_acc[8 * hf + q] = mfma16(alo, bv, o_acc[8 * hf + q], T{});
+#pragma unroll
+        for (int k3 = 0; k3 < kParts; ++k3)
+          o_acc[8 * hf + q] = mfma16(pa[k3], bv, o_acc[8 * hf + q], T{});
       }
     }
     // the next values (this sub-tile's next half, or the next sub-tile), then the
@@ -552,7 +619,7 @@ __device__ __forceinline__ PartialT<8 * NH> tail_item(char* __restrict__ lds_raw
 
   PartialT<8 * NH> res;
 #pragma unroll
-  for (int q = 0; q < 8 * NH; ++q) res.o[q] = o_acc[q];
+  for (int q = 0; q < 8 * NH; ++q) res.o[q] = o_acc[q] * (1.0f / kLift);
   res.m = m_run;
   res.l = l_run;
   return res;
