@@ -241,3 +241,33 @@ def test_int8_decode_head_256_keeps_its_precision(gpu_device, rep):
                                 lens, d ** -0.5)
     err = (got.double().cpu() - want).norm(dim=-1) / want.norm(dim=-1)
     assert err.max() < 2.0 ** -16, err.tolist()
+
+
+@pytest.mark.parametrize("kvh,rep", [(1, 8), (2, 16)])
+@pytest.mark.parametrize("bits", [10, 20, 26, 34])
+def test_decode_head_256_keeps_small_probabilities(gpu_device, kvh, rep, bits):
+    """Head size 256: the position of the largest probability has no value, so the
+    result is all the others', each 2^-bits of it."""
+    from vllm_ascend_quantized_kv_cache.ops.int8_ops import int8_decode_attention
+
+    dev, d, bs, n = gpu_device, 256, 32, 190
+    gen = torch.Generator().manual_seed(bits)
+    key = torch.zeros((7, bs, kvh, d), dtype=torch.int8)
+    value = torch.randint(-127, 128, key.shape, generator=gen, dtype=torch.int8)
+    table = torch.randperm(7, generator=gen, dtype=torch.int32)[None]
+    at = 100  # of the one that counts
+    key[table[0, at // bs], at % bs, :, 0] = 127
+    value[table[0, at // bs], at % bs] = 0
+    q = torch.zeros((1, kvh * rep, d))
+    q[..., 0] = 1.0
+    aq = torch.ones((kvh, d), dtype=torch.bfloat16)
+    scale = bits * 0.6931471805599453 / 127
+    got = int8_decode_attention(q.to(torch.bfloat16).to(dev), key.to(dev), value.to(dev),
+                                aq.to(dev), aq.to(dev), table.to(dev), [n], scale)
+    rows = value[table[0].long()].flatten(0, 1)[:n].double()
+    want = rows.sum(0) * 2.0 ** -bits / (1 + (n - 1) * 2.0 ** -bits)
+    want = want.repeat_interleave(rep, 0)[None]
+    # the bf16 output's half unit and the fp32 score's last bit; where the codes cancel,
+    # 190 products of up to 127 * 2^-bits at 2^-23 each
+    torch.testing.assert_close(got.double().cpu(), want, rtol=2.0 ** -8 + 2.0 ** -18,
+                               atol=190 * 127 * 2.0 ** (-bits - 23))

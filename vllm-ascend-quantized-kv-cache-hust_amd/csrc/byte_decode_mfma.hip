@@ -235,6 +235,11 @@ __device__ __forceinline__ void read_tile_lds(TileRegs<D, FP8>& t, const char* b
   }
 }
 
+// INT8 at 256 dims: p's (and o's) lift on the way through fp16, so that the two
+// parts of a p down to 2^-28 keep their bits and one is lost only below 2^-39.
+template <int D>
+constexpr float kLift = D == 256 ? 16384.0f : 1.0f;
+
 template <int D>
 struct SoftmaxState {
   float m;    // running max of head n (log2 domain), same in the 4 lane groups
@@ -387,13 +392,17 @@ __device__ __forceinline__ void compute_tile(const TileRegs<D, FP8>& t, int p, i
     }
   } else {
     // at 256 dims p goes as fp16 hi + lo parts, at 128 as one fp16
-    constexpr bool kSplitP = D == 256;
+    constexpr bool kSplitP = kLift<D> != 1.0f;
     auto halves = [](const f4 (&x)[2]) {
       return as_h8(h2_bits(static_cast<_Float16>(x[0][0]), static_cast<_Float16>(x[0][1])),
                    h2_bits(static_cast<_Float16>(x[0][2]), static_cast<_Float16>(x[0][3])),
                    h2_bits(static_cast<_Float16>(x[1][0]), static_cast<_Float16>(x[1][1])),
                    h2_bits(static_cast<_Float16>(x[1][2]), static_cast<_Float16>(x[1][3])));
     };
+    if constexpr (kSplitP) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) s[j] *= kLift<D>;
+    }
     const h8 a = halves(s);
     h8 al = a;
     if constexpr (kSplitP) {
@@ -651,7 +660,8 @@ __device__ __forceinline__ void decode_item(
   float va[DPL];
 #pragma unroll
   for (int tt = 0; tt < DPL; ++tt)
-    va[tt] = FP8 ? 1.0f : to_f32(v_aq[static_cast<int64_t>(h) * D + DPL * n + tt]);
+    va[tt] = FP8 ? 1.0f
+                 : to_f32(v_aq[static_cast<int64_t>(h) * D + DPL * n + tt]) * (1.0f / kLift<D>);
   const int64_t head0 = static_cast<int64_t>(wi) * heads;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
