@@ -397,3 +397,38 @@ def test_decode_attends_to_the_rows_the_gather_leaves(gpu_device, d, rows, dtype
                 off = (got[rows * b + j, h].double().cpu() - want).abs() - bound
                 assert off.max() <= 0, (b, j, h, off.max().item())
         at += n
+
+
+@pytest.mark.parametrize("where", ["query", "key code", "value code"])
+def test_decode_of_nans_is_nan(gpu_device, where):
+    """A NaN query row, key or value reaches its heads' outputs and no others, as it
+    does over gathered rows (requests cut into several items, and a whole one)."""
+    d, kvh, rep, bs, lens = 128, 2, 2, 16, [900, 40]
+    gen = torch.Generator().manual_seed(23)
+    nb = sum(-(-n // bs) for n in lens)
+    table = torch.zeros((2, -(-lens[0] // bs)), dtype=torch.int32)
+    table[0] = torch.arange(table.shape[1])
+    table[1, :3] = torch.arange(table.shape[1], nb)
+    _, _, views = _views(gpu_device, nb, bs, kvh, d)
+    x = torch.randn((nb * bs, kvh, d), generator=gen).to(torch.bfloat16).to(gpu_device)
+    fp8_ops.fp8_per_token_head_store(x, x, torch.arange(nb * bs, device=gpu_device), *views)
+    q = torch.randn((2, kvh * rep, d), generator=gen).to(torch.bfloat16)
+    if where == "query":
+        q[:, 2, 7] = float("nan")
+    else:
+        codes = views[0] if where == "key code" else views[2]
+        codes[table[:, 2].long(), 5, 1, 9] = 0x7F  # position 37 of both, kv head 1
+    args = (q.to(gpu_device), *views, table.to(gpu_device), lens)
+    outs = [fp8_ops.fp8_per_token_head_attention(*args, [1, 1], d ** -0.5)]
+    k, v = fp8_ops.fp8_per_token_head_dequant_gather(*args[1:], torch.bfloat16)
+    from vllm_ascend_quantized_kv_cache.ops.attention import prefill_attention
+
+    outs.append(prefill_attention(args[0], k, v, [1, 1], lens, d ** -0.5, True))
+    for out in outs:
+        hit = out.isnan().cpu()
+        if where == "query":
+            assert hit[:, 2].all() and not hit[:, [0, 1, 3]].any()
+        elif where == "key code":
+            assert hit[:, 2:].all() and not hit[:, :2].any()
+        else:
+            assert hit[:, 2:, 9].all() and int(hit.sum()) == 4

@@ -681,7 +681,9 @@ __device__ __forceinline__ void decode_item(
   }
   if (g == 0 && n < cols) {
     const int64_t hh = head0 + col_head(n);
-    ws_ml[2 * hh] = st.m;
+    // E4M3: a NaN score (a NaN query or code) leaves m without it; m = inf then
+    // makes the combine's weights and its result NaN, as the gathered rows give
+    ws_ml[2 * hh] = FP8 && l != l ? INFINITY : st.m;
     ws_ml[2 * hh + 1] = l;
   }
 }
