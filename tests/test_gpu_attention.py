@@ -150,6 +150,33 @@ def test_prefill_attention_keys_in_segments(gpu_device, d, hq, kvh, dtype, causa
     assert not got[20:].any()  # no keys
 
 
+@pytest.mark.parametrize("d", [128, 256])
+@pytest.mark.parametrize("where", ["query", "key", "value"])
+def test_prefill_attention_of_nans_in_segments(gpu_device, d, where):
+    """A NaN among the keys of a segment whose scores are hundreds of powers of two
+    under another's reaches the rows that see it, as it does without segments."""
+    from vllm_ascend_quantized_kv_cache.ops.attention import prefill_attention
+
+    q_lens, kv_lens, hq = [4], [4000], 8
+    g = torch.Generator().manual_seed(d)
+    q = torch.ones(4, hq, d, dtype=torch.bfloat16)
+    k = torch.zeros(4000, 1, d, dtype=torch.bfloat16)
+    k[2000:] = 100.0
+    v = torch.randn(4000, 1, d, generator=g).to(torch.bfloat16)
+    if where == "query":
+        q[1, 5, 3] = float("nan")
+    else:
+        (k if where == "key" else v)[100, 0, 3] = float("nan")
+    got = prefill_attention(q.to(gpu_device), k.to(gpu_device), v.to(gpu_device), q_lens, kv_lens,
+                            d ** -0.5, True).isnan().cpu()
+    if where == "query":
+        assert got[1, 5].all() and int(got.sum()) == d
+    elif where == "key":
+        assert got.all()
+    else:
+        assert got[:, :, 3].all() and int(got.sum()) == 4 * hq
+
+
 def test_prefill_attention_batch_past_the_launch_argument(gpu_device):
     """More requests, and more tiles, than the plan argument carries."""
     from vllm_ascend_quantized_kv_cache.ops.attention import prefill_attention

@@ -777,8 +777,13 @@ prefill_attn_fa_kernel(PlanArg plan_arg, const int32_t* __restrict__ plan, int b
       for (int j = 0; j < DB; ++j)
         *reinterpret_cast<f4*>(seg.o + r * D + 16 * j + 4 * kg) = o[j][g2];
       if (kg == 0) {
-        seg.ml[2 * r] = m_run[g2] == -INFINITY ? -INFINITY : qscale * m_run[g2];
-        seg.ml[2 * r + 1] = l_acc[g2][0];
+        // a NaN score reaches l but not the maximum: m = inf then makes the merge's
+        // weights NaN, where a small m's would drop the segment from the sum
+        const float l = l_acc[g2][0];
+        seg.ml[2 * r] = l != l                    ? INFINITY
+                        : m_run[g2] == -INFINITY ? -INFINITY
+                                                  : qscale * m_run[g2];
+        seg.ml[2 * r + 1] = l;
       }
     }
     return;
@@ -816,7 +821,8 @@ constexpr int kFaTileRows = 128;  // rows (queries x heads of a GQA group) per w
 
 // Merge of the segments of a tile's rows: one wave per row, 8 waves a workgroup,
 // blockIdx.y the tile's group of 8 rows.  A segment without keys for the row
-// (m = -inf) carries weight 0 and its o, possibly unwritten, is selected out.
+// (m = -inf) has its o, possibly unwritten, selected out; one whose weight
+// underflows takes part (a NaN or inf among its values has to show).
 constexpr int kMergeRows = 8;
 template <typename T, int D>
 __global__ void __launch_bounds__(64 * kMergeRows)
@@ -843,6 +849,7 @@ prefill_merge_kernel(PlanArg plan_arg, int batch, int hq, int kvh, FastDiv rep_d
     m = x.x;
     l = x.y;
   }
+  const uint64_t written = __builtin_amdgcn_ballot_w64(m != -INFINITY);
   const float mx = max_wave64(m);
   const float w = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mx);
   const float lsum = sum_wave64(w * l);
@@ -855,7 +862,7 @@ prefill_merge_kernel(PlanArg plan_arg, int batch, int hq, int kvh, FastDiv rep_d
     const float ws = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), s));
     const float* o = seg.o + (first + static_cast<int64_t>(s) * kFaTileRows) * D + PL * lane;
 #pragma unroll
-    for (int i = 0; i < PL; ++i) acc[i] += ws != 0.0f ? ws * o[i] : 0.0f;
+    for (int i = 0; i < PL; ++i) acc[i] += (written >> s) & 1 ? ws * o[i] : 0.0f;
   }
   const float inv = lsum > 0.0f ? 1.0f / lsum : 0.0f;
   const int i = static_cast<int>(rep_div.div(static_cast<uint32_t>(row)));
