@@ -444,7 +444,8 @@ int kvq_fp8_pth_gather_lens(const uint8_t* k_data, const float* k_scale, const u
  * block_size % 16 == 0, at most 16 query heads per kv head; other geometries
  * return KVQ_ERR_GEOMETRY.  Block ids as for kvq_fp8_pth_gather.  The lengths
  * are read during the call and travel with the launches; `workspace` holds
- * kvq_fp8_pth_decode_workspace_bytes for the same lengths.
+ * kvq_fp8_pth_decode_workspace_bytes for the same lengths, rows and device (a
+ * smaller workspace_bytes returns KVQ_ERR_INVALID before anything is launched).
  * The read path the reference lacks for this scheme, as kvq_fp8_pth_gather
  * followed by kvq_prefill_attn would compute it, without the dense rows. */
 int64_t kvq_fp8_pth_decode_workspace_bytes(const int64_t* seq_lens, int64_t batch, int64_t rows,
@@ -455,7 +456,7 @@ int kvq_fp8_pth_decode_attn(const void* query, int dtype, int64_t batch, int64_t
                             const float* k_scale, const uint8_t* v_data, const float* v_scale,
                             int64_t num_blocks, int block_size, const void* block_table,
                             int block_index_type, int64_t max_blocks, const int64_t* seq_lens,
-                            void* workspace, void* out, void* stream);
+                            void* workspace, int64_t workspace_bytes, void* out, void* stream);
 
 /* ---- self-test ---------------------------------------------------------- */
 

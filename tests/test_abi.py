@@ -79,6 +79,24 @@ def test_workspace_sizes_are_host_computable():
     assert lib.kvq_int8_decode_workspace_bytes(3, 32, 128) == 3 * 32 * 130 * 4
 
 
+def test_e4m3_decode_refuses_lengths_past_its_range():
+    """Refused on the host, as the sizing call refuses them, however wide the table."""
+    import numpy as np
+
+    from vllm_ascend_quantized_kv_cache.ops import _native
+
+    if not _native.library_path().exists():
+        pytest.skip("libkvq_hip.so not built")
+    lib, some = _native.lib(), 16  # any pointer: refused before it is read
+    for length in (-1, 0x7FFF0001, 1 << 32):
+        lens = np.array([length], dtype=np.int64)
+        assert lib.kvq_fp8_pth_decode_workspace_bytes(lens.ctypes.data, 1, 1, 4, 2, 128,
+                                                      16) == _native.KVQ_ERR_INVALID
+        assert lib.kvq_fp8_pth_decode_attn(
+            some, 2, 1, 1, 1, 4, 2, 128, 0.1, some, some, some, some, 4, 16, some, 0, 1 << 40,
+            lens.ctypes.data, some, 1 << 40, some, 0) == _native.KVQ_ERR_INVALID
+
+
 def test_ops_refuse_cpu_tensors_loudly():
     """The product path has no CPU fallback: host tensors raise before any launch."""
     import torch

@@ -432,3 +432,33 @@ def test_decode_of_nans_is_nan(gpu_device, where):
             assert hit[:, 2:].all() and not hit[:, :2].any()
         else:
             assert hit[:, 2:, 9].all() and int(hit.sum()) == 4
+
+
+@pytest.mark.parametrize("lens", [[9000, 3], [100] * 800])
+def test_decode_refuses_a_workspace_too_small(gpu_device, lens):
+    """A workspace a byte under any launch's partials is refused before a launch."""
+    from vllm_ascend_quantized_kv_cache.ops import _native
+
+    d, kvh, hq, bs = 128, 2, 4, 16
+    lib, batch = _native.lib(), len(lens)
+    lens_np = np.array(lens, dtype=np.int64)
+    need = lib.kvq_fp8_pth_decode_workspace_bytes(lens_np.ctypes.data, batch, 1, hq, kvh, d, bs)
+    _, _, views = _views(gpu_device, 1, bs, kvh, d)
+    q = torch.zeros((batch, hq, d), dtype=torch.bfloat16, device=gpu_device)
+    out = torch.full_like(q, 7.0)
+    table = torch.zeros((batch, -(-max(lens) // bs)), dtype=torch.int32, device=gpu_device)
+    ws = torch.empty(need, dtype=torch.uint8, device=gpu_device)
+
+    def call(nbytes):
+        return lib.kvq_fp8_pth_decode_attn(
+            q.data_ptr(), _native.dtype_code(q.dtype), batch, 1, 1, hq, kvh, d, 0.1,
+            *(v.data_ptr() for v in views), 1, bs, table.data_ptr(), _native.index_code(table.dtype),
+            table.shape[1], lens_np.ctypes.data, ws.data_ptr(), nbytes, out.data_ptr(),
+            _native.stream_of(q))
+
+    assert call(need - 1) == _native.KVQ_ERR_INVALID
+    torch.cuda.synchronize()
+    assert (out == 7.0).all()
+    assert call(need) == 0
+    torch.cuda.synchronize()
+    assert not out.any()  # all values are zero

@@ -482,7 +482,7 @@ __device__ __forceinline__ bool find_item(int wi, int lane, int& b, int& l, int&
       const int first = __builtin_amdgcn_readlane(upto - items, at);
       b = c + at;
       pb = (wi - first) * split;
-      pe = pb + split < l ? pb + split : l;
+      pe = split < l - pb ? pb + split : l;  // no sum past l
       return true;
     }
     base = __builtin_amdgcn_readlane(upto, 63);
@@ -818,6 +818,7 @@ int64_t fp8_split(const int64_t* lens, int64_t n, int kvh, int d, int cus) {
   return split;
 }
 
+constexpr int64_t kMaxLen = 0x7fff0000;  // positions of a request
 constexpr int64_t kMaxRowHeads = 65536;  // rows * query heads of a request (the combine's grid)
 
 struct Fp8Plan {
@@ -862,7 +863,7 @@ extern "C" int64_t kvq_fp8_pth_decode_workspace_bytes(const int64_t* seq_lens, i
   if (!fp8_decode_geometry(num_heads, num_kv_heads, head_size, block_size))
     return KVQ_ERR_GEOMETRY;
   for (int64_t b = 0; b < batch; ++b)
-    if (seq_lens[b] < 0 || seq_lens[b] > 0x7fff0000) return KVQ_ERR_INVALID;
+    if (seq_lens[b] < 0 || seq_lens[b] > kMaxLen) return KVQ_ERR_INVALID;
   int64_t most = 0;  // launches run one after another on one stream and share it
   const int rc = fp8_launches(seq_lens, batch, num_kv_heads, head_size, [&](const Fp8Plan& p) {
     most = std::max(most, fp8_ws_bytes(p.items, p.n, rows * num_heads, head_size));
@@ -879,7 +880,8 @@ extern "C" int kvq_fp8_pth_decode_attn(const void* query, int dtype, int64_t bat
                                        int64_t num_blocks, int block_size,
                                        const void* block_table, int block_index_type,
                                        int64_t max_blocks, const int64_t* seq_lens,
-                                       void* workspace, void* out, void* stream) {
+                                       void* workspace, int64_t workspace_bytes, void* out,
+                                       void* stream) {
   if (batch == 0) return KVQ_OK;
   if (!query || !k_data || !k_scale || !v_data || !v_scale || !block_table || !seq_lens || !out ||
       !workspace || batch < 0 || num_blocks <= 0 || max_blocks <= 0)
@@ -893,7 +895,8 @@ extern "C" int kvq_fp8_pth_decode_attn(const void* query, int dtype, int64_t bat
       !kvq::aligned16(k_data, v_data))  // 16-byte DMA lanes
     return KVQ_ERR_GEOMETRY;
   for (int64_t b = 0; b < batch; ++b)
-    if (seq_lens[b] < 0 || seq_lens[b] > max_blocks * block_size) return KVQ_ERR_INVALID;
+    if (seq_lens[b] < 0 || seq_lens[b] > kMaxLen || seq_lens[b] > max_blocks * block_size)
+      return KVQ_ERR_INVALID;
   int64_t lds_max = 0;
   const int lrc = kvq::device_lds_max(&lds_max);
   if (lrc != KVQ_OK) return lrc;
@@ -909,6 +912,12 @@ extern "C" int kvq_fp8_pth_decode_attn(const void* query, int dtype, int64_t bat
   const int64_t row = static_cast<int64_t>(heads) * d * 2;  // bytes of its 16-bit query rows
   const int take = std::min<int>(static_cast<int>(rows), 16 / (num_heads / kvh));
   const unsigned passes = static_cast<unsigned>((rows + take - 1) / take);
+  // the launches' items follow from the lengths and the device: every one has to
+  // fit before the first writes
+  const int wrc = fp8_launches(seq_lens, batch, kvh, d, [&](const Fp8Plan& p) -> int {
+    return fp8_ws_bytes(p.items, p.n, heads, d) <= workspace_bytes ? KVQ_OK : KVQ_ERR_INVALID;
+  });
+  if (wrc != KVQ_OK) return wrc;
   return fp8_launches(seq_lens, batch, kvh, d, [&](const Fp8Plan& p) -> int {
     float* ws_ml = ws_o + p.items * heads * d;
     int32_t* meta = reinterpret_cast<int32_t*>(ws_ml + 2 * p.items * heads);

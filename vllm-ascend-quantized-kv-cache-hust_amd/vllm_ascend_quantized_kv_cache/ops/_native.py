@@ -118,7 +118,8 @@ SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
     "kvq_fp8_pth_decode_workspace_bytes": (_I64, [_P, _I64, _I64, _I, _I, _I, _I]),
     "kvq_fp8_pth_decode_attn": (
         _I,
-        [_P, _I, _I64, _I64, _I, _I, _I, _I, _F, _P, _P, _P, _P, _I64, _I, _P, _I, _I64, _P, _P, _P, _P],
+        [_P, _I, _I64, _I64, _I, _I, _I, _I, _F, _P, _P, _P, _P, _I64, _I, _P, _I, _I64, _P, _P, _I64,
+         _P, _P],
     ),
 }
 

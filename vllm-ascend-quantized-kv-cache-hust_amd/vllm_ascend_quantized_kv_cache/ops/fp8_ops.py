@@ -311,7 +311,8 @@ def _decode_attention(query, k_data, k_scale, v_data, v_scale, block_table, seq_
         _native.ptr(q), _native.dtype_code(q.dtype), batch, rows, 1 if causal else 0, hq, kvh, d,
         float(scale), _native.ptr(k_data), _native.ptr(k_scale), _native.ptr(v_data), _native.ptr(v_scale), nb,
         bs, _native.ptr(table), _native.index_code(table.dtype), table.shape[1],
-        lens_np.ctypes.data, _native.ptr(ws), _native.ptr(target), _native.stream_of(q),
+        lens_np.ctypes.data, _native.ptr(ws), ws.numel(), _native.ptr(target),
+        _native.stream_of(q),
     )
     _native.check(rc, "kvq_fp8_pth_decode_attn")
     if target is not out:
