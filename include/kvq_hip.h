@@ -114,7 +114,7 @@ int kvq_kivi_ring_write(const void* src, int src_dtype, const int64_t* src_rows,
  * input rows, ring dst ring rows.  Inputs and rings are [rows, KVH, D] of
  * `dtype`.  Precondition: no ring dst is a pack source of the same side (the
  * batch then has no order inside it).  Head size 128 or 256, group size 64 or 128,
- * bf16/fp16 only: other geometries return KVQ_ERR_GEOMETRY and the caller
+ * bf16/fp16, inputs and rings on 16-byte bounds: others return KVQ_ERR_GEOMETRY and the caller
  * uses the separate entry points.  n_key_pack % group_size == 0 with the
  * group rules of kvq_kivi_pack_key. */
 int kvq_kivi_store(const void* key_input, const void* value_input, void* ring_k,
@@ -312,7 +312,8 @@ int64_t kvq_plan_prefill_attn(const int64_t* q_lens, const int64_t* kv_lens, int
 
 /* kvq_prefill_attn over a plan of kvq_plan_prefill_attn copied to the device:
  * only tiles with rows are launched, the longest first.  bf16 / fp16 and head
- * sizes 64, 128 and 256; KVQ_ERR_GEOMETRY otherwise. */
+ * sizes 64, 128 and 256, key and value on 16-byte bounds; KVQ_ERR_GEOMETRY
+ * otherwise (kvq_prefill_attn takes any). */
 int kvq_prefill_attn_planned(const void* query, const void* key, const void* value, int dtype,
                              const int32_t* plan, int64_t batch, int64_t num_units,
                              int num_heads, int num_kv_heads, int head_size, float scale,
@@ -441,8 +442,8 @@ int kvq_fp8_pth_gather_lens(const uint8_t* k_data, const float* k_scale, const u
  *   K = float(code) * k_scale[token, head] rounded to `dtype`, V likewise (the
  *   gather's rows), softmax in fp32.
  * query/out [batch * rows, num_heads, D] of `dtype` (bf16 / fp16), D 128 or 256,
- * block_size % 16 == 0, at most 16 query heads per kv head; other geometries
- * return KVQ_ERR_GEOMETRY.  Block ids as for kvq_fp8_pth_gather.  The lengths
+ * block_size % 16 == 0, at most 16 query heads per kv head, codes on 16-byte
+ * bounds; others return KVQ_ERR_GEOMETRY.  Block ids as for kvq_fp8_pth_gather.  The lengths
  * are read during the call and travel with the launches; `workspace` holds
  * kvq_fp8_pth_decode_workspace_bytes for the same lengths, rows and device (a
  * smaller workspace_bytes returns KVQ_ERR_INVALID before anything is launched).

@@ -153,6 +153,38 @@ def test_planned_decode_step_equals_general_path(gpu_device, g):
     assert fast.kivi_host_reads == 0
 
 
+def test_planned_step_of_rows_off_their_alignment(gpu_device):
+    """Key and value rows 8 bytes off a 16-byte bound (views into a larger buffer),
+    eager and captured, leave what rows on one leave."""
+    case = _Case(gpu_device, steps=4, seed=7)
+    plain, off, graphed = case.build(), case.build(), case.build()
+    graphed.kivi_decode_graph(case.b, max_blocks=case.table.shape[1])
+    n = case.b * case.kvh * case.d
+    k_s, v_s = (torch.empty(n + 4, dtype=torch.bfloat16, device=gpu_device)[4:].view(
+        case.b, case.kvh, case.d) for _ in range(2))
+    assert k_s.data_ptr() % 16 == v_s.data_ptr() % 16 == 8
+    q_s = torch.empty((case.b, case.hq, case.d), dtype=torch.bfloat16, device=gpu_device)
+    outs = [torch.zeros_like(q_s) for _ in range(3)]
+    graph = None
+    for j in range(4):
+        md, q, k, v = case.step(j)
+        for dst, src in ((q_s, q), (k_s, k), (v_s, v)):
+            dst.copy_(src)
+        plain.forward(None, q, k, v, None, md, outs[0])
+        off.forward(None, q, k_s, v_s, None, md, outs[1])
+        graphed.prepare_kivi_graph_replay(md, k_s, v_s)
+        if graph is None:
+            torch.cuda.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                graphed.forward(None, q_s, k_s, v_s, None, md, outs[2])
+        graph.replay()
+        torch.cuda.synchronize()
+        for impl, out in ((off, outs[1]), (graphed, outs[2])):
+            assert torch.equal(out, outs[0]), f"step {j}"
+            _same_state(impl, plain)
+
+
 def test_layers_share_one_planned_step(gpu_device, monkeypatch):
     """Layers called with one metadata object per engine step: the first
     plans and stages the step, the others whose window mirror matches take

@@ -765,6 +765,82 @@ def test_split_decode_head_256_cache_off_its_alignment(gpu_device, monkeypatch, 
                        lambda s: plan_decode_pieces(s, 1, 256), lens=[300, 129, 1, 700])
 
 
+@pytest.mark.parametrize("kvh,g,bs", [(2, 128, 128),  # split decode
+                                      (8, 128, 128),  # page-streaming
+                                      (8, 64, 128)])
+@pytest.mark.parametrize("side", range(6))
+@pytest.mark.parametrize("pieces", [True, False])
+def test_decode_cache_off_its_alignment(gpu_device, monkeypatch, kvh, g, bs, side, pieces):
+    """Head size 128 likewise, over the kernels that a plan with and without pieces
+    takes when everything is on its bound."""
+    import sys
+
+    from vllm_ascend_quantized_kv_cache.ops.kivi_decode import plan_decode, plan_decode_work
+
+    monkeypatch.setattr(sys.modules[__name__], "to_dev", lambda arrays, dev: tuple(
+        _off_16(t, dev) if i == side else t.to(dev) for i, t in enumerate(arrays)))
+    _split_decode_case(gpu_device, 128, kvh, g, bs, 5, torch.bfloat16,
+                       (lambda s: plan_decode(s, kvh, 256, page_streaming=kvh == 8)) if pieces
+                       else lambda s: plan_decode_work(s, 128), lens=[300, 129, 1, 700])
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_views_off_their_alignment(gpu_device, d):
+    """Dense attention, INT8 decode and (128 dims) the int4 packs and store of
+    contiguous views 8 bytes off a 16-byte bound, against the same on one; entry
+    points without another kernel refuse them."""
+    import ctypes
+
+    from vllm_ascend_quantized_kv_cache.ops import _native, kivi_pack
+    from vllm_ascend_quantized_kv_cache.ops.attention import prefill_attention
+    from vllm_ascend_quantized_kv_cache.ops.int8_ops import int8_decode_attention
+
+    dev, kvh, bs, dtype, puts = gpu_device, 2, 64, torch.bfloat16, (_off_16, torch.Tensor.to)
+    gen = torch.Generator().manual_seed(6)
+    lens = [130, 64, 17]
+    table = torch.tensor([[5, 1, 3], [0, 0, 0], [2, 0, 0]], dtype=torch.int32)
+    rows = torch.randn((sum(lens), kvh, d), generator=gen).to(dtype)
+    q = torch.randn((len(lens), kvh * 4, d), generator=gen).to(dtype).to(dev)
+    tol = dict(atol=1e-2, rtol=1e-2)  # two results within a bf16 rounding or two each
+    for side in range(2):
+        both = []
+        for put in puts:
+            kv = [(put if i == side else torch.Tensor.to)(x, dev)
+                  for i, x in enumerate((rows, rows.flip(0)))]
+            both.append(prefill_attention(q, *kv, [1] * 3, lens, d ** -0.5, True))
+            one, n = (ctypes.c_int64 * 3)(1, 1, 1), (ctypes.c_int64 * 3)(*lens)
+            out = torch.empty_like(q)
+            assert _native.lib().kvq_prefill_attn_lens(
+                q.data_ptr(), kv[0].data_ptr(), kv[1].data_ptr(), _native.dtype_code(dtype), one,
+                n, 3, kvh * 4, kvh, d, d ** -0.5, 1, None, 0, out.data_ptr(),
+                _native.stream_of(q)) == (_native.KVQ_ERR_GEOMETRY if put is _off_16 else 0)
+        torch.testing.assert_close(*both, **tol)
+
+    codes = torch.randint(-127, 128, (2, 8, bs, kvh, d), generator=gen, dtype=torch.int8)
+    aq = (torch.rand((kvh, d), generator=gen) / 100).to(dtype).to(dev)
+    both = [int8_decode_attention(q, put(codes[0], dev), put(codes[1], dev), aq, aq, table.to(dev),
+                                  lens, d ** -0.5) for put in puts]
+    torch.testing.assert_close(*both, **tol)
+
+    if d != 128:
+        return
+    for g in (64, 128):
+        slots = torch.arange(128, device=dev)
+        src = torch.cat([slots + 128, slots, slots + 128, slots])
+        packed = []
+        for put in puts:
+            x = put(rows[:128], dev)
+            ring = torch.zeros(1, 128, kvh, d, dtype=dtype, device=dev)
+            pages = to_dev(empty_kivi_caches(2, 128, kvh, d, g), dev)
+            if not kivi_pack.kivi_store(x, x, ring, ring, src, (128, 128, 0, 0), pages, g):
+                assert put is _off_16
+                kivi_pack.kivi_pack_key_cache(x, slots, *pages[:3], g)
+                kivi_pack.kivi_pack_value_cache(x, slots, *pages[3:], g)
+            packed.append(pages)
+        for a, b in zip(*packed):
+            assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+
+
 def test_head_256_views_off_their_alignment(gpu_device):
     """INT8 decode, dense attention, E4M3 decode and the int4 packs of contiguous
     views that start 8 bytes off a 16-byte bound, against the same on one."""

@@ -765,8 +765,8 @@ int launch_int8_decode_mfma(const void* query, int dtype, int hq, int kvh, int d
                             float* ws_ml, hipStream_t s, bool* launched) {
   *launched = false;
   if ((d != 128 && d != 256) || hq / kvh > 16 || bs % 16) return KVQ_OK;
-  // rows of 256 bytes off the DMA's 16-byte lanes run the generic kernel
-  if (d == 256 && !aligned16(kc, vc)) return KVQ_OK;
+  // rows off the DMA's 16-byte lanes run the generic kernel
+  if (!aligned16(kc, vc)) return KVQ_OK;
   if (num_work * kvh > 0x7fffffff) return KVQ_ERR_INVALID;
   // all kv heads of an item in one workgroup when they fit (at most 8 waves
   // and their tile buffers in the workgroup's LDS), else one wave per head

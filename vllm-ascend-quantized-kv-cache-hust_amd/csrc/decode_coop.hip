@@ -737,6 +737,7 @@ int launch_kivi_decode_coop(const void* query, int q_dtype, int hq, int kvh, int
   *launched = false;
   if (!pieces || num_pieces <= 0 || !coop_decode_applies(q_dtype, hq, kvh, d, ring_dtype, bs, g))
     return KVQ_OK;
+  if (!(aligned16(kq, vq) && aligned16(ks, km) && aligned16(vs, vm))) return KVQ_OK;  // DMA lanes
   // the page softmax orders raw scores, which a positive scale keeps
   if (!(qscale > 0.0f) || qscale == INFINITY) return KVQ_OK;
   int64_t lds_max = 0;

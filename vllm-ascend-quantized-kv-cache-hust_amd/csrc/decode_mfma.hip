@@ -1114,12 +1114,15 @@ int launch_kivi_decode_mfma(const void* query, int q_dtype, int hq, int kvh, int
   *launched = false;
   *tail_done = false;
   *split = false;
+  // every kernel below copies codes and key scales to LDS by 16-byte lanes
+  if (!(aligned16(kq, vq) && aligned16(ks, km))) return KVQ_OK;
   {
-    // the split decode: pieces that the page-streaming kernel does not take, and
-    // head size 256 with or without them
+    // the split decode: pieces that the page-streaming kernel (value scales by
+    // 16-byte lanes too) does not take, and head size 256 with or without them
     const bool with_pieces = pieces && num_pieces > 0;
-    if (d == 256 || (with_pieces && !(qscale > 0.0f && qscale != INFINITY &&
-                                      coop_decode_applies(q_dtype, hq, kvh, d, ring_dtype, bs, g)))) {
+    const bool coop = qscale > 0.0f && qscale != INFINITY && aligned16(vs, vm) &&
+                      coop_decode_applies(q_dtype, hq, kvh, d, ring_dtype, bs, g);
+    if (d == 256 || (with_pieces && !coop)) {
       const int src = launch_kivi_decode_split(
           query, q_dtype, hq, kvh, d, qscale, kq, ks, km, vq, vs, vm, bs, g, nb, block_table,
           maxb, seq_meta, work, num_work, with_pieces ? pieces : nullptr, num_pieces, ring_k,

@@ -426,7 +426,7 @@ int launch_kivi_decode_split(const void* query, int q_dtype, int hq, int kvh, in
   *launched = false;
   if (!split_decode_applies(q_dtype, hq, kvh, d, ring_dtype, bs, g)) return KVQ_OK;
   // caches off the DMA's 16-byte lanes: the generic kernel
-  if (d == 256 && !(aligned16(kq, vq) && aligned16(ks, km))) return KVQ_OK;
+  if (!(aligned16(kq, vq) && aligned16(ks, km))) return KVQ_OK;
   // a plan without pieces: every item is one (its tail items too)
   if (!pieces) num_pieces = num_work;
   // the lane offsets of a tile's DMAs are 32-bit: a page of all heads, and (in

@@ -1094,10 +1094,11 @@ extern "C" int kvq_kivi_pack_key(const void* src_a, int64_t n_a, const void* src
     return KVQ_ERR_GEOMETRY;
   if (num_tokens % group_size) return KVQ_ERR_INVALID;
   if (!src_index && n_a < num_tokens) return KVQ_ERR_INVALID;
-  if ((src_dtype == KVQ_DTYPE_BF16 || src_dtype == KVQ_DTYPE_F16) && kvq::aligned16(src_a, src_b))
+  const bool dma = kvq::aligned16(src_a, src_b);  // the LDS pack's 16-byte lanes
+  if ((src_dtype == KVQ_DTYPE_BF16 || src_dtype == KVQ_DTYPE_F16) && dma)
     halve_heads_of_256(num_kv_heads, head_size, group_size);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (pack_lds_applies(src_dtype, head_size, group_size, num_tokens, num_kv_heads) &&
+  if (dma && pack_lds_applies(src_dtype, head_size, group_size, num_tokens, num_kv_heads) &&
       (slot_index_type == KVQ_INDEX_I32 || slot_index_type == KVQ_INDEX_I64))
     return pack_side(true, src_dtype, src_a, n_a, src_b, src_index, slot_mapping,
                      slot_index_type, num_tokens, num_kv_heads, group_size, block_size, k_quant,
@@ -1154,10 +1155,11 @@ extern "C" int kvq_kivi_pack_value(const void* src_a, int64_t n_a, const void* s
   if (!kivi_geometry_ok(num_kv_heads, head_size, group_size, block_size))
     return KVQ_ERR_GEOMETRY;
   if (!src_index && n_a < num_tokens) return KVQ_ERR_INVALID;
-  if ((src_dtype == KVQ_DTYPE_BF16 || src_dtype == KVQ_DTYPE_F16) && kvq::aligned16(src_a, src_b))
+  const bool dma = kvq::aligned16(src_a, src_b);  // the LDS pack's 16-byte lanes
+  if ((src_dtype == KVQ_DTYPE_BF16 || src_dtype == KVQ_DTYPE_F16) && dma)
     halve_heads_of_256(num_kv_heads, head_size, group_size);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (pack_lds_applies(src_dtype, head_size, group_size, num_tokens, num_kv_heads) &&
+  if (dma && pack_lds_applies(src_dtype, head_size, group_size, num_tokens, num_kv_heads) &&
       (slot_index_type == KVQ_INDEX_I32 || slot_index_type == KVQ_INDEX_I64))
     return pack_side(false, src_dtype, src_a, n_a, src_b, src_index, slot_mapping,
                      slot_index_type, num_tokens, num_kv_heads, group_size, block_size, v_quant,
@@ -1248,9 +1250,10 @@ extern "C" int kvq_kivi_store(const void* key_input, const void* value_input, vo
   if (n_value_pack && (!v_quant || !v_scale || !v_mn)) return KVQ_ERR_INVALID;
   if (!kivi_geometry_ok(num_kv_heads, head_size, group_size, block_size))
     return KVQ_ERR_GEOMETRY;
-  if (kvq::aligned16(key_input, value_input) && kvq::aligned16(ring_k, ring_v))
-    halve_heads_of_256(num_kv_heads, head_size, group_size);
-  // the register key pack's geometry; callers fall back to the separate
+  if (!kvq::aligned16(key_input, value_input) || !kvq::aligned16(ring_k, ring_v))
+    return KVQ_ERR_GEOMETRY;
+  halve_heads_of_256(num_kv_heads, head_size, group_size);
+  // the LDS pack's geometry (and, above, its DMA lanes' bounds); callers fall back to the separate
   // pack and ring-write entry points elsewhere
   if (head_size != 128 || (group_size != 64 && group_size != 128) ||
       (dtype != KVQ_DTYPE_BF16 && dtype != KVQ_DTYPE_F16))
@@ -1286,6 +1289,8 @@ extern "C" int kvq_kivi_store_planned(const void* key_input, const void* value_i
     return KVQ_ERR_GEOMETRY;
   if (head_size != 128 || (group_size != 64 && group_size != 128) ||
       (dtype != KVQ_DTYPE_BF16 && dtype != KVQ_DTYPE_F16))
+    return KVQ_ERR_GEOMETRY;
+  if (!kvq::aligned16(key_input, value_input) || !kvq::aligned16(ring_k, ring_v))
     return KVQ_ERR_GEOMETRY;
   if (cap_key_pack % group_size) return KVQ_ERR_INVALID;
   if (cap_value_pack * num_kv_heads >= 0x7fffffff) return KVQ_ERR_INVALID;

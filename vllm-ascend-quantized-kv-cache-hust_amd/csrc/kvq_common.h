@@ -24,7 +24,9 @@ struct bf16 {
 using f16 = _Float16;
 
 // Both on 16-byte bounds (nullptr is): what 16-byte lanes of a global-to-LDS
-// DMA take.  A contiguous view into a larger buffer may start off them.
+// DMA take, whatever the head size.  A contiguous view into a larger buffer may
+// start off them; the kernels without DMA then run, or the call is refused with
+// KVQ_ERR_GEOMETRY where the caller has another entry point.
 inline bool aligned16(const void* a, const void* b) {
   return ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) == 0;
 }

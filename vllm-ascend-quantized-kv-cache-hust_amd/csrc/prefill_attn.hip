@@ -884,13 +884,13 @@ struct FaTiles {
   int64_t batch, num_units, tiles;
 };
 
-// At head size 256 the keys and values are on 16-byte bounds, which their DMA
-// into LDS takes in 16-byte lanes; views off them run prefill_attn_kernel.
+// The keys and values are on 16-byte bounds, which their DMA into LDS takes in
+// 16-byte lanes; views off them run prefill_attn_kernel.
 int fa_applies(const void* key, const void* value, int dtype, int head_size, bool* applies) {
   *applies = false;
   if (dtype != KVQ_DTYPE_BF16 && dtype != KVQ_DTYPE_F16) return KVQ_OK;
   if (head_size != 64 && head_size != 128 && head_size != 256) return KVQ_OK;
-  if (head_size == 256 && !aligned16(key, value)) return KVQ_OK;
+  if (!aligned16(key, value)) return KVQ_OK;
   int64_t lds_max = 0;  // LDS one workgroup may use on this device
   const int lrc = device_lds_max(&lds_max);
   if (lrc != KVQ_OK) return lrc;

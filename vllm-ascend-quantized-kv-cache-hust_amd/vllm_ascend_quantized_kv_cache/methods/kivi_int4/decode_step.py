@@ -209,6 +209,9 @@ class KiviDecodeLauncher:
         ring = impl._kivi_ring
         kq, ks, km, vq, vs, vm = impl._kivi_caches()
         lib = _native.lib()
+        # rows off the 16-byte bounds of the kernel's DMA lanes go through a copy
+        if (key.data_ptr() | value.data_ptr()) % 16:
+            key, value = key.clone(), value.clone()
         common = (_native.ptr(key), _native.ptr(value), _native.ptr(ring.key),
                   _native.ptr(ring.value), ring.rows * ring.ring_len,
                   _native.dtype_code(ring.dtype), ring.num_kv_heads, ring.head_size,

@@ -49,9 +49,9 @@ def _launch(q, k, v, q_lens: list[int], kv_lens: list[int], scale: float, causal
     kvh = k.shape[1]
     batch = len(q_lens)
     dtype = _native.dtype_code(q.dtype)
-    # 256 dims: keys and values on the 16-byte bounds of the kernel's DMA lanes
-    tiled = d in (64, 128, 256) and q.dtype != torch.float32 and (
-        d != 256 or (k.data_ptr() | v.data_ptr()) % 16 == 0)
+    # keys and values on the 16-byte bounds of the kernel's DMA lanes
+    tiled = (d in (64, 128, 256) and q.dtype != torch.float32
+             and (k.data_ptr() | v.data_ptr()) % 16 == 0)
     if tiled and batch <= 128:
         # small batches: the lengths and tiles travel with the launch
         lens_t = ctypes.c_int64 * batch

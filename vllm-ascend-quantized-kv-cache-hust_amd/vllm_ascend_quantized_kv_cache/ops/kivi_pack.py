@@ -201,21 +201,22 @@ def kivi_store(
     ``jobs`` (int64, on the device) and ``counts`` come from
     ``StorePlan.one_launch_jobs``; inputs are ``[n, KVH, D]`` contiguous in the
     ring dtype.  Returns False (nothing launched) for a geometry the one-launch
-    kernel does not cover.
+    kernel does not cover, and for inputs or rings off a 16-byte bound.
     """
     kq, ks, km, vq, vs, vm = caches
     nb, kvh, d, pbs = kq.shape
     if not store_one_launch_supported(d, group_size, ring_k.dtype):
         return False
-    if d == 256 and any(t is not None and t.data_ptr() % 16
-                        for t in (key_input, value_input, ring_k, ring_v)):
+    ptr_k, ptr_v = _native.ptr(key_input), _native.ptr(value_input)
+    ptr_rk, ptr_rv = ring_k.data_ptr(), ring_v.data_ptr()
+    if ((ptr_k or 0) | (ptr_v or 0) | ptr_rk | ptr_rv) % 16:
         return False  # off the 16-byte lanes of the kernel's DMA
     if sum(counts) == 0:
         return True
     _native.require_gpu_tensors("kivi store", ring_k, ring_v, jobs, kq, key_input, value_input)
     rc = _native.lib().kvq_kivi_store(
-        _native.ptr(key_input), _native.ptr(value_input), _native.ptr(ring_k),
-        _native.ptr(ring_v), ring_k.shape[0] * ring_k.shape[1], _native.dtype_code(ring_k.dtype),
+        ptr_k, ptr_v, ptr_rk, ptr_rv, ring_k.shape[0] * ring_k.shape[1],
+        _native.dtype_code(ring_k.dtype),
         kvh, d, group_size, pbs * 8, _native.ptr(jobs), *counts,
         _native.ptr(kq), _native.ptr(ks), _native.ptr(km), _native.ptr(vq), _native.ptr(vs),
         _native.ptr(vm), _native.stream_of(ring_k),
