@@ -319,6 +319,13 @@ int kvq_prefill_attn_planned(const void* query, const void* key, const void* val
                              int num_heads, int num_kv_heads, int head_size, float scale,
                              int causal, void* out, void* stream);
 
+/* Host-side (no GPU call): the segments kvq_prefill_attn_lens cuts each tile's keys
+ * into on a device of cu_count compute units, 1 when they stay whole; KVQ_ERR_CAPACITY
+ * and KVQ_ERR_INVALID as the call itself. */
+int64_t kvq_prefill_attn_segments(const int64_t* q_lens, const int64_t* kv_lens, int64_t batch,
+                                  int num_heads, int num_kv_heads, int head_size, int causal,
+                                  int cu_count);
+
 /* kvq_prefill_attn with the lengths on the host (int64 [batch], read during the
  * call): the plan travels with the launch, nothing is copied to the device.
  * Calls of few tiles over long keys cut each tile's keys into segments, whose

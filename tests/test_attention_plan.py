@@ -66,22 +66,56 @@ def test_plan_past_the_packed_range_keeps_the_lengths():
     assert plan[:70001].tolist() == list(range(70001)) == plan[70001:].tolist()
 
 
-@pytest.mark.parametrize("q_lens,kv_lens,hq,kvh,d,cut", [
-    ([16], [8192], 8, 1, 128, True),       # one tile, long keys
-    ([16], [500], 8, 1, 128, False),       # too few blocks to cut
-    ([2048] * 8, [10240] * 8, 40, 8, 128, False),  # more tiles than slots
-    ([0, 0], [5, 5], 8, 1, 128, False),
-])
-def test_workspace_follows_the_cut(q_lens, kv_lens, hq, kvh, d, cut):
+def _lens_call(name, q_lens, kv_lens, *args):
     import ctypes
 
+    arr = ctypes.c_int64 * len(q_lens)
+    return getattr(_native.lib(), name)(arr(*q_lens), arr(*kv_lens), len(q_lens), *args)
+
+
+# the segments follow from the tiles and their key blocks: as many as fill the
+# chip's slots (two workgroups a CU, one at 256 dims), of at least 4 blocks of 64
+# keys, at most 32, where that takes 8 blocks off the longest tile
+SEGMENTS = [
+    ([16], [8192], 8, 1, 128, 256, 32),           # one tile, 128 blocks, 512 slots: the most
+    ([16], [8192], 8, 1, 128, 8, 16),             # ... 16 slots
+    ([16], [8192], 8, 1, 256, 8, 8),              # ... 8
+    ([16] * 3, [8192] * 3, 8, 1, 128, 8, 5),      # three tiles share 16 slots
+    ([16], [2000], 8, 1, 128, 256, 8),            # 32 blocks: 8 segments of 4
+    ([16], [500], 8, 1, 128, 256, 1),             # 8 blocks: two segments save 4
+    ([16], [1024], 8, 1, 128, 256, 4),            # 16 blocks: four segments save 12
+    ([1024] * 6, [10240] * 6, 8, 1, 128, 256, 1),   # 384 tiles on 512 slots: one each
+    ([1024] * 4, [10240] * 4, 8, 1, 128, 256, 2),   # 256 tiles: two each
+    ([1024] * 4, [10240] * 4, 8, 1, 256, 256, 1),   # 256 tiles on 256 slots
+    ([700] * 4, [10240] * 4, 40, 8, 128, 256, 1),   # 112 tiles of 8 kv heads: more than slots
+    ([0, 0], [5, 5], 8, 1, 128, 256, 1),
+]
+
+
+@pytest.mark.parametrize("q_lens,kv_lens,hq,kvh,d,cus,segs", SEGMENTS)
+def test_segments_follow_the_rule(q_lens, kv_lens, hq, kvh, d, cus, segs):
+    got = _lens_call("kvq_prefill_attn_segments", q_lens, kv_lens, hq, kvh, d, 1, cus)
+    assert got == segs
+    # without a device, or one of unknown size, the keys stay whole
+    assert _lens_call("kvq_prefill_attn_segments", q_lens, kv_lens, hq, kvh, d, 1, 0) == 1
+
+
+def test_segments_of_a_plan_past_the_argument():
+    """8 x 2048 queries of 5 heads a kv head: 640 tiles, and the argument holds 482."""
+    for name, extra in (("kvq_prefill_attn_segments", (256,)),
+                        ("kvq_prefill_attn_lens_workspace_bytes", ())):
+        got = _lens_call(name, [2048] * 8, [10240] * 8, 40, 8, 128, 1, *extra)
+        assert got == _native.KVQ_ERR_CAPACITY
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("q_lens,kv_lens,hq,kvh,d,cus,segs", SEGMENTS)
+def test_workspace_follows_the_cut(gpu_device, q_lens, kv_lens, hq, kvh, d, cus, segs):
+    """Rows of whole tiles, D + 2 floats each, per segment; none for whole keys."""
     import torch
 
-    lib = _native.lib()
-    arr = ctypes.c_int64 * len(q_lens)
-    got = lib.kvq_prefill_attn_lens_workspace_bytes(arr(*q_lens), arr(*kv_lens), len(q_lens), hq,
-                                                    kvh, d, 1)
-    if torch.cuda.is_available() or not cut:
-        # partial rows of whole tiles, D + 2 floats each (without a GPU: no cut)
-        assert (got > 0) == cut if got != _native.KVQ_ERR_CAPACITY else not cut
-        assert got <= 0 or got % (128 * (d + 2) * 4) == 0
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    segs = _lens_call("kvq_prefill_attn_segments", q_lens, kv_lens, hq, kvh, d, 1, cus)
+    tiles = sum(-(-m * (hq // kvh) // 128) for m in q_lens)
+    got = _lens_call("kvq_prefill_attn_lens_workspace_bytes", q_lens, kv_lens, hq, kvh, d, 1)
+    assert got == (tiles * kvh * segs * 128 * (d + 2) * 4 if segs > 1 else 0)

@@ -1030,12 +1030,17 @@ int64_t plan_units(const int64_t* q_lens, const int64_t* kv_lens, int64_t batch,
 // keys are cut into as many segments as fill the chip, of at least 4 blocks
 // (a segment's start and end cost about 3), where that takes 8 blocks off the
 // longest tile, about what the merge costs.
-int64_t plan_segs(int64_t units, int64_t most, int kvh, int head_size) {
-  int cus = 0;
-  if (device_cu_count(&cus) != KVQ_OK || cus <= 0) return 1;
+int64_t plan_segs(int64_t units, int64_t most, int kvh, int head_size, int cus) {
+  if (cus <= 0) return 1;
   const int64_t slots = static_cast<int64_t>(cus) * (head_size == 256 ? 1 : 2);
   const int64_t segs = std::min<int64_t>({slots / std::max<int64_t>(1, units * kvh), most / 4, 32});
   return segs > 1 && most - most / segs >= 8 ? segs : 1;
+}
+
+int64_t plan_segs(int64_t units, int64_t most, int kvh, int head_size) {
+  int cus = 0;
+  if (device_cu_count(&cus) != KVQ_OK) return 1;
+  return plan_segs(units, most, kvh, head_size, cus);
 }
 
 int64_t seg_rows(int64_t units, int kvh, int64_t segs) { return units * kvh * segs * kFaTileRows; }
@@ -1112,6 +1117,18 @@ extern "C" int kvq_prefill_attn_planned(const void* query, const void* key, cons
                            static_cast<hipStream_t>(stream), &launched);
   if (rc != KVQ_OK) return rc;
   return launched ? KVQ_OK : KVQ_ERR_GEOMETRY;
+}
+
+extern "C" int64_t kvq_prefill_attn_segments(const int64_t* q_lens, const int64_t* kv_lens,
+                                             int64_t batch, int num_heads, int num_kv_heads,
+                                             int head_size, int causal, int cu_count) {
+  if (!plan_args_ok(q_lens, kv_lens, batch, num_heads, num_kv_heads, head_size))
+    return KVQ_ERR_INVALID;
+  if (plan_arg_cap(batch) <= 0) return KVQ_ERR_CAPACITY;
+  int64_t most = 0;
+  const int64_t n = plan_units(q_lens, kv_lens, batch, num_heads / num_kv_heads, causal,
+                               plan_arg_cap(batch), &most, nullptr);
+  return n < 0 ? n : plan_segs(n, most, num_kv_heads, head_size, cu_count);
 }
 
 extern "C" int64_t kvq_prefill_attn_lens_workspace_bytes(const int64_t* q_lens,

@@ -77,6 +77,7 @@ SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
     "kvq_prefill_attn_planned": (
         _I, [_P, _P, _P, _I, _P, _I64, _I64, _I, _I, _I, _F, _I, _P, _P]
     ),
+    "kvq_prefill_attn_segments": (_I64, [_P, _P, _I64, _I, _I, _I, _I, _I]),
     "kvq_prefill_attn_lens_workspace_bytes": (_I64, [_P, _P, _I64, _I, _I, _I, _I]),
     "kvq_prefill_attn_lens": (
         _I, [_P, _P, _P, _I, _P, _P, _I64, _I, _I, _I, _F, _I, _P, _I64, _P, _P]
