@@ -158,6 +158,30 @@ def test_gather_matches_oracle_bit_exact(gpu_device, out_dtype, d, kvh):
         assert torch.equal(dk.cpu(), wk) and torch.equal(dv.cpu(), wv)
 
 
+@pytest.mark.parametrize("index", [torch.int32, torch.int64])
+def test_gather_with_lengths_on_the_device_is_the_same(gpu_device, index):
+    """The entry point that reads the first rows from device memory, over ragged
+    lengths and an empty request."""
+    from vllm_ascend_quantized_kv_cache.ops import _native
+
+    nb, bs, kvh, d, lens = 12, 16, 2, 128, [37, 16, 0, 70]
+    table = torch.tensor([[3, 7, 11, -1, -1], [0, -1, -1, -1, -1], [-1] * 5, [1, 2, 4, 5, 6]],
+                         dtype=index, device=gpu_device)
+    _, _, views = _views(gpu_device, nb, bs, kvh, d)
+    rows = [_inputs(nb * bs, kvh, d, torch.bfloat16, seed=s).to(gpu_device) for s in (1, 2)]
+    fp8_ops.fp8_per_token_head_store(*rows, torch.arange(nb * bs, device=gpu_device), *views)
+    want = fp8_ops.fp8_per_token_head_dequant_gather(*views, table, lens, torch.bfloat16)
+    cu = torch.tensor([0, 37, 53, 53, 123], dtype=torch.int64, device=gpu_device)
+    got = [torch.zeros_like(x) for x in want]
+    rc = _native.lib().kvq_fp8_pth_gather(
+        *(v.data_ptr() for v in views), nb, bs, kvh, d, table.data_ptr(),
+        _native.index_code(index), 5, cu.data_ptr(), 4, got[0].data_ptr(), got[1].data_ptr(),
+        _native.dtype_code(torch.bfloat16), _native.stream_of(cu))
+    assert rc == 0
+    for a, b in zip(got, want):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
 @pytest.mark.parametrize("batch", [256, 257, 600])
 def test_gather_of_batches_past_one_launch(gpu_device, batch):
     """A launch carries 256 requests' rows; short, empty and long ones on both

@@ -271,3 +271,29 @@ def test_decode_head_256_keeps_small_probabilities(gpu_device, kvh, rep, bits):
     # 190 products of up to 127 * 2^-bits at 2^-23 each
     torch.testing.assert_close(got.double().cpu(), want, rtol=2.0 ** -8 + 2.0 ** -18,
                                atol=190 * 127 * 2.0 ** (-bits - 23))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_dequant_gather_with_lengths_on_the_device_is_the_same(gpu_device, dtype):
+    """The entry point that reads the first rows from device memory, over ragged
+    lengths and an empty request."""
+    from vllm_ascend_quantized_kv_cache.ops import _native
+    from vllm_ascend_quantized_kv_cache.ops.int8_ops import int8_dequant_gather
+
+    dev, nb, bs, kvh, d, lens = gpu_device, 12, 16, 3, 64, [37, 16, 0, 70]
+    gen = torch.Generator().manual_seed(31)
+    caches = [torch.randint(-128, 128, (nb, bs, kvh, d), generator=gen, dtype=torch.int8).to(dev)
+              for _ in range(2)]
+    aq = [(torch.rand((kvh, d), generator=gen) / 50).to(dtype).to(dev) for _ in range(2)]
+    table = torch.tensor([[3, 7, 11, 0, 0], [0] * 5, [0] * 5, [1, 2, 4, 5, 6]], dtype=torch.int32,
+                         device=dev)
+    want = int8_dequant_gather(*caches, table, lens, dtype, *aq)
+    cu = torch.tensor([0, 37, 53, 53, 123], dtype=torch.int64, device=dev)
+    got = [torch.zeros_like(x) for x in want]
+    rc = _native.lib().kvq_int8_dequant_gather(
+        caches[0].data_ptr(), caches[1].data_ptr(), nb, bs, kvh, d, aq[0].data_ptr(),
+        aq[1].data_ptr(), _native.dtype_code(dtype), table.data_ptr(), 5, cu.data_ptr(), 4,
+        got[0].data_ptr(), got[1].data_ptr(), _native.stream_of(cu))
+    assert rc == 0
+    for a, b in zip(got, want):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
