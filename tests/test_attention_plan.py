@@ -73,11 +73,11 @@ def _lens_call(name, q_lens, kv_lens, *args):
     return getattr(_native.lib(), name)(arr(*q_lens), arr(*kv_lens), len(q_lens), *args)
 
 
-# the segments follow from the tiles and their key blocks: as many as fill the
+# the segments follow from the tiles, their key blocks and their rows: what fits the
 # chip's slots (two workgroups a CU, one at 256 dims), of at least 4 blocks of 64
-# keys, at most 32, where that takes 8 blocks off the longest tile
+# keys, at most 32, where the blocks saved outweigh the partials' way through memory
 SEGMENTS = [
-    ([16], [8192], 8, 1, 128, 256, 32),           # one tile, 128 blocks, 512 slots: the most
+    ([16], [8192], 8, 1, 128, 256, 26),           # one tile of 128 blocks: 5 blocks each
     ([16], [8192], 8, 1, 128, 8, 16),             # ... 16 slots
     ([16], [8192], 8, 1, 256, 8, 8),              # ... 8
     ([16] * 3, [8192] * 3, 8, 1, 128, 8, 5),      # three tiles share 16 slots
@@ -89,6 +89,12 @@ SEGMENTS = [
     ([1024] * 4, [10240] * 4, 8, 1, 256, 256, 1),   # 256 tiles on 256 slots
     ([700] * 4, [10240] * 4, 40, 8, 128, 256, 1),   # 112 tiles of 8 kv heads: more than slots
     ([0, 0], [5, 5], 8, 1, 128, 256, 1),
+    ([60] * 8, [1024] * 8, 64, 8, 128, 256, 1),   # 16 MB of partials a segment for 8 blocks
+    ([60] * 8, [6000] * 8, 64, 8, 128, 256, 2),   # ... for 47
+    ([60] * 3, [1024] * 3, 64, 8, 128, 256, 1),   # 6 MB a segment, 16 blocks
+    ([60] * 3, [2048] * 3, 64, 8, 128, 256, 3),   # ... 32
+    ([60] * 3, [1024] * 3, 8, 8, 128, 256, 4),    # 0.7 MB
+    ([60] * 8, [768] * 8, 8, 8, 256, 256, 3),     # 4 MB, 12 blocks of 256 dims
 ]
 
 

@@ -1027,20 +1027,48 @@ int64_t plan_units(const int64_t* q_lens, const int64_t* kv_lens, int64_t batch,
 // Segments per tile.  A launch of fewer tiles than the chip holds workgroups
 // leaves the rest of it idle while each tile walks its keys alone (8 query
 // heads on 1 kv head, 16 rows over 8K keys: 128 blocks on 1 of 256 CUs), so its
-// keys are cut into as many segments as fill the chip, of at least 4 blocks
-// (a segment's start and end cost about 3), where that takes 8 blocks off the
-// longest tile, about what the merge costs.
-int64_t plan_segs(int64_t units, int64_t most, int kvh, int head_size, int cus) {
+// keys are cut, into segments of at least 4 blocks (a segment's start and end
+// cost about 3) that fit the chip at once, where the blocks this takes off the
+// longest tile outweigh the partials' way through memory.  In microseconds, as
+// measured on 1 - 256 tiles of 4 - 128 rows over 768 - 12K keys: a block of the
+// longest tile 1.05 (1.5 at 256 dims, 0.85 at 64), 1.4 times that where two workgroups
+// share a CU, the merge 3.5 + 0.2 a segment + 0.5 a MB of partials.  8 requests
+// of 60 rows over 1K keys, 64 heads on 8 kv heads: 27.8 whole, 41.1 in two
+// segments; 3 of them over 2K keys 41.7, 35.6 in three; 1 over 3K on 1 kv head 58,
+// 18 in ten.
+int64_t plan_segs(int64_t units, int64_t most, int64_t rows, int kvh, int head_size, int cus) {
   if (cus <= 0) return 1;
+  const double wgs = static_cast<double>(std::max<int64_t>(1, units * kvh));
   const int64_t slots = static_cast<int64_t>(cus) * (head_size == 256 ? 1 : 2);
-  const int64_t segs = std::min<int64_t>({slots / std::max<int64_t>(1, units * kvh), most / 4, 32});
-  return segs > 1 && most - most / segs >= 8 ? segs : 1;
+  const int64_t fit =
+      std::min<int64_t>({slots / std::max<int64_t>(1, units * kvh), most / 4, 32});
+  const double block = head_size == 256 ? 1.5 : head_size == 128 ? 1.05 : 0.85;
+  const double row_mb = static_cast<double>(rows) * kvh * (head_size + 2) * 4e-6;
+  int64_t best = 1;
+  double least = block * static_cast<double>(most) - 1.5;  // whole, and what a cut has to save
+  for (int64_t segs = 2; segs <= fit; ++segs) {
+    const double share = std::min(1.0, std::max(0.0, wgs * static_cast<double>(segs) / cus - 1.0));
+    const double us = block * static_cast<double>((most + segs - 1) / segs) * (1.0 + 0.4 * share) +
+                      3.5 + static_cast<double>(segs) * (0.2 + 0.5 * row_mb);
+    if (us < least) {
+      least = us;
+      best = segs;
+    }
+  }
+  return best;
 }
 
-int64_t plan_segs(int64_t units, int64_t most, int kvh, int head_size) {
+int64_t plan_segs(int64_t units, int64_t most, int64_t rows, int kvh, int head_size) {
   int cus = 0;
   if (device_cu_count(&cus) != KVQ_OK) return 1;
-  return plan_segs(units, most, kvh, head_size, cus);
+  return plan_segs(units, most, rows, kvh, head_size, cus);
+}
+
+// Rows of one kv head of a batch whose lengths plan_units accepts.
+int64_t head_rows(const int64_t* q_lens, int64_t batch, int64_t rep) {
+  int64_t n = 0;
+  for (int64_t b = 0; b < batch; ++b) n += q_lens[b];
+  return n * rep;
 }
 
 int64_t seg_rows(int64_t units, int kvh, int64_t segs) { return units * kvh * segs * kFaTileRows; }
@@ -1128,7 +1156,9 @@ extern "C" int64_t kvq_prefill_attn_segments(const int64_t* q_lens, const int64_
   int64_t most = 0;
   const int64_t n = plan_units(q_lens, kv_lens, batch, num_heads / num_kv_heads, causal,
                                plan_arg_cap(batch), &most, nullptr);
-  return n < 0 ? n : plan_segs(n, most, num_kv_heads, head_size, cu_count);
+  return n < 0 ? n
+               : plan_segs(n, most, head_rows(q_lens, batch, num_heads / num_kv_heads),
+                           num_kv_heads, head_size, cu_count);
 }
 
 extern "C" int64_t kvq_prefill_attn_lens_workspace_bytes(const int64_t* q_lens,
@@ -1142,7 +1172,8 @@ extern "C" int64_t kvq_prefill_attn_lens_workspace_bytes(const int64_t* q_lens,
   const int64_t n = plan_units(q_lens, kv_lens, batch, num_heads / num_kv_heads, causal,
                                plan_arg_cap(batch), &most, nullptr);
   if (n <= 0) return n;
-  const int64_t segs = plan_segs(n, most, num_kv_heads, head_size);
+  const int64_t segs = plan_segs(n, most, head_rows(q_lens, batch, num_heads / num_kv_heads),
+                                 num_kv_heads, head_size);
   return segs == 1 ? 0 : seg_rows(n, num_kv_heads, segs) * (head_size + 2) * 4;
 }
 
@@ -1168,7 +1199,8 @@ extern "C" int kvq_prefill_attn_lens(const void* query, const void* key, const v
   // without the workspace (or on another device than it was sized on) the keys
   // stay whole
   SegWs seg{nullptr, nullptr, 1};
-  const int64_t segs = plan_segs(n, most, num_kv_heads, head_size);
+  const int64_t segs = plan_segs(n, most, head_rows(q_lens, batch, num_heads / num_kv_heads),
+                                 num_kv_heads, head_size);
   const int64_t rows = seg_rows(n, num_kv_heads, segs);
   if (segs > 1 && workspace && workspace_bytes >= rows * (head_size + 2) * 4) {
     seg.o = static_cast<float*>(workspace);
