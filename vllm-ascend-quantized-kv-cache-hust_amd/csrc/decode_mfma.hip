@@ -742,7 +742,7 @@ __device__ __forceinline__ void tr_item(
     const uint32_t* __restrict__ vq, const float* __restrict__ vs, const float* __restrict__ vm,
     int bs, int g, int64_t nb, const int32_t* __restrict__ block_table, int64_t maxb, int b,
     int pb, int pe, int kind, int wi, char* my_lds, float* xfer, int half, int npair, int lane,
-    int n, int kg, int gpb, int ng, int wpd, float* __restrict__ ws_o,
+    int n, int kg, int gpb, int ng, int wpd, bool pieces, float* __restrict__ ws_o,
     float* __restrict__ ws_ml) {
   using T = tr::Tile<NVG, KSV>;
   constexpr int D = T::D;
@@ -790,11 +790,13 @@ __device__ __forceinline__ void tr_item(
     }
     const uint32_t* W = reinterpret_cast<const uint32_t*>(cur);
     if (new_group) tr::prepare_group<TQ, NVG, KSV, FOLD>(W, n, kg, ql, qscale, qg);
+    if (pieces) __builtin_amdgcn_s_setprio(1);
     const uint32_t off = tr::lds_off(cur);
     if (p0 + GT <= pe)
       tr::compute_tile<NVG, KSV, FOLD, true>(W, off, p0, p0, pe, n, kg, qg, qscale, acc);
     else
       tr::compute_tile<NVG, KSV, FOLD, false>(W, off, p0, p0, pe, n, kg, qg, qscale, acc);
+    if (pieces) __builtin_amdgcn_s_setprio(0);
   };
   if (p_first < pe) issue(my_lds, p_first, true);  // prologue: tile 0 into buffer 0
   int cur = 0;
@@ -849,8 +851,7 @@ __host__ __device__ constexpr int wave_lds_bytes() {
 // takes the int4 (kind-0) items, the second the tail (kind-1) items, so every
 // tail wave is dispatched after every int4 wave and runs in the slots the
 // shorter int4 items free, with no second stream or event between the two.
-// With pieces (32-token tiles with the tail path; 64-token tiles have their pieces
-// in decode_coop.hip and decode_split.hip): one workgroup per (piece, head group) walks the
+// With pieces (TAIL only): one workgroup per (piece, head group) walks the
 // piece's items [pieces[k], pieces[k+1]) in order, int4 and tail alike; the
 // host cuts the pieces to about equal cost, so every workgroup of the single
 // pass ends at about the same time.
@@ -873,7 +874,7 @@ kivi_decode_mfma_kernel(const TQ* __restrict__ query, int hq, int kvh, int hpw, 
   constexpr int WAVE_LDS = wave_lds_bytes<CPG, VG1, KSV, TAIL>();
 
   extern __shared__ __align__(16) char lds_raw[];
-  const int32_t* pieces = TAIL && CPG != 8 ? pieces_arg : nullptr;
+  const int32_t* pieces = TAIL ? pieces_arg : nullptr;
   const int lane0 = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int hw = wave % hpw;    // head within the workgroup's group
@@ -929,7 +930,7 @@ kivi_decode_mfma_kernel(const TQ* __restrict__ query, int hq, int kvh, int hpw, 
     tr_item<TQ, VG1 ? 1 : 2, KSV, FOLD>(query, hq, kvh, h, rep, qscale, kq, ks, km, vq, vs, vm,
                                         bs, g, nb, block_table, maxb, b, pb, pe, kind, wi,
                                         my_lds, xfer, half, npair, lane, n, kg, gpb, ng, wpd,
-                                        ws_o, ws_ml);
+                                        pieces != nullptr, ws_o, ws_ml);
   } else {
 
   const QRegs<TQ> qv = load_q<TQ, FOLD>(query, b, hq, h, rep, n, kg);
@@ -1142,18 +1143,15 @@ int launch_kivi_decode_mfma(const void* query, int q_dtype, int hq, int kvh, int
   const uint32_t* kqu = reinterpret_cast<const uint32_t*>(kq);
   const uint32_t* vqu = reinterpret_cast<const uint32_t*>(vq);
   const bool tail = tail_path_applies(q_dtype, hq, kvh, d, ring_dtype, bs);
-  // pieces need the tail path (a piece mixes int4 and tail items); the kernels of
-  // 64-token pieces are the two above and below, and a plan that neither takes (a
-  // page past their 32-bit offsets) runs item by item
-  const bool with_pieces = tail && pieces && num_pieces > 0;
-  const bool use_pieces = with_pieces && cpg == 4;
+  // pieces need the tail path (a piece mixes int4 and tail items)
+  const bool use_pieces = tail && pieces && num_pieces > 0;
   // GQA groups of at most 8 heads fold the hi/lo score parts into one MFMA
   const bool fold = hq / kvh <= 8;
   // one value group per head row: value scales gathered once per PV k-step
   const bool vg1 = cpg == 8 && g >= 128;
   // a key group per page: its scales are contiguous per head
   const bool ksv = vg1 && bs == g;
-  if (with_pieces && !use_pieces) {
+  if (use_pieces) {
     // whole pages for all kv heads per workgroup where the geometry allows
     bool coop = false;
     const int crc = launch_kivi_decode_coop(query, q_dtype, hq, kvh, d, qscale, kq, ks, km, vq,
