@@ -179,8 +179,9 @@ int kvq_kivi_gather_dequant(const int32_t* k_quant, const float* k_scale, const 
  *               end together.  D 128 or 256 with group_size 64 or 128, blocks
  *               of a power of two from 64 and 16-bit query and ring: four such
  *               waves form a workgroup and leave one partial per request
- *               between them (D 256 runs plans without pieces so too, an item
- *               per wave); the items merged away carry m = -inf.  Where no
+ *               between them (D 128 given 10 pieces a request, 24 where the kv
+ *               heads are no power of two; D 256 runs plans without pieces so
+ *               too, an item per wave); the items merged away carry m = -inf.  Where no
  *               MFMA kernel runs both kinds the pieces are ignored.
  *   workspace   >= kvq_kivi_decode_workspace_bytes(num_work, num_heads, D)
  *   block_table int32 [batch, max_blocks]

@@ -735,6 +735,26 @@ def test_split_decode_matches_oracle(gpu_device, d, kvh, g, bs, rep, dtype, cu_c
                        lambda s: plan_decode_pieces(s, kvh, cu_count))
 
 
+@pytest.mark.parametrize("kvh,cu_count,merges", [(2, 19, False), (2, 20, True), (3, 74, False),
+                                                 (3, 76, True)])
+@pytest.mark.parametrize("g", [64, 128])
+def test_decode_on_both_sides_of_the_merge_rule(gpu_device, kvh, cu_count, merges, g):
+    """Head size 128, 8 requests: a few pieces fewer than the split decode takes (the
+    per-wave kernel's pieces), and a few more."""
+    from vllm_ascend_quantized_kv_cache.ops.kivi_decode import plan_decode_pieces
+
+    counts = []
+
+    def plan(seqs):
+        p = plan_decode_pieces(seqs, kvh, cu_count)
+        counts.append(len(p[2]) - 1)
+        return p
+
+    lens = [6003, 1, 4000, 0, 3500, 77, 5571, 6000]
+    _split_decode_case(gpu_device, 128, kvh, g, 128, 5, torch.bfloat16, plan, lens=lens)
+    assert (counts[0] >= (80 if kvh == 2 else 192)) == merges, counts
+
+
 @pytest.mark.parametrize("d,kvh,rep", [(128, 2, 5), (256, 1, 8), (256, 1, 16)])
 def test_split_decode_query_off_its_alignment(gpu_device, d, kvh, rep):
     """Queries 8 bytes off a 16-byte bound (the staging through LDS needs one)."""

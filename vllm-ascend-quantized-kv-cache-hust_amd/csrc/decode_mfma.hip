@@ -1102,7 +1102,7 @@ int64_t wave_lds_of(int cpg, bool vg1, bool ksv) {
   return vg1 ? wave_lds_bytes<8, true, false, TAIL>() : wave_lds_bytes<8, false, false, TAIL>();
 }
 
-int launch_kivi_decode_mfma(const void* query, int q_dtype, int hq, int kvh, int d, float qscale,
+int launch_kivi_decode_mfma(const void* query, int q_dtype, int64_t batch, int hq, int kvh, int d, float qscale,
                             const int32_t* kq, const float* ks, const float* km,
                             const int32_t* vq, const float* vs, const float* vm, int bs, int g,
                             int64_t nb, const int32_t* block_table, int64_t maxb,
@@ -1120,9 +1120,18 @@ int launch_kivi_decode_mfma(const void* query, int q_dtype, int hq, int kvh, int
     // the split decode: pieces that the page-streaming kernel (value scales by
     // 16-byte lanes too) does not take, and head size 256 with or without them
     const bool with_pieces = pieces && num_pieces > 0;
+    // At head size 128 the split decode pays by merging a request's partials, so
+    // with enough pieces a request: 12 requests of 0.5K-6K positions on 2 kv heads
+    // (85 pieces each) 19.1 us against 36.1 on the per-wave kernel below, 20 on 8
+    // kv heads in 64-position pages (13) 35.6 and 38.2; with few it waits at the
+    // merge for nothing: 100 of 0.1K-1.5K on those 8 heads (2.6) 49.2 and 46.3.
+    // Other head counts than powers of two spread a workgroup's pieces unevenly
+    // over the XCDs: 3 heads level at 21 pieces, 5 lose 12% at 8.5.
+    const int64_t least = (kvh & (kvh - 1)) == 0 ? 10 : 24;
+    const bool merges = num_pieces >= least * batch;
     const bool coop = qscale > 0.0f && qscale != INFINITY && aligned16(vs, vm) &&
                       coop_decode_applies(q_dtype, hq, kvh, d, ring_dtype, bs, g);
-    if (d == 256 || (with_pieces && !coop)) {
+    if (d == 256 || (with_pieces && !coop && merges)) {
       const int src = launch_kivi_decode_split(
           query, q_dtype, hq, kvh, d, qscale, kq, ks, km, vq, vs, vm, bs, g, nb, block_table,
           maxb, seq_meta, work, num_work, with_pieces ? pieces : nullptr, num_pieces, ring_k,

@@ -499,7 +499,7 @@ extern "C" int kvq_kivi_decode_attn(const void* query, int q_dtype, int64_t batc
   // int4 items (kind 0), and the tail items (kind 1) in a second pass of the
   // same grid where the tail path applies
   bool mfma = false, tail = false, split = false;
-  int rc = kvq::launch_kivi_decode_mfma(query, q_dtype, num_heads, num_kv_heads, head_size,
+  int rc = kvq::launch_kivi_decode_mfma(query, q_dtype, batch, num_heads, num_kv_heads, head_size,
                                        qscale, k_quant, k_scale, k_mn, v_quant, v_scale, v_mn,
                                        block_size, group_size, num_blocks, block_table,
                                        max_blocks, seq_meta, work, num_work, pieces,

@@ -52,7 +52,7 @@ inline bool tail_path_applies(int q_dtype, int hq, int kvh, int d, int ring_dtyp
 // pass of the same grid, or, given pieces, in one pass of one wave per (piece,
 // kv head).  *launched / *tail_done tell the caller which kinds still need
 // another kernel, *split that the split decode ran (items merged).
-int launch_kivi_decode_mfma(const void* query, int q_dtype, int hq, int kvh, int d, float qscale,
+int launch_kivi_decode_mfma(const void* query, int q_dtype, int64_t batch, int hq, int kvh, int d, float qscale,
                             const int32_t* kq, const float* ks, const float* km,
                             const int32_t* vq, const float* vs, const float* vm, int bs, int g,
                             int64_t nb, const int32_t* block_table, int64_t maxb,
