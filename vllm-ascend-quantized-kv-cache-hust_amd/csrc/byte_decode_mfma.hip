@@ -237,6 +237,8 @@ __device__ __forceinline__ void read_tile_lds(TileRegs<D, FP8>& t, const char* b
 
 // INT8 at 256 dims: p's (and o's) lift on the way through fp16, so that the two
 // parts of a p down to 2^-28 keep their bits and one is lost only below 2^-39.
+// (Against 64 bits, fp32 activations, 300 - 16K positions: 1.4e-7 - 2.1e-7, where the
+// fp32 kernel these calls had before was 2.7e-7 - 3.3e-7 off.)
 template <int D>
 constexpr float kLift = D == 256 ? 16384.0f : 1.0f;
 

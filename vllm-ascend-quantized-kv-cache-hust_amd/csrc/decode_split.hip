@@ -14,7 +14,7 @@
 //
 // Head size 256 had no MFMA path (the generic fp32 kernel: 4650 us for 64
 // requests of 1K-16K positions on 1 kv head, against 32 us for its 166 MB at
-// the copy rate; 64 here, its combine included).
+// the copy rate; 69 here, its combine included).
 //
 // Tiles: 64 positions, decode_tr.h's layout and compute, double-buffered in the
 // wave's own LDS: the DMA of the next tile is in flight while one computes.  The
@@ -24,8 +24,9 @@
 //   D = 128: 2 workgroups a CU (8 x 19-20 KB of LDS), one piece a wave;
 //   D = 256: 1 workgroup a CU (4 x 38-40 KB), two pieces a wave where the plan
 //            has more of them than the chip holds waves.
-// What bounds it: at D = 256 the issue of one wave per SIMD (some 5 us a tile, of
-// them 0.95 waiting for its DMA, at 1500 vector and 300 scalar instructions), at
+// What bounds it: at D = 256 the issue of one wave per SIMD (a tile's 1600 vector,
+// 128 matrix and 270 scalar instructions take some 6 us, of them 0.95 waiting for
+// its DMA; the wave issues vector instructions in 45% of its cycles), at
 // D = 128 the start: every wave's first tile, 20 MB over the chip, takes 5 - 6 of
 // 22 us on 40 requests of 1K-10K positions and 2 kv heads.  Hence the query rows
 // through LDS (the second tile leaves before the first is there), the key
