@@ -177,6 +177,31 @@ def test_prefill_attention_of_nans_in_segments(gpu_device, d, where):
         assert got[:, :, 3].all() and int(got.sum()) == 4 * hq
 
 
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_prefill_attention_query_and_output_at_odd_addresses(gpu_device, d):
+    """Queries and outputs that start 2 bytes past a 16-byte bound (ordinary vector
+    accesses take any address) give what aligned ones give, whole and in segments."""
+    from vllm_ascend_quantized_kv_cache.ops.attention import prefill_attention
+
+    def odd(shape):
+        n = 1
+        for x in shape:
+            n *= x
+        t = torch.zeros(n + 1, dtype=torch.bfloat16, device=gpu_device)[1:].view(shape)
+        assert t.data_ptr() % 16 == 2
+        return t
+
+    g = torch.Generator().manual_seed(d)
+    for q_lens, kv_lens in (([70, 3], [70, 40]), ([5], [3000])):
+        q = torch.randn(sum(q_lens), 4, d, generator=g).to(torch.bfloat16).to(gpu_device)
+        k, v = (torch.randn(sum(kv_lens), 2, d, generator=g).to(torch.bfloat16).to(gpu_device)
+                for _ in range(2))
+        want = prefill_attention(q, k, v, q_lens, kv_lens, d ** -0.5, True)
+        got = prefill_attention(odd(q.shape).copy_(q), k, v, q_lens, kv_lens, d ** -0.5, True,
+                                out=odd(q.shape))
+        assert torch.equal(got, want)
+
+
 def test_prefill_attention_batch_past_the_launch_argument(gpu_device):
     """More requests, and more tiles, than the plan argument carries."""
     from vllm_ascend_quantized_kv_cache.ops.attention import prefill_attention
